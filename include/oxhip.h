@@ -110,7 +110,7 @@ void oxhip_free_weight(oxhip_ctx* ctx, oxhip_weight* w);
 /* Bytes the weight occupies in HBM. */
 size_t oxhip_weight_bytes(const oxhip_weight* w);
 /* Backend::matmul (src/gpu.rs:160; src/cuda.rs:1428-1493): all jobs share x [t, n_in] (host f32);
- * computes every job or none. Routing as matmul_quant_multi_at's (src/kernels.rs:1731-1879): up to 8 tokens the
+ * computes every job or none. Routing as matmul_quant_multi_at's (src/kernels.rs:1731-1879): up to 16 tokens the
  * Q8 / Q8_0 / Q4_K / Q5_K / Q6_K / MXFP4 / MLX 4-bit jobs share one launch of the int8 decode kernel (the CPU's decode semantics,
  * src/kernels.rs:1908-1928); more than 16 tokens over MLX 4-bit, Q8, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4, NVFP4 or FP8 (128-column
  * blocks) weights run the bf16 matrix-core GEMM; everything else runs the decode kernels over 16 tokens at a time. */
@@ -181,8 +181,8 @@ int oxhip_dev_decode(oxhip_ctx* ctx, const oxhip_weight* w, const oxhip_qact* xa
 int oxhip_dev_decode_noalloc(oxhip_ctx* ctx, const oxhip_weight* w, const oxhip_qact* xa, size_t t, float* y, void* stream);
 /* Several independent decode matmuls in one call (a decode step issues many small matmuls; what
  * matmul_quant_batch does for the CPU, src/kernels.rs:1937-1994). The jobs must not depend on one another: runs of
- * consecutive jobs of at most 8 tokens over Q8 / Q8_0 / Q4_K / Q5_K / Q6_K / Q4_0 / MXFP4 / MLX 4-bit weights share launches: one per
- * kernel among them (Q8_0, Q4_K and Q6_K share one, Q5_K takes Q4_K and Q6_K jobs into its own, each other format has its own), up to 16 jobs each; their latency chains
+ * consecutive jobs over Q8 / Q8_0 / Q4_K / Q5_K / Q6_K / Q4_0 / MXFP4 / MLX 4-bit weights share launches: one per
+ * kernel among them (Q8_0, Q4_K and Q6_K share one, Q5_K takes Q4_K and Q6_K jobs into its own, each other format has its own; jobs of more than 8 tokens apart from the others), up to 16 jobs each; their latency chains
  * overlap, and every job's rows are bit-identical to a launch of its own. The others launch one by one, in order, on
  * `stream` (inside a shared launch the library orders the jobs itself). ev_start / ev_stop (from oxhip_event_create, or
  * NULL) are recorded before / after the launch that holds the job; for jobs that share a launch the first start and the

@@ -720,7 +720,7 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
         }
     }
     float* yd = static_cast<float*>(c->y.p);
-    // Routing, as matmul_quant_multi_at does (src/kernels.rs:1731-1879): up to 8 tokens the jobs that the matrix-core
+    // Routing, as matmul_quant_multi_at does (src/kernels.rs:1731-1879): up to 16 tokens the jobs that the matrix-core
     // decode kernel takes share one launch; more than 16 tokens go to the prefill GEMM where the format has one (MLX
     // 4-bit, FP8 with 128-column blocks: bf16 matrix cores, f32 accumulation); everything else runs the decode
     // kernels over 16 tokens at a time.
@@ -738,7 +738,7 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
     };
     for (size_t j = 0; j < n_jobs; j++) {
         const oxhip_weight* w = jobs[j].w;
-        if (t <= 8 && !is_dense(w) && decode_batchable(w->v, t)) {
+        if (t <= 16 && !is_dense(w) && decode_batchable(w->v, t)) {
             fused.push_back(DecodeBatchItem{w->v, view_of(xa), yd + offs[j], (uint32_t)t, Epi{}});
             continue;
         }

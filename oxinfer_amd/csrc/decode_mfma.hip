@@ -1,4 +1,4 @@
-// Decode (1..8 tokens) on the matrix cores: a dequant-fused skinny GEMM over int8 activations.
+// Decode (1..16 tokens) on the matrix cores: a dequant-fused skinny GEMM over int8 activations.
 //
 // The arithmetic is the CPU decode kernels' (QMat::rows_t1 / rows_tc, src/kernels.rs:1339-1369;
 // dot_row_generic, src/ggml.rs:1288-1315 of the reference): exact int32 sums of int8 weight codes
@@ -70,7 +70,7 @@ constexpr int pf_for() { return FMT == FMT_Q6_K ? 4 : 8; }  // Q6_K records are 
 // activations' own sums; the DUMP variant writes I16 / 16. The m * fs terms of a step's four blocks are one more
 // matrix instruction (f32, 16 x 16 x 4: rows = tokens, K = the four blocks), straight into the accumulators.
 // LDS metadata: xs [nbl][TPAD], and for the formats with mins or offsets fs [nbl][TPAD], over the workgroup's nbl
-// blocks from b0. Q6_K keeps its own three arrays (see its step).
+// blocks from b0.
 // `at`: index of the lane's first token in its block's row
 __device__ __forceinline__ void load_xs(const float* lds, uint32_t at, float* xs) {
     const float4 x = *reinterpret_cast<const float4*>(lds + at);
@@ -153,13 +153,23 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                                             uint32_t* __restrict__ counters, uint32_t bx, uint32_t by, uint32_t nthr,
                                             float* __restrict__ lds_all, Epi epi = Epi{}, Mapping map = Mapping{}) {
     static_assert(NG == 1 || (GROUPED && ALDS && !DUMP && NT == 8), "token groups are for grouped launches");
-    static_assert(!REMAP || (!GROUPED && !DUMP && ALDS && NG == 1), "other mappings are for dense launches over staged activations");
-    constexpr int TPAD = NT <= 4 ? 4 : 8;
+    static_assert(!REMAP || (!GROUPED && !DUMP && ALDS && NG == 1 && NT <= 8), "other mappings are for dense launches over staged activations");
+    // Nine to sixteen tokens (NT = 16): the instruction is v_mfma_i32_16x16x32_i8, one block x 16 tokens x 16 rows, so that the
+    // token rows are all in use without masking (a lane's bytes 0-7 and 8-15 of a record are the operands of two consecutive
+    // instructions, and the lane receives tokens 4 kq + i of both blocks). Every block parity keeps a sum of its own, as the two
+    // lane groups of the 8-token form do, so a token's sums are associated, and its bits are, as in a launch of fewer tokens.
+    // The weights are unpacked once for all tokens and the operands need no masks: a step costs about what it costs at 8 tokens,
+    // where two launches of eight streamed and unpacked everything twice (MLX 4-bit, 16 tokens: gate / up pair of 14336 x 4096
+    // 35.1 -> 21.3 us, 4096 x 14336 24.1 -> 16.0, 4096 x 4096 13.2 -> 10.4). Bound by the staging: 16 to 20 B per column and
+    // workgroup next to rt * 9 B (4-bit) of weights.
+    constexpr bool WIDE = NT == 16;
+    static_assert(!WIDE || (ALDS && !DUMP && !GROUPED && NG == 1), "the 16-token form is for dense launches over staged activations");
+    constexpr int TPAD = NT <= 4 ? 4 : NT <= 8 ? 8 : 16;
     // the swizzled operand array pays at 8 tokens (where the staging stores are many); at fewer its address math costs more
     constexpr bool SWZ = NT >= 8;
     constexpr int NI = NT < 4 ? NT : 4;          // accumulator registers that hold live tokens
     constexpr bool MINS = k45_format(FMT) || FMT == FMT_Q4M;   // m * fs terms (Q4_0 has none)
-    constexpr int NARR = q8_format(FMT) || FMT == FMT_Q40 || FMT == FMT_MXFP4 ? 1 : FMT == FMT_Q6_K ? (DUMP ? 4 : 3) : 2;  // metadata arrays
+    constexpr int NARR = MINS ? 2 : 1;                         // metadata arrays: xs, and fs for the formats with m * fs terms
     // the wave index and everything derived from it (tile, K range) live in scalar registers: branches on them are
     // scalar, and the load counters the compiler keeps stay exact across them
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -195,8 +205,8 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     const uint32_t B0 = BPS * S0, nbl = BPS * fs * sl, M0 = B0 / 2;
     // LDS: [operand-order activations: 512 B per pair of blocks] [scales, sums] [partial sums]; with ALDS the
     // partial sums reuse the activations' space once every wave is done with them
-    uint2* afr = reinterpret_cast<uint2*>(lds_all);  // [NG][nbl / 2][64]
-    float* lds = lds_all + (ALDS ? (size_t)NG * (nbl / 2) * 128 : 0);
+    uint2* afr = reinterpret_cast<uint2*>(lds_all);  // [NG][nbl / 2][64]; 16 tokens: [nbl][64]
+    float* lds = lds_all + (ALDS ? (size_t)NG * (nbl / 2) * (WIDE ? 256 : 128) : 0);
     const uint32_t nm = nbl * TPAD, as = NG * nm;  // scale entries of a token group; floats per array
     float* red = ALDS ? lds_all : lds + (size_t)NARR * as;  // [rt][runs][NG][TPAD][16]
     uint32_t row0 = 0;  // first activation / output row of this launch unit
@@ -225,7 +235,8 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     const int8_t* xrow = xa.q + src_row(a_tok) * w.n_in;
     const uint32_t amask0 = a_half ? 0u : 0xFFFFFFFFu, amask1 = ~amask0;
     // D role: this lane's registers are tokens 4 (kq & 1) + i of block parity kq >> 1
-    const uint32_t d_half = kq >> 1, d_tok0 = 4 * (kq & 1);
+    // (16 tokens: tokens 4 kq + i of either block)
+    const uint32_t d_half = kq >> 1, d_tok0 = WIDE ? 4 * kq : 4 * (kq & 1);
     // Q4_K: the bytes this lane takes from a step's {scales, mins} words (v_perm_b32: 0..3 = the scales, 4..7 = the mins)
     const uint32_t q4k_sel = d_half | ((2 + d_half) << 8) | (kq << 16) | ((4 + kq) << 24);
 
@@ -329,8 +340,10 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     v4f macc[MINS ? NG : 1];
 #pragma unroll
     for (int g = 0; g < (MINS ? NG : 1); g++) macc[g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    float acch[WIDE ? 4 : 1] = {};  // 16 tokens: the blocks of odd parity
     // Q6_K: every lane group sums its own 16-column sub-block for tokens 4 tg + i
-    float acc6a[4] = {0.0f, 0.0f, 0.0f, 0.0f}, acc6b[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // tg = 0, 1
+    constexpr int NTG = NT <= 4 ? 1 : NT <= 8 ? 2 : 4;
+    float acc6[4][4] = {};
     // `m`: index of the instruction along K (pair of blocks 2 m, 2 m + 1); with ALDS its operand comes from LDS
     auto mfma = [&](v4i bw, uint32_t m, int tg, uint32_t d0, uint32_t d1) -> v4i {
         v4i c = {0, 0, 0, 0};
@@ -342,6 +355,20 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
         v4i a = {(int)(d0 & amask0), (int)(d1 & amask0), (int)(d0 & amask1), (int)(d1 & amask1)};
         return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bw, c, 0, 0, 0);
     };
+    // 16 tokens: block `b`'s sums of 16 tokens x 16 rows, `w0`, `w1` the lane's 8 codes of it
+    auto mfma16 = [&](int w0, int w1, uint32_t b) -> v4i {
+        const uint2 av = afr[(size_t)(b - B0) * 64 + opslot(b - B0, lane)];
+        const v4i c = {0, 0, 0, 0};
+        return __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, av), __builtin_bit_cast(long, make_uint2((uint32_t)w0, (uint32_t)w1)), c, 0, 0, 0);
+    };
+    auto wide_block = [&](int w0, int w1, uint32_t b, float d, float* sum) {
+        const v4i D = mfma16(w0, w1, b);
+        float xs[4];
+        load_xs(lds, (min(b, nblk - 1) - B0) * TPAD + d_tok0, xs);
+        const int I[4] = {D.x, D.y, D.z, D.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) sum[i] = fmaf(d, xs[i] * (float)I[i], sum[i]);
+    };
     // The m * fs terms of the step's four blocks (blocks b4 .. b4 + 3): rows = tokens (8 .. 15: none), K = the blocks;
     // this lane supplies fs of (token n, block b4 + kq) and `mk`, row n's m of block b4 + kq. D[4 kq + i][n]: the lane
     // groups 0 and 1 receive the tokens their accumulators hold, the others zeros.
@@ -352,7 +379,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
 #pragma unroll
             for (int tg = 0; tg < NG; tg++) {
                 const float f = lds[(size_t)as + tg * nm + at];
-                macc[tg] = __builtin_amdgcn_mfma_f32_16x16x4f32(n < (uint32_t)TPAD ? f : 0.0f, mk, macc[tg], 0, 0, 0);
+                macc[tg] = __builtin_amdgcn_mfma_f32_16x16x4f32(WIDE || n < (uint32_t)TPAD ? f : 0.0f, mk, macc[tg], 0, 0, 0);
             }
         }
     };
@@ -371,7 +398,12 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     };
     auto compute_step = [&](const Step<FMT>& st, const uint32_t* sw, uint32_t s) {
         const uint4 c = st.w;
-        if constexpr (q8_format(FMT)) {
+        if constexpr (WIDE && q8_format(FMT)) {
+            const float d0 = FMT == FMT_Q8F ? __uint_as_float(sw[0]) : f16_bits_to_f32((uint16_t)(sw[0] & 0xFFFF));
+            const float d1 = FMT == FMT_Q8F ? __uint_as_float(sw[NM - 1]) : f16_bits_to_f32((uint16_t)(sw[0] >> 16));
+            wide_block((int)c.x, (int)c.y, 2 * s, d0, acc[0]);
+            wide_block((int)c.z, (int)c.w, 2 * s + 1, d1, acch);
+        } else if constexpr (q8_format(FMT)) {
             const float d = FMT == FMT_Q8F ? __uint_as_float(d_half ? sw[NM - 1] : sw[0]) : f16_bits_to_f32((uint16_t)(d_half ? sw[0] >> 16 : sw[0] & 0xFFFF));
             v4i bw = {(int)c.x, (int)c.y, (int)c.z, (int)c.w};
             const uint32_t b = 2 * s + d_half;
@@ -410,6 +442,11 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                     const uint32_t x0 = pr ? c.z : c.x, x1 = pr ? c.w : c.y;
                     bw = v4i{centre_lo(x0), centre_lo(x1), centre_hi(x0), centre_hi(x1)};
                 }
+                if constexpr (WIDE) {  // (the sub-blocks' scales are bytes 2 pr and 2 pr + 1 of sw[0])
+                    wide_block(bw.x, bw.y, 4 * s + 2 * pr, d16 * (float)((sw[0] >> (16 * pr)) & 0xFF), acc[0]);
+                    wide_block(bw.z, bw.w, 4 * s + 2 * pr + 1, d16 * (float)((sw[0] >> (16 * pr + 8)) & 0xFF), acch);
+                    continue;
+                }
                 const uint32_t b = 4 * s + 2 * pr + d_half;  // global index of this lane's block of 32
 #pragma unroll
                 for (int tg = 0; tg < NG; tg++) {
@@ -431,43 +468,40 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
             // Scales go per 16 columns, so an instruction's 16 operand slots are (sub-block sb, token t4): lane group kq
             // supplies sub-block kq's 16 activations of token t4 in the slots with sb = kq and zeros elsewhere, and lane
             // (kq, n) receives sub-block kq's exact sums for tokens 4 tg + i of row n. Eight tokens take two instructions.
-            const float d = f16_bits_to_f32((uint16_t)(sw[2] & 0xFFFF));
-            const uint32_t hq[2] = {st.h.x, st.h.y};
+            // The codes centre on 32 and go in as the int8 values 4 (code - 32): nibble in bits 2..5, the high pair on top with
+            // its top bit flipped (one flip for the lane's four operand dwords), so that the sums need no correction by the
+            // activations' own: two LDS arrays less (at 16 tokens a workgroup over 4096 columns stages 72 KB instead of 90, and
+            // two fit a CU: q / k / v of 6144 x 4096 27.6 -> 15.4 us), and one read per instruction less.
+            const float d = f16_bits_to_f32((uint16_t)(sw[2] & 0xFFFF)) * 0.25f;
+            const uint32_t hq[2] = {st.h.x ^ 0xAAAAAAAAu, st.h.y ^ 0xAAAAAAAAu};
             const bool on = (n >> 2) == kq;
             const uint4* afr6 = reinterpret_cast<const uint4*>(afr);  // [64-column group][8 tokens][kq]
 #pragma unroll
             for (int h = 0; h < 2; h++) {  // the step's two groups of 64 columns
                 const uint32_t lo = h ? c.z : c.x, hi = h ? c.w : c.y, hh = hq[h];
-                const v4i bw = {(int)((lo & 0x0F0F0F0Fu) | ((hh & 0x03030303u) << 4)), (int)(((lo >> 4) & 0x0F0F0F0Fu) | (((hh >> 2) & 0x03030303u) << 4)),
-                                (int)((hi & 0x0F0F0F0Fu) | (((hh >> 4) & 0x03030303u) << 4)), (int)(((hi >> 4) & 0x0F0F0F0Fu) | (((hh >> 6) & 0x03030303u) << 4))};
+                constexpr uint32_t NIB = 0x3C3C3C3Cu, TOP = 0xC0C0C0C0u;
+                const v4i bw = {(int)(((lo << 2) & NIB) | ((hh << 6) & TOP)), (int)(((lo >> 2) & NIB) | ((hh << 4) & TOP)),
+                                (int)(((hi << 2) & NIB) | ((hh << 2) & TOP)), (int)(((hi >> 2) & NIB) | (hh & TOP))};
                 const float dsc = d * (float)(int)(int8_t)((sw[h] >> (8 * kq)) & 0xFF);
                 const uint32_t m64 = 2 * s + h, b = 2 * m64 + (kq >> 1);  // the lane's 32-block (its scale's) and its half
                 const uint32_t at = (min(b, nblk - 1) - B0) * TPAD;
 #pragma unroll
-                for (int tg = 0; tg < (NT > 4 ? 2 : 1); tg++) {
-                    const uint4 av = afr6[((size_t)(m64 - M0) * 8 + 4 * tg + (n & 3)) * 4 + kq];
+                for (int tg = 0; tg < NTG; tg++) {
+                    const uint4 av = afr6[((size_t)(m64 - M0) * (WIDE ? 16 : 8) + 4 * tg + (n & 3)) * 4 + kq];
                     const v4i a = {on ? (int)av.x : 0, on ? (int)av.y : 0, on ? (int)av.z : 0, on ? (int)av.w : 0};
                     const v4i z = {0, 0, 0, 0};
                     const v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bw, z, 0, 0, 0);
                     const float4 xs = *reinterpret_cast<const float4*>(lds + at + 4 * tg);
-                    const float4 cc = *reinterpret_cast<const float4*>(lds + (size_t)(1 + (kq & 1)) * as + at + 4 * tg);
-                    const float xv[4] = {xs.x, xs.y, xs.z, xs.w}, cv[4] = {cc.x, cc.y, cc.z, cc.w};
+                    const float xv[4] = {xs.x, xs.y, xs.z, xs.w};
                     const int U[4] = {D.x, D.y, D.z, D.w};
 #pragma unroll
-                    for (int i = 0; i < NI; i++) {
-                        const float v = fmaf(xv[i], (float)U[i], cv[i]);
-                        if (tg == 0) acc6a[i] = fmaf(dsc, v, acc6a[i]);
-                        else acc6b[i] = fmaf(dsc, v, acc6b[i]);
-                    }
+                    for (int i = 0; i < NI; i++) acc6[tg][i] = fmaf(dsc, xv[i] * (float)U[i], acc6[tg][i]);
                     if (DUMP) {
-                        const int4 sp = *reinterpret_cast<const int4*>(lds + (size_t)3 * as + at + 4 * tg);
-                        const int su[4] = {sp.x, sp.y, sp.z, sp.w};
                         const uint32_t row = tile * 16 + n;
 #pragma unroll
                         for (int i = 0; i < 4; i++) {
-                            const int s16 = (kq & 1) ? (su[i] >> 16) : (int)(int16_t)(su[i] & 0xFFFF);
                             if (4 * tg + i < (int)t && row < w.n_out && b < nblk)
-                                dump[((size_t)(4 * tg + i) * w.n_out + row) * (w.n_in / 16) + 4 * m64 + kq] = U[i] - 32 * s16;
+                                dump[((size_t)(4 * tg + i) * w.n_out + row) * (w.n_in / 16) + 4 * m64 + kq] = U[i] >> 2;
                         }
                     }
                 }
@@ -481,6 +515,22 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                 v4i bw = MX ? v4i{(int)mxfp4_values<0>(x0 & NIB), (int)mxfp4_values<0>((x0 >> 4) & NIB), (int)mxfp4_values<0>(x1 & NIB),
                                   (int)mxfp4_values<0>((x1 >> 4) & NIB)}
                             : v4i{centre_lo(x0), centre_hi(x0), centre_lo(x1), centre_hi(x1)};
+                if constexpr (WIDE) {
+                    const uint32_t b = 4 * s + 2 * g;
+                    float d0, d1;
+                    if constexpr (MX) {
+                        d0 = e8m0_half((sw[0] >> (16 * g)) & 0xFF);
+                        d1 = e8m0_half((sw[0] >> (16 * g + 8)) & 0xFF);
+                    } else if constexpr (FMT == FMT_Q40) {
+                        d0 = f16_bits_to_f32((uint16_t)(sw[g] & 0xFFFF)) * 0.0625f;
+                        d1 = f16_bits_to_f32((uint16_t)(sw[g] >> 16)) * 0.0625f;
+                    } else {
+                        d0 = d1 = f16_bits_to_f32((uint16_t)(g ? sw[0] >> 16 : sw[0] & 0xFFFF)) * 0.0625f;
+                    }
+                    wide_block(bw.x, bw.y, b, b < nblk ? d0 : 0.0f, acc[0]);
+                    wide_block(bw.z, bw.w, b + 1, b + 1 < nblk ? d1 : 0.0f, acch);
+                    continue;
+                }
                 const uint32_t b = 4 * s + 2 * g + d_half;
                 // MLX: the group's scale; Q4_0: the lane's block's own scale (word g, half d_half); MXFP4: its scale byte
                 float d;
@@ -551,18 +601,18 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     auto act_store = [&](uint32_t tok, uint32_t c, const uint4* v) {
         if (t4m_format(FMT)) {
             const uint32_t b = c;
-            uint2* dst = afr + ((size_t)(tok >> 3) * (nbl / 2) + (b >> 1)) * 64;
-            const uint32_t s0 = SWZ ? opslot(b >> 1, 8 * (b & 1) + (tok & 7)) : 8 * (b & 1) + (tok & 7);
+            uint2* dst = WIDE ? afr + (size_t)b * 64 : afr + ((size_t)(tok >> 3) * (nbl / 2) + (b >> 1)) * 64;
+            const uint32_t s0 = WIDE ? opslot(b, tok) : SWZ ? opslot(b >> 1, 8 * (b & 1) + (tok & 7)) : 8 * (b & 1) + (tok & 7);
             dst[s0] = make_uint2(v[0].x, v[1].x);
             dst[s0 ^ 16] = make_uint2(v[0].y, v[1].y);
             dst[s0 ^ 32] = make_uint2(v[0].z, v[1].z);
             dst[s0 ^ 48] = make_uint2(v[0].w, v[1].w);
         } else if (FMT == FMT_Q6_K) {  // chunk c = columns 16 c ..: sub-block c % 4 of 64-column group c / 4
-            reinterpret_cast<uint4*>(afr)[((size_t)(c >> 2) * 8 + (tok & 7)) * 4 + (c & 3)] = make_uint4(v[0].x, v[0].y, v[0].z, v[0].w);
+            reinterpret_cast<uint4*>(afr)[((size_t)(c >> 2) * (WIDE ? 16 : 8) + (WIDE ? tok : tok & 7)) * 4 + (c & 3)] = make_uint4(v[0].x, v[0].y, v[0].z, v[0].w);
         } else {
             const uint32_t b = c >> 1;
-            uint2* dst = afr + ((size_t)(tok >> 3) * (nbl / 2) + (b >> 1)) * 64;
-            const uint32_t s0 = SWZ ? opslot(b >> 1, 32 * (c & 1) + 8 * (b & 1) + (tok & 7)) : 32 * (c & 1) + 8 * (b & 1) + (tok & 7);
+            uint2* dst = WIDE ? afr + (size_t)b * 64 : afr + ((size_t)(tok >> 3) * (nbl / 2) + (b >> 1)) * 64;
+            const uint32_t s0 = WIDE ? opslot(b, 32 * (c & 1) + tok) : SWZ ? opslot(b >> 1, 32 * (c & 1) + 8 * (b & 1) + (tok & 7)) : 32 * (c & 1) + 8 * (b & 1) + (tok & 7);
             dst[s0] = make_uint2(v[0].x, v[0].y);
             dst[s0 ^ 16] = make_uint2(v[0].z, v[0].w);
         }
@@ -570,7 +620,6 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     // scales and sums: unit i = (q = i / nbl, block i % nbl of the slice) with q = TPAD group + token of the group
     struct MetaReg {
         float x, f;
-        int sq, sq2;  // Q6_K: the sums of the block's two halves
     };
     const uint32_t m_dq = nthr / nbl, m_dr = nthr - m_dq * nbl;
     auto meta_load = [&](uint32_t q, uint32_t b, MetaReg& r) {
@@ -578,25 +627,12 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
         const bool live = tok < t && B0 + b < nblk;
         const size_t src = (live ? src_row(tok) : 0) * nblk + B0 + (live ? b : 0);
         r.x = live ? xa.scales[src] : 0.0f;
-        if (FMT == FMT_Q6_K) {
-            r.sq = live ? xa.sums16[2 * src] : 0;
-            r.sq2 = live ? xa.sums16[2 * src + 1] : 0;
-            r.f = 0.0f;
-        } else {
-            r.sq = r.sq2 = 0;
-            r.f = MINS && live ? xa.fsums[src] : 0.0f;
-        }
+        r.f = MINS && live ? xa.fsums[src] : 0.0f;
     };
     auto meta_store = [&](uint32_t q, uint32_t b, const MetaReg& r) {
         const uint32_t at = (q / TPAD) * nm + b * TPAD + q % TPAD;
         lds[at] = r.x;
-        if (FMT == FMT_Q6_K) {  // the codes are unsigned (0..63): -32 x the half's activation sum, scaled like the dot
-            lds[(size_t)as + at] = -32.0f * (r.x * (float)r.sq);
-            lds[(size_t)2 * as + at] = -32.0f * (r.x * (float)r.sq2);
-            if (DUMP) reinterpret_cast<int*>(lds)[(size_t)3 * as + at] = (r.sq & 0xFFFF) | (r.sq2 << 16);
-        } else if (MINS) {
-            lds[(size_t)as + at] = r.f;
-        }
+        if (MINS) lds[(size_t)as + at] = r.f;
     };
     uint4 sa[SA];
     MetaReg smr[SM];
@@ -646,10 +682,27 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     }
     // what did not fit the registers (long rows, small workgroups) follows behind the weights
     if (ALDS) {
-        for (; aq < t; advance(aq, ar, a_dq, a_dr, adiv)) {
-            uint4 v[AU];
-            act_load(aq, ar, v);
-            act_store(aq, ar, v);
+        if constexpr (WIDE) {
+            while (aq < t) {  // (as many requests per round trip as at first)
+                const uint32_t q1 = aq, r1 = ar;
+#pragma unroll
+                for (int j = 0; j < SA / AU; j++) {
+                    act_load(min(aq, t - 1), ar, sa + AU * j);
+                    advance(aq, ar, a_dq, a_dr, adiv);
+                }
+                aq = q1, ar = r1;
+#pragma unroll
+                for (int j = 0; j < SA / AU; j++) {
+                    if (aq < t) act_store(aq, ar, sa + AU * j);
+                    advance(aq, ar, a_dq, a_dr, adiv);
+                }
+            }
+        } else {
+            for (; aq < t; advance(aq, ar, a_dq, a_dr, adiv)) {
+                uint4 v[AU];
+                act_load(aq, ar, v);
+                act_store(aq, ar, v);
+            }
         }
     }
     for (; mq < NG * TPAD; advance(mq, mr, m_dq, m_dr, nbl)) {
@@ -665,16 +718,20 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     // The end of a run: its sums as a wave of its own leaves them ...
     auto close_run = [&]() {
         if constexpr (FMT == FMT_Q6_K) {
-            // the four sub-blocks of a token meet across the lane groups; group 0 then holds tokens 0..3, group 1 tokens 4..7
+            // the four sub-blocks of a token meet across the lane groups; group 0 then holds tokens 0..3, group 1 tokens 4..7, ...
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float a = acc6a[i], b = acc6b[i];
-                a += __shfl_xor(a, 16);
-                a += __shfl_xor(a, 32);
-                b += __shfl_xor(b, 16);
-                b += __shfl_xor(b, 32);
-                acc[0][i] = (kq & 1) ? b : a;
-            }
+            for (int tg = 0; tg < NTG; tg++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    float a = acc6[tg][i];
+                    a += __shfl_xor(a, 16);
+                    a += __shfl_xor(a, 32);
+                    acc[0][i] = tg == 0 || (kq & (NTG - 1)) == (uint32_t)tg ? a : acc[0][i];
+                }
+        } else if constexpr (WIDE) {
+            // (the mins' sums join the even blocks', then the odd ones': the order of the 8-token form)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[0][i] = (MINS ? acc[0][i] + macc[0][i] : acc[0][i]) + acch[i];
         } else {
             if constexpr (MINS) {
 #pragma unroll
@@ -691,7 +748,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     };
     // ... go to the run's place among its tile's partial sums ...
     auto store_run = [&](uint32_t run) {
-        if (kq < 2) {
+        if (WIDE || kq < 2) {
 #pragma unroll
             for (int g = 0; g < NG; g++)
 #pragma unroll
@@ -715,7 +772,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                 nrun++;
                 left = per;
 #pragma unroll
-                for (int i = 0; i < 4; i++) acc[0][i] = acc6a[i] = acc6b[i] = 0.0f;
+                for (int i = 0; i < 4; i++) acc[0][i] = acc6[0][i] = acc6[1][i] = 0.0f;
                 macc[0] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
             }
         }
@@ -874,7 +931,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
         if (!combine) return;
         // The chunks of a row group meet like K slices do (below): the last workgroup to arrive, of all the launch's chunks,
         // adds every token's routed rows in route order (multiply, then add: src/moe.rs:608-615).
-        __shared__ uint32_t last_chunk;
+        uint32_t& last_chunk = *reinterpret_cast<uint32_t*>(lds_all);  // (the partial sums there have been read)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -912,7 +969,9 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     // for the next launch. Every access to the partial rows and the counter is a device-scope atomic access, and each
     // thread waits for its stores to complete before the workgroup's arrival is counted, so no cache-wide write-back
     // or invalidation is needed (a device-scope fence here costs tens of microseconds per launch).
-    __shared__ uint32_t is_last;
+    // (the flag takes a word of the dynamic LDS, whose partial sums have been read: with a static word of its own a workgroup
+    // that stages 80 KiB would leave no room for a second one on its CU)
+    uint32_t& is_last = *reinterpret_cast<uint32_t*>(lds_all);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -952,7 +1011,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
 // (Grouped launches keep to 8 waves, which leaves them 256 registers for the accumulators of their token groups.)
 // (Q6_K: bounded at 8 waves like its shared-launch kernel, see decode_batch_kernel)
 template <int FMT, int NT, bool DUMP, bool GROUPED, bool ALDS, int NG>
-__global__ __launch_bounds__(GROUPED || FMT == FMT_Q6_K ? 512 : 1024) void decode_mfma_kernel(WeightView w, QActView xa, uint32_t t, uint32_t rt,
+__global__ __launch_bounds__(GROUPED || FMT == FMT_Q6_K || NT == 16 ? 512 : 1024) void decode_mfma_kernel(WeightView w, QActView xa, uint32_t t, uint32_t rt,
                                                                            uint32_t kw, float* __restrict__ y,
                                                                            int32_t* __restrict__ dump, GroupView grp, uint32_t ksplit,
                                                                            float* __restrict__ partial,
@@ -984,14 +1043,17 @@ struct BatchArgs {
     BatchJob j[BATCH_MAX];
 };
 
-template <int FMT, bool FAT>
+template <int FMT, bool FAT, bool WIDE>
 __device__ __forceinline__ void batch_dispatch(const BatchJob& jb, uint32_t bid, float* lds) {
     const uint32_t nthr = 64 * jb.rt * jb.map.kwp;
     if (threadIdx.x >= nthr) return;  // whole waves (nthr is a multiple of 64), before any barrier
     const GroupView none{};
     const uint32_t ksp = jb.ks >> __builtin_ctz(jb.map.fs);  // slices across workgroups
     const uint32_t bx = bid >> __builtin_ctz(ksp), by = bid & (ksp - 1);  // the slices of a row group are neighbours in launch order (a power of two)
-    if (jb.t == 1) decode_body<FMT, 1, false, false, true, 1, FAT>(jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
+    if constexpr (WIDE) {
+        decode_body<FMT, 16, false, false, true>(jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
+        return;
+    } else if (jb.t == 1) decode_body<FMT, 1, false, false, true, 1, FAT>(jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
     else if (jb.t == 2 && !t4m_format(FMT)) decode_body<FMT, 2, false, false, true, 1, FAT>(  // (MLX at 2 tokens: the 4-token body, which fits the registers)
         jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
     else if (jb.t <= 4) decode_body<FMT, 4, false, false, true, 1, FAT>(jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
@@ -1025,22 +1087,23 @@ inline int set_of(int fmt, uint32_t mask) {
 // matmuls go out in one launch. Q4_0's kernel is bounded at 512 threads, which saves it nine spilled registers; its shapes
 // never exceed 8 waves.)
 // FAT: the launch's jobs use the fat mapping (see place_job); the plain kernels do without its bookkeeping.
-template <uint32_t FSET, bool FAT>
-__global__ __launch_bounds__(FSET == (1u << FMT_Q40) ? 512 : 1024) void decode_batch_kernel(BatchArgs a) {
+// WIDE: the launch's jobs have 9 to 16 tokens each (a kernel of its own, for the registers; plain mapping).
+template <uint32_t FSET, bool FAT, bool WIDE = false>
+__global__ __launch_bounds__(WIDE || FSET == (1u << FMT_Q40) ? 512 : 1024) void decode_batch_kernel(BatchArgs a) {
     extern __shared__ __align__(16) float lds_dyn[];
     uint32_t j = 0;
     while (j + 1 < a.njobs && blockIdx.x >= a.j[j + 1].wg0) j++;  // uniform
     const BatchJob& jb = a.j[j];
     const uint32_t bx = blockIdx.x - jb.wg0;
     switch (jb.w.fmt) {
-        case FMT_Q8_0: if constexpr (FSET & fbit(FMT_Q8_0)) batch_dispatch<FMT_Q8_0, FAT>(jb, bx, lds_dyn); break;
-        case FMT_Q8F: if constexpr (FSET & fbit(FMT_Q8F)) batch_dispatch<FMT_Q8F, FAT>(jb, bx, lds_dyn); break;
-        case FMT_Q4_K: if constexpr (FSET & fbit(FMT_Q4_K)) batch_dispatch<FMT_Q4_K, FAT>(jb, bx, lds_dyn); break;
-        case FMT_Q5_K: if constexpr (FSET & fbit(FMT_Q5_K)) batch_dispatch<FMT_Q5_K, FAT>(jb, bx, lds_dyn); break;
-        case FMT_Q6_K: if constexpr (FSET & fbit(FMT_Q6_K)) batch_dispatch<FMT_Q6_K, FAT>(jb, bx, lds_dyn); break;
-        case FMT_Q4M: if constexpr (FSET & fbit(FMT_Q4M)) batch_dispatch<FMT_Q4M, FAT>(jb, bx, lds_dyn); break;
-        case FMT_Q40: if constexpr (FSET & fbit(FMT_Q40)) batch_dispatch<FMT_Q40, FAT>(jb, bx, lds_dyn); break;
-        case FMT_MXFP4: if constexpr (FSET & fbit(FMT_MXFP4)) batch_dispatch<FMT_MXFP4, FAT>(jb, bx, lds_dyn); break;
+        case FMT_Q8_0: if constexpr (FSET & fbit(FMT_Q8_0)) batch_dispatch<FMT_Q8_0, FAT, WIDE>(jb, bx, lds_dyn); break;
+        case FMT_Q8F: if constexpr (FSET & fbit(FMT_Q8F)) batch_dispatch<FMT_Q8F, FAT, WIDE>(jb, bx, lds_dyn); break;
+        case FMT_Q4_K: if constexpr (FSET & fbit(FMT_Q4_K)) batch_dispatch<FMT_Q4_K, FAT, WIDE>(jb, bx, lds_dyn); break;
+        case FMT_Q5_K: if constexpr (FSET & fbit(FMT_Q5_K)) batch_dispatch<FMT_Q5_K, FAT, WIDE>(jb, bx, lds_dyn); break;
+        case FMT_Q6_K: if constexpr (FSET & fbit(FMT_Q6_K)) batch_dispatch<FMT_Q6_K, FAT, WIDE>(jb, bx, lds_dyn); break;
+        case FMT_Q4M: if constexpr (FSET & fbit(FMT_Q4M)) batch_dispatch<FMT_Q4M, FAT, WIDE>(jb, bx, lds_dyn); break;
+        case FMT_Q40: if constexpr (FSET & fbit(FMT_Q40)) batch_dispatch<FMT_Q40, FAT, WIDE>(jb, bx, lds_dyn); break;
+        case FMT_MXFP4: if constexpr (FSET & fbit(FMT_MXFP4)) batch_dispatch<FMT_MXFP4, FAT, WIDE>(jb, bx, lds_dyn); break;
         default: break;
     }
 }
@@ -1139,7 +1202,7 @@ Shape pair_shape(Shape sh) {
 }
 uint32_t pair_tiles(const Shape& sh, bool pair) { return pair ? pair_shape(sh).rt / 2 : sh.rt; }
 
-constexpr size_t LDS_MAX = 160 * 1024 - 256;  // dynamic LDS on offer (the kernel also holds a static word)
+constexpr size_t LDS_MAX = 160 * 1024;  // dynamic LDS on offer (the kernels hold no static LDS)
 
 // Dynamic LDS of a launch; `alds` comes back false when the operand-order activations do not fit (they are then read
 // from L2 per record).
@@ -1148,9 +1211,9 @@ size_t lds_bytes(int fmt, bool dump, uint32_t nsteps, int tpad, const Shape& sh,
     const uint32_t bps = q8_format(fmt) ? 2 : 4;
     const uint32_t fs = map.fs ? map.fs : 1;
     const uint32_t nbl = bps * fs * ((nsteps + sh.ks - 1) / sh.ks);  // blocks of the workgroup's slices
-    const uint32_t narr = q8_format(fmt) || fmt == FMT_Q40 || fmt == FMT_MXFP4 ? 1 : fmt == FMT_Q6_K ? (dump ? 4 : 3) : 2;  // metadata arrays
+    const uint32_t narr = k45_format(fmt) || fmt == FMT_Q4M ? 2 : 1;  // metadata arrays
     const size_t meta = (size_t)narr * ng * nbl * tpad * 4, red = (size_t)sh.rt * fs * sh.kw * ng * tpad * 16 * 4;
-    const size_t act = (size_t)ng * (nbl / 2) * 512;
+    const size_t act = (size_t)ng * (nbl / 2) * (tpad == 16 ? 1024 : 512);
     const size_t with = act + meta > red ? act + meta : red;  // the partial sums reuse the activations' space
     *alds = with <= LDS_MAX;
     return *alds ? with : meta + red;
@@ -1178,7 +1241,7 @@ hipError_t launch_one(bool alds, dim3 grid, dim3 block, size_t lds, hipStream_t 
         else kern<<<grid, block, lds, s>>>(w, v, t, sh.rt, sh.kw, y, dump, g, sh.ks, sc.partial, sc.counters, epi);
     };
     if (alds) go(decode_mfma_kernel<FMT, NT, DUMP, GROUPED, true, NG>);
-    else if constexpr (NG == 1 && FMT != FMT_Q6_K) go(decode_mfma_kernel<FMT, NT, DUMP, GROUPED, false, 1>);
+    else if constexpr (NG == 1 && FMT != FMT_Q6_K && NT <= 8) go(decode_mfma_kernel<FMT, NT, DUMP, GROUPED, false, 1>);
     else e = hipErrorInvalidValue;  // token groups and Q6_K need the staged activations
     return e != hipSuccess ? e : hipGetLastError();
 }
@@ -1194,18 +1257,25 @@ hipError_t run(const WeightView& w, const QActView& xa, size_t t, float* y, int3
     const uint32_t ntiles = row_tiles(w.n_out), nsteps = steps_of<FMT>(w.n_in);
     const bool pair = !DUMP && epi0.pair_p0 != nullptr;
     Shape sh = shape_for(ntiles, nsteps, true, FMT);
-    // slices need scratch: 8 token rows per slice (of both matrices of a pair) and a counter per row group
-    auto scratch_ok = [&](const Shape& h) {
+    // slices need scratch: 8 (or 16) token rows per slice (of both matrices of a pair) and a counter per row group
+    auto scratch_ok = [&](const Shape& h, size_t rows) {
         const uint32_t groups = (ntiles + pair_tiles(h, pair) - 1) / pair_tiles(h, pair);
-        return h.ks == 1 || (sc.partial && sc.counters && sc.partial_floats >= (size_t)h.ks * 8 * w.n_out * (pair ? 2 : 1) && sc.ncounters >= (size_t)groups * CTR_STRIDE);
+        return h.ks == 1 || (sc.partial && sc.counters && sc.partial_floats >= (size_t)h.ks * rows * w.n_out * (pair ? 2 : 1) && sc.ncounters >= (size_t)groups * CTR_STRIDE);
     };
-    if (!scratch_ok(sh)) sh = shape_for(ntiles, nsteps, false, FMT);
+    if (!scratch_ok(sh, 8)) sh = shape_for(ntiles, nsteps, false, FMT);
     if (pair) sh = pair_shape(sh);
     const uint32_t nblk = w.n_in / 32;
     const uint32_t per_wg = pair ? sh.rt / 2 : sh.rt;  // row tiles of the output per workgroup
     dim3 grid((ntiles + per_wg - 1) / per_wg, sh.ks), block(64 * sh.rt * sh.kw);
+    // Nine to sixteen tokens in one pass over the weights where their staged activations fit the LDS and the scratch their
+    // slices' rows; otherwise eight at a time.
+    bool wide = false;
+    if (!DUMP && t > 8 && t <= 16) {
+        const size_t l = lds_bytes(FMT, false, nsteps, 16, sh, &wide);
+        wide = wide && l <= LDS_MAX && sh.rt * sh.kw <= 8 && scratch_ok(sh, t);
+    }
     // timing events: one launch carries them itself; around several they are recorded on the stream
-    const bool ride = t <= 8;
+    const bool ride = t <= 8 || wide;
     if (!ride && ev_start) {
         hipError_t e = hipEventRecord(ev_start, s);
         if (e != hipSuccess) return e;
@@ -1213,7 +1283,7 @@ hipError_t run(const WeightView& w, const QActView& xa, size_t t, float* y, int3
     hipEvent_t e0 = ride ? ev_start : nullptr, e1 = ride ? ev_stop : nullptr;
     size_t c0 = 0;
     while (c0 < t) {
-        const size_t tc = t - c0 < 8 ? t - c0 : 8;
+        const size_t tc = wide ? t : t - c0 < 8 ? t - c0 : 8;
         QActView v = xa;
         v.q += c0 * w.n_in;
         v.scales += c0 * nblk;
@@ -1223,7 +1293,7 @@ hipError_t run(const WeightView& w, const QActView& xa, size_t t, float* y, int3
         if (v.sums16) v.sums16 += c0 * 2 * nblk;
         float* yo = y ? y + c0 * w.n_out : nullptr;  // no output rows when only the block sums are wanted
         int32_t* du = dump ? dump + c0 * (size_t)w.n_out * nblk * (FMT == FMT_Q6_K ? 2 : 1) : nullptr;
-        const int tpad = tc <= 4 ? 4 : 8;
+        const int tpad = tc <= 4 ? 4 : tc <= 8 ? 8 : 16;
         bool alds;
         const size_t lds = lds_bytes(FMT, DUMP, nsteps, tpad, sh, &alds);
         if (lds > LDS_MAX) return hipErrorInvalidValue;  // rows too long for the staged activation scales
@@ -1234,7 +1304,9 @@ hipError_t run(const WeightView& w, const QActView& xa, size_t t, float* y, int3
         if (tc == 1) e = launch_one<FMT, 1, DUMP, false>(alds, grid, block, lds, s, w, v, tt, sh, yo, du, GroupView{}, sc, e0, e1, epi);
         else if (tc == 2 && !t4m_format(FMT)) e = launch_one<FMT, 2, DUMP, false>(alds, grid, block, lds, s, w, v, tt, sh, yo, du, GroupView{}, sc, e0, e1, epi);
         else if (tc <= 4) e = launch_one<FMT, 4, DUMP, false>(alds, grid, block, lds, s, w, v, tt, sh, yo, du, GroupView{}, sc, e0, e1, epi);
-        else e = launch_one<FMT, 8, DUMP, false>(alds, grid, block, lds, s, w, v, tt, sh, yo, du, GroupView{}, sc, e0, e1, epi);
+        else if (tc <= 8) e = launch_one<FMT, 8, DUMP, false>(alds, grid, block, lds, s, w, v, tt, sh, yo, du, GroupView{}, sc, e0, e1, epi);
+        else if constexpr (!DUMP) e = launch_one<FMT, 16, DUMP, false>(alds, grid, block, lds, s, w, v, tt, sh, yo, du, GroupView{}, sc, e0, e1, epi);
+        else e = hipErrorInvalidValue;
         if (e != hipSuccess) return e;
         c0 += tc;
     }
@@ -1311,11 +1383,11 @@ bool decode_pair_ok(const WeightView& w) {
 
 bool decode_batchable(const WeightView& w, size_t t) {
     if (!mfma_decode_format(w.fmt)) return false;
-    if (t < 1 || t > 8) return false;
+    if (t < 1 || t > 16) return false;
     const Shape sh = shape_for(row_tiles(w.n_out), steps_rt(w), true, w.fmt);  // as a launch of its own: same bits
     bool alds;
-    const size_t lds = lds_bytes(w.fmt, false, steps_rt(w), t <= 4 ? 4 : 8, sh, &alds);
-    return alds && lds <= LDS_MAX;
+    const size_t lds = lds_bytes(w.fmt, false, steps_rt(w), t <= 4 ? 4 : t <= 8 ? 8 : 16, sh, &alds);
+    return alds && lds <= LDS_MAX && (t <= 8 || sh.rt * sh.kw <= 8);
 }
 
 // Scratch a launch of this weight alone takes when its shape slices K across workgroups (floats of partial rows,
@@ -1354,7 +1426,7 @@ Placed place_job(const DecodeBatchItem& it, bool fat, uint32_t fat_steps) {
     const bool pair = it.epi.pair_p0 != nullptr;
     Shape sh = shape_for(ntiles, nsteps, true, it.w.fmt);
     if (pair) sh = pair_shape(sh);
-    const int tpad = it.t <= 4 ? 4 : 8;
+    const int tpad = it.t <= 4 ? 4 : it.t <= 8 ? 8 : 16;
     Placed pl{sh.rt, Mapping{sh.kw, 1}, 0, 0};
     bool alds = false;
     if (fat && nsteps % (sh.ks * sh.kw) == 0) {  // (every run has the same number of steps)
@@ -1417,9 +1489,12 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
     const uint64_t bit = 1ull << (dev & 63);
     if (!(allowed[(dev >> 6) & 3].load(std::memory_order_acquire) & bit)) {
 #define OXHIP_BATCH_KERNELS(F) reinterpret_cast<const void*>(decode_batch_kernel<F, false>), reinterpret_cast<const void*>(decode_batch_kernel<F, true>)
-        for (const void* k : {OXHIP_BATCH_KERNELS(FSET_GGUF), OXHIP_BATCH_KERNELS(FSET_MLX), OXHIP_BATCH_KERNELS(FSET_K5),
+#define OXHIP_BATCH_WIDE(F) reinterpret_cast<const void*>(decode_batch_kernel<F, false, true>)
+        for (const void* k : {OXHIP_BATCH_WIDE(FSET_GGUF), OXHIP_BATCH_WIDE(FSET_MLX), OXHIP_BATCH_WIDE(FSET_K5), OXHIP_BATCH_WIDE(FSET_Q40),
+                              OXHIP_BATCH_WIDE(FSET_MX4), OXHIP_BATCH_WIDE(FSET_Q8F), OXHIP_BATCH_KERNELS(FSET_GGUF), OXHIP_BATCH_KERNELS(FSET_MLX), OXHIP_BATCH_KERNELS(FSET_K5),
                               OXHIP_BATCH_KERNELS(FSET_Q40), OXHIP_BATCH_KERNELS(FSET_MX4), OXHIP_BATCH_KERNELS(FSET_Q8F)}) {
 #undef OXHIP_BATCH_KERNELS
+#undef OXHIP_BATCH_WIDE
             hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_MAX);
             if (e != hipSuccess) return e;
         }
@@ -1429,18 +1504,18 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
     std::vector<size_t> ldss;
     std::vector<uint32_t> threadss;
     std::vector<bool> fats;
-    // the jobs by format set (the caller's order within a set), then launches of up to BATCH_MAX jobs of one set
+    // the jobs by format set and form (up to 8 tokens, more), in the caller's order, then launches of up to BATCH_MAX jobs of one
     std::vector<const DecodeBatchItem*> sorted;
     std::vector<std::pair<size_t, size_t>> runs;  // [first, count) into `sorted`
     sorted.reserve(n);
     uint32_t call_mask = 0;
     for (size_t i = 0; i < n; i++) call_mask |= fbit(items[i].w.fmt);
-    for (int set = 0; set < NSETS; set++) {
+    for (int set = 0; set < 2 * NSETS; set++) {
         const size_t first = sorted.size();
         for (size_t i = 0; i < n; i++) {
             const int so = set_of(items[i].w.fmt, call_mask);
             if (so < 0) return hipErrorInvalidValue;
-            if (so == set) sorted.push_back(&items[i]);
+            if (2 * so + (items[i].t > 8 ? 1 : 0) == set) sorted.push_back(&items[i]);
         }
         for (size_t i0 = first; i0 < sorted.size(); i0 += BATCH_MAX) runs.emplace_back(i0, std::min(sorted.size() - i0, (size_t)BATCH_MAX));
     }
@@ -1484,7 +1559,8 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
 #endif
         uint64_t fat_wgs = 0;
         for (uint32_t j = 0; j < a.njobs; j++) fat_wgs += place_job(*items_of[j], true, fat_steps).wgs;
-        const bool fat = fat_wgs >= fat_min;
+        const bool wide = items_of[0]->t > 8;  // (all of them, or none)
+        const bool fat = !wide && fat_wgs >= fat_min;
         for (uint32_t j = 0; j < a.njobs; j++) {
             const DecodeBatchItem& it = *items_of[order[j]];
             const uint32_t ntiles = row_tiles(it.w.n_out), nsteps = steps_rt(it.w);
@@ -1493,7 +1569,7 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
             if (pair) sh = pair_shape(sh);
             const Placed pl = place_job(it, fat, fat_steps);
             const size_t l = pl.lds;
-            if (l > LDS_MAX || it.t < 1 || it.t > 8) return hipErrorInvalidValue;
+            if (l > LDS_MAX || it.t < 1 || it.t > 16) return hipErrorInvalidValue;
             sh.rt = pl.rt;
             const uint32_t per_wg = pair ? sh.rt / 2 : sh.rt;
             const uint32_t groups = (ntiles + per_wg - 1) / per_wg;
@@ -1530,13 +1606,14 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
         if (!launches[i].nwg) continue;
         uint32_t fset = 0;
         for (uint32_t j = 0; j < launches[i].njobs; j++) fset |= fbit(launches[i].j[j].w.fmt);
-        if (threadss[i] > (fset == FSET_Q40 ? 512u : 1024u)) return hipErrorInvalidValue;  // (the kernels' launch bounds)
+        if (threadss[i] > (fset == FSET_Q40 || launches[i].j[0].t > 8 ? 512u : 1024u)) return hipErrorInvalidValue;  // (the kernels' launch bounds)
         auto go = [&](auto kern) {
             if (ride) hipExtLaunchKernelGGL(kern, dim3(launches[i].nwg), dim3(threadss[i]), (uint32_t)ldss[i], s, ev_start, ev_stop, 0, launches[i]);
             else kern<<<launches[i].nwg, threadss[i], ldss[i], s>>>(launches[i]);
         };
         const bool fat = fats[i];
-#define OXHIP_GO(F) (fat ? go(decode_batch_kernel<F, true>) : go(decode_batch_kernel<F, false>))
+        const bool wide = launches[i].j[0].t > 8;
+#define OXHIP_GO(F) (wide ? go(decode_batch_kernel<F, false, true>) : fat ? go(decode_batch_kernel<F, true>) : go(decode_batch_kernel<F, false>))
         if (!(fset & ~FSET_GGUF)) OXHIP_GO(FSET_GGUF);
         else if (!(fset & ~FSET_MLX)) OXHIP_GO(FSET_MLX);
         else if (!(fset & ~FSET_K5)) OXHIP_GO(FSET_K5);

@@ -165,7 +165,7 @@ hipError_t launch_decode(const WeightView& w, const QActView& xa, const float* x
 // decode kernels only store.
 hipError_t launch_epilogue(const float* v, size_t t, size_t n, float* y, const Epi& epi, hipStream_t s);
 hipError_t launch_isums(const WeightView& w, const QActView& xa, size_t t, int32_t* out, hipStream_t s);
-// Independent matmuls that may share one launch (decode_mfma.hip): each 1..8 tokens over a tile-packed weight.
+// Independent matmuls that may share one launch (decode_mfma.hip): each 1..16 tokens over a tile-packed weight (jobs of more than 8 in launches of their own).
 struct DecodeBatchItem {
     WeightView w;
     QActView xa;

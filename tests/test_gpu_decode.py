@@ -615,6 +615,43 @@ def test_decode_batch_events(be, oxref):
             assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("kind", [Q4_0, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4, "q8", "mlx"])
+@pytest.mark.parametrize("n_out,n_in", [(37, 768), (272, 4096), (48, 14336)])  # ragged rows; two workgroups a CU; K slices
+def test_sixteen_token_form_keeps_the_bits(be, oxref, kind, n_out, n_in):
+    """Nine to sixteen tokens go through the 16-token form in one pass over the weights: every row, stored, added, of a gate /
+    up pair and in a shared launch with jobs of fewer tokens, has the bits of that token's row computed alone (which the
+    other tests hold to the oracle)."""
+    import torch
+    from oxinfer_amd import hip, synth
+
+    def upload(seed):
+        if kind == "q8":
+            return be.upload_q8(*synth.q8_matrix(n_out, n_in, seed), n_out, n_in)
+        if kind == "mlx":
+            return be.upload_mlx_q4(*synth.mlx_q4(n_out, n_in, seed), 64, n_out, n_in)
+        return be.upload_gguf(kind, oxref.random_blocks(kind, n_out * n_in // oxref.block_size(kind), seed)[0], n_out, n_in)
+    w, w2 = upload(71), upload(72)
+    assert w is not None and w2 is not None, be.last_error()
+    x = dev(synth.activations(16, n_in, 73))
+    qa = be.quantize_act(x)
+    ones = [be.quantize_act(x[i:i + 1].contiguous()) for i in range(16)]
+    bits = lambda v: v.cpu().numpy().view(np.uint32)
+    want = torch.cat([be.decode(w, xa=q) for q in ones])
+    base = dev(synth.activations(16, n_out, 74))
+    added, paired = base.clone(), torch.zeros((16, n_out), device="cuda")
+    for i, q in enumerate(ones):
+        assert be.linear(w, added[i:i + 1], xa=q, t=1, mode=hip.LIN_ADD)
+        assert be.linear(w, paired[i:i + 1], xa=q, t=1, mode=hip.LIN_SILU_PAIR, w2=w2)
+    for t in (9, 13, 16):
+        assert np.array_equal(bits(be.decode(w, xa=qa, t=t)), bits(want[:t]))
+        y = base[:t].clone()
+        assert be.linear(w, y, xa=qa, t=t, mode=hip.LIN_ADD) and np.array_equal(bits(y), bits(added[:t]))
+        assert be.linear(w, y, xa=qa, t=t, mode=hip.LIN_SILU_PAIR, w2=w2) and np.array_equal(bits(y), bits(paired[:t]))
+        ys = [torch.full((c, n_out), float("nan"), device="cuda") for c in (t, 3, t)]
+        be.decode_batch(be.decode_jobs([(w, qa, None, y.shape[0], y, None, None) for y in ys]))
+        assert all(np.array_equal(bits(y), bits(want[:y.shape[0]])) for y in ys)
+
+
 def test_works_from_another_thread_and_concurrent_calls_do_not_mix(be, oxref):
     """The Backend surface is Send + Sync (src/gpu.rs:151): a call from another thread, on weights uploaded here, and eight
     threads calling at once, each with its own input, get their own rows (src/cuda.rs:2048-2077, :2411-2439). A call's
