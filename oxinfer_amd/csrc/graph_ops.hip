@@ -77,19 +77,18 @@ hipError_t launch_router_logits(const float* x, const float* router, const float
 //   what `out` then holds goes, per block of 32, to the QAct (optional).
 // The reference sums the squares one after the other in f32 (src/kernels.rs:2109), which no parallel machine can
 // repeat bit for bit in useful time: here the squares are exact in f64 and summed in f64 (a fixed order), the mean and
-// eps added in f32 as the reference does, and r is the correctly rounded power. The quantization of v is quantize_act's,
-// bit for bit (the same code on the same values). VEC: rows of x, out and w start on 16-byte boundaries (float4 access);
-// otherwise every access is one float.
-template <bool VEC>
-__global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(const float* __restrict__ x, const float* __restrict__ w_f32,
-                                                               const uint16_t* __restrict__ w_bf16, float eps, float pre, uint32_t add,
-                                                               uint32_t n, size_t x_stride, size_t out_stride,
-                                                               float* __restrict__ out, int8_t* __restrict__ q, float* __restrict__ scales,
-                                                               int32_t* __restrict__ sums, float* __restrict__ fsums,
-                                                               float* __restrict__ hsums, int32_t* __restrict__ sums16) {
-    __shared__ double part[4];
-    __shared__ float r_s;
-    const uint32_t tok = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// eps added in f32 as the reference does, and r is the power rounded from 45 correct bits. The quantization of v is
+// quantize_act's, bit for bit (the same code on the same values). VEC: rows of x, out and w start on 16-byte boundaries
+// (float4 access); otherwise every access is one float.
+// The kernel is one row's chain of latencies, so a row takes as many threads as it has float4s (up to 1024), its values and
+// weights are requested together and stay in registers (NV float4s a thread; NV = 0: longer rows, read twice), and eight
+// lanes quantize a block where they hold it (4096 values, one row, in a replayed chain: 5.4 -> 4.4 us).
+template <bool VEC, int NV>
+__global__ __launch_bounds__(1024) void rmsnorm_quantize_kernel(const float* __restrict__ x, const float* __restrict__ w_f32,
+                                                                const uint16_t* __restrict__ w_bf16, float eps, float pre, uint32_t add, uint32_t n,
+                                                                size_t x_stride, size_t out_stride, float* __restrict__ out, QActOut q) {
+    __shared__ double part_s[16];
+    const uint32_t tok = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nthr = blockDim.x, nwaves = nthr >> 6;
     const float* xr = x + (size_t)tok * x_stride;
     auto load4 = [&](const float* p, float* v) {
         if constexpr (VEC) {
@@ -99,66 +98,92 @@ __global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(const float* __re
             v[0] = p[0]; v[1] = p[1]; v[2] = p[2]; v[3] = p[3];
         }
     };
+    auto load_w = [&](uint32_t i, float* v) {
+        if (w_f32) {
+            load4(w_f32 + i, v);
+        } else if (w_bf16) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = bf16_bits_to_f32(w_bf16[i + j]);
+        } else {
+            v[0] = v[1] = v[2] = v[3] = 1.0f;  // (x * 1 is x)
+        }
+    };
+    float xv[NV ? NV : 1][4], wv[NV ? NV : 1][4];
     double ss = 0.0;
-    for (uint32_t i = 4 * threadIdx.x; i < n; i += 1024) {  // n is a multiple of 32
-        float v[4];
-        load4(xr + i, v);
+    auto square = [&](const float* v) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const float p = v[j] * pre;
             ss += (double)p * p;
         }
+    };
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            const uint32_t i = 4 * (threadIdx.x + k * nthr);
+            if (i < n) {
+                load4(xr + i, xv[k]);
+                load_w(i, wv[k]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NV; k++)
+            if (4 * (threadIdx.x + k * nthr) < n) square(xv[k]);
+    } else {
+        for (uint32_t i = 4 * threadIdx.x; i < n; i += 4 * nthr) {
+            load4(xr + i, xv[0]);
+            square(xv[0]);
+        }
     }
     for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off);
-    if (lane == 0) part[wave] = ss;
+    if (lane == 0) part_s[wave] = ss;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const double total = ((part[0] + part[1]) + part[2]) + part[3];
-        const float m = (float)total / (float)n + eps;
-        r_s = (float)(1.0 / sqrt((double)m));
-    }
-    __syncthreads();
-    const float r = r_s;
-    const uint32_t nblocks = n / 32;
-    for (uint32_t b = threadIdx.x; b < nblocks; b += 256) {
-        float v[32];
+    double p[16];  // (all requested at once, added in pairs)
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            float f[4];
-            load4(xr + 32 * b + 4 * i, f);
+    for (int i = 0; i < 16; i++) p[i] = part_s[i];
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[4 * i + j] = (f[j] * pre) * r;
-        }
-        if (w_f32) {
+    for (int i = 0; i < 16; i++) p[i] = (uint32_t)i < nwaves ? p[i] : 0.0;
 #pragma unroll
-            for (int i = 0; i < 32; i++) v[i] = v[i] * w_f32[32 * b + i];
-        } else if (w_bf16) {
+    for (int d = 1; d < 16; d *= 2)
 #pragma unroll
-            for (int i = 0; i < 32; i++) v[i] = v[i] * bf16_bits_to_f32(w_bf16[32 * b + i]);
-        }
-        const size_t gb = (size_t)tok * nblocks + b;
-        float* orow = out ? out + (size_t)tok * out_stride + 32 * b : nullptr;
-        if (out && add) {
+        for (int i = 0; i + d < 16; i += 2 * d) p[i] += p[i + d];
+    const float m = (float)p[0] / (float)n + eps;
+    // m^(-1/2): the hardware's estimate (1 ulp) and one Newton step in f64
+    const double y0 = (double)__builtin_amdgcn_rsqf(m);
+    const float r = m > 1.2e-38f && m < 3.0e38f ? (float)(y0 * (1.5 - 0.5 * (double)m * (y0 * y0))) : (float)(1.0 / sqrt((double)m));
+    auto finish = [&](uint32_t i, const float* xs, const float* ws) {  // elements i .. i + 3 of the row
+        float v[4];
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                float f[4];
-                load4(orow + 4 * i, f);
-#pragma unroll
-                for (int j = 0; j < 4; j++) v[4 * i + j] = f[j] + v[4 * i + j];
-            }
-        }
+        for (int j = 0; j < 4; j++) v[j] = ((xs[j] * pre) * r) * ws[j];
         if (out) {
+            float* o = out + (size_t)tok * out_stride + i;
+            if (add) {
+                float f[4];
+                load4(o, f);
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                if constexpr (VEC) {
-                    *reinterpret_cast<float4*>(orow + 4 * i) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-                } else {
+                for (int j = 0; j < 4; j++) v[j] = f[j] + v[j];
+            }
+            if constexpr (VEC) {
+                *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
 #pragma unroll
-                    for (int j = 0; j < 4; j++) orow[4 * i + j] = v[4 * i + j];
-                }
+                for (int j = 0; j < 4; j++) o[j] = v[j];
             }
         }
-        if (q) quantize_act_values(v, gb, q, scales, sums, fsums, hsums, sums16);
+        if (q.q) quantize_act_part(v, (i >> 2) & 7, (size_t)tok * (n / 32) + i / 32, q);
+    };
+    if constexpr (NV > 0) {
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            const uint32_t i = 4 * (threadIdx.x + k * nthr);
+            if (i < n) finish(i, xv[k], wv[k]);
+        }
+    } else {
+        for (uint32_t i = 4 * threadIdx.x; i < n; i += 4 * nthr) {
+            load4(xr + i, xv[0]);
+            load_w(i, wv[0]);
+            finish(i, xv[0], wv[0]);
+        }
     }
 }
 
@@ -170,13 +195,13 @@ hipError_t launch_rmsnorm_quantize(const float* x, const float* w_f32, const uin
     if (!out_stride) out_stride = n;
     auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     const bool vec = al(x) && al(out) && al(w_f32) && x_stride % 4 == 0 && out_stride % 4 == 0;
+    const unsigned threads = (unsigned)(n / 4 >= 1024 ? 1024 : (n / 4 + 63) / 64 * 64);
     auto go = [&](auto kern) {
-        kern<<<(unsigned)t, 256, 0, s>>>(x, w_f32, w_bf16, eps, pre, add ? 1u : 0u, (uint32_t)n, x_stride, out_stride, out, qa ? qa->q : nullptr,
-                                        qa ? qa->scales : nullptr, qa ? qa->sums : nullptr, qa ? qa->fsums : nullptr, qa ? qa->hsums : nullptr,
-                                        qa ? qa->sums16 : nullptr);
+        kern<<<(unsigned)t, threads, 0, s>>>(x, w_f32, w_bf16, eps, pre, add ? 1u : 0u, (uint32_t)n, x_stride, out_stride, out, qa ? qact_out(*qa) : QActOut{});
     };
-    if (vec) go(rmsnorm_quantize_kernel<true>);
-    else go(rmsnorm_quantize_kernel<false>);
+    if (n <= 4096) vec ? go(rmsnorm_quantize_kernel<true, 1>) : go(rmsnorm_quantize_kernel<false, 1>);
+    else if (n <= 16384) vec ? go(rmsnorm_quantize_kernel<true, 4>) : go(rmsnorm_quantize_kernel<false, 4>);
+    else vec ? go(rmsnorm_quantize_kernel<true, 0>) : go(rmsnorm_quantize_kernel<false, 0>);
     return hipGetLastError();
 }
 

@@ -131,20 +131,17 @@ __global__ __launch_bounds__(64 * NW) void route_top_k_kernel(const float* __res
     route_top_k_body<PER, NW>(logits, stride, n, k, idx, wts, expert_scale, blockIdx.x);
 }
 
-// Workgroups 0 .. t - 1 route a token each; the others quantize one block of 32 of x per lane.
+// Workgroups 0 .. t - 1 route a token each; the others quantize x, eight lanes to a block of 32.
 template <int PER>
 __global__ __launch_bounds__(512) void route_quantize_kernel(const float* __restrict__ logits, uint32_t stride, uint32_t n, uint32_t k,
                                                              uint32_t* __restrict__ idx, float* __restrict__ wts,
                                                              const float* __restrict__ expert_scale, uint32_t t, const float* __restrict__ x,
-                                                             size_t nblocks, int8_t* __restrict__ q, float* __restrict__ scales,
-                                                             int32_t* __restrict__ sums, float* __restrict__ fsums, float* __restrict__ hsums,
-                                                             int32_t* __restrict__ sums16) {
+                                                             size_t nblocks, QActOut o) {
     if (blockIdx.x < t) {
         route_top_k_body<PER, 8>(logits, stride, n, k, idx, wts, expert_scale, blockIdx.x);
         return;
     }
-    const size_t b = (size_t)(blockIdx.x - t) * blockDim.x + threadIdx.x;
-    if (b < nblocks) quantize_act_block(x, b, q, scales, sums, fsums, hsums, sums16);
+    quantize_act_lane(x, (size_t)(blockIdx.x - t) * blockDim.x + threadIdx.x, nblocks, o);
 }
 
 hipError_t launch_route_quantize(const float* logits, size_t t, size_t n, size_t k, uint32_t* idx, float* w, size_t stride,
@@ -153,13 +150,11 @@ hipError_t launch_route_quantize(const float* logits, size_t t, size_t n, size_t
     if (n > 256) return hipErrorInvalidValue;
     const uint32_t st = (uint32_t)(stride ? stride : n);
     const size_t nblocks = t * h / 32;
-    const unsigned grid = (unsigned)(t + (nblocks + 511) / 512);
+    const unsigned grid = (unsigned)(t + (nblocks * 8 + 511) / 512);
     if (n <= 128)
-        route_quantize_kernel<2><<<grid, 512, 0, s>>>(logits, st, (uint32_t)n, (uint32_t)k, idx, w, expert_scale, (uint32_t)t, x, nblocks, o.q, o.scales,
-                                                     o.sums, o.fsums, o.hsums, o.sums16);
+        route_quantize_kernel<2><<<grid, 512, 0, s>>>(logits, st, (uint32_t)n, (uint32_t)k, idx, w, expert_scale, (uint32_t)t, x, nblocks, qact_out(o));
     else
-        route_quantize_kernel<4><<<grid, 512, 0, s>>>(logits, st, (uint32_t)n, (uint32_t)k, idx, w, expert_scale, (uint32_t)t, x, nblocks, o.q, o.scales,
-                                                     o.sums, o.fsums, o.hsums, o.sums16);
+        route_quantize_kernel<4><<<grid, 512, 0, s>>>(logits, st, (uint32_t)n, (uint32_t)k, idx, w, expert_scale, (uint32_t)t, x, nblocks, qact_out(o));
     return hipGetLastError();
 }
 
@@ -246,19 +241,16 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const uint32_t* __restri
 }
 
 // The plan and the quantization of the layer's input depend only on the layer's arguments, and each is a few
-// microseconds of latency: one launch runs both (workgroup 0 plans, the others quantize one block of 32 per lane).
+// microseconds of latency: one launch runs both (workgroup 0 plans, the others quantize, eight lanes to a block of 32).
 __global__ __launch_bounds__(1024) void moe_front_kernel(const uint32_t* __restrict__ route_idx, uint32_t pairs, uint32_t k, uint32_t n_exp,
                                                          int cr, int* __restrict__ row_of, int* __restrict__ src, int4* __restrict__ chunks,
-                                                         int* __restrict__ nchunks, const float* __restrict__ x, size_t nblocks,
-                                                         int8_t* __restrict__ q, float* __restrict__ scales, int32_t* __restrict__ sums,
-                                                         float* __restrict__ fsums, float* __restrict__ hsums, int32_t* __restrict__ sums16) {
+                                                         int* __restrict__ nchunks, const float* __restrict__ x, size_t nblocks, QActOut o) {
     extern __shared__ int sh[];
     if (blockIdx.x == 0) {
         moe_plan_body(sh, route_idx, pairs, k, n_exp, cr, row_of, src, chunks, nchunks);
         return;
     }
-    const size_t b = (size_t)(blockIdx.x - 1) * blockDim.x + threadIdx.x;
-    if (b < nblocks) quantize_act_block(x, b, q, scales, sums, fsums, hsums, sums16);
+    quantize_act_lane(x, (size_t)(blockIdx.x - 1) * blockDim.x + threadIdx.x, nblocks, o);
 }
 
 hipError_t launch_moe_plan(const uint32_t* route_idx, size_t pairs, size_t k, size_t n_exp, uint32_t chunk_rows, int* row_of, int* src,
@@ -281,9 +273,8 @@ hipError_t launch_moe_front(const uint32_t* route_idx, size_t pairs, size_t k, s
         hipError_t e = launch_moe_plan(route_idx, pairs, k, n_exp, chunk_rows, row_of, src, chunks, nchunks, s);
         return e != hipSuccess ? e : launch_quantize_act(x, t, h, o, s);
     }
-    moe_front_kernel<<<1 + (unsigned)((nblocks + 1023) / 1024), 1024, lds, s>>>(route_idx, (uint32_t)pairs, (uint32_t)k, (uint32_t)n_exp,
-                                                                              (int)chunk_rows, row_of, src, chunks, nchunks, x, nblocks, o.q, o.scales,
-                                                                              o.sums, o.fsums, o.hsums, o.sums16);
+    moe_front_kernel<<<1 + (unsigned)((nblocks * 8 + 1023) / 1024), 1024, lds, s>>>(route_idx, (uint32_t)pairs, (uint32_t)k, (uint32_t)n_exp, (int)chunk_rows,
+                                                                                  row_of, src, chunks, nchunks, x, nblocks, qact_out(o));
     return hipGetLastError();
 }
 
@@ -320,98 +311,23 @@ hipError_t launch_moe_act(const float* g, const float* u, size_t stride, size_t 
 }
 
 // The same, followed by quantize_act on the result (src/quant.rs:267-292) without the round trip through memory;
-// bit-identical to moe_act_kernel + quantize_act_kernel. A workgroup of 256 threads takes 32 blocks of 32: eight
-// neighbouring lanes read one block's gate and up values as whole lines and apply the activation (four values each);
-// the values meet in LDS and one lane per block forms the sums in the reference's order and the int8 codes.
-__global__ __launch_bounds__(256) void moe_act_quantize_kernel(const float* __restrict__ gp, const float* __restrict__ up, size_t stride,
-                                                              size_t rows, uint32_t inter, uint32_t kind, float param,
-                                                              int8_t* __restrict__ q, float* __restrict__ scales, int32_t* __restrict__ sums,
-                                                              float* __restrict__ fsums, float* __restrict__ hsums,
-                                                              int32_t* __restrict__ sums16) {
-    __shared__ float vals[32][36];  // rows padded: the finishing lanes read their blocks 36 words apart
-    const size_t bpr = inter / 32, nblocks = rows * bpr;
-    const size_t b0 = (size_t)blockIdx.x * 32;
-    {
-        const uint32_t lb = threadIdx.x >> 3, part = threadIdx.x & 7;
-        const size_t b = b0 + lb;
-        if (b < nblocks) {
-            const size_t r = b / bpr, j0 = (b % bpr) * 32 + 4 * part;
-            const float4 gg = *reinterpret_cast<const float4*>(gp + r * stride + j0);
-            const float4 uu = *reinterpret_cast<const float4*>(up + r * stride + j0);
-            const float gs[4] = {gg.x, gg.y, gg.z, gg.w}, us[4] = {uu.x, uu.y, uu.z, uu.w};
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                float g = gs[e], u = us[e], v;
-                if (kind == 1) {
-                    const float K2 = 2.0f * 0.7978846f;
-                    const float t = K2 * (g + 0.044715f * g * g * g);
-                    v = g / (1.0f + fast_exp(-t)) * u;
-                } else {
-                    if (kind == 2) {
-                        g = fminf(g, param);
-                        u = fminf(fmaxf(u, -param), param);
-                    }
-                    v = g / (1.0f + fast_exp(-g)) * u;
-                }
-                vals[lb][4 * part + e] = v;
-            }
-        }
-    }
-    __syncthreads();
-    const size_t b = b0 + threadIdx.x;
-    if (threadIdx.x >= 32 || b >= nblocks) return;
-    float v[32];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const float4 f = *reinterpret_cast<const float4*>(&vals[threadIdx.x][4 * i]);
-        v[4 * i] = f.x;
-        v[4 * i + 1] = f.y;
-        v[4 * i + 2] = f.z;
-        v[4 * i + 3] = f.w;
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; i++) amax = fmaxf(amax, fabsf(v[i]));
-    const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
-    float h0 = -0.0f, h1 = -0.0f, f = -0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; i++) h0 += v[i];
-#pragma unroll
-    for (int i = 16; i < 32; i++) h1 += v[i];
-#pragma unroll
-    for (int i = 0; i < 32; i++) f += v[i];
-    int s0 = 0, s1 = 0;
-    uint32_t packed[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        uint32_t wv = 0;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const float rr = roundf(v[4 * i + e] * inv);
-            const int iv = rr != rr ? 0 : (int)fminf(fmaxf(rr, -128.0f), 127.0f);
-            if (i < 4) s0 += iv; else s1 += iv;
-            wv |= ((uint32_t)iv & 0xFF) << (8 * e);
-        }
-        packed[i] = wv;
-    }
-    uint4* dst = reinterpret_cast<uint4*>(q + b * 32);
-    dst[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-    dst[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
-    scales[b] = amax / 127.0f;
-    sums[b] = s0 + s1;
-    fsums[b] = f;
-    hsums[2 * b] = h0;
-    hsums[2 * b + 1] = h1;
-    sums16[2 * b] = s0;
-    sums16[2 * b + 1] = s1;
+// bit-identical to moe_act_kernel + quantize_act_kernel: eight lanes to a block of 32, four values each.
+__global__ __launch_bounds__(256) void moe_act_quantize_kernel(const float* __restrict__ gp, const float* __restrict__ up, size_t stride, size_t nblocks,
+                                                              uint32_t inter, uint32_t kind, float param, QActOut o) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, b = i >> 3, bpr = inter / 32;
+    if (b >= nblocks) return;  // (uniform over a block's eight lanes)
+    const uint32_t part = (uint32_t)i & 7;
+    const size_t at = b / bpr * stride + (b % bpr) * 32 + 4 * part;
+    const float4 g = *reinterpret_cast<const float4*>(gp + at), u = *reinterpret_cast<const float4*>(up + at);
+    const float v[4] = {gated_act(g.x, u.x, kind, param), gated_act(g.y, u.y, kind, param), gated_act(g.z, u.z, kind, param), gated_act(g.w, u.w, kind, param)};
+    quantize_act_part(v, part, b, o);
 }
 
 hipError_t launch_moe_act_quantize(const float* g, const float* u, size_t stride, size_t rows, size_t inter, uint32_t kind, float param,
                                    const oxhip_qact& o, hipStream_t s) {
     const size_t blocks = rows * (inter / 32);
     if (!blocks) return hipSuccess;
-    moe_act_quantize_kernel<<<(unsigned)((blocks + 31) / 32), 256, 0, s>>>(g, u, stride, rows, (uint32_t)inter, kind, param, o.q, o.scales, o.sums,
-                                                                        o.fsums, o.hsums, o.sums16);
+    moe_act_quantize_kernel<<<(unsigned)((blocks + 31) / 32), 256, 0, s>>>(g, u, stride, blocks, (uint32_t)inter, kind, param, qact_out(o));
     return hipGetLastError();
 }
 

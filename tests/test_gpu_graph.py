@@ -179,6 +179,26 @@ def test_rmsnorm_quantize(be, oxref, n):
             assert np.array_equal(qb.q.cpu().numpy(), q) and np.array_equal(qb.scales.cpu().numpy().view(np.uint32), scales.view(np.uint32))
 
 
+@pytest.mark.parametrize("n", [32, 2080, 4096, 4128, 16384, 16416])  # one block; a ragged wave; one, four and more float4s a thread
+@pytest.mark.parametrize("off", [0, 1])                               # 16-byte rows, unaligned rows
+def test_norm_at_the_edges_of_its_thread_shapes(be, n, off):
+    """The row within f32 rounding of the f64 definition (two products, r, and half of the mean's three: 4.5 x 2^-24), its QAct quantize_act's, bit for bit."""
+    import torch
+    rng = np.random.default_rng(n + off)
+    rows, stride = 2, n + 4
+    buf, w = rng.normal(0, 3, off + rows * stride).astype(np.float32), rng.normal(1, 0.2, off + n).astype(np.float32)
+    xd, wd, out = dev(buf), dev(w), torch.zeros(off + rows * stride, device="cuda")
+    ok, qa = be.norm(xd[off:], n, rows, out=out[off:], w=wd[off:], x_stride=stride, out_stride=stride, want_q=True)
+    assert ok, be.last_error()
+    got = np.stack([out.cpu().numpy()[off + r * stride: off + r * stride + n] for r in range(rows)])
+    x = np.stack([buf[off + r * stride: off + r * stride + n] for r in range(rows)]).astype(np.float64)
+    want = x / np.sqrt((x * x).mean(axis=1, keepdims=True) + 1e-6) * w[off:].astype(np.float64)
+    assert (np.abs(got - want) <= 5 * 2.0 ** -24 * np.abs(want) + 1e-30).all()
+    ref = be.quantize_act(dev(got))
+    for f in ("q", "scales", "sums", "fsums", "hsums", "sums16"):
+        assert torch.equal(getattr(qa, f).view(torch.uint8), getattr(ref, f).view(torch.uint8)), f
+
+
 def test_norm_with_all_fields(be, oxref):
     """Op::Norm as the reference defines it (src/gpu_decode.rs:53-66, src/cuda_decode.cu:314-327): rows with strides
     inside a larger buffer, the `pre` factor, `out +=`, and views that do not start on 16-byte boundaries. Against the f64
