@@ -2,6 +2,8 @@
 // reference) over the kernels of this library.
 #include "backend.hpp"
 
+#include <system_error>
+#include <thread>
 #include <vector>
 
 namespace oxhip {
@@ -39,6 +41,41 @@ hipError_t launch_fill_zero(uint32_t* p, size_t n, hipStream_t s) {
 }  // namespace oxhip
 
 namespace {
+
+// Copies the pieces between host buffers, large ones by several threads: a thread moves some 10 GB/s between page-locked and
+// ordinary memory, a fifth of what the host link does. Every piece of work is done when it returns, also where no thread
+// could be started.
+struct HostCopy {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+constexpr size_t COPY_THREADS = 8, COPY_PER_THREAD = (size_t)2 << 20;
+constexpr size_t MAX_PINNED = (size_t)256 << 20;  // of page-locked staging a context keeps
+
+void host_copy(const HostCopy* pieces, size_t n) {
+    size_t total = 0;
+    for (size_t i = 0; i < n; i++) total += pieces[i].bytes;
+    auto range = [pieces, n](size_t lo, size_t hi) {  // bytes lo .. hi of the pieces in a row
+        size_t at = 0;
+        for (size_t i = 0; i < n && at < hi; at += pieces[i++].bytes) {
+            const size_t a = lo > at ? lo - at : 0, b = hi - at < pieces[i].bytes ? hi - at : pieces[i].bytes;
+            if (a < b) std::memcpy(static_cast<char*>(pieces[i].dst) + a, static_cast<const char*>(pieces[i].src) + a, b - a);
+        }
+    };
+    size_t parts = total / COPY_PER_THREAD;
+    parts = parts < 1 ? 1 : parts > COPY_THREADS ? COPY_THREADS : parts;
+    const size_t per = align_up((total + parts - 1) / parts, 4096);
+    std::thread th[COPY_THREADS];
+    size_t k = 1;  // part 0 is the caller's
+    try {
+        for (; k < parts; k++) th[k] = std::thread(range, k * per < total ? k * per : total, (k + 1) * per < total ? (k + 1) * per : total);
+    } catch (const std::system_error&) {  // no more threads: the caller does the rest
+    }
+    range(0, per < total ? per : total);
+    if (k < parts) range(k * per < total ? k * per : total, total);
+    for (size_t i = 1; i < k; i++) th[i].join();
+}
 
 struct Planes {
     size_t off[4] = {0, 0, 0, 0};
@@ -165,6 +202,7 @@ void oxhip_close(oxhip_ctx* c) {
     c->xq.release();
     c->y.release();
     c->gemm_ws.release();
+    c->pin.release();
     free_stream_scratch(c);
     (void)hipFree(c->dec.partial);
     (void)hipFree(c->dec.counters);
@@ -704,7 +742,12 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
         set_error("matmul: hipEventCreate failed");
         return done(0);
     }
-    // Everything is computed into device staging first; y is written only once all jobs ran.
+    // Everything is computed into device staging and comes to the host as a whole first; y is written only once all jobs ran.
+    // It comes through page-locked memory that the context keeps: an ordinary buffer made for each call costs its page faults
+    // and the runtime's own staging, 16.6 ms a call for 512 tokens through two 14336 x 4096 matrices (59 MB of results)
+    // against 2.0 ms, of which 1.0 are the link's. Calls with more results than MAX_PINNED take the ordinary buffer. (x is as
+    // fast from where it is: 0.34 ms for 8 MB either way.)
+    uint8_t* pin = c->pin.grow(y_total * 4, MAX_PINNED) ? static_cast<uint8_t*>(c->pin.p) : nullptr;
     (void)hipEventRecord(e0, s);
     if (hipMemcpyAsync(c->x.p, x, t * n_in * 4, hipMemcpyHostToDevice, s) != hipSuccess) {
         set_error("matmul: copy-in failed");
@@ -777,26 +820,17 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
         }
     }
     (void)hipEventRecord(e2, s);
-    if (hipStreamSynchronize(s) != hipSuccess) {
-        set_error("matmul: kernels failed");
-        return done(0);
-    }
-    off = 0;
-    std::vector<float> host(y_total);
-    if (hipMemcpyAsync(host.data(), yd, y_total * 4, hipMemcpyDeviceToHost, s) != hipSuccess) {
-        set_error("matmul: copy-out failed");
-        return done(0);
-    }
+    std::vector<float> host(pin ? 0 : y_total);
+    float* yh = pin ? reinterpret_cast<float*>(pin) : host.data();
+    const hipError_t out = hipMemcpyAsync(yh, yd, y_total * 4, hipMemcpyDeviceToHost, s);
     (void)hipEventRecord(e3, s);
-    if (hipStreamSynchronize(s) != hipSuccess) {
-        set_error("matmul: copy-out failed");
+    if (hipStreamSynchronize(s) != hipSuccess || out != hipSuccess) {
+        set_error("matmul: kernels or copy-out failed");
         return done(0);
     }
-    for (size_t j = 0; j < n_jobs; j++) {
-        size_t n = t * jobs[j].w->v.n_out;
-        std::memcpy(jobs[j].y, host.data() + off, n * 4);
-        off += n;
-    }
+    std::vector<HostCopy> outs(n_jobs);
+    for (size_t j = 0; j < n_jobs; j++) outs[j] = HostCopy{jobs[j].y, yh + offs[j], t * jobs[j].w->v.n_out * 4};
+    host_copy(outs.data(), n_jobs);
     float a = 0, b = 0, d = 0;
     (void)hipEventElapsedTime(&a, e0, e1);
     (void)hipEventElapsedTime(&b, e1, e2);

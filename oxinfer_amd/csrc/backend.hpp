@@ -12,6 +12,8 @@
 
 namespace oxhip {
 
+inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
+
 #define HIP_TRY(expr, what)                                                              \
     do {                                                                                 \
         hipError_t e__ = (expr);                                                         \
@@ -46,6 +48,32 @@ struct DevBuf {
     }
 };
 
+// Page-locked host staging of one context's host-pointer calls: kept from call to call, at most `max` bytes (a call that
+// needs more does without), given back with the context.
+struct PinnedBuf {
+    void* p = nullptr;
+    size_t cap = 0;
+    bool grow(size_t need, size_t max) {
+        if (need > max) return false;
+        if (cap >= need && p) return true;
+        release();
+        size_t want = align_up(need + need / 2, 4096);
+        if (want > max) want = max;
+        if (hipHostMalloc(&p, want, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();  // the caller goes on without staging
+            p = nullptr;
+            return false;
+        }
+        cap = want;
+        return true;
+    }
+    void release() {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        cap = 0;
+    }
+};
+
 // Scratch of the device-pointer entry points on one stream: the decode kernels' K-slice rows and counters, the
 // products of a gate / up pair (and of formats whose kernels only store) before their epilogue, the prefill GEMMs'
 // packed activations.
@@ -71,6 +99,7 @@ struct oxhip_ctx {
     hipStream_t stream = nullptr;
     std::mutex mu;  // serializes the host-pointer surface (staging is shared), as Mutex<Staging> does
     oxhip::DevBuf x, xq, y;
+    oxhip::PinnedBuf pin;   // results of oxhip_matmul on their way over the host link
     oxhip::DevBuf gemm_ws;  // packed activations of the prefill GEMMs
     oxhip::DecodeScratch dec;  // partial rows and counters of the decode kernels that split K across workgroups (host surface, on `stream`)
     std::mutex smu;            // guards per_stream
@@ -106,8 +135,6 @@ inline bool may_allocate(oxhip_ctx* c, hipStream_t s, const char* who) {
     set_error(std::string(who) + ": this call would have to allocate device memory while a plan records on its stream (run the chain once before recording)");
     return false;
 }
-
-inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 inline QActView view_of(const oxhip_qact& a) { return QActView{a.q, a.scales, a.sums, a.fsums, a.hsums, a.sums16}; }
 

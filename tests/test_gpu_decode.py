@@ -442,6 +442,21 @@ def test_host_matmul_matches_device_path_and_declines(be, oxref):
     assert "calls" in be.stats()
 
 
+@pytest.mark.parametrize("t,n_outs", [(1, (8,)), (33, (15889, 1, 16001)), (150, (7001, 24, 13999)), (2080, (32280,))])
+def test_host_matmul_results_come_whole(be, oxref, t, n_outs):
+    # results of one thread's copy, of a few threads with a piece's edge inside a job (4.2 and 12.6 MB), and of more than
+    # the page-locked staging holds (269 MB): the device path's bits, every one of them
+    n_in = 64
+    ws = [be.upload_gguf(Q8_0, oxref.random_blocks(Q8_0, n * n_in // 32, 71 + n)[0], n, n_in) for n in n_outs]
+    x = lcg_input(t, n_in, 72, oxref)
+    ys = [np.full((t, n), np.nan, np.float32) for n in n_outs]
+    assert be.matmul(x, t, n_in, list(zip(ws, ys))), be.last_error()
+    xd = dev(x)
+    for w, y in zip(ws, ys):
+        ref = be.gemm(w, xd, out_bf16=False) if t > 16 else be.decode(w, xa=be.quantize_act(xd))
+        assert np.array_equal(y.view(np.uint32), ref.cpu().numpy().view(np.uint32))
+
+
 def test_upload_declines(be):
     assert be.upload_gguf(10, np.zeros(84, np.uint8), 1, 256) is None  # Q2_K: no device kernels
     assert "no device kernels" in be.last_error()
