@@ -238,6 +238,33 @@ def test_moe_prefill_rows_do_not_depend_on_the_batch(be, oxref, mlx_experts):
         assert np.array_equal(ys.view(np.uint32), y[keep].view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt", ["mlx", "Q4_K", "Q8_0"])
+def test_moe_few_rows_per_expert(be, oxref, fmt):
+    """Passes below three routed rows per expert run in chunks of four rows with the activation in the gate / up launch:
+    on both sides of that line, one expert having every token (several chunks, a ragged last one), each token's row is
+    bit for bit what it is alone."""
+    from oxinfer_amd import synth
+    ne, h, inter, k = 16, 512, 256, 2
+    if fmt == "mlx":
+        descs = [[be.desc_mlx_q4(*synth.mlx_q4(n, c, s + e), 64, n, c) for e in range(ne)] for n, c, s in ((2 * inter, h, 2100), (h, inter, 2200))]
+    else:
+        kind, make = {"Q4_K": (Q4_K, synth.gguf_q4_k), "Q8_0": (Q8_0, synth.gguf_q8_0)}[fmt]
+        descs = [[be.desc_gguf(kind, make(n, c, s + e), n, c) for e in range(ne)] for n, c, s in ((2 * inter, h, 2100), (h, inter, 2200))]
+    dev = be.upload_moe(*descs, h, inter)
+    assert dev is not None, be.last_error()
+    for t in (5, 8, 9, 23, 24):  # 46 routed rows over 16 experts: the last pass under the line
+        x = synth.activations(t, h, 2300 + t)
+        _, idx, w = make_routes(oxref, t, ne, k, 2400 + t)
+        other = np.where(idx[:, 1] == 0, 1, idx[:, 1])
+        idx = np.ascontiguousarray(np.stack([np.zeros_like(other), other], 1))
+        y = np.zeros((t, h), np.float32)
+        assert be.moe(x, t, h, inter, idx, w, k, dev, y), be.last_error()
+        for i in range(t):
+            y1 = np.zeros((1, h), np.float32)
+            assert be.moe(x[i:i + 1], 1, h, inter, idx[i:i + 1], w[i:i + 1], k, dev, y1)
+            assert np.array_equal(y1[0].view(np.uint32), y[i].view(np.uint32)), (t, i)
+
+
 def test_moe_config_shapes(be, oxref):
     """The benchmark's expert shapes (h 2048, inter 768, top-8) over 16 experts: one token on the integer kernels against
     the oracle's decode path, 32 tokens (16 routed rows per expert: the bf16 form) against its grouped f32 path."""
