@@ -123,7 +123,7 @@ namespace {
 __host__ __device__ constexpr bool t4_geometry(int f) { return t4m_format(f) || f == FMT_NVFP4; }
 
 typedef uint32_t u32x4g __attribute__((ext_vector_type(4)));
-constexpr int WG_NT = 8;   // row tiles per workgroup (128 rows), or 7 where that fills more CUs (gemm_row_tiles)
+constexpr int WG_NT = 8;   // row tiles per workgroup (128 rows), or 7 where that fills more CUs (gemm_plan)
 constexpr int AR = 4;      // blocks of A fragments held ahead (a whole K-step: two starve the FP8 shapes, whose activations do not stay in L2)
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -170,8 +170,11 @@ __device__ __forceinline__ uint4 dequant_q4m(uint32_t w, float d, float c) {
 // FMT: FMT_Q4M (tile-packed MLX 4-bit), FMT_Q8_0 / FMT_Q8F / FMT_Q4_K / FMT_Q6_K (their tile records) or FMT_FP8 (e4m3 bytes with 128 x 128 block scales: the bytes are
 // exact in bf16, the block scale multiplies in f32 before the rounding, and a lane takes 32 consecutive row bytes
 // per step, which pack_a's mode 2 mirrors on the activation side).
+// (Eight waves of one token tile: two workgroups share a CU if they take at most 128 registers. Q4_K took 130: bounded it spills 12
+// bytes, 9472 columns x 5000 rows 42.7 -> 31.9 us at 128 tokens with the slices that allows. The 8-bit formats would spill 24 to 44
+// bytes, 33.6 -> 43.9 us on 14336 -> 4096: they keep a CU to a workgroup.)
 template <int FMT, bool OUT_BF16, int NV, int WAVES, int NT>
-__global__ __launch_bounds__(64 * WAVES) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
+__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && FMT != FMT_Q8_0 && FMT != FMT_Q8F ? 4 : 2) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
                                                         void* __restrict__ yv) {
     extern __shared__ uint4 bfrag[];  // [2][4 blocks][NT row tiles][64 lanes]
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -511,44 +514,59 @@ static void run_gemm_reduce(const float* partial, size_t n, uint32_t slices, voi
     }
 }
 
-// K slices for a launch: enough workgroups to cover the CUs while each keeps at least 8 steps.
 // Token tiles per wave and waves per workgroup: one tile and four waves when the launch has at most four tiles (64 tokens),
 // one tile and eight waves up to eight tiles (128 tokens), else two tiles and eight waves.
 static int gemm_nv(size_t mtiles) { return mtiles <= 8 ? 1 : 2; }
 static int gemm_waves(size_t mtiles) { return mtiles <= 4 ? 4 : 8; }  // (5 to 8 token tiles: eight waves of one tile each)
 
-static uint32_t k_slices_for(const WeightView& w, size_t mtiles, uint32_t nt) {
-    const uint32_t per_wg = gemm_waves(mtiles) * gemm_nv(mtiles);
-    const uint32_t wgs = ((row_tiles(w.n_out) + nt - 1) / nt) * (uint32_t)((mtiles + per_wg - 1) / per_wg);
-    const uint32_t steps = (w.n_in + 127) / 128;
-    uint32_t z = 1;
-    // (one token tile per wave: a K-step is short, two workgroups fit a CU, and what counts is requests in flight)
-    const uint32_t places = gemm_nv(mtiles) == 1 ? 512 : 256, min_steps = gemm_nv(mtiles) == 1 ? 4 : 8;
-    while (z < 8 && wgs * z * 2 <= places && steps / (z * 2) >= min_steps) {
-        // every slice must own a step: the kernel gives slice i the steps from i * ceil(steps / z) (33 steps in 8 slices
-        // of 5 would start the last one past the end)
-        const uint32_t z2 = z * 2, per = (steps + z2 - 1) / z2;
-        if ((z2 - 1) * per >= steps) break;
-        z = z2;
-    }
-    return z;
-}
-
-// Row tiles per workgroup: 8, or 7 where that costs less by this count: rounds of workgroups over the 256 CUs x row tiles
-// per workgroup x K-steps per slice (14336 rows x 512 tokens: one round of 256 workgroups of 112 rows instead of 224 of 128,
-// 63 -> 60 us; x 1024 tokens: two full rounds of 256 instead of 256 + 192).
-static int gemm_row_tiles(const WeightView& w, size_t mtiles) {
-    if (gemm_nv(mtiles) == 1) return WG_NT;
+// Row tiles per workgroup (8, or 7 with two token tiles per wave) and K slices of a launch: the pair that costs least, in units
+// of one K-step of an eight-tile workgroup (0.9 us with one token tile per wave, 1.2 to 1.5 us with two):
+//   rounds of workgroups over the 256 CUs x K-steps per slice. Two workgroups with one token tile per wave share a CU and
+//     take 1.55 steps' time for a step of each; a workgroup with two tiles per wave, or with eight waves of an 8-bit format, has
+//     its CU to itself. A slice of four steps costs 4.65 (the pipeline fills as often): 5120 -> 2816, MLX 4-bit, 100 tokens 20.2 us
+//     in 8 slices, 21.2 in 10.
+//   1 for every million partial sums written and read back, 1.9 for those past six million, and 2 for the launch that adds them
+//     (14336 -> 4096, MLX 4-bit, 420 tokens, 4 slices -> 8: 6.9 million more, as many steps, 63.6 -> 69.7 us).
+// Any number of slices counts, not only powers of two: 9472 columns, MLX 4-bit x 9000 rows are 71 workgroups of 74 steps, at
+// 24 tokens 36 us in 3 slices, 38.7 in 4 (284 workgroups), 27.9 in 7 (497); 4352 columns, Q6_K x 5001 rows at 24 tokens
+// 20.7 us in 4, 18.4 in 6 (240 workgroups), 20.6 in 8. With two tiles: 14336 -> 4096, MLX 4-bit, 1100 tokens (160 workgroups) 167.6 us
+// whole, 153.0 in 3 slices, 190.8 in 2; FP8 7168 x 18432 at 1100 tokens 397 us whole, 331 in 3. Four steps per slice at least
+// (7168 -> 1536, Q8_0, 200 tokens: 30.7 us at 14 steps, 24.4 at 7, 23.5 at 5).
+// Seven row tiles: 14336 rows x 512 tokens are one round of 256 workgroups of 112 rows instead of 224 of 128, 63 -> 60 us.
+struct GemmPlan {
+    uint32_t nt, slices;
+};
+static GemmPlan gemm_plan(const WeightView& w, size_t mtiles) {
+    const bool one = gemm_nv(mtiles) == 1;
     const uint32_t per_wg = gemm_waves(mtiles) * gemm_nv(mtiles), cols = (uint32_t)((mtiles + per_wg - 1) / per_wg);
     const uint32_t steps = (w.n_in + 127) / 128;
-    auto cost = [&](uint32_t nt) {
-        const uint32_t z = k_slices_for(w, mtiles, nt), wgs = ((row_tiles(w.n_out) + nt - 1) / nt) * cols * z;
-        return (uint64_t)((wgs + 255) / 256) * nt * ((steps + z - 1) / z);
-    };
-    return cost(7) < cost(8) ? 7 : WG_NT;
+    const bool alone = !one || (gemm_waves(mtiles) == 8 && q8_format(w.fmt));
+    const double millions = (double)mtiles * 16 * w.n_out * 1e-6;
+    auto sums = [](double m) { return m < 6 ? m : 6 + 1.9 * (m - 6); };
+    GemmPlan best{WG_NT, 1};
+    double least = 0;
+    for (uint32_t nt : {(uint32_t)WG_NT, 7u}) {
+        if (one && nt == 7) break;
+        const uint64_t wgs = (uint64_t)((row_tiles(w.n_out) + nt - 1) / nt) * cols;
+        for (uint32_t z = 1; z <= 16; z++) {
+            const uint32_t per = (steps + z - 1) / z;
+            if (z > 1 && steps / z < 4) break;
+            // every slice must own a step: the kernel gives slice i the steps from i * per (33 steps in 8 slices of 5 would
+            // start the last one past the end)
+            if ((z - 1) * per >= steps) continue;
+            const uint64_t rounds = (wgs * z + 255) / 256;
+            const double held = alone ? (double)rounds : (double)(rounds / 2) * 1.55 + (double)(rounds % 2);
+            const double cost = held * (per < 5 && z > 1 ? per + 0.65 : per) * nt / WG_NT + (z > 1 ? sums(z * millions) + 2 : 0);
+            if ((nt == WG_NT && z == 1) || cost < least) {
+                least = cost;
+                best = GemmPlan{nt, z};
+            }
+        }
+    }
+    return best;
 }
 
-uint32_t gemm_k_slices(const WeightView& w, size_t mtiles) { return k_slices_for(w, mtiles, (uint32_t)gemm_row_tiles(w, mtiles)); }
+uint32_t gemm_k_slices(const WeightView& w, size_t mtiles) { return gemm_plan(w, mtiles).slices; }
 
 namespace {
 template <int FMT, int NV, int NT, int WAVES = (NV == 1 ? 4 : 8)>
@@ -581,7 +599,7 @@ hipError_t run_gemm_bf16(const WeightView& w, const void* apk, size_t t, size_t 
                          hipStream_t s) {
     if (gemm_nv(mtiles) == 1 && gemm_waves(mtiles) == 4) return run_gemm_bf16_nv<FMT, 1, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
     if (gemm_nv(mtiles) == 1) return run_gemm_bf16_nv<FMT, 1, WG_NT, 8>(w, apk, t, mtiles, y, out_bf16, partial, s);
-    if (gemm_row_tiles(w, mtiles) == 7) return run_gemm_bf16_nv<FMT, 2, 7>(w, apk, t, mtiles, y, out_bf16, partial, s);
+    if (gemm_plan(w, mtiles).nt == 7) return run_gemm_bf16_nv<FMT, 2, 7>(w, apk, t, mtiles, y, out_bf16, partial, s);
     return run_gemm_bf16_nv<FMT, 2, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
 }
 }  // namespace

@@ -100,7 +100,7 @@ def gguf_raw(name, n_out, n_in, seed):
     return {"Q4_0": synth.gguf_q4_0, "Q8_0": synth.gguf_q8_0, "Q4_K": synth.gguf_q4_k, "Q5_K": synth.gguf_q5_k, "Q6_K": synth.gguf_q6_k, "MXFP4": synth.gguf_mxfp4}[name](n_out, n_in, seed)
 
 
-# 4352 columns = 34 steps of 128: K slices of 9 steps, so slices start inside a Q4_K super-block record; 1120 and 96
+# 4352 columns = 34 steps of 128: K slices of a few steps, so slices start inside a Q4_K super-block record; 1120 and 96
 # columns (Q8_0 only): a last step of one record, and of one block
 @pytest.mark.parametrize("name,n_out,n_in", [(k, n, c) for k in GGUF_KINDS for n, c in ((37, 1024), (256, 512), (200, 256), (130, 4352))]
                          + [("Q8_0", 100, 96), ("Q8_0", 64, 1120), ("Q4_0", 100, 96), ("Q4_0", 64, 1120), ("MXFP4", 64, 1120)])
@@ -125,6 +125,24 @@ def test_gemm_bf16_gguf_matches_oracle(be, oxref, name, n_out, n_in):
             assert row_err(y, exact_bf16) < 1e-3, (t, xd.dtype)
     yb = be.gemm(w, torch.from_numpy(x).cuda(), out_bf16=True).float().cpu().numpy()
     assert row_err(yb, ref) < 2e-2
+
+
+@pytest.mark.parametrize("n_out,n_in", [(130, 9472), (37, 8448), (650, 4864)])
+@pytest.mark.parametrize("name", ["Q4_K", "Q6_K", "Q8_0"])
+def test_gemm_bf16_odd_slice_counts(be, oxref, name, n_out, n_in):
+    """K slices in numbers that are no power of two, up to sixteen, ragged last ones (74, 66 and 38 steps of 128 columns), in
+    each form of the kernel (up to 64 tokens, up to 128, above): the product of the operands rounded to bf16, in 64 bits. 1e-3 as
+    above: the f32 sums of n_in exact products are off by about sqrt(n_in) 2^-24, 6e-6."""
+    import torch
+    from oxinfer_amd import synth
+    raw = gguf_raw(name, n_out, n_in, 23)
+    w = be.upload_gguf(GGUF_KINDS[name], raw, n_out, n_in)
+    assert w is not None, be.last_error()
+    wb = synth.bf16_round(oxref.dequantize_rows(GGUF_KINDS[name], raw, n_out, n_in)).astype(np.float64)
+    for t in (17, 64, 65, 128, 129, 260):
+        x = synth.activations(t, n_in, 400 + t, bf16=True)
+        y = be.gemm(w, torch.from_numpy(x).cuda()).cpu().numpy()
+        assert row_err(y, (x.astype(np.float64) @ wb.T).astype(np.float32)) < 1e-3, t
 
 
 def test_gemm_bf16_gguf_reference_fixtures(be, oxref):
