@@ -70,7 +70,7 @@ constexpr int pf_for() { return FMT == FMT_Q6_K ? 4 : 8; }  // Q6_K records are 
 // activations' own sums; the DUMP variant writes I16 / 16. The m * fs terms of a step's four blocks are one more
 // matrix instruction (f32, 16 x 16 x 4: rows = tokens, K = the four blocks), straight into the accumulators.
 // LDS metadata: xs [nbl][TPAD], and for the formats with mins or offsets fs [nbl][TPAD], over the workgroup's nbl
-// blocks from b0.
+// blocks from b0. Q6_K keeps one or two arrays for its second term (Q6PACK).
 // `at`: index of the lane's first token in its block's row
 __device__ __forceinline__ void load_xs(const float* lds, uint32_t at, float* xs) {
     const float4 x = *reinterpret_cast<const float4*>(lds + at);
@@ -169,7 +169,12 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     constexpr bool SWZ = NT >= 8;
     constexpr int NI = NT < 4 ? NT : 4;          // accumulator registers that hold live tokens
     constexpr bool MINS = k45_format(FMT) || FMT == FMT_Q4M;   // m * fs terms (Q4_0 has none)
-    constexpr int NARR = MINS ? 2 : 1;                         // metadata arrays: xs, and fs for the formats with m * fs terms
+    // Q6_K's second term: up to 8 tokens its two values per block (of either half) are staged ready made; at 16 (and for the
+    // integer sums) the halves' sums themselves are, as 16 bits each, and every use makes its value: a workgroup over 4096
+    // columns then stages 80 KB, not 88, and two fit a CU (14336 x 4096 at 16 tokens 23.4 us, two launches of eight 27.4; four
+    // such matrices together 89.7 and 109). At 8 tokens LDS is not what bounds it: 14.2 us ready made, 16.2 this way.
+    constexpr bool Q6PACK = FMT == FMT_Q6_K && (WIDE || DUMP);
+    constexpr int NARR = MINS || Q6PACK ? 2 : FMT == FMT_Q6_K ? 3 : 1;  // metadata arrays: xs, and fs for the formats with m * fs terms
     // the wave index and everything derived from it (tile, K range) live in scalar registers: branches on them are
     // scalar, and the load counters the compiler keeps stay exact across them
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -468,20 +473,17 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
             // Scales go per 16 columns, so an instruction's 16 operand slots are (sub-block sb, token t4): lane group kq
             // supplies sub-block kq's 16 activations of token t4 in the slots with sb = kq and zeros elsewhere, and lane
             // (kq, n) receives sub-block kq's exact sums for tokens 4 tg + i of row n. Eight tokens take two instructions.
-            // The codes centre on 32 and go in as the int8 values 4 (code - 32): nibble in bits 2..5, the high pair on top with
-            // its top bit flipped (one flip for the lane's four operand dwords), so that the sums need no correction by the
-            // activations' own: two LDS arrays less (at 16 tokens a workgroup over 4096 columns stages 72 KB instead of 90, and
-            // two fit a CU: q / k / v of 6144 x 4096 27.6 -> 15.4 us), and one read per instruction less.
-            const float d = f16_bits_to_f32((uint16_t)(sw[2] & 0xFFFF)) * 0.25f;
-            const uint32_t hq[2] = {st.h.x ^ 0xAAAAAAAAu, st.h.y ^ 0xAAAAAAAAu};
+            // The codes stay unsigned (0..63): a sub-block's value is xs * I - 32 * (xs * its activations' sum), the order of the
+            // reference's terms; see Q6PACK for the second one.
+            const float d = f16_bits_to_f32((uint16_t)(sw[2] & 0xFFFF));
+            const uint32_t hq[2] = {st.h.x, st.h.y};
             const bool on = (n >> 2) == kq;
-            const uint4* afr6 = reinterpret_cast<const uint4*>(afr);  // [64-column group][8 tokens][kq]
+            const uint4* afr6 = reinterpret_cast<const uint4*>(afr);  // [64-column group][8 tokens (16 in the 16-token form)][kq]
 #pragma unroll
             for (int h = 0; h < 2; h++) {  // the step's two groups of 64 columns
                 const uint32_t lo = h ? c.z : c.x, hi = h ? c.w : c.y, hh = hq[h];
-                constexpr uint32_t NIB = 0x3C3C3C3Cu, TOP = 0xC0C0C0C0u;
-                const v4i bw = {(int)(((lo << 2) & NIB) | ((hh << 6) & TOP)), (int)(((lo >> 2) & NIB) | ((hh << 4) & TOP)),
-                                (int)(((hi << 2) & NIB) | ((hh << 2) & TOP)), (int)(((hi >> 2) & NIB) | (hh & TOP))};
+                const v4i bw = {(int)((lo & 0x0F0F0F0Fu) | ((hh & 0x03030303u) << 4)), (int)(((lo >> 4) & 0x0F0F0F0Fu) | (((hh >> 2) & 0x03030303u) << 4)),
+                                (int)((hi & 0x0F0F0F0Fu) | (((hh >> 4) & 0x03030303u) << 4)), (int)(((hi >> 4) & 0x0F0F0F0Fu) | (((hh >> 6) & 0x03030303u) << 4))};
                 const float dsc = d * (float)(int)(int8_t)((sw[h] >> (8 * kq)) & 0xFF);
                 const uint32_t m64 = 2 * s + h, b = 2 * m64 + (kq >> 1);  // the lane's 32-block (its scale's) and its half
                 const uint32_t at = (min(b, nblk - 1) - B0) * TPAD;
@@ -494,14 +496,25 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                     const float4 xs = *reinterpret_cast<const float4*>(lds + at + 4 * tg);
                     const float xv[4] = {xs.x, xs.y, xs.z, xs.w};
                     const int U[4] = {D.x, D.y, D.z, D.w};
+                    int sq[4];
+                    float cv[4];
+                    if constexpr (Q6PACK) {
+                        const int2 sp = *reinterpret_cast<const int2*>(reinterpret_cast<const int16_t*>(lds + as) + 2 * at + TPAD * (kq & 1) + 4 * tg);
+                        sq[0] = (int16_t)sp.x, sq[1] = sp.x >> 16, sq[2] = (int16_t)sp.y, sq[3] = sp.y >> 16;
 #pragma unroll
-                    for (int i = 0; i < NI; i++) acc6[tg][i] = fmaf(dsc, xv[i] * (float)U[i], acc6[tg][i]);
+                        for (int i = 0; i < NI; i++) cv[i] = -32.0f * (xv[i] * (float)sq[i]);
+                    } else {
+                        const float4 cc = *reinterpret_cast<const float4*>(lds + (size_t)(1 + (kq & 1)) * as + at + 4 * tg);
+                        cv[0] = cc.x, cv[1] = cc.y, cv[2] = cc.z, cv[3] = cc.w;
+                    }
+#pragma unroll
+                    for (int i = 0; i < NI; i++) acc6[tg][i] = fmaf(dsc, fmaf(xv[i], (float)U[i], cv[i]), acc6[tg][i]);
                     if (DUMP) {
                         const uint32_t row = tile * 16 + n;
 #pragma unroll
                         for (int i = 0; i < 4; i++) {
                             if (4 * tg + i < (int)t && row < w.n_out && b < nblk)
-                                dump[((size_t)(4 * tg + i) * w.n_out + row) * (w.n_in / 16) + 4 * m64 + kq] = U[i] >> 2;
+                                dump[((size_t)(4 * tg + i) * w.n_out + row) * (w.n_in / 16) + 4 * m64 + kq] = U[i] - 32 * sq[i];
                         }
                     }
                 }
@@ -620,6 +633,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     // scales and sums: unit i = (q = i / nbl, block i % nbl of the slice) with q = TPAD group + token of the group
     struct MetaReg {
         float x, f;
+        int sq, sq2;  // Q6_K: the sums of the block's two halves
     };
     const uint32_t m_dq = nthr / nbl, m_dr = nthr - m_dq * nbl;
     auto meta_load = [&](uint32_t q, uint32_t b, MetaReg& r) {
@@ -628,11 +642,24 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
         const size_t src = (live ? src_row(tok) : 0) * nblk + B0 + (live ? b : 0);
         r.x = live ? xa.scales[src] : 0.0f;
         r.f = MINS && live ? xa.fsums[src] : 0.0f;
+        if (FMT == FMT_Q6_K) {
+            r.sq = live ? xa.sums16[2 * src] : 0;
+            r.sq2 = live ? xa.sums16[2 * src + 1] : 0;
+        }
     };
     auto meta_store = [&](uint32_t q, uint32_t b, const MetaReg& r) {
         const uint32_t at = (q / TPAD) * nm + b * TPAD + q % TPAD;
         lds[at] = r.x;
-        if (MINS) lds[(size_t)as + at] = r.f;
+        if (MINS) {
+            lds[(size_t)as + at] = r.f;
+        } else if constexpr (Q6PACK) {  // [block][half][token]
+            int16_t* sp = reinterpret_cast<int16_t*>(lds + as) + 2 * (at - q % TPAD) + q % TPAD;
+            sp[0] = (int16_t)r.sq;
+            sp[TPAD] = (int16_t)r.sq2;
+        } else if (FMT == FMT_Q6_K) {
+            lds[(size_t)as + at] = -32.0f * (r.x * (float)r.sq);
+            lds[(size_t)2 * as + at] = -32.0f * (r.x * (float)r.sq2);
+        }
     };
     uint4 sa[SA];
     MetaReg smr[SM];
@@ -1211,7 +1238,7 @@ size_t lds_bytes(int fmt, bool dump, uint32_t nsteps, int tpad, const Shape& sh,
     const uint32_t bps = q8_format(fmt) ? 2 : 4;
     const uint32_t fs = map.fs ? map.fs : 1;
     const uint32_t nbl = bps * fs * ((nsteps + sh.ks - 1) / sh.ks);  // blocks of the workgroup's slices
-    const uint32_t narr = k45_format(fmt) || fmt == FMT_Q4M ? 2 : 1;  // metadata arrays
+    const uint32_t narr = k45_format(fmt) || fmt == FMT_Q4M ? 2 : fmt == FMT_Q6_K ? (dump || tpad == 16 ? 2 : 3) : 1;  // metadata arrays
     const size_t meta = (size_t)narr * ng * nbl * tpad * 4, red = (size_t)sh.rt * fs * sh.kw * ng * tpad * 16 * 4;
     const size_t act = (size_t)ng * (nbl / 2) * (tpad == 16 ? 1024 : 512);
     const size_t with = act + meta > red ? act + meta : red;  // the partial sums reuse the activations' space

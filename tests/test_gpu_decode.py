@@ -148,6 +148,42 @@ def test_gguf_decode_matches_oracle(be, oxref, kind, t):
         assert np.array_equal(y1[0].view(np.uint32), y[c].view(np.uint32)), c
 
 
+def q6k_decode_by_hand(raw, n_out, qa, isums, waves):
+    """Rows of one Q6_K super-block as the decode kernels round them: a sub-block of 16 columns is d * sc times
+    fma(xs, sum of the unsigned codes, -32 * (xs * sum of the activations)), each f32 operation rounded once, added to what its place in
+    a step's group of four has (the groups of a wave one after the other, `waves` waves one after the other), then pairs of places."""
+    f32, wide = np.float32, np.longdouble  # (64 bits of mantissa hold the products exactly)
+    fma = lambda a, b, c: (a.astype(wide) * b.astype(wide) + c.astype(wide)).astype(f32)
+    blk = raw.reshape(n_out, 210)
+    d = blk[:, 208:210].copy().view(np.float16)[:, 0].astype(f32)
+    dsc = d[:, None] * blk[:, 192:208].copy().view(np.int8).astype(f32)              # [n_out, 16]
+    s16 = qa.sums16.cpu().numpy()                                                   # [t, 16]
+    xs = np.repeat(qa.scales.cpu().numpy(), 2, axis=1)                              # [t, 16]
+    codes = (isums + 32 * s16[:, None, :]).astype(f32)                              # [t, n_out, 16]
+    v = fma(np.broadcast_to(xs[:, None, :], codes.shape), codes, np.broadcast_to((f32(-32) * (xs * s16.astype(f32)))[:, None, :], codes.shape))
+    v, dsc = v.reshape(*v.shape[:2], waves, -1, 4), np.broadcast_to(dsc.reshape(1, n_out, waves, -1, 4), (v.shape[0], n_out, waves, 4 // waves, 4))
+    total = np.zeros(v.shape[:2], f32)
+    for w in range(waves):
+        acc = np.zeros(v.shape[:2] + (4,), f32)
+        for g in range(v.shape[3]):
+            acc = fma(dsc[:, :, w, g], v[:, :, w, g], acc)
+        total = total + ((acc[..., 0] + acc[..., 1]) + (acc[..., 2] + acc[..., 3]))
+    return total
+
+
+@pytest.mark.parametrize("t", [1, 2, 4, 8, 9, 16])
+def test_q6_k_rounds_as_the_terms_are_written(be, oxref, t):
+    """Every Q6_K product is rounded in one way, whatever the form of the kernel: with the unsigned codes' sum and the activations'
+    as separate terms. Bit for bit (one super-block, whose two steps go to one wave or to two)."""
+    n_out, n_in = 48, 256
+    raw, seed = oxref.random_blocks(Q6_K, n_out, 91)
+    w = be.upload_gguf(Q6_K, raw, n_out, n_in)
+    qa = be.quantize_act(dev(lcg_input(t, n_in, seed, oxref)))
+    got = be.decode(w, xa=qa).cpu().numpy().view(np.uint32)
+    isums = be.isums(w, qa, 16).cpu().numpy()
+    assert any(np.array_equal(got, q6k_decode_by_hand(raw, n_out, qa, isums, waves).view(np.uint32)) for waves in (1, 2))
+
+
 @pytest.mark.parametrize("kind", [Q4_0, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4])
 def test_gguf_decode_row_magnitudes(be, oxref, kind):
     n_out, n_in, t = 64, 4096, 4
