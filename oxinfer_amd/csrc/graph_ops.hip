@@ -77,7 +77,7 @@ hipError_t launch_router_logits(const float* x, const float* router, const float
 //   what `out` then holds goes, per block of 32, to the QAct (optional).
 // The reference sums the squares one after the other in f32 (src/kernels.rs:2109), which no parallel machine can
 // repeat bit for bit in useful time: here the squares are exact in f64 and summed in f64 (a fixed order), the mean and
-// eps added in f32 as the reference does, and r is the power rounded from 45 correct bits. The quantization of v is
+// eps added in f32 as the reference does, and r is the correctly rounded power. The quantization of v is
 // quantize_act's, bit for bit (the same code on the same values). VEC: rows of x, out and w start on 16-byte boundaries
 // (float4 access); otherwise every access is one float.
 // The kernel is one row's chain of latencies, so a row takes as many threads as it has float4s (up to 1024), its values and
@@ -148,9 +148,7 @@ __global__ __launch_bounds__(1024) void rmsnorm_quantize_kernel(const float* __r
 #pragma unroll
         for (int i = 0; i + d < 16; i += 2 * d) p[i] += p[i + d];
     const float m = (float)p[0] / (float)n + eps;
-    // m^(-1/2): the hardware's estimate (1 ulp) and one Newton step in f64
-    const double y0 = (double)__builtin_amdgcn_rsqf(m);
-    const float r = m > 1.2e-38f && m < 3.0e38f ? (float)(y0 * (1.5 - 0.5 * (double)m * (y0 * y0))) : (float)(1.0 / sqrt((double)m));
+    const float r = (float)(1.0 / sqrt((double)m));
     auto finish = [&](uint32_t i, const float* xs, const float* ws) {  // elements i .. i + 3 of the row
         float v[4];
 #pragma unroll

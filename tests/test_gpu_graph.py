@@ -199,6 +199,26 @@ def test_norm_at_the_edges_of_its_thread_shapes(be, n, off):
         assert torch.equal(getattr(qa, f).view(torch.uint8), getattr(ref, f).view(torch.uint8)), f
 
 
+def test_norm_rounds_the_reciprocal_root_correctly(be):
+    """r = m^(-1/2) is the f32 value nearest to the exact one also where that lies closest to the middle between two f32 values: the
+    4096 such means of [1, 4) (every exponent's r is one of theirs, times a power of two). A row's squares add up to 32 m in f32, and
+    a small power of two among its values shows r."""
+    m = np.arange(np.float32(1).view(np.uint32), np.float32(4).view(np.uint32), dtype=np.uint32).view(np.float32)
+    exact = 1.0 / np.sqrt(m.astype(np.float64))
+    ulps = exact / np.spacing(exact.astype(np.float32)).astype(np.float64)  # (both scalings are exact)
+    m = m[np.argsort(np.abs(ulps - np.floor(ulps) - 0.5))[:4096]]
+    want = (1.0 / np.sqrt(m.astype(np.float64))).astype(np.float32)
+    total = 32.0 * m.astype(np.float64)
+    x = np.zeros((len(m), 32), np.float32)
+    x[:, 0] = np.sqrt(total).astype(np.float32)
+    x[:, 0] = np.where(x[:, 0].astype(np.float64) ** 2 > total, np.nextafter(x[:, 0], np.float32(0)), x[:, 0])
+    x[:, 1] = np.sqrt(total - x[:, 0].astype(np.float64) ** 2)
+    x[:, 2] = 2.0 ** -20
+    assert np.array_equal((x.astype(np.float64) ** 2).sum(axis=1).astype(np.float32) / np.float32(32), m)
+    out, _ = be.rmsnorm_quantize(dev(x), None, 0.0)
+    assert np.array_equal(out.cpu().numpy()[:, 2].view(np.uint32), (want * np.float32(2.0 ** -20)).view(np.uint32))
+
+
 def test_norm_with_all_fields(be, oxref):
     """Op::Norm as the reference defines it (src/gpu_decode.rs:53-66, src/cuda_decode.cu:314-327): rows with strides
     inside a larger buffer, the `pre` factor, `out +=`, and views that do not start on 16-byte boundaries. Against the f64
