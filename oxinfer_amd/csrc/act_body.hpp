@@ -29,7 +29,8 @@ __device__ __forceinline__ int dpp_i32(int v) {
 // each, the eight lanes take about 120 and read whole lines (quantize_act of 4096 values 3.9 -> 3.6 us, RMSNorm and
 // quantization 5.4 -> 4.4 us, in a replayed chain, launch boundary included; on an idle stream 3.05 -> 2.35 us).
 __device__ __forceinline__ void quantize_act_part(const float* v, uint32_t part, size_t b, const QActOut& o) {
-    float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    // (from zero, as the reference: the maximum passes NaNs over, and a block of nothing else has the scale 0)
+    float amax = fmaxf(fmaxf(fmaxf(0.0f, fabsf(v[0])), fabsf(v[1])), fmaxf(fmaxf(0.0f, fabsf(v[2])), fabsf(v[3])));
     amax = fmaxf(amax, dpp_f32<0xB1>(amax));   // quad_perm [1,0,3,2]
     amax = fmaxf(amax, dpp_f32<0x4E>(amax));   // quad_perm [2,3,0,1]
     amax = fmaxf(amax, dpp_f32<0x141>(amax));  // row_half_mirror: the other four lanes

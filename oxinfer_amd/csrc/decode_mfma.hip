@@ -882,7 +882,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                 const bool live = tok < t && blk < bpr;  // uniform over the 32 lanes of a block
                 const float* src = aval + (size_t)gt * cols + bl * 32;
                 const float v = src[e];
-                float amax = fabsf(v);
+                float amax = fmaxf(0.0f, fabsf(v));  // (a block of NaNs alone has the scale 0)
 #pragma unroll
                 for (int off = 16; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
                 const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;

@@ -77,6 +77,25 @@ def test_quantize_act_bit_exact(be, oxref):
     assert np.array_equal(xa.sums16.cpu().numpy(), s16)
 
 
+def test_quantize_act_passes_nans_over(be, oxref):
+    """A block's maximum starts from zero and passes NaNs over (src/quant.rs:267-292): a block of NaNs alone has the scale 0 and
+    the codes 0, one with some NaNs the scale of its numbers. The f32 sums are NaN with them."""
+    t, n = 3, 256
+    x = lcg_input(t, n, 17, oxref)
+    x[0, :32] = np.nan
+    x[0, 64:95] = np.nan    # one number left, in the last lane's share
+    x[1, 32:48] = -np.nan   # one half
+    x[1, 100] = np.nan
+    x[2, :] = np.nan
+    xa = be.quantize_act(dev(x))
+    q, scales, sums, fsums, hsums = oxref.quantize_act(x, t, n)
+    assert not scales[0, 0] and not scales[2].any() and scales[0, 2] > 0
+    assert np.array_equal(xa.q.cpu().numpy(), q)
+    assert np.array_equal(xa.scales.cpu().numpy().view(np.uint32), scales.view(np.uint32))
+    assert np.array_equal(xa.sums.cpu().numpy(), sums)
+    assert np.array_equal(xa.fsums.cpu().numpy(), fsums, equal_nan=True) and np.array_equal(xa.hsums.cpu().numpy(), hsums, equal_nan=True)
+
+
 def test_quantize_act_batch_bit_exact(be, oxref):
     """Several matrices in one launch: every output equal to the reference's, as for one at a time."""
     from oxinfer_amd.hip import QAct

@@ -219,6 +219,18 @@ def test_norm_rounds_the_reciprocal_root_correctly(be):
     assert np.array_equal(out.cpu().numpy()[:, 2].view(np.uint32), (want * np.float32(2.0 ** -20)).view(np.uint32))
 
 
+def test_norm_of_a_nan_has_no_scale(be):
+    """One NaN makes the whole normed row NaN; its quantization is that of a row of NaNs (scale 0), the other rows' unchanged."""
+    x = np.random.default_rng(3).normal(0, 1, (3, 128)).astype(np.float32)
+    _, clean = be.rmsnorm_quantize(dev(x), None, 1e-6)
+    x[1, 77] = np.nan
+    out, qa = be.rmsnorm_quantize(dev(x), None, 1e-6)
+    assert np.isnan(out.cpu().numpy()[1]).all()
+    assert not qa.q[1].any() and not qa.scales[1].any() and not qa.sums[1].any() and not qa.sums16[1].any()
+    for i in (0, 2):
+        assert np.array_equal(qa.q[i].cpu().numpy(), clean.q[i].cpu().numpy()) and np.array_equal(qa.scales[i].cpu().numpy(), clean.scales[i].cpu().numpy())
+
+
 def test_norm_with_all_fields(be, oxref):
     """Op::Norm as the reference defines it (src/gpu_decode.rs:53-66, src/cuda_decode.cu:314-327): rows with strides
     inside a larger buffer, the `pre` factor, `out +=`, and views that do not start on 16-byte boundaries. Against the f64

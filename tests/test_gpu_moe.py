@@ -72,7 +72,7 @@ def test_route_top_k_other_sizes(be, oxref, ne, k):
         assert np.allclose(w[i], rw, rtol=1e-6, atol=0), i
 
 
-def moe_reference(oxref, kind, gate_up, down, h, inter, x, idx, w, y0):
+def moe_reference(oxref, kind, gate_up, down, h, inter, x, idx, w, y0, down_kind=None):
     """Each (token, route) pair on the oracle's decode kernels, combined in route order (what
     forward_batched computes row by row, src/moe.rs:438-617)."""
     y = y0.copy()
@@ -88,7 +88,7 @@ def moe_reference(oxref, kind, gate_up, down, h, inter, x, idx, w, y0):
             if kind == "mlx":
                 o = oxref.q4_decode(*down[e], 64, h, inter, a, 1)[0]
             else:
-                o = oxref.gguf_decode(kind, down[e], h, inter, a, 1)[0]
+                o = oxref.gguf_decode(down_kind or kind, down[e], h, inter, a, 1)[0]
             y[i] = y[i] + w[i, j] * o
     return y
 
@@ -263,6 +263,37 @@ def test_moe_few_rows_per_expert(be, oxref, fmt):
             y1 = np.zeros((1, h), np.float32)
             assert be.moe(x[i:i + 1], 1, h, inter, idx[i:i + 1], w[i:i + 1], k, dev, y1)
             assert np.array_equal(y1[0].view(np.uint32), y[i].view(np.uint32)), (t, i)
+
+
+@pytest.mark.parametrize("t", [1, 3, 11, 40])  # one token's three launches; the activation in the gate / up launch; above six tokens per expert not
+@pytest.mark.parametrize("split", [False, True])
+def test_moe_activation_of_nans_has_no_scale(be, oxref, t, split):
+    """Q4_K gate and up rows of a token with a NaN are NaN throughout; the activation's blocks then have the scale 0 (as the oracle
+    has it), which Q8_0 down matrices turn into zeros. The other tokens' rows are what they are without it."""
+    from oxinfer_amd import synth
+    ne, h, inter, k = 12, 256, 128, 2
+    gu = [synth.gguf_q4_k(2 * inter, h, 2500 + e) for e in range(ne)]
+    dn = [synth.gguf_q8_0(h, inter, 2600 + e) for e in range(ne)]
+    down = [be.desc_gguf(Q8_0, d, h, inter) for d in dn]
+    if split:
+        halves = [(np.ascontiguousarray(g.reshape(2, -1)[0]), np.ascontiguousarray(g.reshape(2, -1)[1])) for g in gu]
+        layer = be.upload_moe([be.desc_gguf(Q4_K, g, inter, h) for g, _ in halves], down, h, inter, up=[be.desc_gguf(Q4_K, u, inter, h) for _, u in halves])
+    else:
+        layer = be.upload_moe([be.desc_gguf(Q4_K, g, 2 * inter, h) for g in gu], down, h, inter)
+    assert layer is not None, be.last_error()
+    x = synth.activations(t, h, 2700 + t)
+    _, idx, w = make_routes(oxref, t, ne, k, 2800 + t)
+    from oxinfer_amd import hip
+    layer.set_mode(hip.MOE_INT8)
+    y, clean = np.zeros((t, h), np.float32), np.zeros((t, h), np.float32)
+    assert be.moe(x, t, h, inter, idx, w, k, layer, clean), be.last_error()
+    x[t // 2, 5] = np.nan
+    assert np.array_equal(moe_reference(oxref, Q4_K, gu, dn, h, inter, x[t // 2:t // 2 + 1], idx[t // 2:t // 2 + 1], w[t // 2:t // 2 + 1], np.zeros((1, h), np.float32), Q8_0),
+                          np.zeros((1, h)))
+    assert be.moe(x, t, h, inter, idx, w, k, layer, y), be.last_error()
+    assert not y[t // 2].any()
+    keep = np.arange(t) != t // 2
+    assert np.array_equal(y[keep].view(np.uint32), clean[keep].view(np.uint32))
 
 
 def test_moe_config_shapes(be, oxref):
