@@ -1,0 +1,63 @@
+"""The threaded copy of the host surface's results (csrc/host_copy.hpp), compiled for the CPU."""
+import os
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oxinfer_amd", "csrc")
+
+PROGRAM = r"""
+#include "host_copy.hpp"
+#include <cstdlib>
+#include <new>
+#include <vector>
+
+// allocations that still succeed (-1: all of them); std::thread allocates its state
+static long left = -1;
+void* operator new(size_t n) {
+    if (left == 0) throw std::bad_alloc();
+    if (left > 0) left--;
+    if (void* p = std::malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
+int main(int argc, char** argv) {
+    const long threads = std::atol(argv[1]);  // that may start
+    std::vector<size_t> sizes;
+    for (int i = 2; i < argc; i++) sizes.push_back((size_t)std::atoll(argv[i]));
+    std::vector<std::vector<unsigned char>> src, dst;
+    std::vector<oxhip::HostCopy> pieces;
+    for (size_t i = 0; i < sizes.size(); i++) {
+        src.emplace_back(sizes[i]);
+        for (size_t k = 0; k < sizes[i]; k++) src[i][k] = (unsigned char)(k * 31 + (k >> 12) + i);
+        dst.emplace_back(sizes[i] + 1, 0xEE);
+    }
+    for (size_t i = 0; i < sizes.size(); i++) pieces.push_back({dst[i].data(), src[i].data(), sizes[i]});
+    left = threads;
+    oxhip::host_copy(pieces.data(), pieces.size());
+    left = -1;
+    for (size_t i = 0; i < sizes.size(); i++)
+        if (std::memcmp(dst[i].data(), src[i].data(), sizes[i]) || dst[i][sizes[i]] != 0xEE) return 1;
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def build(tmp_path_factory):
+    def build(program):
+        d = tmp_path_factory.mktemp("host_copy")
+        (d / "main.cpp").write_text(program)
+        subprocess.run(["g++", "-std=c++17", "-O1", "-pthread", "-I", CSRC, str(d / "main.cpp"), "-o", str(d / "main")], check=True)
+        return str(d / "main")
+    return build
+
+
+def test_every_byte_arrives_whatever_threads_start(build):
+    exe = build(PROGRAM)
+    for sizes in ((0,), (1,), (4096, 0, 5), (3 << 20, 1, (5 << 20) + 77), (40 << 20,), tuple([1000003] * 20)):
+        for threads in (-1, 0, 1, 3):  # all, none for want of memory, one, three
+            r = subprocess.run([exe, str(threads), *map(str, sizes)], timeout=60)
+            assert r.returncode == 0, (sizes, threads, r.returncode)
