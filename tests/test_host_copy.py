@@ -61,3 +61,34 @@ def test_every_byte_arrives_whatever_threads_start(build):
         for threads in (-1, 0, 1, 3):  # all, none for want of memory, one, three
             r = subprocess.run([exe, str(threads), *map(str, sizes)], timeout=60)
             assert r.returncode == 0, (sizes, threads, r.returncode)
+
+
+OVERLAP = r"""
+#include "host_copy.hpp"
+#include <algorithm>
+#include <vector>
+
+int main() {
+    // two results to one place, and one that begins in the middle of another (both ways round in address order): the later job's stay
+    const size_t n = 24 << 20;
+    std::vector<unsigned char> a(n, 1), b(n, 2), y(2 * n);
+    for (int k = 0; k < 3; k++) {
+        std::fill(y.begin(), y.end(), 0);
+        unsigned char *first = y.data() + (k == 2 ? n / 2 : 0), *second = y.data() + (k == 1 ? n / 2 : 0);
+        const oxhip::HostCopy pieces[] = {{first, a.data(), n}, {second, b.data(), n}};
+        oxhip::host_copy(pieces, 2);
+        for (size_t i = 0; i < 2 * n; i++) {
+            const unsigned char* p = y.data() + i;
+            const unsigned char want = p >= second && p < second + n ? 2 : p >= first && p < first + n ? 1 : 0;
+            if (*p != want) return 1;
+        }
+    }
+    return 0;
+}
+"""
+
+
+def test_overlapping_results_keep_the_order_of_the_jobs(build):
+    exe = build(OVERLAP)
+    for _ in range(3):
+        assert subprocess.run([exe], timeout=60).returncode == 0
