@@ -121,13 +121,7 @@ int moe_pass(oxhip_ctx* c, oxhip_moe* m, const float* x, size_t t, const uint32_
     uint32_t max_rows = (uint32_t)(t < 8 ? t : 8);
     const size_t avg = pairs / m->n_exp;
     if (avg >= 6 && mfma_format(m->gate_up[0])) max_rows = avg >= 20 ? 32 : 16;
-    // Fewer than three routed rows per expert: chunks of four rows. Such an expert rarely has a fifth row, and the four-row
-    // form stages half the activations and multiplies two operand halves less per record. 128 experts of 2048 / 768, eight
-    // a token, chunks of eight -> four rows: MLX 4-bit 81.3 -> 66.1 us at 24 tokens, Q4_K 88.2 -> 84.5 and Q8_0 119.4 ->
-    // 117.3 us at 40 tokens (2.5 rows); from three rows on the second pass over an expert's weights costs more than that
-    // (32 experts of 2560 / 1024, four a token, 24 tokens: Q4_K 48.5 -> 50.6, Q8_0 61.7 -> 63.4 us).
-    const bool sparse = pairs < 3 * m->n_exp;
-    if (sparse && max_rows > 4) max_rows = 4;
+    const bool sparse = pairs < 3 * m->n_exp;  // fewer than three routed rows per expert
 #ifdef OXHIP_TUNING  // tuning builds only: rows per chunk in OXHIP_MOE_CHUNK
     if (const char* e = getenv("OXHIP_MOE_CHUNK")) {
         const int v = atoi(e);
@@ -149,6 +143,7 @@ int moe_pass(oxhip_ctx* c, oxhip_moe* m, const float* x, size_t t, const uint32_
                    (fused || decode_grouped_fits(m->up[0]->v, rows));
         };
         while (max_rows > 8 && !fits(max_rows)) max_rows /= 2;
+        if (sparse && max_rows > 4 && !fits(max_rows)) max_rows = 4;  // (rows of some 80 thousand columns: the staged scales of four rows fit)
         if (!fits(max_rows)) {
             set_error("moe: rows of these experts are too long for the grouped kernel's staging");
             return 0;
@@ -199,8 +194,8 @@ int moe_pass(oxhip_ctx* c, oxhip_moe* m, const float* x, size_t t, const uint32_
         // are the launch's own output stage; the down launch then also combines (the last workgroup of a row group to
         // finish adds the routed rows in route order): three launches for a decode-sized pass
         // (decode-sized passes only: a large pass has enough rows to fill launches of their own, and its combination is
-        // too much work for the one workgroup per row group that would do it; the activation alone pays as long as the
-        // chunks are short, see above: MLX 4-bit, 128 experts, 24 tokens 66.1 -> 64.2 us, 32 experts 46.4 -> 44.3 us)
+        // too much work for the one workgroup per row group that would do it; the activation alone pays as long as experts have few
+        // rows: MLX 4-bit at 24 tokens, 128 experts 66.1 -> 64.2 us, 32 experts 46.4 -> 44.3 us)
         const bool small = t <= 8;
         const bool glu_fused = (small || sparse) && fused && decode_grouped_glu_ok(m->gate_up[0]->v, inter);
         const bool comb_fused = small && row_tiles((uint32_t)h) <= COMB_GROUPS;

@@ -581,8 +581,9 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     // only arrive behind them and no step could start before the whole ring had landed.
     constexpr int PF = pf_for<FMT, NT>();
     // 16-byte activation chunks / scale entries a thread holds in registers (more go later): every one is a request of
-    // every wave whether or not it has a unit to fetch, so few tokens get few
-    constexpr int SA = NG > 1 ? 8 : NT == 1 ? 2 : NT <= 4 ? 4 : 8, SM = NT <= 4 && NG == 1 ? 2 : 4;
+    // every wave whether or not it has a unit to fetch, so few tokens get few (grouped MLX 4-bit launches take four for eight
+    // rows too, all there is up to 2048 columns, and keep a fifth wave per SIMD: 104 -> 88 registers)
+    constexpr int SA = NG > 1 ? 8 : NT == 1 ? 2 : NT <= 4 || (GROUPED && FMT == FMT_Q4M) ? 4 : 8, SM = NT <= 4 && NG == 1 ? 2 : 4;
     const uint32_t nb = min(nblk, B0 + nbl) - min(nblk, B0);  // real blocks of the slice
     // slot (m, lane) of the operand array: lane = 16 kq + 8 half + token holds the 8 values of block 2 m + half that
     // the weights' lane group kq pairs with (Q4: positions 4 kq.. and 16 + 4 kq..; else 8 kq..). A thread moves 16
@@ -1035,15 +1036,30 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
 
 // Dynamic LDS is declared 16-byte aligned whatever static LDS a kernel also holds: the 8- and 16-byte LDS reads are split
 // into dwords (and the kernel runs two to three times longer) when the array starts at an odd dword.
-// (Grouped launches keep to 8 waves, which leaves them 256 registers for the accumulators of their token groups.)
+// (Grouped launches keep to 8 waves, which leaves them 256 registers for the accumulators of their token groups; with chunks of
+// five to eight rows they are bounded to four waves per SIMD, MLX 4-bit to five: unbounded that kernel took 139 registers and
+// spilled 36 scalar ones.)
 // (Q6_K: bounded at 8 waves like its shared-launch kernel, see decode_batch_kernel)
+// Such a launch has chunks of any length up to its own, and those of up to four rows, the most of them where an expert has few
+// routed rows, run the four-row body. 128 MLX 4-bit experts of 2048 / 768, eight a token, every chunk in the eight-row body of
+// before -> this: 24 tokens routed at random 85.5 -> 64.1 us, 47 tokens all to the same eight experts 53.8 -> 42.0 us. (Chunks of
+// four rows throughout make two passes over the weights of an expert with more: 63.0 and 55.1 us.)
 template <int FMT, int NT, bool DUMP, bool GROUPED, bool ALDS, int NG>
-__global__ __launch_bounds__(GROUPED || FMT == FMT_Q6_K || NT == 16 ? 512 : 1024) void decode_mfma_kernel(WeightView w, QActView xa, uint32_t t, uint32_t rt,
+__global__ __launch_bounds__(GROUPED || FMT == FMT_Q6_K || NT == 16 ? 512 : 1024, GROUPED && NG == 1 && NT == 8 ? (FMT == FMT_Q4M && ALDS ? 5 : 4) : 1) void decode_mfma_kernel(WeightView w, QActView xa, uint32_t t, uint32_t rt,
                                                                            uint32_t kw, float* __restrict__ y,
                                                                            int32_t* __restrict__ dump, GroupView grp, uint32_t ksplit,
                                                                            float* __restrict__ partial,
                                                                            uint32_t* __restrict__ counters, Epi epi) {
     extern __shared__ __align__(16) float lds_dyn[];
+    if constexpr (GROUPED && NT == 8 && NG == 1) {
+        if (!grp.direct) {  // uniform over the workgroup
+            if (blockIdx.y >= (uint32_t)*grp.nchunks) return;
+            if (grp.chunks[blockIdx.y].z <= 4) {
+                decode_body<FMT, 4, DUMP, GROUPED, ALDS, NG>(w, xa, t, rt, kw, y, dump, grp, ksplit, partial, counters, blockIdx.x, blockIdx.y, blockDim.x, lds_dyn, epi);
+                return;
+            }
+        }
+    }
     decode_body<FMT, NT, DUMP, GROUPED, ALDS, NG>(w, xa, t, rt, kw, y, dump, grp, ksplit, partial, counters, blockIdx.x, blockIdx.y,
                                                   blockDim.x, lds_dyn, epi);
 }

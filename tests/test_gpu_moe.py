@@ -238,17 +238,17 @@ def test_moe_prefill_rows_do_not_depend_on_the_batch(be, oxref, mlx_experts):
         assert np.array_equal(ys.view(np.uint32), y[keep].view(np.uint32))
 
 
-@pytest.mark.parametrize("fmt", ["mlx", "Q4_K", "Q8_0"])
+@pytest.mark.parametrize("fmt", ["mlx", "Q4_K", "Q8_0", "Q4_0", "MXFP4"])
 def test_moe_few_rows_per_expert(be, oxref, fmt):
-    """Passes below three routed rows per expert run in chunks of four rows with the activation in the gate / up launch:
-    on both sides of that line, one expert having every token (several chunks, a ragged last one), each token's row is
-    bit for bit what it is alone."""
+    """A launch's chunks of up to four rows run in another form than its longer ones, and below three routed rows per expert the
+    activation is in the gate / up launch: on both sides of these lines, one expert having every token (chunks of eight, a ragged
+    last one), each token's row is bit for bit what it is alone."""
     from oxinfer_amd import synth
     ne, h, inter, k = 16, 512, 256, 2
     if fmt == "mlx":
         descs = [[be.desc_mlx_q4(*synth.mlx_q4(n, c, s + e), 64, n, c) for e in range(ne)] for n, c, s in ((2 * inter, h, 2100), (h, inter, 2200))]
     else:
-        kind, make = {"Q4_K": (Q4_K, synth.gguf_q4_k), "Q8_0": (Q8_0, synth.gguf_q8_0)}[fmt]
+        kind, make = {"Q4_K": (Q4_K, synth.gguf_q4_k), "Q8_0": (Q8_0, synth.gguf_q8_0), "Q4_0": (Q4_0, synth.gguf_q4_0), "MXFP4": (MXFP4, synth.gguf_mxfp4)}[fmt]
         descs = [[be.desc_gguf(kind, make(n, c, s + e), n, c) for e in range(ne)] for n, c, s in ((2 * inter, h, 2100), (h, inter, 2200))]
     dev = be.upload_moe(*descs, h, inter)
     assert dev is not None, be.last_error()
@@ -263,6 +263,22 @@ def test_moe_few_rows_per_expert(be, oxref, fmt):
             y1 = np.zeros((1, h), np.float32)
             assert be.moe(x[i:i + 1], 1, h, inter, idx[i:i + 1], w[i:i + 1], k, dev, y1)
             assert np.array_equal(y1[0].view(np.uint32), y[i].view(np.uint32)), (t, i)
+
+
+def test_moe_rows_too_long_for_eight_at_once(be, oxref):
+    """Rows of 90112 columns: the staged scales of eight routed rows are more than LDS holds, those of four are not."""
+    from oxinfer_amd import synth
+    ne, h, inter = 2, 90112, 32
+    layer = be.upload_moe([be.desc_mlx_q4(*synth.mlx_q4(2 * inter, h, 2900 + e), 64, 2 * inter, h) for e in range(ne)],
+                          [be.desc_gguf(Q8_0, synth.gguf_q8_0(h, inter, 2910 + e), h, inter) for e in range(ne)], h, inter)
+    assert layer is not None, be.last_error()
+    x, idx, w = synth.activations(5, h, 2920), np.array([[0], [0], [0], [1], [0]], np.uint32), np.ones((5, 1), np.float32)
+    y = np.zeros((5, h), np.float32)
+    assert be.moe(x, 5, h, inter, idx, w, 1, layer, y), be.last_error()
+    for i in range(5):
+        y1 = np.zeros((1, h), np.float32)
+        assert be.moe(x[i:i + 1], 1, h, inter, idx[i:i + 1], w[i:i + 1], 1, layer, y1), be.last_error()
+        assert np.array_equal(y1[0].view(np.uint32), y[i].view(np.uint32)), i
 
 
 @pytest.mark.parametrize("t", [1, 3, 11, 40])  # one token's three launches; the activation in the gate / up launch; above six tokens per expert not
