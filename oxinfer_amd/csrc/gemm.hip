@@ -532,7 +532,9 @@ static int gemm_waves(size_t mtiles) { return mtiles <= 4 ? 4 : 8; }  // (5 to 8
 // 20.7 us in 4, 18.4 in 6 (240 workgroups), 20.6 in 8. With two tiles: 14336 -> 4096, MLX 4-bit, 1100 tokens (160 workgroups) 167.6 us
 // whole, 153.0 in 3 slices, 190.8 in 2; FP8 7168 x 18432 at 1100 tokens 397 us whole, 331 in 3. Four steps per slice at least
 // (7168 -> 1536, Q8_0, 200 tokens: 30.7 us at 14 steps, 24.4 at 7, 23.5 at 5).
-// Seven row tiles: 14336 rows x 512 tokens are one round of 256 workgroups of 112 rows instead of 224 of 128, 63 -> 60 us.
+// Seven row tiles: 14336 rows x 512 tokens are one round of 256 workgroups of 112 rows instead of 224 of 128, 63 -> 60 us: a step of
+// theirs costs 0.94 of one of eight, not 7/8 (counted as 7/8, 8192 rows x 512 tokens of 4096 columns went from 256 workgroups in two
+// slices to 148 of seven tiles whole, Q4_K 46.5 -> 53.2 us; 7895 x 5888 at 224 tokens 37.1 -> 39.6).
 struct GemmPlan {
     uint32_t nt, slices;
 };
@@ -558,7 +560,7 @@ static GemmPlan gemm_plan(const WeightView& w, size_t mtiles) {
             if ((z - 1) * per >= steps) continue;
             const uint64_t rounds = (wgs * z + 255) / 256;
             const double held = alone ? (double)rounds : (double)(rounds / 2) * 1.55 + (double)(rounds % 2);
-            const double cost = held * (per < 5 && z > 1 ? per + 0.65 : per) * nt / WG_NT + (z > 1 ? sums(z * millions) + 2 : 0);
+            const double cost = held * (per < 5 && z > 1 ? per + 0.65 : per) * (nt == 7 ? 0.94 : 1.0) + (z > 1 ? sums(z * millions) + 2 : 0);
             if ((nt == WG_NT && z == 1) || cost < least) {
                 least = cost;
                 best = GemmPlan{nt, z};
