@@ -127,7 +127,7 @@ struct Step<FMT_Q6_K> {
     uint32_t a[1];
 };
 
-// FMT: FMT_Q8_0 / FMT_Q8F (the same codes with f32 scales) / FMT_Q4_K / FMT_Q6_K / FMT_Q4M. NT: tokens handled (1, 2, 4 or 8). DUMP: also write the exact
+// FMT: FMT_Q8_0 / FMT_Q8F (the same codes with f32 scales) / FMT_Q4_K / FMT_Q6_K / FMT_Q4M. NT: tokens handled (1, 2, 4, 8 or 16). DUMP: also write the exact
 // integer block sums to `dump` ([t][n_out][n_in/32]) for parity checks.
 // GROUPED: blockIdx.y walks the chunks of a grouped launch (MoE experts over their routed tokens): chunk c is
 // {expert, first row, rows (<= 8 NG)}; the weights are expert's, activation row i of the chunk is row
@@ -374,9 +374,9 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
 #pragma unroll
         for (int i = 0; i < 4; i++) sum[i] = fmaf(d, xs[i] * (float)I[i], sum[i]);
     };
-    // The m * fs terms of the step's four blocks (blocks b4 .. b4 + 3): rows = tokens (8 .. 15: none), K = the blocks;
+    // The m * fs terms of the step's four blocks (blocks b4 .. b4 + 3): rows = tokens (past TPAD: none), K = the blocks;
     // this lane supplies fs of (token n, block b4 + kq) and `mk`, row n's m of block b4 + kq. D[4 kq + i][n]: the lane
-    // groups 0 and 1 receive the tokens their accumulators hold, the others zeros.
+    // groups 0 and 1 receive the tokens their accumulators hold, the others zeros; in the 16-token form all four hold tokens.
     auto mins = [&](uint32_t b4, float mk) {
         if constexpr (MINS) {
             // (a block past the row lies inside the slice's arrays all the same, staged as zero)
@@ -586,7 +586,8 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     constexpr int SA = NG > 1 ? 8 : NT == 1 ? 2 : NT <= 4 || (GROUPED && FMT == FMT_Q4M) ? 4 : 8, SM = NT <= 4 && NG == 1 ? 2 : 4;
     const uint32_t nb = min(nblk, B0 + nbl) - min(nblk, B0);  // real blocks of the slice
     // slot (m, lane) of the operand array: lane = 16 kq + 8 half + token holds the 8 values of block 2 m + half that
-    // the weights' lane group kq pairs with (Q4: positions 4 kq.. and 16 + 4 kq..; else 8 kq..). A thread moves 16
+    // the weights' lane group kq pairs with (Q4: positions 4 kq.. and 16 + 4 kq..; else 8 kq..); in the 16-token form slot
+    // (b, 16 kq + token) holds those of block b. A thread moves 16
     // (Q4: 32) consecutive bytes of one token's row, so the global reads are whole lines. Absent tokens and a padding
     // block keep whatever LDS holds: those products meet zero weights or are dropped.
     constexpr int AU = t4m_format(FMT) ? 2 : 1;  // 16-byte loads per unit of staging work
@@ -1600,9 +1601,9 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
             }
         }
 #endif
+        const bool wide = items_of[0]->t > 8;  // (all of them, or none; the 16-token form has the plain mapping only)
         uint64_t fat_wgs = 0;
-        for (uint32_t j = 0; j < a.njobs; j++) fat_wgs += place_job(*items_of[j], true, fat_steps).wgs;
-        const bool wide = items_of[0]->t > 8;  // (all of them, or none)
+        for (uint32_t j = 0; !wide && j < a.njobs; j++) fat_wgs += place_job(*items_of[j], true, fat_steps).wgs;
         const bool fat = !wide && fat_wgs >= fat_min;
         for (uint32_t j = 0; j < a.njobs; j++) {
             const DecodeBatchItem& it = *items_of[order[j]];

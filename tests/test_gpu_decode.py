@@ -685,8 +685,11 @@ def test_decode_batch_events(be, oxref):
             assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
 
 
-@pytest.mark.parametrize("kind", [Q4_0, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4, "q8", "mlx"])
-@pytest.mark.parametrize("n_out,n_in", [(37, 768), (272, 4096), (48, 14336)])  # ragged rows; two workgroups a CU; K slices
+# ragged rows; two workgroups a CU; K slices; rows that end inside a step of 64 or 128 columns; a pair whose workgroup has 16 waves,
+# which goes eight tokens at a time
+@pytest.mark.parametrize("kind,n_out,n_in", [(k, *s) for k in (Q4_0, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4, "q8", "mlx") for s in ((37, 768), (272, 4096), (48, 14336))]
+                         + [(k, *s) for k in (Q4_0, Q8_0, MXFP4, "q8") for s in ((33, 96), (40, 1120))] + [("mlx", 33, 64), ("mlx", 40, 320), ("mlx", 24, 4160)]
+                         + [(k, 64, 6144) for k in (Q8_0, "q8")])
 def test_sixteen_token_form_keeps_the_bits(be, oxref, kind, n_out, n_in):
     """Nine to sixteen tokens go through the 16-token form in one pass over the weights: every row, stored, added, of a gate /
     up pair and in a shared launch with jobs of fewer tokens, has the bits of that token's row computed alone (which the

@@ -81,6 +81,24 @@ def test_no_alloc_call_leaves_device_memory_alone(be, oxref):
         assert free1 == free0, (free0, free1)
 
 
+def test_no_alloc_goes_eight_at_a_time_where_the_scratch_holds_no_more(be, oxref):
+    """Rows of 32768 columns in 8 K slices: the static scratch (1 Mi floats) holds the partial rows of nine tokens of 12000 rows, which
+    go in one pass, but not those of sixteen, which go eight at a time. Each row as that token's alone."""
+    import torch
+    n_out, n_in, part = 12000, 32768, 250
+    raw, seed = oxref.random_blocks(Q4_K, part * n_in // 256, 4300)
+    w = be.upload_gguf(Q4_K, np.tile(raw, n_out // part), n_out, n_in)
+    assert w is not None, be.last_error()
+    v, _ = oxref.lcg_stream(seed, 16 * n_in)
+    x = dev(((v % 2001).astype(np.float32) / np.float32(1000.0) - np.float32(1.0)).reshape(16, n_in))
+    want = torch.cat([be.decode(w, xa=be.quantize_act(x[i:i + 1].contiguous())) for i in range(16)])
+    qa = be.quantize_act(x)
+    for t in (8, 9, 16):
+        y = torch.full((t, n_out), float("nan"), dtype=torch.float32, device="cuda")
+        assert be.decode_noalloc(w, qa, t=t, y=y) is not None, be.last_error()
+        assert torch.equal(y.view(torch.int32), want[:t].view(torch.int32)), t
+
+
 def test_no_alloc_rejects_what_the_scratch_cannot_hold(be):
     n_out, n_in = 16640, 32768  # 8 K slices x 8 x 16640 floats of partial rows > 4 MiB
     raw = np.zeros(n_out * (n_in // 256) * 144, np.uint8)
