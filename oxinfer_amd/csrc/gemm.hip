@@ -170,11 +170,11 @@ __device__ __forceinline__ uint4 dequant_q4m(uint32_t w, float d, float c) {
 // FMT: FMT_Q4M (tile-packed MLX 4-bit), FMT_Q8_0 / FMT_Q8F / FMT_Q4_K / FMT_Q6_K (their tile records) or FMT_FP8 (e4m3 bytes with 128 x 128 block scales: the bytes are
 // exact in bf16, the block scale multiplies in f32 before the rounding, and a lane takes 32 consecutive row bytes
 // per step, which pack_a's mode 2 mirrors on the activation side).
-// (Eight waves of one token tile: two workgroups share a CU if they take at most 128 registers. Q4_K took 130: bounded it spills 12
-// bytes, 9472 columns x 5000 rows 42.7 -> 31.9 us at 128 tokens with the slices that allows. The 8-bit formats would spill 24 to 44
-// bytes, 33.6 -> 43.9 us on 14336 -> 4096: they keep a CU to a workgroup.)
-template <int FMT, bool OUT_BF16, int NV, int WAVES, int NT>
-__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && FMT != FMT_Q8_0 && FMT != FMT_Q8F ? 4 : 2) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
+// ALONE: see run_gemm_bf16_nv. (Eight waves of one token tile: two workgroups share a CU if they take at most 128 registers. Q4_K took 130:
+// bounded it spills 12 bytes, 9472 columns x 5000 rows 42.7 -> 31.9 us at 128 tokens with the slices that allows. The 8-bit formats
+// would spill 24 to 44 bytes, 33.6 -> 43.9 us on 14336 -> 4096: they keep a CU to a workgroup.)
+template <int FMT, bool OUT_BF16, int NV, int WAVES, int NT, bool ALONE>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 : 2) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
                                                         void* __restrict__ yv) {
     extern __shared__ uint4 bfrag[];  // [2][4 blocks][NT row tiles][64 lanes]
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -581,17 +581,24 @@ hipError_t run_gemm_bf16_nv(const WeightView& w, const void* apk, size_t t, size
     const size_t lds = 2 * 4 * NT * 64 * 16;  // 64 KiB with 8 row tiles
     const bool direct_bf16 = out_bf16 && slices == 1;
     void* dst = slices > 1 ? static_cast<void*>(partial) : y;
-    hipError_t e;
+    hipError_t e = hipSuccess;
+    auto go = [&](auto kern) {
+        e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e == hipSuccess) kern<<<grid, 64 * WAVES, lds, s>>>(w, static_cast<const uint4*>(apk), (uint32_t)t, (uint32_t)mtiles, dst);
+    };
+    // Eight waves of one token tile that leave a second workgroup no room on their CU: the 8-bit formats always; Q4_K in launches of
+    // at most a workgroup per CU, which need none, while the spill of the bounded kernel costs a start half a microsecond later
+    // (2048 columns x 7168 rows at 80 tokens, 224 workgroups: 19.0 us bounded, 18.4 this way).
+    constexpr bool ALWAYS = NV == 1 && WAVES == 8 && q8_format(FMT), CHOICE = NV == 1 && WAVES == 8 && FMT == FMT_Q4_K;
     span_start(s);
-    if (direct_bf16) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_kernel<FMT, true, NV, WAVES, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        gemm_bf16_kernel<FMT, true, NV, WAVES, NT><<<grid, 64 * WAVES, lds, s>>>(w, static_cast<const uint4*>(apk), (uint32_t)t, (uint32_t)mtiles, dst);
+    if (CHOICE && (uint64_t)grid.x * grid.y * grid.z <= 256) {
+        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, WAVES, NT, CHOICE || ALWAYS>);
+        else go(gemm_bf16_kernel<FMT, false, NV, WAVES, NT, CHOICE || ALWAYS>);
     } else {
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_bf16_kernel<FMT, false, NV, WAVES, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        gemm_bf16_kernel<FMT, false, NV, WAVES, NT><<<grid, 64 * WAVES, lds, s>>>(w, static_cast<const uint4*>(apk), (uint32_t)t, (uint32_t)mtiles, dst);
+        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, WAVES, NT, ALWAYS>);
+        else go(gemm_bf16_kernel<FMT, false, NV, WAVES, NT, ALWAYS>);
     }
+    if (e != hipSuccess) return e;
     e = hipGetLastError();
     span_stop(s);
     if (e != hipSuccess || slices == 1) return e;

@@ -145,6 +145,26 @@ def test_gemm_bf16_odd_slice_counts(be, oxref, name, n_out, n_in):
         assert row_err(y, (x.astype(np.float64) @ wb.T).astype(np.float32)) < 1e-3, t
 
 
+@pytest.mark.parametrize("t", [65, 128])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_gemm_q4_k_workgroups_alone_on_their_cus(be, oxref, t, bf16):
+    """Q4_K at 65 to 128 tokens: 256 workgroups (32768 rows, one slice) run the kernel that keeps all its registers, 257 the one
+    bounded for two workgroups per CU. The same sums in the same order: the same bits, and the last workgroup's rows against the
+    product of the operands rounded to bf16 (2e-2 of the row for results in bf16, as above)."""
+    import torch
+    from oxinfer_amd import synth
+    n_out, n_in = 32769, 256
+    raw = gguf_raw("Q4_K", n_out, n_in, 29)
+    full, part = (be.upload_gguf(GGUF_KINDS["Q4_K"], raw[: n * 144], n, n_in) for n in (n_out, 32768))
+    assert full is not None and part is not None, be.last_error()
+    x = synth.activations(t, n_in, 500 + t, bf16=True)
+    xd = torch.from_numpy(x).cuda()
+    y = be.gemm(full, xd, out_bf16=bf16)
+    assert torch.equal(y[:, :32768].contiguous(), be.gemm(part, xd, out_bf16=bf16))
+    wb = synth.bf16_round(oxref.dequantize_rows(GGUF_KINDS["Q4_K"], raw[-40 * 144:], 40, n_in)).astype(np.float64)
+    assert row_err(y[:, -40:].float().cpu().numpy(), (x.astype(np.float64) @ wb.T).astype(np.float32)) < (2e-2 if bf16 else 1e-3)
+
+
 def test_gemm_bf16_gguf_reference_fixtures(be, oxref):
     """The reference's own block fixtures (random_blocks, src/ggml.rs:1446-1496: every bit pattern of codes and packed
     scales, signed Q6_K scales, d of either sign) through the GEMM."""
