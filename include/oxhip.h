@@ -113,7 +113,9 @@ size_t oxhip_weight_bytes(const oxhip_weight* w);
  * computes every job or none. Routing as matmul_quant_multi_at's (src/kernels.rs:1731-1879): up to 16 tokens the
  * Q8 / Q8_0 / Q4_K / Q5_K / Q6_K / MXFP4 / MLX 4-bit jobs share one launch of the int8 decode kernel (the CPU's decode semantics,
  * src/kernels.rs:1908-1928); more than 16 tokens over MLX 4-bit, Q8, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4, NVFP4 or FP8 (128-column
- * blocks) weights run the bf16 matrix-core GEMM; everything else runs the decode kernels over 16 tokens at a time. */
+ * blocks) weights run the bf16 matrix-core GEMM; everything else runs the decode kernels over 16 tokens at a time.
+ * The results of a call come through page-locked host memory that the context keeps until oxhip_close: half more than the largest
+ * call so far needed, at most 256 MiB (a call with more results does without it). Jobs whose y overlap are copied in their order. */
 int oxhip_matmul(oxhip_ctx* ctx, const float* x, size_t t, size_t n_in, oxhip_job* jobs, size_t n_jobs);
 /* Backend::matvec_rows (src/gpu.rs:165): t in 1..=4. The jobs over the matrix-core formats share one launch, a gate / up
  * job as a pair (see oxhip_dev_linear). */
