@@ -199,6 +199,26 @@ def test_norm_at_the_edges_of_its_thread_shapes(be, n, off):
         assert torch.equal(getattr(qa, f).view(torch.uint8), getattr(ref, f).view(torch.uint8)), f
 
 
+@pytest.mark.parametrize("n", [1056, 4096, 4128, 8192, 8224, 16384])  # a part of one block, whole parts, one, two and four float4s a thread
+@pytest.mark.parametrize("rows,off", [(1, 0), (3, 1)])
+def test_norm_over_several_workgroups_keeps_the_bits(be, n, rows, off):
+    """A row shared by several workgroups has the bits of one that a single workgroup norms (the form that rows normed in place
+    take), in `out` and in its QAct, with `add` too."""
+    import torch
+    rng = np.random.default_rng(n + rows)
+    x, w, old = dev(rng.normal(0, 3, off + rows * n).astype(np.float32)), dev(rng.normal(1, 0.2, off + n).astype(np.float32)), rng.normal(0, 1, off + rows * n).astype(np.float32)
+    out, inplace = torch.zeros_like(x), x.clone()
+    ok, qa = be.norm(x[off:], n, rows, out=out[off:], w=w[off:], want_q=True)
+    ok2, qb = be.norm(inplace[off:], n, rows, out=inplace[off:], w=w[off:], want_q=True)
+    assert ok and ok2, be.last_error()
+    assert torch.equal(out[off:].view(torch.int32), inplace[off:].view(torch.int32))
+    for f in ("q", "scales", "sums", "fsums", "hsums", "sums16"):
+        assert torch.equal(getattr(qa, f).view(torch.uint8), getattr(qb, f).view(torch.uint8)), f
+    added = dev(old)
+    assert be.norm(x[off:], n, rows, out=added[off:], w=w[off:], add=True)[0]
+    assert torch.equal(added[off:], dev(old)[off:] + out[off:])
+
+
 def test_norm_rounds_the_reciprocal_root_correctly(be):
     """r = m^(-1/2) is the f32 value nearest to the exact one also where that lies closest to the middle between two f32 values: the
     4096 such means of [1, 4) (every exponent's r is one of theirs, times a power of two). A row's squares add up to 32 m in f32, and
