@@ -532,6 +532,7 @@ static int decode_one(oxhip_ctx* c, const oxhip_weight* w, const oxhip_qact* xa,
                                                                      : "decode: device memory short");
         return 0;
     }
+    sc->streamed += w->bytes;
     HIP_TRY(launch_decode(w->v, v, x, t, y, static_cast<hipStream_t>(stream), sc->dec, ev_start, ev_stop), "decode launch");
     return 1;
 }
@@ -617,6 +618,7 @@ int oxhip_dev_decode_batch(oxhip_ctx* c, const oxhip_decode_job* jobs, size_t n_
                     else HIP_TRY(hipEventRecord(static_cast<hipEvent_t>(jobs[k].ev_start), s), "event record");
                 }
                 items.push_back(DecodeBatchItem{jobs[k].w->v, view_of(*jobs[k].xa), jobs[k].y, (uint32_t)jobs[k].t, Epi{}});
+                ssc->streamed += jobs[k].w->bytes;
             }
             for (size_t k = e; k-- > j;)
                 if (jobs[k].ev_stop) {

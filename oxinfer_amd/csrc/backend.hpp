@@ -1,5 +1,6 @@
 // Definitions shared by the files that implement the C ABI: the context, the device weight, staging.
 #pragma once
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -81,6 +82,7 @@ struct StreamScratch {
     DecodeScratch dec;
     DevBuf tmp;
     DevBuf gemm_ws;
+    std::atomic<uint64_t> streamed{0};  // bytes of the weights that decode calls on this stream have been given: what a plan recorded there reads
 };
 
 }  // namespace oxhip
@@ -105,6 +107,7 @@ struct oxhip_ctx {
     std::mutex smu;            // guards per_stream
     std::map<hipStream_t, oxhip::StreamScratch*> per_stream;  // the device-pointer entry points' scratch, by calling stream
     std::set<hipStream_t> record_failed;  // streams whose plan recording met a call that had to allocate (guarded by smu)
+    std::mutex replay_mu;  // one plan's launches at a time
     double ms_in = 0, ms_gpu = 0, ms_out = 0;
     size_t calls = 0;
 };

@@ -196,6 +196,7 @@ int oxhip_dev_linear(oxhip_ctx* c, const oxhip_weight* w, const oxhip_weight* w2
                                       : "linear: device memory short");
         return 0;
     }
+    sc->streamed += w->bytes + (w2 ? w2->bytes : 0);
     const size_t n_out = w->v.n_out;
     Epi epi;
     epi.mode = mode == OXHIP_LIN_ADD ? EPI_ADD : mode == OXHIP_LIN_ADD_GATED ? EPI_ADD_GATED : EPI_STORE;

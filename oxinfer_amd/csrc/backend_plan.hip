@@ -9,6 +9,12 @@
 // fill kernel). Scratch that grows on first use (a stream's K-slice rows, an MoE layer's pass buffers, packed GEMM
 // activations) must exist before recording starts: run the chain once on the same stream first. A call that would have to
 // allocate while recording fails the recording (oxhip_plan_end reports it), and nothing is replayable then.
+//
+// A short plan is replayed launch by launch, from the list that the finished graph holds: the submission of a graph costs the
+// stream 5 us of its own, 8 behind an ordinary launch, where a launch from the list costs the device what a graph's node does
+// and the host 2.45 us, which it has while the kernels before it run. See DIRECT_MAX.
+#include <unordered_map>
+
 #include "backend.hpp"
 
 using namespace oxhip;
@@ -20,7 +26,54 @@ struct oxhip_plan {
     hipGraphExec_t exec = nullptr;
     bool recording = false;
     size_t nodes = 0;
+    uint64_t streamed0 = 0;  // the stream's count of weight bytes when the recording began
+    std::vector<hipKernelNodeParams> direct;  // the launches in order (arguments live in `graph`); empty: the graph is submitted
 };
+
+// The longest plan that goes out launch by launch, and the weight bytes per launch that it has to stream at least. 16 kernels of
+// 8 us (4, 2): 148.7 us as a graph, 143.6 this way (84.7, 79.7; 54.1, 47.9), behind a copy kernel 153.0 and 145.3; two Q4_K_M
+// layers at one token 114.2 -> 106.5 us, one layer of 1536 / 4096 in MLX 4-bit 36.8 -> 31.5, three of them 92.1 -> 92.5. The gain
+// does not grow with the plan, while the host's share does, so longer plans stay one submission. A chain with hardly any matrix
+// in it would be bound by the host (24 quantizations: 48.6 us as a graph, 55.3 this way), so it stays one too.
+constexpr size_t DIRECT_MAX = 24;
+constexpr uint64_t DIRECT_BYTES = 1 << 20;
+
+static uint64_t streamed_on(oxhip_ctx* c, hipStream_t s) {
+    std::lock_guard<std::mutex> lk(c->smu);
+    auto it = c->per_stream.find(s);
+    return it == c->per_stream.end() ? 0 : it->second->streamed.load();
+}
+
+// The launches of a graph that is one chain of kernels this process can launch by their symbols; empty for any other graph.
+static std::vector<hipKernelNodeParams> chain_of(hipGraph_t g) {
+    size_t n = 0, ne = 0;
+    if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || !n || n > DIRECT_MAX || hipGraphGetEdges(g, nullptr, nullptr, &ne) != hipSuccess || ne != n - 1) return {};
+    std::vector<hipGraphNode_t> nodes(n), from(ne + 1), to(ne + 1);
+    if (hipGraphGetNodes(g, nodes.data(), &n) != hipSuccess || (ne && hipGraphGetEdges(g, from.data(), to.data(), &ne) != hipSuccess)) return {};
+    std::unordered_map<hipGraphNode_t, hipGraphNode_t> next;
+    std::set<hipGraphNode_t> entered;
+    for (size_t i = 0; i < ne; i++)
+        if (!next.emplace(from[i], to[i]).second || !entered.insert(to[i]).second) return {};
+    hipGraphNode_t at = nullptr;
+    for (hipGraphNode_t v : nodes)
+        if (!entered.count(v)) at = v;  // (n - 1 edges, each into a node of its own: one start)
+    std::vector<hipKernelNodeParams> out;
+    while (at && out.size() < n) {
+        hipGraphNodeType type;
+        hipKernelNodeParams k{};
+        hipFunction_t f = nullptr;
+        if (hipGraphNodeGetType(at, &type) != hipSuccess || type != hipGraphNodeTypeKernel || hipGraphKernelNodeGetParams(at, &k) != hipSuccess || !k.func ||
+            !k.kernelParams || k.extra || hipGetFuncBySymbol(&f, k.func) != hipSuccess) {
+            (void)hipGetLastError();
+            return {};
+        }
+        out.push_back(k);
+        auto it = next.find(at);
+        at = it == next.end() ? nullptr : it->second;
+    }
+    if (out.size() != n) out.clear();
+    return out;
+}
 
 extern "C" {
 
@@ -45,6 +98,7 @@ oxhip_plan* oxhip_plan_begin(oxhip_ctx* c, void* stream) {
         c->record_failed.erase(s);
     }
     auto* p = new oxhip_plan();
+    p->streamed0 = streamed_on(c, s);
     p->ctx = c;
     p->stream = s;
     p->recording = true;
@@ -92,6 +146,7 @@ int oxhip_plan_end(oxhip_plan* p) {
     p->graph = g;
     p->exec = x;
     p->nodes = n;
+    if (streamed_on(p->ctx, p->stream) - p->streamed0 >= n * DIRECT_BYTES) p->direct = chain_of(g);
     return 1;
 }
 
@@ -103,7 +158,14 @@ int oxhip_plan_replay(oxhip_plan* p, void* stream) {
         return 0;
     }
     HIP_TRY(hipSetDevice(p->ctx->device), "hipSetDevice");
-    HIP_TRY(hipGraphLaunch(p->exec, stream ? static_cast<hipStream_t>(stream) : p->stream), "plan_replay: hipGraphLaunch");
+    hipStream_t s = stream ? static_cast<hipStream_t>(stream) : p->stream;
+    if (p->direct.empty() || stream_recording(s)) {  // (into a recording: as ever)
+        HIP_TRY(hipGraphLaunch(p->exec, s), "plan_replay: hipGraphLaunch");
+        return 1;
+    }
+    std::lock_guard<std::mutex> lk(p->ctx->replay_mu);  // the launches of a replay follow one another, whatever other threads replay
+    for (const hipKernelNodeParams& k : p->direct)
+        HIP_TRY(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes, s), "plan_replay: hipLaunchKernel");
     return 1;
 }
 

@@ -484,6 +484,48 @@ def test_plan_replays_a_layer_bit_for_bit(be, oxref, ne, h, inter, k, t):
         del plan
 
 
+@pytest.mark.parametrize("pairs,other", [(1, None), (12, None), (12, "kernel"), (2, "copy")])  # 2 and 24 launches go out one by one, 25 as one submission
+def test_plan_launched_one_by_one_or_as_one(be, pairs, other):
+    """The two ways a plan goes out (launch by launch, and as one submission: longer plans, or with anything but kernels in them) give
+    the bits of the calls themselves, on the stream it was recorded on and on another one."""
+    import torch
+    from oxinfer_amd import hip, synth
+    n = 1536  # (2.5 MB of weights for two launches)
+    w = be.upload_gguf(Q8_0, synth.gguf_q8_0(n, n, 5800), n, n)
+    x, y, z, qa = torch.zeros((2, n), device="cuda"), torch.zeros((2, n), device="cuda"), torch.zeros(n, device="cuda"), hip.QAct(2, n, "cuda")
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def chain():
+        for _ in range(pairs):
+            be.quantize_act(x, out=qa)
+            assert be.linear(w, y, xa=qa, t=2, mode=hip.LIN_ADD), be.last_error()
+        if other == "kernel": z.add_(1.0)
+        if other == "copy": z.copy_(y[1])
+
+    def load(i):
+        x.copy_(dev(synth.activations(2, n, 5900 + i)))
+        y.fill_(float(i))
+        z.zero_()
+        torch.cuda.synchronize()
+
+    def results(i, go):
+        load(i)
+        go()
+        torch.cuda.synchronize()
+        return y.clone(), z.clone()
+
+    with torch.cuda.stream(first):
+        want = [results(i, chain) for i in range(3)]
+        plan = be.plan_record(chain)
+        assert plan.launches == 2 * pairs + (other is not None)
+        for i in (2, 0, 1, 2):
+            for go in (plan.replay, lambda: plan.replay(second.cuda_stream)):
+                got = results(i, go)
+                assert torch.equal(got[0].view(torch.int32), want[i][0].view(torch.int32)) and torch.equal(got[1], want[i][1]), i
+            be.quantize_act(y, out=qa)  # the program's own work between the replays
+        del plan
+
+
 def test_plan_recording_on_a_cold_stream_declines(be, oxref):
     """Recording on a stream whose scratch does not exist yet: the call that would have to allocate declines, the
     recording is refused as a whole (oxhip_plan_end returns 0, nothing is replayable) and the stream works again
