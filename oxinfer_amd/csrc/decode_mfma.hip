@@ -57,9 +57,11 @@ __device__ __forceinline__ uint32_t opslot(uint32_t row, uint32_t slot) { return
 namespace {
 
 // Records a wave keeps in flight. HBM delivers about 8 TB/s at about 2 us of loaded latency, so some 16 MB must be
-// on request across the chip at any moment: about 4000 resident waves x PF KiB.
+// on request across the chip at any moment: about 4000 resident waves x PF KiB. Q6_K's records are 1.7 KiB and its step needs
+// the registers; so does that of the 8-bit formats at 9 to 16 tokens, which with eight records took 139 of them, one workgroup of
+// eight waves per CU, with four 103 (a pair of 14336 x 4096 in Q8_0 at 16 tokens 30.7 -> 25.5 us, 4096 x 4096 9.3 -> 7.2).
 template <int FMT, int NT>
-constexpr int pf_for() { return FMT == FMT_Q6_K ? 4 : 8; }  // Q6_K records are 1.7 KiB and its step needs the registers
+constexpr int pf_for() { return FMT == FMT_Q6_K || (NT == 16 && q8_format(FMT)) ? 4 : 8; }
 
 // The kernels evaluate a block's contribution as the reference does (src/ggml.rs:1288-1315, src/kernels.rs:1287-1297):
 //   Q8_0:        d * (xs * I)                                  I = sum of codes * activation codes (exact)
@@ -153,7 +155,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                                             uint32_t* __restrict__ counters, uint32_t bx, uint32_t by, uint32_t nthr,
                                             float* __restrict__ lds_all, Epi epi = Epi{}, Mapping map = Mapping{}) {
     static_assert(NG == 1 || (GROUPED && ALDS && !DUMP && NT == 8), "token groups are for grouped launches");
-    static_assert(!REMAP || (!GROUPED && !DUMP && ALDS && NG == 1 && NT <= 8), "other mappings are for dense launches over staged activations");
+    static_assert(!REMAP || (!GROUPED && !DUMP && ALDS && NG == 1), "other mappings are for dense launches over staged activations");
     // Nine to sixteen tokens (NT = 16): the instruction is v_mfma_i32_16x16x32_i8, one block x 16 tokens x 16 rows, so that the
     // token rows are all in use without masking (a lane's bytes 0-7 and 8-15 of a record are the operands of two consecutive
     // instructions, and the lane receives tokens 4 kq + i of both blocks). Every block parity keeps a sum of its own, as the two
@@ -785,9 +787,9 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                     if (d_tok0 + i < (uint32_t)TPAD) red[((((size_t)r * runs + run) * NG + g) * TPAD + d_tok0 + i) * 16 + n] = acc[g][i];
         }
     };
-    // A wave with further runs (up to MAXRUNS in all) keeps the closed run's sums in registers (the partial sums' place in
+    // A wave with further runs (up to MAXRUNS in all; place_job) keeps the closed run's sums in registers (the partial sums' place in
     // LDS still holds the activations) and starts the next run from zero. `left`: steps to the end of the run in hand.
-    constexpr int MAXRUNS = 4;
+    constexpr int MAXRUNS = WIDE ? 2 : 4;
     float held[REMAP ? MAXRUNS - 1 : 1][4] = {};
     uint32_t nrun = 0, left = per;  // runs closed so far
     auto step_done = [&]() {
@@ -801,7 +803,11 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                 nrun++;
                 left = per;
 #pragma unroll
-                for (int i = 0; i < 4; i++) acc[0][i] = acc6[0][i] = acc6[1][i] = 0.0f;
+                for (int i = 0; i < 4; i++) {
+                    acc[0][i] = acch[WIDE ? i : 0] = 0.0f;
+#pragma unroll
+                    for (int tg = 0; tg < NTG; tg++) acc6[tg][i] = 0.0f;
+                }
                 macc[0] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
             }
         }
@@ -838,7 +844,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     close_run();
     if (ALDS) __syncthreads();  // the partial sums overwrite the staged activations
     if constexpr (REMAP) {
-        if (rpw > 1 && kq < 2) {  // the runs closed on the way
+        if (rpw > 1 && (WIDE || kq < 2)) {  // the runs closed on the way
 #pragma unroll
             for (int h = 0; h < MAXRUNS - 1; h++)
                 if ((uint32_t)h < rpw - 1) {
@@ -1035,34 +1041,73 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
 }
 
 
+// The arguments of a launch of one matmul: what decode_body reads, and the group's only where there are groups (a launch that is not
+// a graph's node fetches its arguments over the host link: 104 bytes instead of 410; with it a replayed
+// chain of 1536 x 1536 products takes 4.0 us each, 4.25 before).
+template <bool GROUPED>
+struct LaunchArgs;
+template <>
+struct LaunchArgs<false> {
+    const uint8_t *p0, *pair_p0;
+    const int8_t* q;
+    const float* scales;
+    const void* sums;  // Q6_K: the halves' integer sums, else the f32 block sums
+    float *y, *partial;
+    uint32_t* counters;
+    const float* gate;
+    int32_t* dump;
+    uint32_t n_out, n_in, t;
+    uint8_t rt, kw, ks, mode, pair_act;
+};
+template <>
+struct LaunchArgs<true> : LaunchArgs<false> {
+    GroupView grp;
+};
+// The activations as a kernel gets them: the codes, the scales and the one kind of sums that the format reads.
+template <int FMT>
+__device__ __forceinline__ QActView act_view(const int8_t* q, const float* scales, const void* sums) {
+    QActView v{};
+    v.q = q;
+    v.scales = scales;
+    if constexpr (FMT == FMT_Q6_K) v.sums16 = static_cast<const int32_t*>(sums);
+    else v.fsums = static_cast<const float*>(sums);
+    return v;
+}
+inline const void* sums_of(int fmt, const QActView& v) { return fmt == FMT_Q6_K ? static_cast<const void*>(v.sums16) : v.fsums; }
+
 // Dynamic LDS is declared 16-byte aligned whatever static LDS a kernel also holds: the 8- and 16-byte LDS reads are split
 // into dwords (and the kernel runs two to three times longer) when the array starts at an odd dword.
 // (Grouped launches keep to 8 waves, which leaves them 256 registers for the accumulators of their token groups; with chunks of
 // five to eight rows they are bounded to four waves per SIMD, MLX 4-bit to five: unbounded that kernel took 139 registers and
 // spilled 36 scalar ones.)
-// (Q6_K: bounded at 8 waves like its shared-launch kernel, see decode_batch_kernel)
 // Such a launch has chunks of any length up to its own, and those of up to four rows, the most of them where an expert has few
 // routed rows, run the four-row body. 128 MLX 4-bit experts of 2048 / 768, eight a token, every chunk in the eight-row body of
 // before -> this: 24 tokens routed at random 85.5 -> 64.1 us, 47 tokens all to the same eight experts 53.8 -> 42.0 us. (Chunks of
 // four rows throughout make two passes over the weights of an expert with more: 63.0 and 55.1 us.)
 template <int FMT, int NT, bool DUMP, bool GROUPED, bool ALDS, int NG>
-__global__ __launch_bounds__(GROUPED || FMT == FMT_Q6_K || NT == 16 ? 512 : 1024, GROUPED && NG == 1 && NT == 8 ? (FMT == FMT_Q4M && ALDS ? 5 : 4) : 1) void decode_mfma_kernel(WeightView w, QActView xa, uint32_t t, uint32_t rt,
-                                                                           uint32_t kw, float* __restrict__ y,
-                                                                           int32_t* __restrict__ dump, GroupView grp, uint32_t ksplit,
-                                                                           float* __restrict__ partial,
-                                                                           uint32_t* __restrict__ counters, Epi epi) {
+__global__ __launch_bounds__(GROUPED ? 512 : 1024, GROUPED && NG == 1 && NT == 8 ? (FMT == FMT_Q4M && ALDS ? 5 : 4) : 1) void decode_mfma_kernel(LaunchArgs<GROUPED> a) {
     extern __shared__ __align__(16) float lds_dyn[];
-    if constexpr (GROUPED && NT == 8 && NG == 1) {
-        if (!grp.direct) {  // uniform over the workgroup
-            if (blockIdx.y >= (uint32_t)*grp.nchunks) return;
-            if (grp.chunks[blockIdx.y].z <= 4) {
-                decode_body<FMT, 4, DUMP, GROUPED, ALDS, NG>(w, xa, t, rt, kw, y, dump, grp, ksplit, partial, counters, blockIdx.x, blockIdx.y, blockDim.x, lds_dyn, epi);
-                return;
+    WeightView w{};
+    w.fmt = FMT;
+    w.n_out = a.n_out;
+    w.n_in = a.n_in;
+    w.p0 = a.p0;
+    const QActView xa = act_view<FMT>(a.q, a.scales, a.sums);
+    Epi epi{a.mode, a.gate, a.pair_p0, a.pair_act};
+    GroupView grp{};
+    if constexpr (GROUPED) {
+        grp = a.grp;
+        if constexpr (NT == 8 && NG == 1) {
+            if (!grp.direct) {  // uniform over the workgroup
+                if (blockIdx.y >= (uint32_t)*grp.nchunks) return;
+                if (grp.chunks[blockIdx.y].z <= 4) {
+                    decode_body<FMT, 4, DUMP, GROUPED, ALDS, NG>(w, xa, a.t, a.rt, a.kw, a.y, a.dump, grp, a.ks, a.partial, a.counters, blockIdx.x, blockIdx.y, blockDim.x, lds_dyn, epi);
+                    return;
+                }
             }
         }
     }
-    decode_body<FMT, NT, DUMP, GROUPED, ALDS, NG>(w, xa, t, rt, kw, y, dump, grp, ksplit, partial, counters, blockIdx.x, blockIdx.y,
-                                                  blockDim.x, lds_dyn, epi);
+    decode_body<FMT, NT, DUMP, GROUPED, ALDS, NG>(w, xa, a.t, a.rt, a.kw, a.y, a.dump, grp, a.ks, a.partial, a.counters, blockIdx.x, blockIdx.y, blockDim.x, lds_dyn, epi);
 }
 
 // Several independent matmuls in one launch (the jobs of one Backend::matmul call, src/gpu.rs:160: Q/K/V, gate/up ...):
@@ -1072,36 +1117,50 @@ __global__ __launch_bounds__(GROUPED || FMT == FMT_Q6_K || NT == 16 ? 512 : 1024
 // about 6 us before the first byte of bandwidth counts), and here the chains of neighbouring jobs overlap instead of
 // queueing behind kernel boundaries.
 constexpr int BATCH_MAX = 16;
+// What a job's workgroups need, and no more: the arguments of a launch that is not a graph's node come over the host link, and a
+// workgroup starts with two dependent reads of them (its job, then that job's line). 200 bytes a job and a walk over the jobs'
+// first workgroups one after the other: three products of 1536 columns, launched from a plan's list, 4.9 us, 4.15 this way.
 struct BatchJob {
-    WeightView w;
-    QActView xa;
-    float* y;
-    float* partial;      // this job's share of the scratch (K slices across workgroups)
+    const uint8_t *p0, *pair_p0;  // the records; those of the pair's second matrix, or none
+    const int8_t* q;
+    const float* scales;
+    const void* sums;             // the block sums the format reads: Q6_K's of the halves, else the f32 ones
+    float *y, *partial;           // partial, counters: this job's share of the scratch (K slices across workgroups)
     uint32_t* counters;
-    uint32_t t, rt, kw, ks, wg0;
-    Mapping map;  // (ks / fs slices across workgroups, 64 rt kwp threads)
-    Epi epi;
+    uint32_t n_out, n_in;
+    uint8_t fmt, t, rt, kw, ks, kwp, fs, pair_act;  // kwp, fs: the Mapping (ks / fs slices across workgroups, 64 rt kwp threads)
 };
 struct BatchArgs {
     uint32_t njobs, nwg;
+    uint32_t first[BATCH_MAX];  // job j's first workgroup (past the last job: none)
     BatchJob j[BATCH_MAX];
 };
 
 template <int FMT, bool FAT, bool WIDE>
 __device__ __forceinline__ void batch_dispatch(const BatchJob& jb, uint32_t bid, float* lds) {
-    const uint32_t nthr = 64 * jb.rt * jb.map.kwp;
+    const uint32_t nthr = 64 * jb.rt * jb.kwp;
     if (threadIdx.x >= nthr) return;  // whole waves (nthr is a multiple of 64), before any barrier
     const GroupView none{};
-    const uint32_t ksp = jb.ks >> __builtin_ctz(jb.map.fs);  // slices across workgroups
+    const uint32_t ksp = (uint32_t)jb.ks >> __builtin_ctz(jb.fs);  // slices across workgroups
     const uint32_t bx = bid >> __builtin_ctz(ksp), by = bid & (ksp - 1);  // the slices of a row group are neighbours in launch order (a power of two)
+    WeightView w{};
+    w.fmt = FMT;
+    w.n_out = jb.n_out;
+    w.n_in = jb.n_in;
+    w.p0 = jb.p0;
+    const QActView xa = act_view<FMT>(jb.q, jb.scales, jb.sums);
+    Epi epi{};
+    epi.pair_p0 = jb.pair_p0;
+    epi.pair_act = jb.pair_act;
+    const Mapping map{jb.kwp, jb.fs};
     if constexpr (WIDE) {
-        decode_body<FMT, 16, false, false, true>(jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
+        decode_body<FMT, 16, false, false, true, 1, FAT>(w, xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, epi, map);
         return;
-    } else if (jb.t == 1) decode_body<FMT, 1, false, false, true, 1, FAT>(jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
+    } else if (jb.t == 1) decode_body<FMT, 1, false, false, true, 1, FAT>(w, xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, epi, map);
     else if (jb.t == 2 && !t4m_format(FMT)) decode_body<FMT, 2, false, false, true, 1, FAT>(  // (MLX at 2 tokens: the 4-token body, which fits the registers)
-        jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
-    else if (jb.t <= 4) decode_body<FMT, 4, false, false, true, 1, FAT>(jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
-    else decode_body<FMT, 8, false, false, true, 1, FAT>(jb.w, jb.xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, jb.epi, jb.map);
+        w, xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, epi, map);
+    else if (jb.t <= 4) decode_body<FMT, 4, false, false, true, 1, FAT>(w, xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, epi, map);
+    else decode_body<FMT, 8, false, false, true, 1, FAT>(w, xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, epi, map);
 }
 
 // FSET: the formats compiled in, one bit per Fmt. The compiler allocates registers over the whole kernel, so every
@@ -1128,18 +1187,22 @@ inline int set_of(int fmt, uint32_t mask) {
     return -1;
 }
 // (Q6_K shares the kernel of Q8_0 and Q4_K since its step keeps 111 registers: a Q4_K_M file's layers mix the three, and their
-// matmuls go out in one launch. Q4_0's kernel is bounded at 512 threads, which saves it nine spilled registers; its shapes
-// never exceed 8 waves.)
+// matmuls go out in one launch. Q4_0's kernel is bounded at 512 threads, which saves it nine spilled registers.)
 // FAT: the launch's jobs use the fat mapping (see place_job); the plain kernels do without its bookkeeping.
-// WIDE: the launch's jobs have 9 to 16 tokens each (a kernel of its own, for the registers; plain mapping).
+// WIDE: the launch's jobs have 9 to 16 tokens each (kernels of their own, for the registers; plain mappings, but compiled as FAT,
+// which keeps the GGUF set at 118 registers and two workgroups per CU: 143 without).
 template <uint32_t FSET, bool FAT, bool WIDE = false>
 __global__ __launch_bounds__(WIDE || FSET == (1u << FMT_Q40) ? 512 : 1024) void decode_batch_kernel(BatchArgs a) {
     extern __shared__ __align__(16) float lds_dyn[];
-    uint32_t j = 0;
-    while (j + 1 < a.njobs && blockIdx.x >= a.j[j + 1].wg0) j++;  // uniform
+    uint32_t j = 0, bx = blockIdx.x;  // (uniform; every job's first workgroup is read at once)
+#pragma unroll
+    for (int i = 1; i < BATCH_MAX; i++)
+        if (blockIdx.x >= a.first[i]) {
+            j = i;
+            bx = blockIdx.x - a.first[i];
+        }
     const BatchJob& jb = a.j[j];
-    const uint32_t bx = blockIdx.x - jb.wg0;
-    switch (jb.w.fmt) {
+    switch (jb.fmt) {
         case FMT_Q8_0: if constexpr (FSET & fbit(FMT_Q8_0)) batch_dispatch<FMT_Q8_0, FAT, WIDE>(jb, bx, lds_dyn); break;
         case FMT_Q8F: if constexpr (FSET & fbit(FMT_Q8F)) batch_dispatch<FMT_Q8F, FAT, WIDE>(jb, bx, lds_dyn); break;
         case FMT_Q4_K: if constexpr (FSET & fbit(FMT_Q4_K)) batch_dispatch<FMT_Q4_K, FAT, WIDE>(jb, bx, lds_dyn); break;
@@ -1174,7 +1237,17 @@ constexpr uint32_t NCU = 256;
 //    dealt round-robin, and prefers a few records per wave, four or more waves, enough workgroups for every CU, and
 //    little restaging (every workgroup stages its slice of the activations: 11 bytes per column next to the
 //    rt * bytes-per-column of weights it streams).
-Shape search_shape(uint32_t ntiles, uint32_t nsteps, uint32_t cols_per_step, double weight_bytes_per_col) {
+//
+// One class of shapes the model does not see as they are: at most a workgroup per CU (rt = 1) and long rows that need no slices. The
+// CU is the workgroup's alone, and eight waves step through the row in half the time of four. Lone launches at 1 / 8 / 16 tokens,
+// before -> this: 2048 x 5632 MLX 4-bit 6.8 / 8.6 / 12.0 -> 6.0 / 7.4 / 9.5 us, Q8_0 7.4 / 8.5 / 11.5 -> 6.5 / 7.1 / 9.4, Q6_K 7.5 / 10.6 /
+// 17.1 -> 6.6 / 9.1 / 13.6. Up to 5120 columns it pays where a step is a short run of bytes or many instructions (4096 x 4096: Q8_0
+// 6.9 / 7.2 / 9.9 -> 6.4 / 7.2 / 7.8, Q6_K 6.8 / 8.6 / 13.4 -> 6.3 / 8.2 / 10.9), not for 4-bit records (Q4_K 5.5 -> 5.9 at 1 token), and not
+// in matrices taller than wide, which come in pairs (sixteen waves to a workgroup). (More runs of fewer steps: the rows' error
+// against 64 bits is 1 to 10 % smaller. Eight runs of 8192 columns in place of two slices of four were as fast again, 8.6 -> 7.3 us at
+// 1 token of 3072 rows, but summed one after the other their error is 2 to 4 % larger; two runs of a Q8_0 row of 4096 columns
+// in place of four, 23.3 -> 22.6 us for a pair of 14336 rows, 20 %.)
+Shape search_shape(uint32_t ntiles, uint32_t nsteps, uint32_t cols_per_step, double weight_bytes_per_col, int fmt) {
     uint32_t ks0 = 1;
     while (ks0 < 32 && (size_t)nsteps * cols_per_step * 11 / ks0 > 80 * 1024 && nsteps / (ks0 * 2) >= 4) ks0 *= 2;
     while (ks0 > 1 && (nsteps + ks0 - 1) / ks0 * (ks0 - 1) >= nsteps) ks0 /= 2;  // no empty slice
@@ -1202,6 +1275,8 @@ Shape search_shape(uint32_t ntiles, uint32_t nsteps, uint32_t cols_per_step, dou
                 }
             }
     }
+    const uint32_t cols = nsteps * cols_per_step;
+    if (ntiles <= NCU && ks0 == 1 && (cols > 5120 || (cols >= 3072 && cols >= 16 * ntiles && (q8_format(fmt) || fmt == FMT_Q6_K)))) best = Shape{1, 8, 1};
 #ifdef OXHIP_TUNING  // tuning builds only (never the shipped library): "tiles:steps=rt,kw,ks;..." in OXHIP_DECODE_SHAPE
     if (const char* e = getenv("OXHIP_DECODE_SHAPE")) {
         for (const char* p = e; p && *p;) {
@@ -1232,7 +1307,7 @@ Shape shape_for(uint32_t ntiles, uint32_t nsteps, bool allow_slices, int fmt) {
     std::lock_guard<std::mutex> g(mu);
     auto it = cache.find(key);
     if (it != cache.end()) return it->second;
-    Shape sh = search_shape(ntiles, nsteps, cols_per_step, bytes_per_col);
+    Shape sh = search_shape(ntiles, nsteps, cols_per_step, bytes_per_col, fmt);
     if (!allow_slices) sh.ks = 1;
     cache.emplace(key, sh);
     return sh;
@@ -1240,11 +1315,24 @@ Shape shape_for(uint32_t ntiles, uint32_t nsteps, bool allow_slices, int fmt) {
 
 // A gate / up pair: a workgroup holds the tiles of the same rows of both matrices, so its tile count is even; kw and ks (the
 // order of a row's sum) stay what the weight's shape alone gives, which keeps each product's bits those of a launch of its own.
-Shape pair_shape(Shape sh) {
-    if (sh.rt % 2) sh.rt = (sh.rt + 1) * sh.kw <= 8 ? sh.rt + 1 : sh.rt > 1 ? sh.rt - 1 : 2;  // (rt = 1 with kw = 8: 16 waves)
+// Of the tile counts that eight waves allow (two tiles at least) the one whose tiles take the busiest CU least, each workgroup's
+// staging counted as a tile more, as four more of nine and more tokens; of equals the largest. (A pair of 11008
+// x 4096, 1 / 8 / 16 tokens, four tiles -> two, two, four: MLX 4-bit 15.6 / 18.0 / 20.5 -> 13.5 / 15.9 / 20.5 us; of 8192 x 3072, two ->
+// four: Q8_0 11.6 / 12.1 / 14.5 -> 11.6 / 11.9 / 13.1.)
+Shape pair_shape(Shape sh, uint32_t ntiles, size_t t) {
+    const uint32_t stage = t > 8 ? 4 : 1;
+    uint32_t best = 0;
+    uint64_t least = 0;
+    for (uint32_t rt = 2; rt == 2 || rt * sh.kw <= 8; rt += 2) {
+        const uint64_t wgs = (uint64_t)((ntiles + rt / 2 - 1) / (rt / 2)) * sh.ks, cost = (wgs + NCU - 1) / NCU * (rt + stage);
+        if (!best || cost <= least) {
+            best = rt;
+            least = cost;
+        }
+    }
+    sh.rt = best;
     return sh;
 }
-uint32_t pair_tiles(const Shape& sh, bool pair) { return pair ? pair_shape(sh).rt / 2 : sh.rt; }
 
 constexpr size_t LDS_MAX = 160 * 1024;  // dynamic LDS on offer (the kernels hold no static LDS)
 
@@ -1279,10 +1367,13 @@ hipError_t launch_one(bool alds, dim3 grid, dim3 block, size_t lds, hipStream_t 
             if (e == hipSuccess) allowed[(dev >> 6) & 3].fetch_or(bit, std::memory_order_release);
         }
         if (e != hipSuccess) return;
+        LaunchArgs<GROUPED> a{};
+        static_cast<LaunchArgs<false>&>(a) = LaunchArgs<false>{w.p0, epi.pair_p0, v.q, v.scales, sums_of(FMT, v), y, sc.partial, sc.counters, epi.gate, dump, w.n_out, w.n_in, t,
+                                                               (uint8_t)sh.rt, (uint8_t)sh.kw, (uint8_t)sh.ks, (uint8_t)epi.mode, (uint8_t)epi.pair_act};
+        if constexpr (GROUPED) a.grp = g;
         // timing events ride on the dispatch: its start and end as the device saw them
-        if (ev_start || ev_stop)
-            hipExtLaunchKernelGGL(kern, grid, block, (uint32_t)lds, s, ev_start, ev_stop, 0, w, v, t, sh.rt, sh.kw, y, dump, g, sh.ks, sc.partial, sc.counters, epi);
-        else kern<<<grid, block, lds, s>>>(w, v, t, sh.rt, sh.kw, y, dump, g, sh.ks, sc.partial, sc.counters, epi);
+        if (ev_start || ev_stop) hipExtLaunchKernelGGL(kern, grid, block, (uint32_t)lds, s, ev_start, ev_stop, 0, a);
+        else kern<<<grid, block, lds, s>>>(a);
     };
     if (alds) go(decode_mfma_kernel<FMT, NT, DUMP, GROUPED, true, NG>);
     else if constexpr (NG == 1 && FMT != FMT_Q6_K && NT <= 8) go(decode_mfma_kernel<FMT, NT, DUMP, GROUPED, false, 1>);
@@ -1300,14 +1391,17 @@ hipError_t run(const WeightView& w, const QActView& xa, size_t t, float* y, int3
                hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr, const Epi& epi0 = Epi{}) {
     const uint32_t ntiles = row_tiles(w.n_out), nsteps = steps_of<FMT>(w.n_in);
     const bool pair = !DUMP && epi0.pair_p0 != nullptr;
-    Shape sh = shape_for(ntiles, nsteps, true, FMT);
+    auto shaped = [&](bool allow_slices) {
+        const Shape h = shape_for(ntiles, nsteps, allow_slices, FMT);
+        return pair ? pair_shape(h, ntiles, t) : h;
+    };
+    Shape sh = shaped(true);
     // slices need scratch: 8 (or 16) token rows per slice (of both matrices of a pair) and a counter per row group
     auto scratch_ok = [&](const Shape& h, size_t rows) {
-        const uint32_t groups = (ntiles + pair_tiles(h, pair) - 1) / pair_tiles(h, pair);
+        const uint32_t per = pair ? h.rt / 2 : h.rt, groups = (ntiles + per - 1) / per;
         return h.ks == 1 || (sc.partial && sc.counters && sc.partial_floats >= (size_t)h.ks * rows * w.n_out * (pair ? 2 : 1) && sc.ncounters >= (size_t)groups * CTR_STRIDE);
     };
-    if (!scratch_ok(sh, 8)) sh = shape_for(ntiles, nsteps, false, FMT);
-    if (pair) sh = pair_shape(sh);
+    if (!scratch_ok(sh, 8)) sh = shaped(false);
     const uint32_t nblk = w.n_in / 32;
     const uint32_t per_wg = pair ? sh.rt / 2 : sh.rt;  // row tiles of the output per workgroup
     dim3 grid((ntiles + per_wg - 1) / per_wg, sh.ks), block(64 * sh.rt * sh.kw);
@@ -1316,7 +1410,7 @@ hipError_t run(const WeightView& w, const QActView& xa, size_t t, float* y, int3
     bool wide = false;
     if (!DUMP && t > 8 && t <= 16) {
         const size_t l = lds_bytes(FMT, false, nsteps, 16, sh, &wide);
-        wide = wide && l <= LDS_MAX && sh.rt * sh.kw <= 8 && scratch_ok(sh, t);
+        wide = wide && l <= LDS_MAX && scratch_ok(sh, t);
     }
     // timing events: one launch carries them itself; around several they are recorded on the stream
     const bool ride = t <= 8 || wide;
@@ -1417,12 +1511,12 @@ uint32_t steps_rt(const WeightView& w) {
 }
 }  // namespace
 
-// Whether a gate / up pair of this weight's shape and format runs as one launch (its workgroup of paired tiles fits the
-// kernel's bound: Q6_K's kernels take at most 8 waves).
-bool decode_pair_ok(const WeightView& w) {
+// Whether a gate / up pair of this weight's shape and format runs as one launch: its workgroup of paired tiles fits the kernel's
+// bound. `shared`: in the shared launch, where Q4_0's kernel is bounded at 8 waves.
+bool decode_pair_ok(const WeightView& w, bool shared) {
     if (!mfma_decode_format(w.fmt)) return false;
-    const Shape sh = pair_shape(shape_for(row_tiles(w.n_out), steps_rt(w), true, w.fmt));
-    return sh.rt * sh.kw <= (w.fmt == FMT_Q6_K || w.fmt == FMT_Q40 ? 8u : 16u);  // (their shared-launch kernels are bounded at 8 waves)
+    const Shape sh = pair_shape(shape_for(row_tiles(w.n_out), steps_rt(w), true, w.fmt), row_tiles(w.n_out), 1);
+    return sh.rt * sh.kw <= (shared && w.fmt == FMT_Q40 ? 8u : 16u);
 }
 
 bool decode_batchable(const WeightView& w, size_t t) {
@@ -1442,7 +1536,7 @@ void decode_scratch_need(const WeightView& w, size_t* partial_floats, size_t* nc
     const uint32_t ntiles = row_tiles(w.n_out);
     const Shape sh = shape_for(ntiles, steps_rt(w), true, w.fmt);
     if (sh.ks <= 1) return;
-    const uint32_t per_wg = pair_tiles(sh, pair);
+    const uint32_t per_wg = pair ? std::min(pair_shape(sh, ntiles, 1).rt, pair_shape(sh, ntiles, 16).rt) / 2 : sh.rt;
     *partial_floats = (size_t)sh.ks * 8 * w.n_out * (pair ? 2 : 1);
     *ncounters = (size_t)((ntiles + per_wg - 1) / per_wg) * CTR_STRIDE;
 }
@@ -1469,7 +1563,7 @@ Placed place_job(const DecodeBatchItem& it, bool fat, uint32_t fat_steps) {
     const uint32_t ntiles = row_tiles(it.w.n_out), nsteps = steps_rt(it.w);
     const bool pair = it.epi.pair_p0 != nullptr;
     Shape sh = shape_for(ntiles, nsteps, true, it.w.fmt);
-    if (pair) sh = pair_shape(sh);
+    if (pair) sh = pair_shape(sh, ntiles, it.t);
     const int tpad = it.t <= 4 ? 4 : it.t <= 8 ? 8 : 16;
     Placed pl{sh.rt, Mapping{sh.kw, 1}, 0, 0};
     bool alds = false;
@@ -1533,7 +1627,7 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
     const uint64_t bit = 1ull << (dev & 63);
     if (!(allowed[(dev >> 6) & 3].load(std::memory_order_acquire) & bit)) {
 #define OXHIP_BATCH_KERNELS(F) reinterpret_cast<const void*>(decode_batch_kernel<F, false>), reinterpret_cast<const void*>(decode_batch_kernel<F, true>)
-#define OXHIP_BATCH_WIDE(F) reinterpret_cast<const void*>(decode_batch_kernel<F, false, true>)
+#define OXHIP_BATCH_WIDE(F) reinterpret_cast<const void*>(decode_batch_kernel<F, true, true>)
         for (const void* k : {OXHIP_BATCH_WIDE(FSET_GGUF), OXHIP_BATCH_WIDE(FSET_MLX), OXHIP_BATCH_WIDE(FSET_K5), OXHIP_BATCH_WIDE(FSET_Q40),
                               OXHIP_BATCH_WIDE(FSET_MX4), OXHIP_BATCH_WIDE(FSET_Q8F), OXHIP_BATCH_KERNELS(FSET_GGUF), OXHIP_BATCH_KERNELS(FSET_MLX), OXHIP_BATCH_KERNELS(FSET_K5),
                               OXHIP_BATCH_KERNELS(FSET_Q40), OXHIP_BATCH_KERNELS(FSET_MX4), OXHIP_BATCH_KERNELS(FSET_Q8F)}) {
@@ -1567,6 +1661,7 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
         const DecodeBatchItem* const* items_of = sorted.data() + run.first;
         BatchArgs a{};
         a.njobs = (uint32_t)run.second;
+        for (uint32_t& f : a.first) f = 0xFFFFFFFFu;
         size_t lds = 0, pf = 0, nc = 0;  // scratch is shared by the jobs of one launch, reused by the next launch
         uint32_t wg = 0, threads = 64;
         // Block order within the launch. Workgroups start in block order, so the last jobs make the tail of the launch,
@@ -1610,9 +1705,10 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
             const uint32_t ntiles = row_tiles(it.w.n_out), nsteps = steps_rt(it.w);
             const bool pair = it.epi.pair_p0 != nullptr;
             Shape sh = shape_for(ntiles, nsteps, true, it.w.fmt);
-            if (pair) sh = pair_shape(sh);
+            if (pair) sh = pair_shape(sh, ntiles, it.t);
             const Placed pl = place_job(it, fat, fat_steps);
             const size_t l = pl.lds;
+            if (it.epi.mode != EPI_STORE) return hipErrorInvalidValue;  // (a shared launch's jobs store)
             if (l > LDS_MAX || it.t < 1 || it.t > 16) return hipErrorInvalidValue;
             sh.rt = pl.rt;
             const uint32_t per_wg = pair ? sh.rt / 2 : sh.rt;
@@ -1629,7 +1725,9 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
             }
             lds = l > lds ? l : lds;
             threads = 64 * sh.rt * pl.map.kwp > threads ? 64 * sh.rt * pl.map.kwp : threads;
-            a.j[j] = BatchJob{it.w, it.xa, it.y, partial, counters, it.t, sh.rt, sh.kw, sh.ks, wg, pl.map, it.epi};
+            a.j[j] = BatchJob{it.w.p0, it.epi.pair_p0, it.xa.q, it.xa.scales, sums_of(it.w.fmt, it.xa), it.y, partial, counters,
+                              it.w.n_out, it.w.n_in, (uint8_t)it.w.fmt, (uint8_t)it.t, (uint8_t)sh.rt, (uint8_t)sh.kw, (uint8_t)sh.ks, (uint8_t)pl.map.kwp, (uint8_t)pl.map.fs, (uint8_t)it.epi.pair_act};
+            a.first[j] = wg;
             wg += groups * (sh.ks / pl.map.fs);
         }
         a.nwg = wg;
@@ -1649,7 +1747,7 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
     for (size_t i = 0; i < launches.size(); i++) {
         if (!launches[i].nwg) continue;
         uint32_t fset = 0;
-        for (uint32_t j = 0; j < launches[i].njobs; j++) fset |= fbit(launches[i].j[j].w.fmt);
+        for (uint32_t j = 0; j < launches[i].njobs; j++) fset |= fbit(launches[i].j[j].fmt);
         if (threadss[i] > (fset == FSET_Q40 || launches[i].j[0].t > 8 ? 512u : 1024u)) return hipErrorInvalidValue;  // (the kernels' launch bounds)
         auto go = [&](auto kern) {
             if (ride) hipExtLaunchKernelGGL(kern, dim3(launches[i].nwg), dim3(threadss[i]), (uint32_t)ldss[i], s, ev_start, ev_stop, 0, launches[i]);
@@ -1657,7 +1755,7 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
         };
         const bool fat = fats[i];
         const bool wide = launches[i].j[0].t > 8;
-#define OXHIP_GO(F) (wide ? go(decode_batch_kernel<F, false, true>) : fat ? go(decode_batch_kernel<F, true>) : go(decode_batch_kernel<F, false>))
+#define OXHIP_GO(F) (wide ? go(decode_batch_kernel<F, true, true>) : fat ? go(decode_batch_kernel<F, true>) : go(decode_batch_kernel<F, false>))
         if (!(fset & ~FSET_GGUF)) OXHIP_GO(FSET_GGUF);
         else if (!(fset & ~FSET_MLX)) OXHIP_GO(FSET_MLX);
         else if (!(fset & ~FSET_K5)) OXHIP_GO(FSET_K5);

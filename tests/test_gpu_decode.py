@@ -519,7 +519,8 @@ def test_upload_declines(be):
     assert be.upload_gguf(Q4_K, np.zeros(144, np.uint8), 1, 256) is not None
 
 
-@pytest.mark.parametrize("kind,n_out,n_in", [(Q8_0, 14336, 4096), (Q8_0, 4096, 14336), (Q4_K, 14336, 4096), (Q4_K, 4096, 14336), (Q6_K, 14336, 4096), (Q6_K, 4096, 14336), (Q5_K, 4096, 14336), (MXFP4, 14336, 4096)])
+@pytest.mark.parametrize("kind,n_out,n_in", [(Q8_0, 14336, 4096), (Q8_0, 4096, 14336), (Q4_K, 14336, 4096), (Q4_K, 4096, 14336), (Q6_K, 14336, 4096), (Q6_K, 4096, 14336), (Q5_K, 4096, 14336), (MXFP4, 14336, 4096),
+                                              (Q4_K, 2048, 5632), (Q8_0, 2560, 6912), (Q6_K, 4096, 4096)])
 def test_full_size_rows_against_oracle(be, oxref, kind, n_out, n_in):
     """The benchmark shapes: a sample of rows of the full-size product against the oracle, plus properties
     that hold at any size: the all-ones-activation row sums and batch invariance."""
@@ -685,11 +686,11 @@ def test_decode_batch_events(be, oxref):
             assert np.array_equal(y.cpu().numpy().view(np.uint32), want.view(np.uint32))
 
 
-# ragged rows; two workgroups a CU; K slices; rows that end inside a step of 64 or 128 columns; a pair whose workgroup has 16 waves,
-# which goes eight tokens at a time
+# ragged rows; two workgroups a CU; K slices; rows that end inside a step of 64 or 128 columns; eight runs to a row (long rows, and
+# 3072 columns in 8 and 6 bits), whose last runs are shorter, and pairs of sixteen waves
 @pytest.mark.parametrize("kind,n_out,n_in", [(k, *s) for k in (Q4_0, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4, "q8", "mlx") for s in ((37, 768), (272, 4096), (48, 14336))]
                          + [(k, *s) for k in (Q4_0, Q8_0, MXFP4, "q8") for s in ((33, 96), (40, 1120))] + [("mlx", 33, 64), ("mlx", 40, 320), ("mlx", 24, 4160)]
-                         + [(k, 64, 6144) for k in (Q8_0, "q8")])
+                         + [(k, 64, 6144) for k in (Q8_0, "q8")] + [(k, 40, 5376) for k in (Q4_0, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4, "q8", "mlx")] + [(Q6_K, 37, 3072), (Q8_0, 37, 3136)])
 def test_sixteen_token_form_keeps_the_bits(be, oxref, kind, n_out, n_in):
     """Nine to sixteen tokens go through the 16-token form in one pass over the weights: every row, stored, added, of a gate /
     up pair and in a shared launch with jobs of fewer tokens, has the bits of that token's row computed alone (which the

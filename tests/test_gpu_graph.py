@@ -106,7 +106,7 @@ def test_linear_store_add_gated(be, oxref, kind, n_out, n_in):
     assert float(y.min()) == 7.0 and float(y.max()) == 7.0  # declined: nothing written
 
 
-@pytest.mark.parametrize("kind,n_out,n_in", [(Q4_K, 96, 512), (Q8_0, 40, 864), ("mlx", 80, 640), (Q4_K, 32, 14336), ("q4", 10, 512), ("bf16", 21, 520),
+@pytest.mark.parametrize("kind,n_out,n_in", [(Q4_K, 96, 512), (Q8_0, 40, 864), ("mlx", 80, 640), (Q4_K, 32, 14336), (Q6_K, 48, 3072), (Q4_K, 48, 5376), ("q4", 10, 512), ("bf16", 21, 520),
                                              (Q6_K, 48, 512), (Q4_K, 1000, 768), (Q8_0, 272, 14336), (Q4_0, 130, 1120), (Q6_K, 40, 14336)])
 def test_linear_pairs(be, oxref, kind, n_out, n_in):
     """LinMode SiluPair / GeluPair: y = act(W x) * (W2 x) with silu_mul / gelu_mul (src/kernels.rs:2188-2198, :2234-2257). Over
