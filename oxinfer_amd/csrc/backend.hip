@@ -42,6 +42,7 @@ hipError_t launch_fill_zero(uint32_t* p, size_t n, hipStream_t s) {
 
 namespace {
 
+constexpr size_t OUT_CHUNKED = (size_t)8 << 20;  // results of this size and more come in chunks
 constexpr size_t MAX_PINNED = (size_t)256 << 20;  // of page-locked staging a context keeps
 
 struct Planes {
@@ -170,6 +171,10 @@ void oxhip_close(oxhip_ctx* c) {
     c->y.release();
     c->gemm_ws.release();
     c->pin.release();
+    for (hipEvent_t e : c->span)
+        if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->chunk_came)
+        if (e) (void)hipEventDestroy(e);
     free_stream_scratch(c);
     (void)hipFree(c->dec.partial);
     (void)hipFree(c->dec.counters);
@@ -700,35 +705,36 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
         set_error("matmul: device memory short");
         return 0;
     }
-    hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, e3 = nullptr;
-    auto done = [&](int rc) {
-        for (hipEvent_t e : {e0, e1, e2, e3})
-            if (e) (void)hipEventDestroy(e);
-        return rc;
-    };
-    if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess || hipEventCreate(&e2) != hipSuccess ||
-        hipEventCreate(&e3) != hipSuccess) {
-        set_error("matmul: hipEventCreate failed");
-        return done(0);
-    }
+    for (hipEvent_t* e : {&c->span[0], &c->span[1], &c->span[2], &c->span[3]})
+        if (!*e && hipEventCreate(e) != hipSuccess) {
+            *e = nullptr;
+            set_error("matmul: hipEventCreate failed");
+            return 0;
+        }
+    for (hipEvent_t& e : c->chunk_came)
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            e = nullptr;
+            set_error("matmul: hipEventCreate failed");
+            return 0;
+        }
     // Everything is computed into device staging and comes to the host as a whole first; y is written only once all jobs ran.
     // It comes through page-locked memory that the context keeps: an ordinary buffer made for each call costs its page faults
     // and the runtime's own staging, 16.6 ms a call for 512 tokens through two 14336 x 4096 matrices (59 MB of results)
-    // against 2.0 ms, of which 1.0 are the link's. Calls with more results than MAX_PINNED take the ordinary buffer. (x is as
-    // fast from where it is: 0.34 ms for 8 MB either way.)
+    // against 2.0 ms, 1.7 copied out in chunks, of which 1.0 are the link's. Calls with more results than MAX_PINNED take the ordinary
+    // buffer. (x is as fast from where it is: 0.34 ms for 8 MB either way.)
     uint8_t* pin = c->pin.grow(y_total * 4, MAX_PINNED) ? static_cast<uint8_t*>(c->pin.p) : nullptr;
-    (void)hipEventRecord(e0, s);
+    (void)hipEventRecord(c->span[0], s);
     if (hipMemcpyAsync(c->x.p, x, t * n_in * 4, hipMemcpyHostToDevice, s) != hipSuccess) {
         set_error("matmul: copy-in failed");
-        return done(0);
+        return 0;
     }
-    (void)hipEventRecord(e1, s);
+    (void)hipEventRecord(c->span[1], s);
     oxhip_qact xa{};
     if (any_q) {
         xa = carve_qact(c->xq.p, t, n_in);
         if (launch_quantize_act(static_cast<const float*>(c->x.p), t, n_in, xa, s) != hipSuccess) {
             set_error("matmul: quantize_act launch failed");
-            return done(0);
+            return 0;
         }
     }
     float* yd = static_cast<float*>(c->y.p);
@@ -746,7 +752,7 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
     auto fail = [&](const char* what) {
         set_error(std::string("matmul: ") + what);
         (void)hipStreamSynchronize(s);
-        return done(0);
+        return 0;
     };
     for (size_t j = 0; j < n_jobs; j++) {
         const oxhip_weight* w = jobs[j].w;
@@ -758,7 +764,7 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
         if (gemm) {
             if (!gemm_bf16_run(c->gemm_ws, w, c->x.p, false, t, yd + offs[j], false, s)) {
                 (void)hipStreamSynchronize(s);
-                return done(0);
+                return 0;
             }
             continue;
         }
@@ -788,27 +794,43 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
             return fail("decode batch launch failed");
         }
     }
-    (void)hipEventRecord(e2, s);
-    std::vector<float> host(pin ? 0 : y_total);
-    float* yh = pin ? reinterpret_cast<float*>(pin) : host.data();
-    const hipError_t out = hipMemcpyAsync(yh, yd, y_total * 4, hipMemcpyDeviceToHost, s);
-    (void)hipEventRecord(e3, s);
-    if (hipStreamSynchronize(s) != hipSuccess || out != hipSuccess) {
-        set_error("matmul: kernels or copy-out failed");
-        return done(0);
+    (void)hipEventRecord(c->span[2], s);
+    // Large results cross the link in five chunks, each copied out while the next ones still come, the last one the smallest: what is
+    // left to do when it has come. (A copy of its own costs some 20 us: 59 MB in 56 chunks take longer than in one.) Nothing reaches y
+    // before the first chunk has come, that is before all jobs have run.
+    const size_t bytes = y_total * 4, chunks = pin && bytes >= OUT_CHUNKED ? OUT_CHUNKS : 1;
+    size_t ends[OUT_CHUNKS];
+    for (size_t k = 0, parts = 0; k < chunks; k++) {
+        parts += chunks - k;
+        ends[k] = k + 1 == chunks ? bytes : bytes * parts / (chunks * (chunks + 1) / 2) / 4096 * 4096;
     }
+    std::vector<float> host(pin ? 0 : y_total);
+    uint8_t* yh = pin ? pin : reinterpret_cast<uint8_t*>(host.data());
+    hipError_t out = hipSuccess;
+    for (size_t k = 0, at = 0; k < chunks && out == hipSuccess; at = ends[k++]) {
+        out = hipMemcpyAsync(yh + at, reinterpret_cast<uint8_t*>(yd) + at, ends[k] - at, hipMemcpyDeviceToHost, s);
+        if (out == hipSuccess && k + 1 < chunks) out = hipEventRecord(c->chunk_came[k], s);
+    }
+    (void)hipEventRecord(c->span[3], s);
     std::vector<HostCopy> outs(n_jobs);
-    for (size_t j = 0; j < n_jobs; j++) outs[j] = HostCopy{jobs[j].y, yh + offs[j], t * jobs[j].w->v.n_out * 4};
-    host_copy(outs.data(), n_jobs);
+    for (size_t j = 0; j < n_jobs; j++) outs[j] = HostCopy{jobs[j].y, yh + offs[j] * 4, t * jobs[j].w->v.n_out * 4};
+    const bool whole = out == hipSuccess && host_copy_arriving(outs.data(), n_jobs, ends, chunks, chunks > 1 ? COPY_SHARE : COPY_PER_THREAD, [&](size_t k) {
+        return (k + 1 < chunks ? hipEventSynchronize(c->chunk_came[k]) : hipStreamSynchronize(s)) == hipSuccess;
+    });
+    if (!whole) {
+        (void)hipStreamSynchronize(s);  // (whatever still comes goes to the staging)
+        set_error("matmul: kernels or copy-out failed");
+        return 0;
+    }
     float a = 0, b = 0, d = 0;
-    (void)hipEventElapsedTime(&a, e0, e1);
-    (void)hipEventElapsedTime(&b, e1, e2);
-    (void)hipEventElapsedTime(&d, e2, e3);
+    (void)hipEventElapsedTime(&a, c->span[0], c->span[1]);
+    (void)hipEventElapsedTime(&b, c->span[1], c->span[2]);
+    (void)hipEventElapsedTime(&d, c->span[2], c->span[3]);
     c->ms_in += a;
     c->ms_gpu += b;
     c->ms_out += d;
     c->calls++;
-    return done(1);
+    return 1;
 }
 
 }  // extern "C"

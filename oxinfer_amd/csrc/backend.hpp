@@ -24,6 +24,8 @@ inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
         }                                                                                \
     } while (0)
 
+constexpr size_t OUT_CHUNKS = 5;  // large results of oxhip_matmul cross the host link in this many copies
+
 constexpr size_t VRAM_RESERVE = 512ull << 20;  // kept free for activations (src/cuda.rs:573-588)
 
 struct DevBuf {
@@ -102,6 +104,8 @@ struct oxhip_ctx {
     std::mutex mu;  // serializes the host-pointer surface (staging is shared), as Mutex<Staging> does
     oxhip::DevBuf x, xq, y;
     oxhip::PinnedBuf pin;   // results of oxhip_matmul on their way over the host link
+    hipEvent_t span[4] = {};                          // its call's timing: start, input there, kernels done, results there
+    hipEvent_t chunk_came[oxhip::OUT_CHUNKS - 1] = {};  // a chunk of its results has come (the last one: the stream is done)
     oxhip::DevBuf gemm_ws;  // packed activations of the prefill GEMMs
     oxhip::DecodeScratch dec;  // partial rows and counters of the decode kernels that split K across workgroups (host surface, on `stream`)
     std::mutex smu;            // guards per_stream

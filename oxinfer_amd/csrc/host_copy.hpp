@@ -1,5 +1,6 @@
 // Copies between host buffers by several threads (the results of the host surface on their way out of page-locked memory).
 #pragma once
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
@@ -14,14 +15,16 @@ struct HostCopy {
     size_t bytes;
 };
 
-constexpr size_t COPY_THREADS = 8, COPY_PER_THREAD = (size_t)2 << 20;
+constexpr size_t COPY_THREADS = 8, COPY_PER_THREAD = (size_t)2 << 20, COPY_SHARE = (size_t)256 << 10;
 
-// Copies the pieces, large ones by several threads: a thread moves some 10 GB/s between page-locked and ordinary memory, a
-// fifth of what the host link does. Every piece of work is done when it returns, also where no thread could be started. Pieces whose
-// destinations overlap go one after the other, by the caller: what a later one writes stays.
-inline void host_copy(const HostCopy* pieces, size_t n) {
-    size_t total = 0;
-    for (size_t i = 0; i < n; i++) total += pieces[i].bytes;
+// Copies the pieces while their bytes arrive: chunk c of `chunks` ends at byte ends[c] of all of them in a row (the last one at their
+// end). wait(c), called by the caller's thread for c = 0, 1, ... in order, returns once chunk c is there, or false if it never will be
+// (then what is not copied yet stays as it was, and the result is false). Large chunks go by several threads, each its share of every chunk: a thread moves some
+// 10 GB/s between page-locked and ordinary memory, a fifth of what the host link does. Every piece of work is done when it
+// returns, also where no thread could be started. Pieces whose destinations overlap go one after the other, by the caller: what a
+// later one writes stays.
+template <class Wait>
+inline bool host_copy_arriving(const HostCopy* pieces, size_t n, const size_t* ends, size_t chunks, size_t per_thread, Wait wait) {
     auto range = [pieces, n](size_t lo, size_t hi) {  // bytes lo .. hi of the pieces in a row
         size_t at = 0;
         for (size_t i = 0; i < n && at < hi; at += pieces[i++].bytes) {
@@ -35,18 +38,45 @@ inline void host_copy(const HostCopy* pieces, size_t n) {
             const uintptr_t a = reinterpret_cast<uintptr_t>(pieces[i].dst), b = reinterpret_cast<uintptr_t>(pieces[j].dst);
             overlap |= a < b + pieces[j].bytes && b < a + pieces[i].bytes;
         }
-    size_t parts = overlap ? 1 : total / COPY_PER_THREAD;
+    size_t parts = overlap ? 1 : ends[chunks - 1] / chunks / per_thread;
     parts = parts < 1 ? 1 : parts > COPY_THREADS ? COPY_THREADS : parts;
-    const size_t per = ((total + parts - 1) / parts + 4095) / 4096 * 4096;
+    auto share = [=](size_t k, size_t c) {  // thread k's share of chunk c
+        const size_t lo = c ? ends[c - 1] : 0, hi = ends[c], per = ((hi - lo + parts - 1) / parts + 4095) / 4096 * 4096;
+        range(lo + k * per < hi ? lo + k * per : hi, lo + (k + 1) * per < hi ? lo + (k + 1) * per : hi);
+    };
+    std::atomic<size_t> arrived{0};  // chunks; NEVER: no more will come
+    constexpr size_t NEVER = ~(size_t)0;
+    auto work = [&](size_t k) {
+        for (size_t c = 0; c < chunks; c++) {
+            size_t a;
+            while ((a = arrived.load(std::memory_order_acquire)) <= c) std::this_thread::yield();
+            if (a == NEVER) return;
+            share(k, c);
+        }
+    };
     std::thread th[COPY_THREADS];
-    size_t k = 1;  // part 0 is the caller's
+    size_t k = 1;  // share 0 is the caller's
     try {
-        for (; k < parts; k++) th[k] = std::thread(range, k * per < total ? k * per : total, (k + 1) * per < total ? (k + 1) * per : total);
+        for (; k < parts; k++) th[k] = std::thread(work, k);
     } catch (const std::exception&) {  // no more threads, or no memory for one's state: the caller does the rest
     }
-    range(0, per < total ? per : total);
-    if (k < parts) range(k * per < total ? k * per : total, total);
+    bool ok = true;
+    for (size_t c = 0; c < chunks && ok; c++) {
+        ok = wait(c);
+        arrived.store(ok ? c + 1 : NEVER, std::memory_order_release);
+        if (!ok) break;
+        share(0, c);
+        for (size_t i = k; i < parts; i++) share(i, c);
+    }
     for (size_t i = 1; i < k; i++) th[i].join();
+    return ok;
+}
+
+// The same for bytes that are there.
+inline void host_copy(const HostCopy* pieces, size_t n) {
+    size_t total = 0;
+    for (size_t i = 0; i < n; i++) total += pieces[i].bytes;
+    (void)host_copy_arriving(pieces, n, &total, 1, COPY_PER_THREAD, [](size_t) { return true; });
 }
 
 }  // namespace oxhip

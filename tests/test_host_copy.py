@@ -92,3 +92,39 @@ def test_overlapping_results_keep_the_order_of_the_jobs(build):
     exe = build(OVERLAP)
     for _ in range(3):
         assert subprocess.run([exe], timeout=60).returncode == 0
+
+
+ARRIVING = r"""
+#include "host_copy.hpp"
+#include <cstdlib>
+#include <vector>
+
+// argv: the chunk that never comes (-1: all come), the chunks' ends; two pieces, the second a third of the bytes
+int main(int argc, char** argv) {
+    const long never = std::atol(argv[1]);
+    std::vector<size_t> ends;
+    for (int i = 2; i < argc; i++) ends.push_back((size_t)std::atoll(argv[i]));
+    const size_t total = ends.back(), first = total - total / 3;
+    std::vector<unsigned char> src(total + 1, 0), dst(total + 2, 0xEE);
+    const oxhip::HostCopy pieces[2] = {{dst.data(), src.data(), first}, {dst.data() + first + 1, src.data() + first, total - first}};
+    size_t told = 0;
+    const bool ok = oxhip::host_copy_arriving(pieces, 2, ends.data(), ends.size(), 4096, [&](size_t c) {
+        if (c != told++ || (long)c == never) return false;
+        for (size_t k = c ? ends[c - 1] : 0; k < ends[c]; k++) src[k] = (unsigned char)(k * 31 + (k >> 12) + 1);
+        return true;
+    });
+    const size_t there = never < 0 ? total : never ? ends[never - 1] : 0;
+    if (ok != (never < 0) || told != (never < 0 ? ends.size() : (size_t)never + 1)) return 1;
+    for (size_t k = 0; k < total; k++)
+        if (dst[k + (k >= first)] != (k < there ? (unsigned char)(k * 31 + (k >> 12) + 1) : 0xEE)) return 2;
+    return dst[first] != 0xEE || dst[total + 1] != 0xEE;
+}
+"""
+
+
+def test_chunks_are_copied_as_they_come_and_no_others(build):
+    """Each chunk by all threads once it has come, in order; after one that never comes nothing more."""
+    exe = build(ARRIVING)
+    for ends in ((1,), (4096,), (3000, 3000, 9001), (5 << 20, 9 << 20, 12 << 20, 14 << 20, (15 << 20) - 3)):
+        for never in (-1, *range(len(ends))):
+            assert subprocess.run([exe, str(never), *map(str, ends)], timeout=60).returncode == 0, (ends, never)
