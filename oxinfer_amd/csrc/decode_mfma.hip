@@ -58,8 +58,9 @@ namespace {
 
 // Records a wave keeps in flight. HBM delivers about 8 TB/s at about 2 us of loaded latency, so some 16 MB must be
 // on request across the chip at any moment: about 4000 resident waves x PF KiB. Q6_K's records are 1.7 KiB and its step needs
-// the registers; so does that of the 8-bit formats at 9 to 16 tokens, which with eight records took 139 of them, one workgroup of
-// eight waves per CU, with four 103 (a pair of 14336 x 4096 in Q8_0 at 16 tokens 30.7 -> 25.5 us, 4096 x 4096 9.3 -> 7.2).
+// the registers; so did that of the 8-bit formats at 9 to 16 tokens, which with eight records took 139 of them, one workgroup of
+// eight waves per CU, with four 103 (a pair of 14336 x 4096 in Q8_0 at 16 tokens 30.7 -> 25.5 us, 4096 x 4096 9.3 -> 7.2); with its
+// LDS reads ahead of their use it takes 88.
 template <int FMT, int NT>
 constexpr int pf_for() { return FMT == FMT_Q6_K || (NT == 16 && q8_format(FMT)) ? 4 : 8; }
 
@@ -209,7 +210,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     const uint32_t slice = GROUPED ? 0 : by;
     const uint32_t sl = (nsteps + ksplit - 1) >> kssh;
     const uint32_t S0 = min(nsteps, slice * fs * sl), S1 = min(nsteps, S0 + fs * sl);  // (the workgroup's fs slices)
-    const uint32_t B0 = BPS * S0, nbl = BPS * fs * sl, M0 = B0 / 2;
+    const uint32_t B0 = BPS * S0, nbl = BPS * fs * sl;
     // LDS: [operand-order activations: 512 B per pair of blocks] [scales, sums] [partial sums]; with ALDS the
     // partial sums reuse the activations' space once every wave is done with them
     uint2* afr = reinterpret_cast<uint2*>(lds_all);  // [NG][nbl / 2][64]; 16 tokens: [nbl][64]
@@ -304,8 +305,8 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     // before its other half is asked for: Q6_K's launch fetched 7.5 % more than its records hold, one line per record.)
     constexpr int NM = FMT == FMT_Q8_0 || FMT == FMT_MXFP4 ? 1 : (k45_format(FMT) || FMT == FMT_Q6_K) ? 3 : 2;  // (Q8F: the two f32 scales)
     uint32_t slast = max(s1, 1u) - 1;
-    // (Q6_K: with the clamp's bound opaque the compiler keeps 111 registers instead of 141 and a fourth wave per SIMD fits: the
-    // shared launch of four Q6_K matmuls 47.9 -> 45.6 us. The other formats' kernels do not gain, Q4_0's loses.)
+    // (Q6_K: with the clamp's bound opaque the compiler kept 111 registers instead of 141 and a fourth wave per SIMD fits: the
+    // shared launch of four Q6_K matmuls 47.9 -> 45.6 us. The other formats' kernels did not gain, Q4_0's lost.)
     if constexpr (FMT == FMT_Q6_K) asm volatile("" : "+v"(slast));
     auto load_scales = [&](uint32_t* m, uint32_t first) {
         const uint32_t s = min(first + kq, slast);
@@ -351,44 +352,78 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     // Q6_K: every lane group sums its own 16-column sub-block for tokens 4 tg + i
     constexpr int NTG = NT <= 4 ? 1 : NT <= 8 ? 2 : 4;
     float acc6[4][4] = {};
-    // `m`: index of the instruction along K (pair of blocks 2 m, 2 m + 1); with ALDS its operand comes from LDS
-    auto mfma = [&](v4i bw, uint32_t m, int tg, uint32_t d0, uint32_t d1) -> v4i {
-        v4i c = {0, 0, 0, 0};
-        if (ALDS) {
-            const uint2 av = afr[((size_t)tg * (nbl / 2) + (m - M0)) * 64 + (SWZ ? opslot(m - M0, lane) : lane)];
-            d0 = av.x;
-            d1 = av.y;
+    // What a step reads from LDS: the operands of its NA instructions, the activation scales of the lane's tokens in their blocks
+    // and, for the mins' instruction, the lane's block sum. Each of these reads takes a hundred cycles and more, and a step that
+    // waits for its own, instruction by instruction, spends most of its time there with the few waves per SIMD that a lone launch
+    // has. So a step asks for its scales first, issues its products on operands that have come during the step before, asks for
+    // the next step's, and then adds up. Two MLX 4-bit layers (4096 / 14336) at 16 tokens 141.0 -> 126.7 us, MoE decode of
+    // one token 19.05 -> 18.4, two Q8_0 layers at 8 tokens 130.3 -> 128.6, two
+    // Q6_K layers of 2560 / 6912 at 2 / 8 / 16 tokens 76.8 / 96.1 / 131.1 -> 72.9 / 91.9 / 125.9. What bounds a lone launch of 4096 rows
+    // now is its ramp (arguments, staging, the first records) and the join of its waves. (All reads in one batch a step ahead: 20 to
+    // 30 registers more, spilled at 16 tokens.)
+    // (Blocks past the row lie inside the slice's arrays all the same: their scales and sums are staged as zero.)
+    constexpr int NA = WIDE ? (int)BPS : (int)BPS / 2;
+    struct Meta {
+        float xs[NA][4];
+        float f;
+    };
+    const uint32_t ulast = fs * sl - 1;  // the slice's last step, for reads ahead of its end
+    const uint32_t xs_lane = WIDE ? d_tok0 : d_half * TPAD + d_tok0;
+    const uint32_t f_lane = kq * TPAD + min(n, (uint32_t)TPAD - 1);
+    uint2 av[NA];
+    auto load_av = [&](uint32_t s, int tg, int i0, int i1) {  // instructions [i0, i1) of step `s` (of the slice's last one, if that lies before it)
+        if (!ALDS) return;
+        const uint32_t r0 = NA * min(s - S0, ulast);  // the step's first row of the operand array; NA divides it
+        const uint32_t xor0 = SWZ ? (r0 & 7u) ^ ((r0 & 8u) << 1) : 0u;
+#pragma unroll
+        for (int i = i0; i < i1; i++) av[i] = (afr + (size_t)tg * (nbl / 2) * 64 + 64 * i)[64 * r0 + ((lane ^ (SWZ ? i : 0)) ^ xor0)];
+    };
+    auto load_meta = [&](Meta& o, uint32_t s, int tg, int i0, int i1) {
+        const uint32_t at = BPS * TPAD * (s - S0);
+#pragma unroll
+        for (int i = i0; i < i1; i++) load_xs(lds + (size_t)tg * nm + i * (WIDE ? 1 : 2) * TPAD, at + xs_lane, o.xs[i]);
+        if (MINS && i1 == NA) o.f = (lds + (size_t)as + tg * nm)[at + f_lane];
+    };
+    // Q6_K: the operands of products 2 j and 2 j + 1 of step `s` (of the slice's last one, if that lies before it): the lane's
+    // sub-block of 16 columns, token 4 tg + n % 4, in [64-column group][8 tokens (16 in the 16-token form)][kq]
+    uint4 av6[2];
+    auto load_av6 = [&](uint32_t s, int j) {
+        const uint4* at = reinterpret_cast<const uint4*>(afr) + (size_t)min(s - S0, ulast) * (WIDE ? 128 : 64) + (n & 3) * 4 + kq;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int h = (2 * j + k) / NTG, tg = (2 * j + k) % NTG;
+            av6[k] = at[h * (WIDE ? 64 : 32) + 16 * tg];
         }
-        v4i a = {(int)(d0 & amask0), (int)(d1 & amask0), (int)(d0 & amask1), (int)(d1 & amask1)};
+    };
+    // (not where a step has several token groups, nor for Q6_K, which reads its own way, nor for Q5_K at 16 tokens, which has no
+    // registers left)
+    constexpr bool AHEAD = NG == 1 && FMT != FMT_Q6_K && !(WIDE && FMT == FMT_Q5_K);
+    // instruction `i` of a step on the lane's 16 codes `bw` (a pair of blocks) ...
+    auto mfma = [&](v4i bw, int i, uint32_t d0, uint32_t d1) -> v4i {
+        const v4i c = {0, 0, 0, 0};
+        if (ALDS) {
+            d0 = av[i].x;
+            d1 = av[i].y;
+        }
+        const v4i a = {(int)(d0 & amask0), (int)(d1 & amask0), (int)(d0 & amask1), (int)(d1 & amask1)};
         return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bw, c, 0, 0, 0);
     };
-    // 16 tokens: block `b`'s sums of 16 tokens x 16 rows, `w0`, `w1` the lane's 8 codes of it
-    auto mfma16 = [&](int w0, int w1, uint32_t b) -> v4i {
-        const uint2 av = afr[(size_t)(b - B0) * 64 + opslot(b - B0, lane)];
+    // ... in the 16-token form on its 8 codes `w0`, `w1` of block `i`
+    auto mfma16 = [&](int w0, int w1, int i) -> v4i {
         const v4i c = {0, 0, 0, 0};
-        return __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, av), __builtin_bit_cast(long, make_uint2((uint32_t)w0, (uint32_t)w1)), c, 0, 0, 0);
+        return __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, av[i]), __builtin_bit_cast(long, make_uint2((uint32_t)w0, (uint32_t)w1)), c, 0, 0, 0);
     };
-    auto wide_block = [&](int w0, int w1, uint32_t b, float d, float* sum) {
-        const v4i D = mfma16(w0, w1, b);
-        float xs[4];
-        load_xs(lds, (min(b, nblk - 1) - B0) * TPAD + d_tok0, xs);
+    // sum += d (xs I) over the lane's tokens
+    auto scale_add = [&](const v4i& D, float d, const float* xs, float* sum) {
         const int I[4] = {D.x, D.y, D.z, D.w};
 #pragma unroll
-        for (int i = 0; i < 4; i++) sum[i] = fmaf(d, xs[i] * (float)I[i], sum[i]);
+        for (int i = 0; i < NI; i++) sum[i] = fmaf(d, xs[i] * (float)I[i], sum[i]);
     };
-    // The m * fs terms of the step's four blocks (blocks b4 .. b4 + 3): rows = tokens (past TPAD: none), K = the blocks;
-    // this lane supplies fs of (token n, block b4 + kq) and `mk`, row n's m of block b4 + kq. D[4 kq + i][n]: the lane
+    // The m * fs terms of the step's four blocks: rows = tokens (past TPAD: none), K = the blocks;
+    // this lane supplies fs of (token n, block kq) and `mk`, row n's m of block kq. D[4 kq + i][n]: the lane
     // groups 0 and 1 receive the tokens their accumulators hold, the others zeros; in the 16-token form all four hold tokens.
-    auto mins = [&](uint32_t b4, float mk) {
-        if constexpr (MINS) {
-            // (a block past the row lies inside the slice's arrays all the same, staged as zero)
-            const uint32_t at = (b4 + kq - B0) * TPAD + min(n, (uint32_t)TPAD - 1);
-#pragma unroll
-            for (int tg = 0; tg < NG; tg++) {
-                const float f = lds[(size_t)as + tg * nm + at];
-                macc[tg] = __builtin_amdgcn_mfma_f32_16x16x4f32(WIDE || n < (uint32_t)TPAD ? f : 0.0f, mk, macc[tg], 0, 0, 0);
-            }
-        }
+    auto mins = [&](const Meta& o, int tg, float mk) {
+        if constexpr (MINS) macc[tg] = __builtin_amdgcn_mfma_f32_16x16x4f32(WIDE || n < (uint32_t)TPAD ? o.f : 0.0f, mk, macc[tg], 0, 0, 0);
     };
     // a nibble moved to the top of its byte with its top bit flipped: one three-input bit operation per operand dword
     // (plus the shift for the low nibbles)
@@ -405,25 +440,56 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     };
     auto compute_step = [&](const Step<FMT>& st, const uint32_t* sw, uint32_t s) {
         const uint4 c = st.w;
-        if constexpr (WIDE && q8_format(FMT)) {
-            const float d0 = FMT == FMT_Q8F ? __uint_as_float(sw[0]) : f16_bits_to_f32((uint16_t)(sw[0] & 0xFFFF));
-            const float d1 = FMT == FMT_Q8F ? __uint_as_float(sw[NM - 1]) : f16_bits_to_f32((uint16_t)(sw[0] >> 16));
-            wide_block((int)c.x, (int)c.y, 2 * s, d0, acc[0]);
-            wide_block((int)c.z, (int)c.w, 2 * s + 1, d1, acch);
-        } else if constexpr (q8_format(FMT)) {
-            const float d = FMT == FMT_Q8F ? __uint_as_float(d_half ? sw[NM - 1] : sw[0]) : f16_bits_to_f32((uint16_t)(d_half ? sw[0] >> 16 : sw[0] & 0xFFFF));
-            v4i bw = {(int)c.x, (int)c.y, (int)c.z, (int)c.w};
-            const uint32_t b = 2 * s + d_half;
+        Meta o;
+        if constexpr (AHEAD) {
+            load_meta(o, s, 0, 0, NA);
+            __builtin_amdgcn_sched_barrier(0);  // (the compiler would put the reads back to their uses)
+        }
+        // `bw[i]`: the operand of instruction i (a pair of blocks); `d(i, half)`: the scale of its block `half` for
+        // this lane's row.
+        auto products = [&](const v4i* bw, auto d, float mk) {
+            auto add_up = [&](const v4i& D, int tg, int i) {
+                if constexpr (WIDE) {
+                    scale_add(D, d(i / 2, i & 1), o.xs[i], i & 1 ? acch : acc[0]);
+                } else {
+                    scale_add(D, d(i, d_half), o.xs[i], acc[tg]);
+                    if (DUMP) {
+                        constexpr int SH = q8_format(FMT) || FMT == FMT_MXFP4 ? 0 : FMT == FMT_Q5_K ? 3 : 4;
+                        const int isum[4] = {D.x >> SH, D.y >> SH, D.z >> SH, D.w >> SH};
+                        dump_block(BPS * s + 2 * i + d_half, isum);
+                    }
+                }
+            };
+            auto product = [&](int i) {
+                if constexpr (WIDE) return i & 1 ? mfma16(bw[i / 2].z, bw[i / 2].w, i) : mfma16(bw[i / 2].x, bw[i / 2].y, i);
+                else return mfma(bw[i], i, st.a[2 * i], st.a[2 * i + 1]);
+            };
+            if constexpr (AHEAD) {
+                v4i D[NA];
 #pragma unroll
-            for (int tg = 0; tg < NG; tg++) {
-                v4i D = mfma(bw, s, tg, st.a[0], st.a[1]);
-                float xs[4];
-                load_xs(lds, tg * nm + (min(b, nblk - 1) - B0) * TPAD + d_tok0, xs);
-                int isum[4] = {D.x, D.y, D.z, D.w};
+                for (int i = 0; i < NA; i++) D[i] = product(i);
+                load_av(s + 1, 0, 0, NA);
+                __builtin_amdgcn_sched_barrier(0);
+                mins(o, 0, mk);
 #pragma unroll
-                for (int i = 0; i < NI; i++) acc[tg][i] = fmaf(d, xs[i] * (float)isum[i], acc[tg][i]);
-                dump_block(b, isum);
+                for (int i = 0; i < NA; i++) add_up(D[i], 0, i);
+            } else {
+#pragma unroll
+                for (int i = 0; i < NA; i++)
+#pragma unroll
+                    for (int tg = 0; tg < NG; tg++) {
+                        load_av(s, tg, i, i + 1);
+                        load_meta(o, s, tg, i, i + 1);
+                        add_up(product(i), tg, i);
+                        if (i == NA - 1) mins(o, tg, mk);
+                    }
             }
+        };
+        if constexpr (q8_format(FMT)) {
+            const v4i bw = {(int)c.x, (int)c.y, (int)c.z, (int)c.w};
+            products(&bw, [&](int, uint32_t half) {
+                return FMT == FMT_Q8F ? __uint_as_float(half ? sw[NM - 1] : sw[0]) : f16_bits_to_f32((uint16_t)(half ? sw[0] >> 16 : sw[0] & 0xFFFF));
+            }, 0.0f);
         } else if constexpr (k45_format(FMT)) {
             // sw[0]: the step's four sub-block scales, sw[1]: its four mins (bytes), sw[2]: (d, dmin). One byte permute
             // gathers this lane's four: the scales of its two blocks (sub-blocks d_half and 2 + d_half of the step) and,
@@ -434,85 +500,81 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
             // byte, the inverted fifth bit on top
             constexpr bool FIVE = FMT == FMT_Q5_K;
             const float d16 = d * (FIVE ? 0.125f : 0.0625f);
-            const float dsc[2] = {d16 * (float)(pk & 0xFF), d16 * (float)((pk >> 8) & 0xFF)};
             // decode_i8's m of sub-block kq: 8 s - dmin * mn, 16 s for Q5_K (src/ggml.rs:1046-1073)
             const float mk = fmaf((FIVE ? 16.0f : 8.0f) * d, (float)((pk >> 16) & 0xFF), -(dmin * (float)(pk >> 24)));
+            v4i bw[2];
 #pragma unroll
             for (int pr = 0; pr < 2; pr++) {  // the two byte pairs of the lane's chunk
-                v4i bw;
+                const uint32_t x0 = pr ? c.z : c.x, x1 = pr ? c.w : c.y;
                 if constexpr (FIVE) {
                     constexpr uint32_t NIB = 0x78787878u, TOP = 0x80808080u;
-                    const uint32_t x0 = pr ? c.z : c.x, x1 = pr ? c.w : c.y, hb = ~st.h;
-                    bw = v4i{(int)(((x0 << 3) & NIB) | ((hb << (7 - 4 * pr)) & TOP)), (int)(((x1 << 3) & NIB) | ((hb << (6 - 4 * pr)) & TOP)),
-                             (int)(((x0 >> 1) & NIB) | ((hb << (5 - 4 * pr)) & TOP)), (int)(((x1 >> 1) & NIB) | ((hb << (4 - 4 * pr)) & TOP))};
+                    const uint32_t hb = ~st.h;
+                    bw[pr] = v4i{(int)(((x0 << 3) & NIB) | ((hb << (7 - 4 * pr)) & TOP)), (int)(((x1 << 3) & NIB) | ((hb << (6 - 4 * pr)) & TOP)),
+                                 (int)(((x0 >> 1) & NIB) | ((hb << (5 - 4 * pr)) & TOP)), (int)(((x1 >> 1) & NIB) | ((hb << (4 - 4 * pr)) & TOP))};
                 } else {
-                    const uint32_t x0 = pr ? c.z : c.x, x1 = pr ? c.w : c.y;
-                    bw = v4i{centre_lo(x0), centre_lo(x1), centre_hi(x0), centre_hi(x1)};
-                }
-                if constexpr (WIDE) {  // (the sub-blocks' scales are bytes 2 pr and 2 pr + 1 of sw[0])
-                    wide_block(bw.x, bw.y, 4 * s + 2 * pr, d16 * (float)((sw[0] >> (16 * pr)) & 0xFF), acc[0]);
-                    wide_block(bw.z, bw.w, 4 * s + 2 * pr + 1, d16 * (float)((sw[0] >> (16 * pr + 8)) & 0xFF), acch);
-                    continue;
-                }
-                const uint32_t b = 4 * s + 2 * pr + d_half;  // global index of this lane's block of 32
-#pragma unroll
-                for (int tg = 0; tg < NG; tg++) {
-                    v4i D = mfma(bw, 2 * s + pr, tg, st.a[2 * pr], st.a[2 * pr + 1]);
-                    float xs[4];
-                    load_xs(lds, tg * nm + (b - B0) * TPAD + d_tok0, xs);
-                    const int I[4] = {D.x, D.y, D.z, D.w};
-#pragma unroll
-                    for (int i = 0; i < NI; i++) acc[tg][i] = fmaf(dsc[pr], xs[i] * (float)I[i], acc[tg][i]);
-                    if (DUMP) {
-                        constexpr int SH = FIVE ? 3 : 4;
-                        int isum[4] = {I[0] >> SH, I[1] >> SH, I[2] >> SH, I[3] >> SH};
-                        dump_block(b, isum);
-                    }
+                    bw[pr] = v4i{centre_lo(x0), centre_lo(x1), centre_hi(x0), centre_hi(x1)};
                 }
             }
-            mins(4 * s, mk);
+            // (16 tokens: sub-block b's scale is byte b of sw[0]; else byte i of the permute's result is instruction i's)
+            products(bw, [&](int i, uint32_t half) { return d16 * (float)(WIDE ? (sw[0] >> (16 * i + 8 * half)) & 0xFF : (pk >> (8 * i)) & 0xFF); }, mk);
         } else if constexpr (FMT == FMT_Q6_K) {
             // Scales go per 16 columns, so an instruction's 16 operand slots are (sub-block sb, token t4): lane group kq
             // supplies sub-block kq's 16 activations of token t4 in the slots with sb = kq and zeros elsewhere, and lane
             // (kq, n) receives sub-block kq's exact sums for tokens 4 tg + i of row n. Eight tokens take two instructions.
             // The codes stay unsigned (0..63): a sub-block's value is xs * I - 32 * (xs * its activations' sum), the order of the
             // reference's terms; see Q6PACK for the second one.
+            // A step is 2 NTG products (its two groups of 64 columns times the groups of four tokens), taken two at a time: their
+            // scales and second terms are asked for, the products issued on operands that have come during the pair before, the
+            // next pair's asked for, the sums formed.
             const float d = f16_bits_to_f32((uint16_t)(sw[2] & 0xFFFF));
             const uint32_t hq[2] = {st.h.x, st.h.y};
             const bool on = (n >> 2) == kq;
-            const uint4* afr6 = reinterpret_cast<const uint4*>(afr);  // [64-column group][8 tokens (16 in the 16-token form)][kq]
 #pragma unroll
-            for (int h = 0; h < 2; h++) {  // the step's two groups of 64 columns
-                const uint32_t lo = h ? c.z : c.x, hi = h ? c.w : c.y, hh = hq[h];
-                const v4i bw = {(int)((lo & 0x0F0F0F0Fu) | ((hh & 0x03030303u) << 4)), (int)(((lo >> 4) & 0x0F0F0F0Fu) | (((hh >> 2) & 0x03030303u) << 4)),
-                                (int)((hi & 0x0F0F0F0Fu) | (((hh >> 4) & 0x03030303u) << 4)), (int)(((hi >> 4) & 0x0F0F0F0Fu) | (((hh >> 6) & 0x03030303u) << 4))};
-                const float dsc = d * (float)(int)(int8_t)((sw[h] >> (8 * kq)) & 0xFF);
-                const uint32_t m64 = 2 * s + h, b = 2 * m64 + (kq >> 1);  // the lane's 32-block (its scale's) and its half
-                const uint32_t at = (min(b, nblk - 1) - B0) * TPAD;
+            for (int j = 0; j < NTG; j++) {
+                float4 xs[2], cc[2];
+                int2 sp[2];
+                const uint32_t u = s - S0;
 #pragma unroll
-                for (int tg = 0; tg < NTG; tg++) {
-                    const uint4 av = afr6[((size_t)(m64 - M0) * (WIDE ? 16 : 8) + 4 * tg + (n & 3)) * 4 + kq];
-                    const v4i a = {on ? (int)av.x : 0, on ? (int)av.y : 0, on ? (int)av.z : 0, on ? (int)av.w : 0};
+                for (int k = 0; k < 2; k++) {
+                    const int h = (2 * j + k) / NTG, tg = (2 * j + k) % NTG;
+                    const uint32_t at = (4 * u + 2 * h + (kq >> 1)) * TPAD + 4 * tg;  // (the lane's 32-block and its half)
+                    xs[k] = *reinterpret_cast<const float4*>(lds + at);
+                    if constexpr (Q6PACK) sp[k] = *reinterpret_cast<const int2*>(reinterpret_cast<const int16_t*>(lds + as) + 2 * (at - 4 * tg) + TPAD * (kq & 1) + 4 * tg);
+                    else cc[k] = *reinterpret_cast<const float4*>(lds + (size_t)(1 + (kq & 1)) * as + at);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // (the compiler would put the reads back to their uses)
+                v4i D[2];
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const int h = (2 * j + k) / NTG;
+                    const uint32_t lo = h ? c.z : c.x, hi = h ? c.w : c.y, hh = hq[h];
+                    const v4i bw = {(int)((lo & 0x0F0F0F0Fu) | ((hh & 0x03030303u) << 4)), (int)(((lo >> 4) & 0x0F0F0F0Fu) | (((hh >> 2) & 0x03030303u) << 4)),
+                                    (int)((hi & 0x0F0F0F0Fu) | (((hh >> 4) & 0x03030303u) << 4)), (int)(((hi >> 4) & 0x0F0F0F0Fu) | (((hh >> 6) & 0x03030303u) << 4))};
+                    const v4i a = {on ? (int)av6[k].x : 0, on ? (int)av6[k].y : 0, on ? (int)av6[k].z : 0, on ? (int)av6[k].w : 0};
                     const v4i z = {0, 0, 0, 0};
-                    const v4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bw, z, 0, 0, 0);
-                    const float4 xs = *reinterpret_cast<const float4*>(lds + at + 4 * tg);
-                    const float xv[4] = {xs.x, xs.y, xs.z, xs.w};
-                    const int U[4] = {D.x, D.y, D.z, D.w};
+                    D[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bw, z, 0, 0, 0);
+                }
+                load_av6(j + 1 < NTG ? s : s + 1, j + 1 < NTG ? j + 1 : 0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const int h = (2 * j + k) / NTG, tg = (2 * j + k) % NTG;
+                    const float dsc = d * (float)(int)(int8_t)((sw[h] >> (8 * kq)) & 0xFF);
+                    const float xv[4] = {xs[k].x, xs[k].y, xs[k].z, xs[k].w};
+                    const int U[4] = {D[k].x, D[k].y, D[k].z, D[k].w};
                     int sq[4];
                     float cv[4];
                     if constexpr (Q6PACK) {
-                        const int2 sp = *reinterpret_cast<const int2*>(reinterpret_cast<const int16_t*>(lds + as) + 2 * at + TPAD * (kq & 1) + 4 * tg);
-                        sq[0] = (int16_t)sp.x, sq[1] = sp.x >> 16, sq[2] = (int16_t)sp.y, sq[3] = sp.y >> 16;
+                        sq[0] = (int16_t)sp[k].x, sq[1] = sp[k].x >> 16, sq[2] = (int16_t)sp[k].y, sq[3] = sp[k].y >> 16;
 #pragma unroll
                         for (int i = 0; i < NI; i++) cv[i] = -32.0f * (xv[i] * (float)sq[i]);
                     } else {
-                        const float4 cc = *reinterpret_cast<const float4*>(lds + (size_t)(1 + (kq & 1)) * as + at + 4 * tg);
-                        cv[0] = cc.x, cv[1] = cc.y, cv[2] = cc.z, cv[3] = cc.w;
+                        cv[0] = cc[k].x, cv[1] = cc[k].y, cv[2] = cc[k].z, cv[3] = cc[k].w;
                     }
 #pragma unroll
                     for (int i = 0; i < NI; i++) acc6[tg][i] = fmaf(dsc, fmaf(xv[i], (float)U[i], cv[i]), acc6[tg][i]);
                     if (DUMP) {
-                        const uint32_t row = tile * 16 + n;
+                        const uint32_t row = tile * 16 + n, m64 = 2 * s + h, b = 2 * m64 + (kq >> 1);
 #pragma unroll
                         for (int i = 0; i < 4; i++) {
                             if (4 * tg + i < (int)t && row < w.n_out && b < nblk)
@@ -522,58 +584,25 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                 }
             }
         } else {
+            constexpr bool MX = FMT == FMT_MXFP4;  // table codes: the int8 operand is the code's doubled value itself
+            constexpr uint32_t NIB = 0x0F0F0F0Fu;
+            v4i bw[2];
 #pragma unroll
             for (int g = 0; g < 2; g++) {  // the two groups of 64 of the step
                 const uint32_t x0 = g ? c.z : c.x, x1 = g ? c.w : c.y;  // blocks 2 g, 2 g + 1
-                constexpr bool MX = FMT == FMT_MXFP4;  // table codes: the int8 operand is the code's doubled value itself
-                constexpr uint32_t NIB = 0x0F0F0F0Fu;
-                v4i bw = MX ? v4i{(int)mxfp4_values<0>(x0 & NIB), (int)mxfp4_values<0>((x0 >> 4) & NIB), (int)mxfp4_values<0>(x1 & NIB),
-                                  (int)mxfp4_values<0>((x1 >> 4) & NIB)}
-                            : v4i{centre_lo(x0), centre_hi(x0), centre_lo(x1), centre_hi(x1)};
-                if constexpr (WIDE) {
-                    const uint32_t b = 4 * s + 2 * g;
-                    float d0, d1;
-                    if constexpr (MX) {
-                        d0 = e8m0_half((sw[0] >> (16 * g)) & 0xFF);
-                        d1 = e8m0_half((sw[0] >> (16 * g + 8)) & 0xFF);
-                    } else if constexpr (FMT == FMT_Q40) {
-                        d0 = f16_bits_to_f32((uint16_t)(sw[g] & 0xFFFF)) * 0.0625f;
-                        d1 = f16_bits_to_f32((uint16_t)(sw[g] >> 16)) * 0.0625f;
-                    } else {
-                        d0 = d1 = f16_bits_to_f32((uint16_t)(g ? sw[0] >> 16 : sw[0] & 0xFFFF)) * 0.0625f;
-                    }
-                    wide_block(bw.x, bw.y, b, b < nblk ? d0 : 0.0f, acc[0]);
-                    wide_block(bw.z, bw.w, b + 1, b + 1 < nblk ? d1 : 0.0f, acch);
-                    continue;
-                }
-                const uint32_t b = 4 * s + 2 * g + d_half;
-                // MLX: the group's scale; Q4_0: the lane's block's own scale (word g, half d_half); MXFP4: its scale byte
-                float d;
-                if constexpr (MX) d = e8m0_half((sw[0] >> (8 * (2 * g + d_half))) & 0xFF);
-                else if constexpr (FMT == FMT_Q40) d = f16_bits_to_f32((uint16_t)(d_half ? sw[g] >> 16 : sw[g] & 0xFFFF));
-                else d = f16_bits_to_f32((uint16_t)(g ? sw[0] >> 16 : sw[0] & 0xFFFF));
-                // padding blocks hold zero codes (which centre to -8) and zero scales: they add zeros (as a select, not a
-                // branch: a divergent branch here makes every step wait for all requests)
-                const float dz = b < nblk ? (MX ? d : d * 0.0625f) : 0.0f;
-#pragma unroll
-                for (int tg = 0; tg < NG; tg++) {
-                    v4i D = mfma(bw, 2 * s + g, tg, st.a[2 * g], st.a[2 * g + 1]);
-                    float xs[4];
-                    load_xs(lds, tg * nm + (min(b, nblk - 1) - B0) * TPAD + d_tok0, xs);
-                    const int I[4] = {D.x, D.y, D.z, D.w};
-#pragma unroll
-                    for (int i = 0; i < NI; i++) acc[tg][i] = fmaf(dz, xs[i] * (float)I[i], acc[tg][i]);
-                    if (DUMP) {
-                        constexpr int SH = MX ? 0 : 4;
-                        int isum[4] = {I[0] >> SH, I[1] >> SH, I[2] >> SH, I[3] >> SH};
-                        dump_block(b, isum);
-                    }
-                }
+                bw[g] = MX ? v4i{(int)mxfp4_values<0>(x0 & NIB), (int)mxfp4_values<0>((x0 >> 4) & NIB), (int)mxfp4_values<0>(x1 & NIB),
+                                 (int)mxfp4_values<0>((x1 >> 4) & NIB)}
+                           : v4i{centre_lo(x0), centre_hi(x0), centre_lo(x1), centre_hi(x1)};
             }
-            if constexpr (FMT == FMT_Q4M) {  // the offset of block kq's group of 64, times the block's exact activation sum
-                const float off = bf16_bits_to_f32((uint16_t)(kq >> 1 ? sw[1] >> 16 : sw[1] & 0xFFFF));
-                mins(4 * s, 4 * s + kq < nblk ? off : 0.0f);
-            }
+            // MLX: the scale of the block's group; Q4_0: the block's own (word b / 2, half b % 2); MXFP4: its scale byte. Padding
+            // blocks hold zero codes (which centre to -8), zero scales and zero activation scales: they add zeros.
+            float off = 0.0f;  // MLX: the offset of block kq's group of 64, times the block's exact activation sum
+            if constexpr (FMT == FMT_Q4M) off = bf16_bits_to_f32((uint16_t)(kq >> 1 ? sw[1] >> 16 : sw[1] & 0xFFFF));
+            products(bw, [&](int i, uint32_t half) {
+                if constexpr (MX) return e8m0_half((sw[0] >> (16 * i + 8 * half)) & 0xFF);
+                else if constexpr (FMT == FMT_Q40) return f16_bits_to_f32((uint16_t)(half ? sw[i] >> 16 : sw[i] & 0xFFFF)) * 0.0625f;
+                else return f16_bits_to_f32((uint16_t)(i ? sw[0] >> 16 : sw[0] & 0xFFFF)) * 0.0625f;
+            }, off);
         }
     };
 
@@ -812,6 +841,8 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
             }
         }
     };
+    if constexpr (AHEAD) load_av(s0, 0, 0, NA);
+    if constexpr (FMT == FMT_Q6_K) load_av6(s0, 0);
     uint32_t sb = s0;
     for (; sb + PF < s1; sb += PF) {
 #pragma unroll
@@ -1079,13 +1110,13 @@ inline const void* sums_of(int fmt, const QActView& v) { return fmt == FMT_Q6_K 
 // into dwords (and the kernel runs two to three times longer) when the array starts at an odd dword.
 // (Grouped launches keep to 8 waves, which leaves them 256 registers for the accumulators of their token groups; with chunks of
 // five to eight rows they are bounded to four waves per SIMD, MLX 4-bit to five: unbounded that kernel took 139 registers and
-// spilled 36 scalar ones.)
+// spilled 36 scalar ones; those of several token groups to four, MXFP4's would take 184.)
 // Such a launch has chunks of any length up to its own, and those of up to four rows, the most of them where an expert has few
 // routed rows, run the four-row body. 128 MLX 4-bit experts of 2048 / 768, eight a token, every chunk in the eight-row body of
 // before -> this: 24 tokens routed at random 85.5 -> 64.1 us, 47 tokens all to the same eight experts 53.8 -> 42.0 us. (Chunks of
 // four rows throughout make two passes over the weights of an expert with more: 63.0 and 55.1 us.)
 template <int FMT, int NT, bool DUMP, bool GROUPED, bool ALDS, int NG>
-__global__ __launch_bounds__(GROUPED ? 512 : 1024, GROUPED && NG == 1 && NT == 8 ? (FMT == FMT_Q4M && ALDS ? 5 : 4) : 1) void decode_mfma_kernel(LaunchArgs<GROUPED> a) {
+__global__ __launch_bounds__(GROUPED ? 512 : 1024, GROUPED && NT == 8 ? (FMT == FMT_Q4M && ALDS && NG == 1 ? 5 : 4) : 1) void decode_mfma_kernel(LaunchArgs<GROUPED> a) {
     extern __shared__ __align__(16) float lds_dyn[];
     WeightView w{};
     w.fmt = FMT;
@@ -1186,13 +1217,13 @@ inline int set_of(int fmt, uint32_t mask) {
     }
     return -1;
 }
-// (Q6_K shares the kernel of Q8_0 and Q4_K since its step keeps 111 registers: a Q4_K_M file's layers mix the three, and their
-// matmuls go out in one launch. Q4_0's kernel is bounded at 512 threads, which saves it nine spilled registers.)
+// (Q6_K shares the kernel of Q8_0 and Q4_K since its step leaves room for four waves per SIMD: a Q4_K_M file's layers mix the three,
+// and their matmuls go out in one launch. All are bounded to 128 registers: nothing spills, two workgroups of eight waves fit a CU.)
 // FAT: the launch's jobs use the fat mapping (see place_job); the plain kernels do without its bookkeeping.
 // WIDE: the launch's jobs have 9 to 16 tokens each (kernels of their own, for the registers; plain mappings, but compiled as FAT,
-// which keeps the GGUF set at 118 registers and two workgroups per CU: 143 without).
+// which keeps the GGUF set at 123 registers).
 template <uint32_t FSET, bool FAT, bool WIDE = false>
-__global__ __launch_bounds__(WIDE || FSET == (1u << FMT_Q40) ? 512 : 1024) void decode_batch_kernel(BatchArgs a) {
+__global__ __launch_bounds__(1024) void decode_batch_kernel(BatchArgs a) {
     extern __shared__ __align__(16) float lds_dyn[];
     uint32_t j = 0, bx = blockIdx.x;  // (uniform; every job's first workgroup is read at once)
 #pragma unroll
