@@ -473,45 +473,68 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 
 }
 
 // Adds the K slices in order: y = p[0] + p[1] + ... (f32 or bf16 out). VEC outputs per thread (4 when n is a multiple of 4 and
-// the buffers are 16-byte aligned).
-template <bool OUT_BF16, int VEC>
+// the buffers are 16-byte aligned). A launch that does not fill the chip is bound by its trips to memory, one per slice where a slice
+// is requested when the one before it has been added: BATCH requests eight, four, two and one at a time, the sums as they were
+// (rows of 4096 and 4095 floats, 16 slices of 17 to 49 tokens 4.8-5.3 -> 3.9-4.1 us, 8 slices of 65 to 193 tokens 4.8-7.1 -> 4.1-5.6).
+template <bool OUT_BF16, int VEC, bool BATCH>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ p, size_t n, uint32_t slices, void* __restrict__ yv) {
     const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * VEC;
     if (i >= n) return;
     float v[VEC];
-    if (VEC == 4) {
-        const float4 a = *reinterpret_cast<const float4*>(p + i);
-        v[0] = a.x; v[1 % VEC] = a.y; v[2 % VEC] = a.z; v[3 % VEC] = a.w;
-        for (uint32_t z = 1; z < slices; z++) {
-            const float4 b = *reinterpret_cast<const float4*>(p + (size_t)z * n + i);
-            v[0] += b.x; v[1 % VEC] += b.y; v[2 % VEC] += b.z; v[3 % VEC] += b.w;
+#pragma unroll
+    for (int k = 0; k < VEC; k++) v[k] = -0.0f;  // (the zero that leaves every first term as it is)
+    uint32_t z = 0;
+    auto add = [&](auto many) {
+        constexpr int M = decltype(many)::value;
+        float b[M][VEC];
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            const float* at = p + (size_t)(z + m) * n + i;
+            if constexpr (VEC == 4) {
+                const float4 f = *reinterpret_cast<const float4*>(at);
+                b[m][0] = f.x; b[m][1] = f.y; b[m][2] = f.z; b[m][3] = f.w;
+            } else {
+                b[m][0] = *at;
+            }
         }
+#pragma unroll
+        for (int m = 0; m < M; m++)
+#pragma unroll
+            for (int k = 0; k < VEC; k++) v[k] += b[m][k];
+        z += M;
+    };
+    if constexpr (BATCH) {
+        while (slices - z >= 8) add(std::integral_constant<int, 8>{});
+        if ((slices - z) & 4) add(std::integral_constant<int, 4>{});
+        if ((slices - z) & 2) add(std::integral_constant<int, 2>{});
+        if ((slices - z) & 1) add(std::integral_constant<int, 1>{});
+    } else {
+        while (z < slices) add(std::integral_constant<int, 1>{});
+    }
+    if constexpr (VEC == 4) {
         if (OUT_BF16) {
             *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(yv) + i) =
-                make_uint2(f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1 % VEC]) << 16),
-                           f32_to_bf16_bits(v[2 % VEC]) | ((uint32_t)f32_to_bf16_bits(v[3 % VEC]) << 16));
+                make_uint2(f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16), f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16));
         } else {
-            *reinterpret_cast<float4*>(reinterpret_cast<float*>(yv) + i) = make_float4(v[0], v[1 % VEC], v[2 % VEC], v[3 % VEC]);
+            *reinterpret_cast<float4*>(reinterpret_cast<float*>(yv) + i) = make_float4(v[0], v[1], v[2], v[3]);
         }
+    } else if (OUT_BF16) {
+        reinterpret_cast<uint16_t*>(yv)[i] = f32_to_bf16_bits(v[0]);
     } else {
-        v[0] = p[i];
-        for (uint32_t z = 1; z < slices; z++) v[0] += p[(size_t)z * n + i];
-        if (OUT_BF16) reinterpret_cast<uint16_t*>(yv)[i] = f32_to_bf16_bits(v[0]);
-        else reinterpret_cast<float*>(yv)[i] = v[0];
+        reinterpret_cast<float*>(yv)[i] = v[0];
     }
 }
 
+// Four outputs a thread: past 1.4 million of them the waves in flight cover the trips, and the plain loop streams better (4096 floats x 321
+// tokens, 4 slices 5.56 us plain, 5.44 batched; 385 tokens 5.76 and 5.88; 512 tokens of the 14336-column matrix 7.2 and 7.9).
+// One output a thread: 4 slices of 449 tokens 7.9 plain, 7.7 batched, and at most 2 % apart beyond.
 static void run_gemm_reduce(const float* partial, size_t n, uint32_t slices, void* y, bool out_bf16, hipStream_t s) {
     const bool wide = n % 4 == 0 && reinterpret_cast<uintptr_t>(partial) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
-    if (wide) {
-        const unsigned grid = (unsigned)((n / 4 + 255) / 256);
-        if (out_bf16) gemm_reduce_kernel<true, 4><<<grid, 256, 0, s>>>(partial, n, slices, y);
-        else gemm_reduce_kernel<false, 4><<<grid, 256, 0, s>>>(partial, n, slices, y);
-    } else {
-        const unsigned grid = (unsigned)((n + 255) / 256);
-        if (out_bf16) gemm_reduce_kernel<true, 1><<<grid, 256, 0, s>>>(partial, n, slices, y);
-        else gemm_reduce_kernel<false, 1><<<grid, 256, 0, s>>>(partial, n, slices, y);
-    }
+    const unsigned grid = (unsigned)((n / (wide ? 4 : 1) + 255) / 256);
+    auto go = [&](auto kern) { kern<<<grid, 256, 0, s>>>(partial, n, slices, y); };
+    if (!wide) out_bf16 ? go(gemm_reduce_kernel<true, 1, true>) : go(gemm_reduce_kernel<false, 1, true>);
+    else if (n <= 1400000) out_bf16 ? go(gemm_reduce_kernel<true, 4, true>) : go(gemm_reduce_kernel<false, 4, true>);
+    else out_bf16 ? go(gemm_reduce_kernel<true, 4, false>) : go(gemm_reduce_kernel<false, 4, false>);
 }
 
 // Token tiles per wave and waves per workgroup: one tile and four waves when the launch has at most four tiles (64 tokens),

@@ -390,6 +390,27 @@ def test_gemm_fp8_wide_scale_blocks_and_k_slices(be, oxref):
         assert row_err(y1, ref[:3]) < 1e-3
 
 
+@pytest.mark.parametrize("slices", [2, 3, 4, 7, 8, 9, 15, 16])
+def test_gemm_slice_sums(be, oxref, slices):
+    """The slices' sums are requested eight, four, two and one at a time, four outputs or one per thread (272 and 289 outputs): none is
+    left out or taken twice. Slices of four steps of 128 columns are what the plan picks for one row group. Against 64 bits within
+    f32 summation's bound (columns x 2^-24 of the terms' magnitudes; half a unit of bf16 more for a bf16 result)."""
+    import torch
+    from oxinfer_amd import synth
+    n_in, t = 512 * slices, 17
+    x = synth.activations(t, n_in, 75, bf16=True)
+    for n_out in (16, 17):
+        raw = synth.gguf_q8_0(n_out, n_in, 74)
+        w = be.upload_gguf(8, raw, n_out, n_in)
+        assert w is not None, be.last_error()
+        wb = synth.bf16_round(oxref.dequantize_rows(8, raw, n_out, n_in)).astype(np.float64)
+        ref, size = x.astype(np.float64) @ wb.T, np.abs(x).astype(np.float64) @ np.abs(wb).T
+        for out_bf16 in (False, True):
+            y = be.gemm(w, torch.from_numpy(x).cuda().to(torch.bfloat16), out_bf16=out_bf16).float().cpu().numpy()
+            bound = n_in * 2.0**-24 * size
+            assert (np.abs(y - ref) <= bound + (2.0**-8 * (np.abs(ref) + bound) if out_bf16 else 0)).all(), (n_out, out_bf16)
+
+
 def test_gemm_fp8_declines_other_shapes(be):
     import torch
     from oxinfer_amd import synth
