@@ -411,6 +411,33 @@ def test_gemm_slice_sums(be, oxref, slices):
             assert (np.abs(y - ref) <= bound + (2.0**-8 * (np.abs(ref) + bound) if out_bf16 else 0)).all(), (n_out, out_bf16)
 
 
+@pytest.mark.parametrize("t", [1, 4, 5, 8, 9, 16, 17, 31, 32])
+def test_fp8_few_tokens_packs_rows_at_any_alignment(be, oxref, t):
+    """The few-token FP8 kernel's fragments, one plane and two: rows that start on any element give the bits of aligned ones, and those
+    are the product's (f32 summation's bound, and the input's rounding: bf16's, or 2^-16 with the value kept in two planes)."""
+    import torch
+    from oxinfer_amd import synth
+    n_out, n_in = 48, 1152
+    data, scales = synth.fp8_e4m3(n_out, n_in, 77)
+    w = be.upload_fp8(data, scales, n_out, n_in)
+    wf = be.dequantize(w).cpu().numpy().astype(np.float64)
+    x = torch.from_numpy(synth.activations(t, n_in, 78)).cuda()
+    xf = x.cpu().numpy().astype(np.float64)
+    ref, size = xf @ wf.T, np.abs(xf) @ np.abs(wf).T
+
+    def shifted(v):
+        out = torch.empty(v.numel() + 1, dtype=v.dtype, device="cuda")[1:].view(v.shape)
+        return out.copy_(v)
+
+    runs = [(x, 2.0**-8, be.gemm), (x.to(torch.bfloat16), 2.0**-8, be.gemm)]
+    if t <= 16:
+        runs.append((x, 2.0**-16, lambda w, v: be.decode(w, x=v)))
+    for v, rounding, call in runs:
+        y = call(w, v)
+        assert torch.equal(y.view(torch.int32), call(w, shifted(v)).view(torch.int32))
+        assert (np.abs(y.cpu().numpy() - ref) <= (n_in * 2.0**-24 + rounding) * size).all()
+
+
 def test_gemm_fp8_declines_other_shapes(be):
     import torch
     from oxinfer_amd import synth
