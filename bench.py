@@ -438,7 +438,7 @@ def bench_moe(be, torch, synth, steps, warmup, pool_gb, t, experts, int8=False):
                 plans.append(be.plan_record(lambda d=d: be.moe_routed(d, x, logits, k, y, sel=sel)))
             pwall, pms = timed_steps(torch, lambda i: plans[i % len(plans)].replay(), steps, warmup)
             side.synchronize()
-        replayed = {"what": "the same pass as a recorded plan (oxhip_plan_replay: one submission for its launches)", "launches": int(plans[0].launches),
+        replayed = {"what": "the same pass as a recorded plan (oxhip_plan_replay: one call for its launches)", "launches": int(plans[0].launches),
                     "ms_per_step": round(pwall / steps * 1e3, 5), "value": round(nbytes * steps / pwall / 1e9, 2), "avg_us_by_events": round(pms * 1e3, 2)}
         del plans
     return dict(base_line(steps, warmup), value=round(nbytes * steps / wall / 1e9, 2), unit="GB/s", ms_per_step=round(wall / steps * 1e3, 5),

@@ -115,7 +115,9 @@ size_t oxhip_weight_bytes(const oxhip_weight* w);
  * src/kernels.rs:1908-1928); more than 16 tokens over MLX 4-bit, Q8, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4, NVFP4 or FP8 (128-column
  * blocks) weights run the bf16 matrix-core GEMM; everything else runs the decode kernels over 16 tokens at a time.
  * The results of a call come through page-locked host memory that the context keeps until oxhip_close: half more than the largest
- * call so far needed, at most 256 MiB (a call with more results does without it). Jobs whose y overlap are copied in their order. */
+ * call so far needed, at most 256 MiB (a call with more results does without it). Jobs whose y overlap are copied in their order.
+ * Results of 8 MiB and more are copied out chunk by chunk once all jobs have run: if the link fails between two of them, the call
+ * returns 0 with some of y written (every other 0 leaves y as it was). */
 int oxhip_matmul(oxhip_ctx* ctx, const float* x, size_t t, size_t n_in, oxhip_job* jobs, size_t n_jobs);
 /* Backend::matvec_rows (src/gpu.rs:165): t in 1..=4. The jobs over the matrix-core formats share one launch, a gate / up
  * job as a pair (see oxhip_dev_linear). */
@@ -319,7 +321,7 @@ int oxhip_dev_experts(oxhip_ctx* ctx, oxhip_moe* m, const float* x, size_t t, co
 int oxhip_dev_moe_routed(oxhip_ctx* ctx, oxhip_moe* m, const float* x, size_t t, const float* logits, size_t logit_stride, size_t k,
                          const float* expert_scale, uint32_t* sel, float* y, int add, void* stream);
 
-/* ---- a recorded chain of device-pointer ops, replayed as one submission ---------------------------------------------
+/* ---- a recorded chain of device-pointer ops, replayed with one call ---------------------------------------------
  * The matmul side of DecodePlan::step (src/gpu_decode.rs:572-587; CUDA's per-graph launch list, src/cuda_decode.rs:1044-1049):
  * a token's ops (norm + quantize, linears, route, experts, ...) are issued once between oxhip_plan_begin and
  * oxhip_plan_end on `stream` (a stream of the caller's, not the null stream), where they are recorded instead of run; every

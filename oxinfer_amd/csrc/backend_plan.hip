@@ -1,4 +1,4 @@
-// A recorded run of device-pointer ops that replays as one submission: the matmul side of the reference's DecodePlan
+// A recorded run of device-pointer ops that replays with one call: the matmul side of the reference's DecodePlan
 // (src/gpu_decode.rs:572-587; the CUDA backend builds a fixed launch list per graph once and re-issues it every token,
 // src/cuda_decode.rs:1044-1049). Here the list is a HIP graph captured from the library's own launches: between
 // oxhip_plan_begin and oxhip_plan_end every oxhip_dev_* call on the plan's stream is recorded instead of run, and

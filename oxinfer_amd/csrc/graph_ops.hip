@@ -84,20 +84,6 @@ __device__ __forceinline__ float rms_factor(double ss, uint32_t n, float eps) {
     return (float)y;
 }
 
-// RMSNorm of one row per workgroup (Op::Norm, src/gpu_decode.rs:53-66), then quantize_act of the row that was written,
-// without a round trip through memory:
-//   x' = x * pre;  r = (sum x'^2 / n + eps)^(-1/2);  v = (x' * r) * w  (or x' * r);  out = v, or out += v with `add`;
-//   what `out` then holds goes, per block of 32, to the QAct (optional).
-// The reference sums the squares one after the other in f32 (src/kernels.rs:2109), which no parallel machine can
-// repeat bit for bit in useful time: here the squares are exact in f64 and summed in f64 (a fixed order), the mean and
-// eps added in f32 as the reference does, and r is the correctly rounded power. The quantization of v is
-// quantize_act's, bit for bit (the same code on the same values). VEC: rows of x, out and w start on 16-byte boundaries
-// (float4 access); otherwise every access is one float.
-// The kernel is one row's chain of latencies, so a row takes as many threads as it has float4s (up to 1024), its values and
-// weights are requested together and stay in registers (NV float4s a thread; NV = 0: longer rows, read twice), and eight
-// lanes quantize a block where they hold it (4096 values, one row, in a replayed chain: 5.4 -> 4.4 us).
-// ONE row in one workgroup: rows that share memory with an output, very long rows, and launches of so many rows that they fill
-// the chip; the others go to rmsnorm_parts_kernel below, value for value.
 // The sum over a wave's 64 lanes, in every lane: lanes 32 apart first, then 16, 8, 4, 2 and 1 (a fixed order). In registers: the
 // halves and quarters change places with the lane swaps; from 8 on the values repeat, so that rotations within 16 lanes bring them.
 template <int CTRL>
@@ -120,6 +106,20 @@ __device__ __forceinline__ double wave_xor_sum(double v) {
     return v;
 }
 
+// RMSNorm of one row per workgroup (Op::Norm, src/gpu_decode.rs:53-66), then quantize_act of the row that was written,
+// without a round trip through memory:
+//   x' = x * pre;  r = (sum x'^2 / n + eps)^(-1/2);  v = (x' * r) * w  (or x' * r);  out = v, or out += v with `add`;
+//   what `out` then holds goes, per block of 32, to the QAct (optional).
+// The reference sums the squares one after the other in f32 (src/kernels.rs:2109), which no parallel machine can
+// repeat bit for bit in useful time: here the squares are exact in f64 and summed in f64 (a fixed order), the mean and
+// eps added in f32 as the reference does, and r is the correctly rounded power. The quantization of v is
+// quantize_act's, bit for bit (the same code on the same values). VEC: rows of x, out and w start on 16-byte boundaries
+// (float4 access); otherwise every access is one float.
+// The kernel is one row's chain of latencies, so a row takes as many threads as it has float4s (up to 1024), its values and
+// weights are requested together and stay in registers (NV float4s a thread; NV = 0: longer rows, read twice), and eight
+// lanes quantize a block where they hold it (4096 values, one row, in a replayed chain: 5.4 -> 4.4 us).
+// ONE row in one workgroup: rows that share memory with an output, very long rows, and launches of so many rows that they fill
+// the chip; the others go to rmsnorm_parts_kernel below, value for value.
 template <bool VEC, int NV>
 __global__ __launch_bounds__(1024) void rmsnorm_quantize_kernel(const float* __restrict__ x, const float* __restrict__ w_f32,
                                                                 const uint16_t* __restrict__ w_bf16, float eps, float pre, uint32_t add, uint32_t n,
