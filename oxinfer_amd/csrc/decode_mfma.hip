@@ -462,7 +462,14 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
             };
             auto product = [&](int i) {
                 if constexpr (WIDE) return i & 1 ? mfma16(bw[i / 2].z, bw[i / 2].w, i) : mfma16(bw[i / 2].x, bw[i / 2].y, i);
-                else return mfma(bw[i], i, st.a[2 * i], st.a[2 * i + 1]);
+                else if constexpr (FMT == FMT_MXFP4 && NG > 1) {
+                    // A pair's codes are looked up where they are used, pair after pair (the barrier below): with both pairs' made
+                    // ahead the kernels of two and four token groups take 184 and 194 registers, or spill 17 and 154 of them; this way 100
+                    // and 116. 128 / 32 experts of 2048 / 768 at 256 tokens: 238 / 152 us, spilled 203 / 209, this way 163 / 117.
+                    constexpr uint32_t NIB = 0x0F0F0F0Fu;
+                    uint32_t x0 = i ? c.z : c.x, x1 = i ? c.w : c.y;
+                    return mfma(v4i{(int)mxfp4_values<0>(x0 & NIB), (int)mxfp4_values<0>((x0 >> 4) & NIB), (int)mxfp4_values<0>(x1 & NIB), (int)mxfp4_values<0>((x1 >> 4) & NIB)}, i, 0, 0);
+                } else return mfma(bw[i], i, st.a[2 * i], st.a[2 * i + 1]);
             };
             if constexpr (AHEAD) {
                 v4i D[NA];
@@ -475,7 +482,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                 for (int i = 0; i < NA; i++) add_up(D[i], 0, i);
             } else {
 #pragma unroll
-                for (int i = 0; i < NA; i++)
+                for (int i = 0; i < NA; i++) {
 #pragma unroll
                     for (int tg = 0; tg < NG; tg++) {
                         load_av(s, tg, i, i + 1);
@@ -483,6 +490,8 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                         add_up(product(i), tg, i);
                         if (i == NA - 1) mins(o, tg, mk);
                     }
+                    if constexpr (NG > 1 && FMT == FMT_MXFP4) __builtin_amdgcn_sched_barrier(0);
+                }
             }
         };
         if constexpr (q8_format(FMT)) {
@@ -1110,7 +1119,7 @@ inline const void* sums_of(int fmt, const QActView& v) { return fmt == FMT_Q6_K 
 // into dwords (and the kernel runs two to three times longer) when the array starts at an odd dword.
 // (Grouped launches keep to 8 waves, which leaves them 256 registers for the accumulators of their token groups; with chunks of
 // five to eight rows they are bounded to four waves per SIMD, MLX 4-bit to five: unbounded that kernel took 139 registers and
-// spilled 36 scalar ones; those of several token groups to four, MXFP4's would take 184.)
+// spilled 36 scalar ones; those of several token groups to four.)
 // Such a launch has chunks of any length up to its own, and those of up to four rows, the most of them where an expert has few
 // routed rows, run the four-row body. 128 MLX 4-bit experts of 2048 / 768, eight a token, every chunk in the eight-row body of
 // before -> this: 24 tokens routed at random 85.5 -> 64.1 us, 47 tokens all to the same eight experts 53.8 -> 42.0 us. (Chunks of
