@@ -1,10 +1,11 @@
 // Copies between host buffers by several threads (the results of the host surface on their way out of page-locked memory).
 #pragma once
-#include <atomic>
+#include <condition_variable>
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <thread>
 
 namespace oxhip {
@@ -19,10 +20,11 @@ constexpr size_t COPY_THREADS = 8, COPY_PER_THREAD = (size_t)2 << 20, COPY_SHARE
 
 // Copies the pieces while their bytes arrive: chunk c of `chunks` ends at byte ends[c] of all of them in a row (the last one at their
 // end). wait(c), called by the caller's thread for c = 0, 1, ... in order, returns once chunk c is there, or false if it never will be
-// (then what is not copied yet stays as it was, and the result is false). Large chunks go by several threads, each its share of every chunk: a thread moves some
-// 10 GB/s between page-locked and ordinary memory, a fifth of what the host link does. Every piece of work is done when it
-// returns, also where no thread could be started. Pieces whose destinations overlap go one after the other, by the caller: what a
-// later one writes stays.
+// (then what is not copied yet stays as it was, and the result is false). Large chunks go by several threads, each its share of every
+// chunk: a thread moves some 10 GB/s between page-locked and ordinary memory, a fifth of what the host link does. The threads start
+// when the first chunk has come and sleep until the next one: what it takes before (the kernels that make the bytes) costs no core.
+// Every piece of work is done when it returns, also where no thread could be started. Pieces whose destinations overlap go one after
+// the other, by the caller: what a later one writes stays.
 template <class Wait>
 inline bool host_copy_arriving(const HostCopy* pieces, size_t n, const size_t* ends, size_t chunks, size_t per_thread, Wait wait) {
     auto range = [pieces, n](size_t lo, size_t hi) {  // bytes lo .. hi of the pieces in a row
@@ -44,13 +46,18 @@ inline bool host_copy_arriving(const HostCopy* pieces, size_t n, const size_t* e
         const size_t lo = c ? ends[c - 1] : 0, hi = ends[c], per = ((hi - lo + parts - 1) / parts + 4095) / 4096 * 4096;
         range(lo + k * per < hi ? lo + k * per : hi, lo + (k + 1) * per < hi ? lo + (k + 1) * per : hi);
     };
-    std::atomic<size_t> arrived{0};  // chunks; NEVER: no more will come
-    constexpr size_t NEVER = ~(size_t)0;
+    if (!wait(0)) return false;
+    std::mutex mu;
+    std::condition_variable more;
+    size_t arrived = 1;  // chunks (guarded by mu)
+    bool never = false;  // no more will come (guarded by mu)
     auto work = [&](size_t k) {
         for (size_t c = 0; c < chunks; c++) {
-            size_t a;
-            while ((a = arrived.load(std::memory_order_acquire)) <= c) std::this_thread::yield();
-            if (a == NEVER) return;
+            {
+                std::unique_lock<std::mutex> lk(mu);
+                more.wait(lk, [&] { return arrived > c || never; });
+                if (arrived <= c) return;
+            }
             share(k, c);
         }
     };
@@ -61,12 +68,17 @@ inline bool host_copy_arriving(const HostCopy* pieces, size_t n, const size_t* e
     } catch (const std::exception&) {  // no more threads, or no memory for one's state: the caller does the rest
     }
     bool ok = true;
-    for (size_t c = 0; c < chunks && ok; c++) {
-        ok = wait(c);
-        arrived.store(ok ? c + 1 : NEVER, std::memory_order_release);
-        if (!ok) break;
+    for (size_t c = 0; ok; c++) {
         share(0, c);
         for (size_t i = k; i < parts; i++) share(i, c);
+        if (c + 1 == chunks) break;
+        ok = wait(c + 1);
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            if (ok) arrived++;
+            else never = true;
+        }
+        more.notify_all();
     }
     for (size_t i = 1; i < k; i++) th[i].join();
     return ok;

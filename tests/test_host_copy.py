@@ -128,3 +128,42 @@ def test_chunks_are_copied_as_they_come_and_no_others(build):
     for ends in ((1,), (4096,), (3000, 3000, 9001), (5 << 20, 9 << 20, 12 << 20, 14 << 20, (15 << 20) - 3)):
         for never in (-1, *range(len(ends))):
             assert subprocess.run([exe, str(never), *map(str, ends)], timeout=60).returncode == 0, (ends, never)
+
+
+WAITING = r"""
+#include "host_copy.hpp"
+#include <chrono>
+#include <filesystem>
+#include <sys/resource.h>
+#include <vector>
+
+static long threads() {
+    long n = 0;
+    for (const auto& e : std::filesystem::directory_iterator("/proc/self/task")) n += e.path().filename() != ".";
+    return n;
+}
+static double cpu_seconds() {
+    rusage u{};
+    getrusage(RUSAGE_SELF, &u);
+    return u.ru_utime.tv_sec + u.ru_stime.tv_sec + 1e-6 * (u.ru_utime.tv_usec + u.ru_stime.tv_usec);
+}
+
+int main() {
+    std::vector<size_t> ends = {1 << 20, 2 << 20, 3 << 20};
+    std::vector<unsigned char> src(ends.back(), 1), dst(ends.back(), 0);
+    const oxhip::HostCopy piece{dst.data(), src.data(), ends.back()};
+    const double before = cpu_seconds();
+    bool early = false;
+    const bool ok = oxhip::host_copy_arriving(&piece, 1, ends.data(), ends.size(), 4096, [&](size_t c) {
+        std::this_thread::sleep_for(std::chrono::milliseconds(200));
+        early |= c == 0 && threads() != 1;
+        return true;
+    });
+    return !ok || early || cpu_seconds() - before > 0.15 || dst != src;  // (a thread that spins through the waits alone takes 0.6 s)
+}
+"""
+
+
+def test_waiting_for_chunks_costs_no_core(build):
+    """No thread before the first chunk has come, and none that spins until the next one."""
+    assert subprocess.run([build(WAITING)], timeout=60).returncode == 0
