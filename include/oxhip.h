@@ -116,8 +116,8 @@ size_t oxhip_weight_bytes(const oxhip_weight* w);
  * blocks) weights run the bf16 matrix-core GEMM; everything else runs the decode kernels over 16 tokens at a time.
  * The results of a call come through page-locked host memory that the context keeps until oxhip_close: half more than the largest
  * call so far needed, at most 256 MiB (a call with more results does without it). Jobs whose y overlap are copied in their order.
- * Results of 8 MiB and more are copied out chunk by chunk once all jobs have run: if the link fails between two of them, the call
- * returns 0 with some of y written (every other 0 leaves y as it was). */
+ * Results of 8 MiB and more are copied out chunk by chunk once all jobs have run; should the link fail between two of them, what y
+ * held is put back before the call returns 0. */
 int oxhip_matmul(oxhip_ctx* ctx, const float* x, size_t t, size_t n_in, oxhip_job* jobs, size_t n_jobs);
 /* Backend::matvec_rows (src/gpu.rs:165): t in 1..=4. The jobs over the matrix-core formats share one launch, a gate / up
  * job as a pair (see oxhip_dev_linear). */

@@ -797,7 +797,7 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
     (void)hipEventRecord(c->span[2], s);
     // Large results cross the link in five chunks, each copied out while the next ones still come, the last one the smallest: what is
     // left to do when it has come. (A copy of its own costs some 20 us: 59 MB in 56 chunks take longer than in one.) Nothing reaches y
-    // before the first chunk has come, that is before all jobs have run.
+    // before the first chunk has come, that is before all jobs have run, and should a later one not come, what y held is put back.
     const size_t bytes = y_total * 4, chunks = pin && bytes >= OUT_CHUNKED ? OUT_CHUNKS : 1;
     size_t ends[OUT_CHUNKS];
     for (size_t k = 0, parts = 0; k < chunks; k++) {

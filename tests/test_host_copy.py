@@ -96,38 +96,53 @@ def test_overlapping_results_keep_the_order_of_the_jobs(build):
 
 ARRIVING = r"""
 #include "host_copy.hpp"
+#include <algorithm>
 #include <cstdlib>
 #include <vector>
 
-// argv: the chunk that never comes (-1: all come), the chunks' ends; two pieces, the second a third of the bytes
+static unsigned char old_byte(size_t k) { return (unsigned char)(k * 7 + (k >> 11) + 5); }
+static unsigned char new_byte(size_t k) { return (unsigned char)(k * 31 + (k >> 12) + 1); }
+
+// argv: the chunk that never comes (-1: all come), bytes by which the second piece's destination lies inside the first's, the chunks'
+// ends; two pieces, the second a third of the bytes
 int main(int argc, char** argv) {
     const long never = std::atol(argv[1]);
     std::vector<size_t> ends;
-    for (int i = 2; i < argc; i++) ends.push_back((size_t)std::atoll(argv[i]));
-    const size_t total = ends.back(), first = total - total / 3;
-    std::vector<unsigned char> src(total + 1, 0), dst(total + 2, 0xEE);
-    const oxhip::HostCopy pieces[2] = {{dst.data(), src.data(), first}, {dst.data() + first + 1, src.data() + first, total - first}};
+    for (int i = 3; i < argc; i++) ends.push_back((size_t)std::atoll(argv[i]));
+    const size_t total = ends.back(), first = total - total / 3, back = std::min((size_t)std::atoll(argv[2]), first);
+    const size_t at2 = first + 1 - (back ? back + 1 : 0);  // (one byte lies between them where they do not overlap)
+    std::vector<unsigned char> src(total + 1, 0), dst(total + 2), want;
+    for (size_t k = 0; k < dst.size(); k++) dst[k] = old_byte(k);
+    want = dst;
+    if (never < 0) {
+        for (size_t k = 0; k < first; k++) want[k] = new_byte(k);
+        // overlapping ranges are written chunk by chunk, the later piece's bytes of a chunk last
+        for (size_t c = 0; back && c < ends.size(); c++)
+            for (size_t k = c ? ends[c - 1] : 0; k < ends[c]; k++) want[k < first ? k : at2 + k - first] = new_byte(k);
+        for (size_t k = first; !back && k < total; k++) want[at2 + k - first] = new_byte(k);
+    }
+    const oxhip::HostCopy pieces[2] = {{dst.data(), src.data(), first}, {dst.data() + at2, src.data() + first, total - first}};
     size_t told = 0;
     const bool ok = oxhip::host_copy_arriving(pieces, 2, ends.data(), ends.size(), 4096, [&](size_t c) {
         if (c != told++ || (long)c == never) return false;
-        for (size_t k = c ? ends[c - 1] : 0; k < ends[c]; k++) src[k] = (unsigned char)(k * 31 + (k >> 12) + 1);
+        for (size_t k = c ? ends[c - 1] : 0; k < ends[c]; k++) src[k] = new_byte(k);
         return true;
     });
-    const size_t there = never < 0 ? total : never ? ends[never - 1] : 0;
     if (ok != (never < 0) || told != (never < 0 ? ends.size() : (size_t)never + 1)) return 1;
-    for (size_t k = 0; k < total; k++)
-        if (dst[k + (k >= first)] != (k < there ? (unsigned char)(k * 31 + (k >> 12) + 1) : 0xEE)) return 2;
-    return dst[first] != 0xEE || dst[total + 1] != 0xEE;
+    return dst == want ? 0 : 2;
 }
 """
 
 
-def test_chunks_are_copied_as_they_come_and_no_others(build):
-    """Each chunk by all threads once it has come, in order; after one that never comes nothing more."""
+def test_all_chunks_are_copied_or_nothing_is(build):
+    """Each chunk by all threads once it has come, in order; after one that never comes every destination is as it was, also where
+    destinations overlap."""
     exe = build(ARRIVING)
     for ends in ((1,), (4096,), (3000, 3000, 9001), (5 << 20, 9 << 20, 12 << 20, 14 << 20, (15 << 20) - 3)):
         for never in (-1, *range(len(ends))):
-            assert subprocess.run([exe, str(never), *map(str, ends)], timeout=60).returncode == 0, (ends, never)
+            for back in (0, ends[-1] // 4):
+                r = subprocess.run([exe, str(never), str(back), *map(str, ends)], timeout=60)
+                assert r.returncode == 0, (ends, never, back)
 
 
 WAITING = r"""
@@ -159,7 +174,7 @@ int main() {
         early |= c == 0 && threads() != 1;
         return true;
     });
-    return !ok || early || cpu_seconds() - before > 0.15 || dst != src;  // (a thread that spins through the waits alone takes 0.6 s)
+    return !ok || early || cpu_seconds() - before > 0.15 || dst != std::vector<unsigned char>(ends.back(), 1);  // (a thread that spins through the waits alone takes 0.6 s)
 }
 """
 
