@@ -338,8 +338,10 @@ oxhip_plan* oxhip_plan_begin(oxhip_ctx* ctx, void* stream);
 int oxhip_plan_end(oxhip_plan* plan);
 /* Launches the plan holds (0 before oxhip_plan_end succeeded). */
 size_t oxhip_plan_launches(const oxhip_plan* plan);
+/* 1 if replays of the plan go out launch by launch, 0 if as one submission. */
+int oxhip_plan_one_by_one(const oxhip_plan* plan);
 /* Submits the recorded chain on `stream` (NULL: the stream it was recorded on): as one submission, or, where that is faster (a
- * chain of at most 24 kernels that streams weights), launch by launch in the recorded order. Other work on `stream` goes before or
+ * chain of at most 24 kernels, all of them this library's, that streams weights), launch by launch in the recorded order. Other work on `stream` goes before or
  * behind a replay as the caller orders its calls; replays of one context that threads start together take turns. */
 int oxhip_plan_replay(oxhip_plan* plan, void* stream);
 /* Also abandons a recording in progress. */

@@ -13,6 +13,8 @@
 // A short plan is replayed launch by launch, from the list that the finished graph holds: the submission of a graph costs the
 // stream 5 us of its own, 8 behind an ordinary launch, where a launch from the list costs the device what a graph's node does
 // and the host 2.45 us, which it has while the kernels before it run. See DIRECT_MAX.
+#include <dlfcn.h>
+
 #include <unordered_map>
 
 #include "backend.hpp"
@@ -44,7 +46,14 @@ static uint64_t streamed_on(oxhip_ctx* c, hipStream_t s) {
     return it == c->per_stream.end() ? 0 : it->second->streamed.load();
 }
 
-// The launches of a graph that is one chain of kernels this process can launch by their symbols; empty for any other graph.
+// Whether a kernel is this library's (its symbol lies in the library's own image). The caller's are left to the graph: a node does not
+// tell everything that its launch asked for (a cooperative kernel's reads as an ordinary one, which could never pass its grid barrier).
+static bool own_kernel(const void* symbol) {
+    Dl_info k{}, here{};
+    return dladdr(symbol, &k) && dladdr(reinterpret_cast<const void*>(&oxhip_plan_begin), &here) && k.dli_fbase == here.dli_fbase;
+}
+
+// The launches of a graph that is one chain of this library's kernels; empty for any other graph.
 static std::vector<hipKernelNodeParams> chain_of(hipGraph_t g) {
     size_t n = 0, ne = 0;
     if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || !n || n > DIRECT_MAX || hipGraphGetEdges(g, nullptr, nullptr, &ne) != hipSuccess || ne != n - 1) return {};
@@ -61,9 +70,8 @@ static std::vector<hipKernelNodeParams> chain_of(hipGraph_t g) {
     while (at && out.size() < n) {
         hipGraphNodeType type;
         hipKernelNodeParams k{};
-        hipFunction_t f = nullptr;
         if (hipGraphNodeGetType(at, &type) != hipSuccess || type != hipGraphNodeTypeKernel || hipGraphKernelNodeGetParams(at, &k) != hipSuccess || !k.func ||
-            !k.kernelParams || k.extra || hipGetFuncBySymbol(&f, k.func) != hipSuccess) {
+            !own_kernel(k.func) || !k.kernelParams || k.extra) {
             (void)hipGetLastError();
             return {};
         }
@@ -151,6 +159,8 @@ int oxhip_plan_end(oxhip_plan* p) {
 }
 
 size_t oxhip_plan_launches(const oxhip_plan* p) { return p ? p->nodes : 0; }
+
+int oxhip_plan_one_by_one(const oxhip_plan* p) { return p && !p->direct.empty(); }
 
 int oxhip_plan_replay(oxhip_plan* p, void* stream) {
     if (!p || !p->exec) {

@@ -115,6 +115,7 @@ def load_library():
         "oxhip_plan_begin": (vp, [vp, vp]),
         "oxhip_plan_end": (C.c_int, [vp]),
         "oxhip_plan_launches": (sz, [vp]),
+        "oxhip_plan_one_by_one": (C.c_int, [vp]),
         "oxhip_plan_replay": (C.c_int, [vp, vp]),
         "oxhip_plan_free": (None, [vp]),
         "oxhip_event_create": (vp, []),
@@ -183,6 +184,11 @@ class Plan:
     @property
     def launches(self):
         return load_library().oxhip_plan_launches(self.handle)
+
+    @property
+    def one_by_one(self):
+        """Whether replays go out launch by launch (short plans of the library's own kernels), not as one submission."""
+        return bool(load_library().oxhip_plan_one_by_one(self.handle))
 
     def replay(self, stream=None):
         if not load_library().oxhip_plan_replay(self.handle, C.c_void_p(stream) if stream else None):

@@ -526,6 +526,38 @@ def test_plan_launched_one_by_one_or_as_one(be, pairs, other):
         del plan
 
 
+@pytest.mark.parametrize("pairs,other,one_by_one", [(1, None, True), (12, None, True), (13, None, False), (3, "kernel", False), (3, "copy", False), (0, "light", False)])
+def test_which_way_a_plan_goes_out(be, pairs, other, one_by_one):
+    """Launch by launch: up to 24 launches, all of them kernels of the library's own, over 1 MiB of weights a launch."""
+    import torch
+    from oxinfer_amd import hip, synth
+    n = 1536
+    w = be.upload_gguf(Q8_0, synth.gguf_q8_0(n, n, 5800), n, n)
+    x, y, z, qa = torch.ones((2, n), device="cuda"), torch.zeros((2, n), device="cuda"), torch.zeros(n, device="cuda"), hip.QAct(2, n, "cuda")
+
+    def chain():
+        for _ in range(pairs):  # (7.5 MB of weights and a seventh launch: without the foreign one 3 pairs would go out one by one)
+            be.quantize_act(x, out=qa)
+            assert be.linear(w, y, xa=qa, t=2), be.last_error()
+        if other == "kernel": z.add_(1.0)
+        if other == "copy": z.copy_(y[1])
+        if other == "light": be.quantize_act(x, out=qa)
+
+    with torch.cuda.stream(torch.cuda.Stream()):
+        chain()
+        torch.cuda.synchronize()
+        plan = be.plan_record(chain)
+        assert plan.launches == 2 * pairs + (other is not None) and plan.one_by_one == one_by_one
+        want = (y.clone(), float(z[0]))
+        y.zero_()
+        plan.replay()
+        torch.cuda.synchronize()
+        if pairs: assert torch.equal(y, want[0])
+        if other == "kernel": assert float(z[0]) == want[1] + 1
+        if other == "copy": assert torch.equal(z, y[1])
+        del plan
+
+
 def test_plan_recording_on_a_cold_stream_declines(be, oxref):
     """Recording on a stream whose scratch does not exist yet: the call that would have to allocate declines, the
     recording is refused as a whole (oxhip_plan_end returns 0, nothing is replayable) and the stream works again
