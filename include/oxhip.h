@@ -6,7 +6,8 @@
  *
  * Conventions (those of `trait Backend`, src/gpu.rs:151-294):
  *   - functions returning int: 1 = done, 0 = declined and NOTHING was written; the caller then runs
- *     its CPU path (src/gpu.rs:158-160, src/model.rs:877-882). Handle-returning calls give NULL.
+ *     its CPU path (src/gpu.rs:158-160, src/model.rs:877-882). Handle-returning calls give NULL. (A device that refuses a
+ *     launch of a device-pointer call or a replay in the middle is the exception: the launches before it have gone out.)
  *   - oxhip_last_error() holds the reason of the calling thread's last decline.
  *   - every call may come from any thread, concurrently (src/cuda.rs:2047-2077, :2410-2438).
  *   - matrices are [n_out, n_in] row-major, outputs y[t][n_out] f32 (src/kernels.rs:54-57).
@@ -341,8 +342,12 @@ size_t oxhip_plan_launches(const oxhip_plan* plan);
 /* 1 if replays of the plan go out launch by launch, 0 if as one submission. */
 int oxhip_plan_one_by_one(const oxhip_plan* plan);
 /* Submits the recorded chain on `stream` (NULL: the stream it was recorded on): as one submission, or, where that is faster (a
- * chain of at most 24 kernels, all of them this library's, that streams weights), launch by launch in the recorded order. Other work on `stream` goes before or
- * behind a replay as the caller orders its calls; replays of one context that threads start together take turns. */
+ * chain of at most 24 kernels, all of them this library's, that streams weights), launch by launch in the recorded order. Other
+ * work on `stream` goes before or behind a replay as the caller orders its calls. Replays of one context that threads start
+ * together are submitted one after the other; this orders their submission only: plans that share buffers or were recorded on one
+ * stream (whose scratch they then share) must not run on two streams at once. Should the device refuse a launch, the call returns 0
+ * and oxhip_last_error names it: the launches before it have gone out, and what they write is written (the first one refused:
+ * nothing is). */
 int oxhip_plan_replay(oxhip_plan* plan, void* stream);
 /* Also abandons a recording in progress. */
 void oxhip_plan_free(oxhip_plan* plan);

@@ -111,7 +111,7 @@ struct oxhip_ctx {
     std::mutex smu;            // guards per_stream
     std::map<hipStream_t, oxhip::StreamScratch*> per_stream;  // the device-pointer entry points' scratch, by calling stream
     std::set<hipStream_t> record_failed;  // streams whose plan recording met a call that had to allocate (guarded by smu)
-    std::mutex replay_mu;  // one plan's launches at a time
+    std::mutex replay_mu;  // one replay is handed to the runtime at a time
     double ms_in = 0, ms_gpu = 0, ms_out = 0;
     size_t calls = 0;
 };

@@ -169,13 +169,19 @@ int oxhip_plan_replay(oxhip_plan* p, void* stream) {
     }
     HIP_TRY(hipSetDevice(p->ctx->device), "hipSetDevice");
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : p->stream;
+    std::lock_guard<std::mutex> lk(p->ctx->replay_mu);  // whichever way they go out: a submission would split another plan's launches
     if (p->direct.empty() || stream_recording(s)) {  // (into a recording: as ever)
         HIP_TRY(hipGraphLaunch(p->exec, s), "plan_replay: hipGraphLaunch");
         return 1;
     }
-    std::lock_guard<std::mutex> lk(p->ctx->replay_mu);  // the launches of a replay follow one another, whatever other threads replay
-    for (const hipKernelNodeParams& k : p->direct)
-        HIP_TRY(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes, s), "plan_replay: hipLaunchKernel");
+    for (size_t i = 0; i < p->direct.size(); i++) {
+        const hipKernelNodeParams& k = p->direct[i];
+        const hipError_t e = hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes, s);
+        if (e != hipSuccess) {
+            set_error("plan_replay: launch " + std::to_string(i + 1) + " of " + std::to_string(p->direct.size()) + ": " + hipGetErrorString(e));
+            return 0;
+        }
+    }
     return 1;
 }
 

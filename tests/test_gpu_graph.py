@@ -558,6 +558,55 @@ def test_which_way_a_plan_goes_out(be, pairs, other, one_by_one):
         del plan
 
 
+def test_replays_of_threads_follow_one_another(be):
+    """A plan launched one by one is not split by another thread's replay on the same stream, whichever way that one goes out."""
+    import threading
+
+    import torch
+    from oxinfer_amd import hip, synth
+    n, rounds = 1536, 300
+    w = be.upload_gguf(Q8_0, synth.gguf_q8_0(n, n, 5800), n, n)
+    xs = [dev(synth.activations(1, n, 5910 + i)) for i in range(3)]
+    y, qa = torch.zeros((1, n), device="cuda"), hip.QAct(1, n, "cuda")  # (every plan goes through the same quantized rows)
+    stream = torch.cuda.Stream()
+
+    def matrices():
+        for _ in range(12):
+            be.quantize_act(xs[0], out=qa)
+            assert be.linear(w, y, xa=qa, t=1, mode=hip.LIN_ADD), be.last_error()
+
+    with torch.cuda.stream(stream):
+        matrices()
+        torch.cuda.synchronize()
+        plan = be.plan_record(matrices)
+        others = [be.plan_record(lambda: [be.quantize_act(xs[1], out=qa) for _ in range(4)]), be.plan_record(lambda: [be.quantize_act(xs[2], out=qa) for _ in range(30)])]
+        assert plan.one_by_one and not any(o.one_by_one for o in others)
+
+        def accumulated(*beside):
+            y.zero_()
+            torch.cuda.synchronize()
+            errors = []
+
+            def go(p):
+                try:
+                    for _ in range(rounds):
+                        p.replay()
+                except Exception as e:  # (in a thread)
+                    errors.append(e)
+
+            threads = [threading.Thread(target=go, args=(p,)) for p in (plan, *beside)]
+            for th in threads: th.start()
+            for th in threads: th.join()
+            torch.cuda.synchronize()
+            assert not errors, errors
+            return y.clone()
+
+        want = accumulated()
+        for other in others:
+            assert torch.equal(accumulated(other).view(torch.int32), want.view(torch.int32))
+        del plan, others
+
+
 def test_plan_recording_on_a_cold_stream_declines(be, oxref):
     """Recording on a stream whose scratch does not exist yet: the call that would have to allocate declines, the
     recording is refused as a whole (oxhip_plan_end returns 0, nothing is replayable) and the stream works again
