@@ -1355,10 +1355,10 @@ Shape shape_for(uint32_t ntiles, uint32_t nsteps, bool allow_slices, int fmt) {
 
 // A gate / up pair: a workgroup holds the tiles of the same rows of both matrices, so its tile count is even; kw and ks (the
 // order of a row's sum) stay what the weight's shape alone gives, which keeps each product's bits those of a launch of its own.
-// Of the tile counts that eight waves allow (two tiles at least) the one whose tiles take the busiest CU least, each workgroup's
-// staging counted as a tile more, as four more of nine and more tokens; of equals the largest. (A pair of 11008
-// x 4096, 1 / 8 / 16 tokens, four tiles -> two, two, four: MLX 4-bit 15.6 / 18.0 / 20.5 -> 13.5 / 15.9 / 20.5 us; of 8192 x 3072, two ->
-// four: Q8_0 11.6 / 12.1 / 14.5 -> 11.6 / 11.9 / 13.1.)
+// Of the tile counts that eight waves allow (two tiles at least: sixteen waves, the kernels' bound, where a row has eight runs) the
+// one whose tiles take the busiest CU least, each workgroup's staging counted as a tile more, as four more of nine and more tokens; of
+// equals the largest. (A pair of 11008 x 4096, 1 / 8 / 16 tokens, four tiles -> two, two, four: MLX 4-bit 15.6 / 18.0 / 20.5 -> 13.5 /
+// 15.9 / 20.5 us; of 8192 x 3072, two -> four: Q8_0 11.6 / 12.1 / 14.5 -> 11.6 / 11.9 / 13.1.)
 Shape pair_shape(Shape sh, uint32_t ntiles, size_t t) {
     const uint32_t stage = t > 8 ? 4 : 1;
     uint32_t best = 0;
@@ -1551,21 +1551,13 @@ uint32_t steps_rt(const WeightView& w) {
 }
 }  // namespace
 
-// Whether a gate / up pair of this weight's shape and format runs as one launch: its workgroup of paired tiles fits the kernel's
-// bound. `shared`: in the shared launch, where Q4_0's kernel is bounded at 8 waves.
-bool decode_pair_ok(const WeightView& w, bool shared) {
-    if (!mfma_decode_format(w.fmt)) return false;
-    const Shape sh = pair_shape(shape_for(row_tiles(w.n_out), steps_rt(w), true, w.fmt), row_tiles(w.n_out), 1);
-    return sh.rt * sh.kw <= (shared && w.fmt == FMT_Q40 ? 8u : 16u);
-}
-
 bool decode_batchable(const WeightView& w, size_t t) {
     if (!mfma_decode_format(w.fmt)) return false;
     if (t < 1 || t > 16) return false;
     const Shape sh = shape_for(row_tiles(w.n_out), steps_rt(w), true, w.fmt);  // as a launch of its own: same bits
     bool alds;
     const size_t lds = lds_bytes(w.fmt, false, steps_rt(w), t <= 4 ? 4 : t <= 8 ? 8 : 16, sh, &alds);
-    return alds && lds <= LDS_MAX && (t <= 8 || sh.rt * sh.kw <= 8);
+    return alds && lds <= LDS_MAX;
 }
 
 // Scratch a launch of this weight alone takes when its shape slices K across workgroups (floats of partial rows,
@@ -1788,7 +1780,7 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
         if (!launches[i].nwg) continue;
         uint32_t fset = 0;
         for (uint32_t j = 0; j < launches[i].njobs; j++) fset |= fbit(launches[i].j[j].fmt);
-        if (threadss[i] > (fset == FSET_Q40 || launches[i].j[0].t > 8 ? 512u : 1024u)) return hipErrorInvalidValue;  // (the kernels' launch bounds)
+        if (threadss[i] > 1024) return hipErrorInvalidValue;  // (the kernels' launch bound)
         auto go = [&](auto kern) {
             if (ride) hipExtLaunchKernelGGL(kern, dim3(launches[i].nwg), dim3(threadss[i]), (uint32_t)ldss[i], s, ev_start, ev_stop, 0, launches[i]);
             else kern<<<launches[i].nwg, threadss[i], ldss[i], s>>>(launches[i]);

@@ -6,7 +6,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-Q4_0, Q8_0, Q4_K, MXFP4 = 2, 8, 12, 39
+Q4_0, Q8_0, Q4_K, Q5_K, Q6_K, MXFP4 = 2, 8, 12, 13, 14, 39
 
 
 @pytest.fixture(scope="module")
@@ -534,10 +534,12 @@ def test_matvec_rows(be, oxref):
     assert not be.matvec_rows(np.zeros((5, n_in), np.float32), 5, n_in, [(w, None, np.zeros((5, n_out), np.float32))])
 
 
-@pytest.mark.parametrize("kind,n_out,n_in", [(Q4_K, 1000, 768), (Q8_0, 272, 14336), (Q4_K, 48, 14336)])
+@pytest.mark.parametrize("kind,n_out,n_in", [(Q4_K, 1000, 768), (Q8_0, 272, 14336), (Q4_K, 48, 14336),
+                                             (Q6_K, 48, 3072), (Q8_0, 48, 5120), (Q4_0, 40, 5376), (Q4_K, 48, 5376), (Q5_K, 40, 5376)])
 def test_matvec_rows_shares_a_launch_and_pairs_keep_the_bits(be, oxref, kind, n_out, n_in):
     """Several RowsJobs of one call (plain and gate / up) share one launch; a gate / up job's rows are silu_mul of the two
-    products as separate plain jobs give them, bit for bit (K-sliced shapes and ragged row groups included)."""
+    products as separate plain jobs give them, bit for bit (K-sliced shapes and ragged row groups included; the last five have rows of
+    eight runs, whose pairs' workgroups are sixteen waves)."""
     from oxinfer_amd import synth
     raws = [oxref.random_blocks(kind, n_out * n_in // oxref.block_size(kind), 70 + i)[0] for i in range(3)]
     ws = [be.upload_gguf(kind, r, n_out, n_in) for r in raws]
