@@ -156,7 +156,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                                             uint32_t* __restrict__ counters, uint32_t bx, uint32_t by, uint32_t nthr,
                                             float* __restrict__ lds_all, Epi epi = Epi{}, Mapping map = Mapping{}) {
     static_assert(NG == 1 || (GROUPED && ALDS && !DUMP && NT == 8), "token groups are for grouped launches");
-    static_assert(!REMAP || (!GROUPED && !DUMP && ALDS && NG == 1), "other mappings are for dense launches over staged activations");
+    static_assert(!REMAP || (!GROUPED && !DUMP && ALDS && NG == 1 && NT <= 8), "other mappings are for dense launches over staged activations");
     // Nine to sixteen tokens (NT = 16): the instruction is v_mfma_i32_16x16x32_i8, one block x 16 tokens x 16 rows, so that the
     // token rows are all in use without masking (a lane's bytes 0-7 and 8-15 of a record are the operands of two consecutive
     // instructions, and the lane receives tokens 4 kq + i of both blocks). Every block parity keeps a sum of its own, as the two
@@ -827,7 +827,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     };
     // A wave with further runs (up to MAXRUNS in all; place_job) keeps the closed run's sums in registers (the partial sums' place in
     // LDS still holds the activations) and starts the next run from zero. `left`: steps to the end of the run in hand.
-    constexpr int MAXRUNS = WIDE ? 2 : 4;
+    constexpr int MAXRUNS = 4;
     float held[REMAP ? MAXRUNS - 1 : 1][4] = {};
     uint32_t nrun = 0, left = per;  // runs closed so far
     auto step_done = [&]() {
@@ -841,11 +841,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                 nrun++;
                 left = per;
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    acc[0][i] = acch[WIDE ? i : 0] = 0.0f;
-#pragma unroll
-                    for (int tg = 0; tg < NTG; tg++) acc6[tg][i] = 0.0f;
-                }
+                for (int i = 0; i < 4; i++) acc[0][i] = acc6[0][i] = acc6[1][i] = 0.0f;
                 macc[0] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
             }
         }
@@ -884,7 +880,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     close_run();
     if (ALDS) __syncthreads();  // the partial sums overwrite the staged activations
     if constexpr (REMAP) {
-        if (rpw > 1 && (WIDE || kq < 2)) {  // the runs closed on the way
+        if (rpw > 1 && kq < 2) {  // the runs closed on the way
 #pragma unroll
             for (int h = 0; h < MAXRUNS - 1; h++)
                 if ((uint32_t)h < rpw - 1) {
@@ -1194,7 +1190,7 @@ __device__ __forceinline__ void batch_dispatch(const BatchJob& jb, uint32_t bid,
     epi.pair_act = jb.pair_act;
     const Mapping map{jb.kwp, jb.fs};
     if constexpr (WIDE) {
-        decode_body<FMT, 16, false, false, true, 1, FAT>(w, xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, epi, map);
+        decode_body<FMT, 16, false, false, true>(w, xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, epi, map);
         return;
     } else if (jb.t == 1) decode_body<FMT, 1, false, false, true, 1, FAT>(w, xa, jb.t, jb.rt, jb.kw, jb.y, nullptr, none, jb.ks, jb.partial, jb.counters, bx, by, nthr, lds, epi, map);
     else if (jb.t == 2 && !t4m_format(FMT)) decode_body<FMT, 2, false, false, true, 1, FAT>(  // (MLX at 2 tokens: the 4-token body, which fits the registers)
@@ -1229,8 +1225,7 @@ inline int set_of(int fmt, uint32_t mask) {
 // (Q6_K shares the kernel of Q8_0 and Q4_K since its step leaves room for four waves per SIMD: a Q4_K_M file's layers mix the three,
 // and their matmuls go out in one launch. All are bounded to 128 registers: nothing spills, two workgroups of eight waves fit a CU.)
 // FAT: the launch's jobs use the fat mapping (see place_job); the plain kernels do without its bookkeeping.
-// WIDE: the launch's jobs have 9 to 16 tokens each (kernels of their own, for the registers; plain mappings, but compiled as FAT,
-// which keeps the GGUF set at 123 registers).
+// WIDE: the launch's jobs have 9 to 16 tokens each (kernels of their own, for the registers; plain mapping).
 template <uint32_t FSET, bool FAT, bool WIDE = false>
 __global__ __launch_bounds__(1024) void decode_batch_kernel(BatchArgs a) {
     extern __shared__ __align__(16) float lds_dyn[];
@@ -1659,7 +1654,7 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
     const uint64_t bit = 1ull << (dev & 63);
     if (!(allowed[(dev >> 6) & 3].load(std::memory_order_acquire) & bit)) {
 #define OXHIP_BATCH_KERNELS(F) reinterpret_cast<const void*>(decode_batch_kernel<F, false>), reinterpret_cast<const void*>(decode_batch_kernel<F, true>)
-#define OXHIP_BATCH_WIDE(F) reinterpret_cast<const void*>(decode_batch_kernel<F, true, true>)
+#define OXHIP_BATCH_WIDE(F) reinterpret_cast<const void*>(decode_batch_kernel<F, false, true>)
         for (const void* k : {OXHIP_BATCH_WIDE(FSET_GGUF), OXHIP_BATCH_WIDE(FSET_MLX), OXHIP_BATCH_WIDE(FSET_K5), OXHIP_BATCH_WIDE(FSET_Q40),
                               OXHIP_BATCH_WIDE(FSET_MX4), OXHIP_BATCH_WIDE(FSET_Q8F), OXHIP_BATCH_KERNELS(FSET_GGUF), OXHIP_BATCH_KERNELS(FSET_MLX), OXHIP_BATCH_KERNELS(FSET_K5),
                               OXHIP_BATCH_KERNELS(FSET_Q40), OXHIP_BATCH_KERNELS(FSET_MX4), OXHIP_BATCH_KERNELS(FSET_Q8F)}) {
@@ -1787,7 +1782,7 @@ hipError_t launch_decode_mfma_batch(const DecodeBatchItem* items, size_t n, cons
         };
         const bool fat = fats[i];
         const bool wide = launches[i].j[0].t > 8;
-#define OXHIP_GO(F) (wide ? go(decode_batch_kernel<F, true, true>) : fat ? go(decode_batch_kernel<F, true>) : go(decode_batch_kernel<F, false>))
+#define OXHIP_GO(F) (wide ? go(decode_batch_kernel<F, false, true>) : fat ? go(decode_batch_kernel<F, true>) : go(decode_batch_kernel<F, false>))
         if (!(fset & ~FSET_GGUF)) OXHIP_GO(FSET_GGUF);
         else if (!(fset & ~FSET_MLX)) OXHIP_GO(FSET_MLX);
         else if (!(fset & ~FSET_K5)) OXHIP_GO(FSET_K5);
