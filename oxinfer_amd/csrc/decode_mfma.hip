@@ -396,8 +396,8 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
         }
     };
     // (not where a step has several token groups, nor for Q6_K, which reads its own way, nor for Q5_K at 16 tokens, which has no
-    // registers left)
-    constexpr bool AHEAD = NG == 1 && FMT != FMT_Q6_K && !(WIDE && FMT == FMT_Q5_K);
+    // registers left, nor for Q4_K and Q5_K on operands from L2, where it spills them)
+    constexpr bool AHEAD = NG == 1 && (ALDS || !k45_format(FMT)) && FMT != FMT_Q6_K && !(WIDE && FMT == FMT_Q5_K);
     // instruction `i` of a step on the lane's 16 codes `bw` (a pair of blocks) ...
     auto mfma = [&](v4i bw, int i, uint32_t d0, uint32_t d1) -> v4i {
         const v4i c = {0, 0, 0, 0};
@@ -1115,13 +1115,14 @@ inline const void* sums_of(int fmt, const QActView& v) { return fmt == FMT_Q6_K 
 // into dwords (and the kernel runs two to three times longer) when the array starts at an odd dword.
 // (Grouped launches keep to 8 waves, which leaves them 256 registers for the accumulators of their token groups; with chunks of
 // five to eight rows they are bounded to four waves per SIMD, MLX 4-bit to five: unbounded that kernel took 139 registers and
-// spilled 36 scalar ones; those of several token groups to four.)
+// spilled 36 scalar ones; those of several token groups to four. The integer-sum forms, for which there are no pairs, keep to 8 waves
+// too: with room for 16, Q6_K's spilled 228 registers instead of 64.)
 // Such a launch has chunks of any length up to its own, and those of up to four rows, the most of them where an expert has few
 // routed rows, run the four-row body. 128 MLX 4-bit experts of 2048 / 768, eight a token, every chunk in the eight-row body of
 // before -> this: 24 tokens routed at random 85.5 -> 64.1 us, 47 tokens all to the same eight experts 53.8 -> 42.0 us. (Chunks of
 // four rows throughout make two passes over the weights of an expert with more: 63.0 and 55.1 us.)
 template <int FMT, int NT, bool DUMP, bool GROUPED, bool ALDS, int NG>
-__global__ __launch_bounds__(GROUPED ? 512 : 1024, GROUPED && NT == 8 ? (FMT == FMT_Q4M && ALDS && NG == 1 ? 5 : 4) : 1) void decode_mfma_kernel(LaunchArgs<GROUPED> a) {
+__global__ __launch_bounds__(GROUPED || DUMP ? 512 : 1024, GROUPED && NT == 8 ? (FMT == FMT_Q4M && ALDS && NG == 1 ? 5 : 4) : 1) void decode_mfma_kernel(LaunchArgs<GROUPED> a) {
     extern __shared__ __align__(16) float lds_dyn[];
     WeightView w{};
     w.fmt = FMT;
@@ -1440,6 +1441,7 @@ hipError_t run(const WeightView& w, const QActView& xa, size_t t, float* y, int3
     const uint32_t nblk = w.n_in / 32;
     const uint32_t per_wg = pair ? sh.rt / 2 : sh.rt;  // row tiles of the output per workgroup
     dim3 grid((ntiles + per_wg - 1) / per_wg, sh.ks), block(64 * sh.rt * sh.kw);
+    if (block.x > (DUMP ? 512 : 1024)) return hipErrorInvalidValue;  // (the kernels' launch bounds)
     // Nine to sixteen tokens in one pass over the weights where their staged activations fit the LDS and the scratch their
     // slices' rows; otherwise eight at a time.
     bool wide = false;
