@@ -768,3 +768,35 @@ def test_works_from_another_thread_and_concurrent_calls_do_not_mix(be, oxref):
     for th in threads:
         th.join()
     assert not errors, errors
+
+
+@pytest.mark.parametrize("n_out,n_in", [(256, 3072), (256, 4096), (250, 5120), (250, 5632)])
+def test_rows_of_eight_runs_sum_in_their_order(be, oxref, n_out, n_in):
+    """Long rows of low matrices are summed in eight runs of steps: the bits of that order (a run keeps a sum per block parity, the runs
+    are added one after the other), whose distance from 64 bits is not larger than that of four runs."""
+    from oxinfer_amd import synth
+    t, nblk = 16, n_in // 32
+    raw = synth.gguf_q8_0(n_out, n_in, n_in)
+    blocks = raw.reshape(n_out, nblk, 34)
+    d = blocks[:, :, :2].copy().view(np.float16)[:, :, 0].astype(np.float64)
+    codes = blocks[:, :, 2:].copy().view(np.int8).astype(np.float32)
+    xa = be.quantize_act(dev(synth.activations(t, n_in, 90)))
+    xq, xs = xa.q.cpu().numpy().reshape(t, nblk, 32).astype(np.float32), xa.scales.cpu().numpy()
+    sums = np.einsum("obk,tbk->tob", codes, xq)  # (below 2^24: exact)
+    terms = (xs[:, None, :] * sums).astype(np.float32)
+
+    def in_runs(runs):
+        per = -(-(nblk // 2) // runs)  # steps (of two blocks) of a run
+        total = np.zeros((t, n_out), np.float32)
+        for r in range(runs):
+            parity = [np.zeros((t, n_out), np.float32) for _ in range(2)]
+            for b in range(2 * r * per, min(2 * (r + 1) * per, nblk)):
+                parity[b & 1] = (d[:, b] * terms[:, :, b] + parity[b & 1]).astype(np.float32)  # one rounding: the product is exact
+            total = total + (parity[0] + parity[1])
+        return total
+
+    exact = np.einsum("tob,ob->to", sums.astype(np.float64) * xs[:, None, :].astype(np.float64), d)
+    eight, four = in_runs(8), in_runs(4)
+    y = be.decode(be.upload_gguf(Q8_0, raw, n_out, n_in), xa=xa).cpu().numpy()
+    assert np.array_equal(y.view(np.uint32), eight.view(np.uint32))
+    assert np.linalg.norm(eight - exact) <= np.linalg.norm(four - exact)

@@ -219,6 +219,22 @@ def test_norm_over_several_workgroups_keeps_the_bits(be, n, rows, off):
     assert torch.equal(added[off:], dev(old)[off:] + out[off:])
 
 
+@pytest.mark.parametrize("n,rows", [(1056, 256), (4096, 128), (8192, 64), (16384, 32)])
+def test_norm_on_both_sides_of_the_workgroup_limit(be, n, rows):
+    """As many rows as go out over several workgroups each (512 in all), and one row more, which takes one workgroup a row: the same bits."""
+    import torch
+    rng = np.random.default_rng(n + rows)
+    x, w = dev(rng.normal(0, 3, (rows + 1) * n).astype(np.float32)), dev(rng.normal(1, 0.2, n).astype(np.float32))
+    outs = []
+    for r in (rows, rows + 1):
+        out = torch.zeros_like(x)
+        ok, qa = be.norm(x, n, r, out=out, w=w, want_q=True)
+        assert ok, be.last_error()
+        outs.append((out[: rows * n], *(getattr(qa, f)[:rows] for f in ("q", "scales", "sums", "fsums", "hsums", "sums16"))))
+    for a, b in zip(*outs):
+        assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
 def test_norm_rounds_the_reciprocal_root_correctly(be):
     """r = m^(-1/2) is the f32 value nearest to the exact one also where that lies closest to the middle between two f32 values: the
     4096 such means of [1, 4) (every exponent's r is one of theirs, times a power of two). A row's squares add up to 32 m in f32, and
