@@ -720,7 +720,7 @@ int oxhip_matmul(oxhip_ctx* c, const float* x, size_t t, size_t n_in, oxhip_job*
     // Everything is computed into device staging and comes to the host as a whole first; y is written only once all jobs ran.
     // It comes through page-locked memory that the context keeps: an ordinary buffer made for each call costs its page faults
     // and the runtime's own staging, 16.6 ms a call for 512 tokens through two 14336 x 4096 matrices (59 MB of results)
-    // against 2.0 ms, 1.7 copied out in chunks, of which 1.0 are the link's. Calls with more results than MAX_PINNED take the ordinary
+    // against 2.0 ms, 1.7 to 1.9 copied out in chunks, of which 1.0 are the link's. Calls with more results than MAX_PINNED take the ordinary
     // buffer. (x is as fast from where it is: 0.34 ms for 8 MB either way.)
     uint8_t* pin = c->pin.grow(y_total * 4, MAX_PINNED) ? static_cast<uint8_t*>(c->pin.p) : nullptr;
     (void)hipEventRecord(c->span[0], s);

@@ -10,9 +10,9 @@
 // activations) must exist before recording starts: run the chain once on the same stream first. A call that would have to
 // allocate while recording fails the recording (oxhip_plan_end reports it), and nothing is replayable then.
 //
-// A short plan is replayed launch by launch, from the list that the finished graph holds: the submission of a graph costs the
-// stream 5 us of its own, 8 behind an ordinary launch, where a launch from the list costs the device what a graph's node does
-// and the host 2.45 us, which it has while the kernels before it run. See DIRECT_MAX.
+// A short plan of the library's own kernels is replayed launch by launch, from the list that the finished graph holds: the submission
+// of a graph costs the stream 5 us of its own, 8 behind an ordinary launch, where a launch from the list costs the device what a
+// graph's node does and the host 2.45 us, which it has while the kernels before it run. See DIRECT_MAX.
 #include <dlfcn.h>
 
 #include <unordered_map>

@@ -475,7 +475,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 
 // Adds the K slices in order: y = p[0] + p[1] + ... (f32 or bf16 out). VEC outputs per thread (4 when n is a multiple of 4 and
 // the buffers are 16-byte aligned). A launch that does not fill the chip is bound by its trips to memory, one per slice where a slice
 // is requested when the one before it has been added: BATCH requests eight, four, two and one at a time, the sums as they were
-// (rows of 4096 and 4095 floats, 16 slices of 17 to 49 tokens 4.8-5.3 -> 3.9-4.1 us, 8 slices of 65 to 193 tokens 4.8-7.1 -> 4.1-5.6).
+// (16 slices of 17 to 49 tokens, rows of 4096 and of 4095 floats 4.8-5.3 -> 3.9-4.1 us; 8 slices of 65 to 129 tokens, 4096 floats
+// 4.8-5.0 -> 4.2-4.4, 4095 floats, one output a thread, 4.8-6.0 -> 4.1-4.5).
 template <bool OUT_BF16, int VEC, bool BATCH>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ p, size_t n, uint32_t slices, void* __restrict__ yv) {
     const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * VEC;
