@@ -13,9 +13,9 @@
 // dequantize at the same time: the waves 0-3 do so in a step's first block, the waves 4-7 in its second. Sharing the
 // token dimension keeps the activation requests at one per fragment and workgroup (sharing the rows instead would
 // request every fragment twice and run into the vector memory path's 64 bytes per cycle and CU). A
-// launch of at most 64 tokens runs 4 waves with one token tile each (64 tokens x 128 rows per workgroup), one of 65 to
-// 128 tokens 8 waves with one tile each (34 -> 27 us on the Llama-8B MLP shapes against two tiles per wave).
-//   B (weights): each K-step of 128 the waves dequantize the step's 8 row tiles (one each; two each with 4 waves) from the packed
+// launch of 65 to 128 tokens runs one tile per wave (34 -> 27 us on the Llama-8B MLP shapes against two); up to 64 tokens are
+// gemm_short.hip's.
+//   B (weights): each K-step of 128 the waves dequantize the step's 8 row tiles (one each) from the packed
 //     records into bf16 MFMA fragments in LDS (double-buffered, one barrier per step); every wave then reads all
 //     8 x 4 fragments with ds_read_b128. A weight is dequantized once per workgroup: (code - 8) * d + offset in
 //     f32 as one fma(code, d, offset - 8 d), rounded to bf16. The GGUF formats likewise, from their own records:
@@ -26,13 +26,9 @@
 //     16-byte-per-lane load straight from global memory / L2, a block ahead of its use.
 #include <type_traits>
 
-#include "internal.hpp"
-#include "layout.hpp"
+#include "gemm_tile.hpp"
 
 namespace oxhip {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Activations [t][n_in] (f32 or bf16) -> fragments [mtile][block][lane][8 bf16]; lane = 16 kq + m holds token
 // 16 mtile + m at K positions 32 b + 4 kq + {0..3} then 32 b + 16 + 4 kq + {0..3} (SPLIT, the order of the
@@ -113,53 +109,11 @@ hipError_t launch_pack_a(const void* x, bool src_bf16, int mode, size_t t, size_
     return hipGetLastError();
 }
 
-#ifndef OXHIP_GEMM_EARLY_RAW
-#define OXHIP_GEMM_EARLY_RAW 1
-#endif
-
 namespace {
 
-// the formats in the T4M code geometry (NVFP4's records too: float-stored, so not one of the int8 decode formats)
-__host__ __device__ constexpr bool t4_geometry(int f) { return t4m_format(f) || f == FMT_NVFP4; }
-
-typedef uint32_t u32x4g __attribute__((ext_vector_type(4)));
 constexpr int WG_NT = 8;   // row tiles per workgroup (128 rows), or 7 where that fills more CUs (gemm_plan)
+constexpr int WAVES = 8;
 constexpr int AR = 4;      // blocks of A fragments held ahead (a whole K-step: two starve the FP8 shapes, whose activations do not stay in L2)
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-// Two f32 -> packed bf16 (round to nearest even) with the hardware conversion, one instruction, no branches.
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
-}
-
-// Eight unsigned byte codes (the bytes of lo, then of hi) -> 8 bf16 of code * d + c.
-template <int K>
-__device__ __forceinline__ float byte_f32(uint32_t x) {  // byte K of x as f32: one conversion that selects the byte itself
-    float f;
-    if constexpr (K == 0) asm("v_cvt_f32_ubyte0_e32 %0, %1" : "=v"(f) : "v"(x));
-    else if constexpr (K == 1) asm("v_cvt_f32_ubyte1_e32 %0, %1" : "=v"(f) : "v"(x));
-    else if constexpr (K == 2) asm("v_cvt_f32_ubyte2_e32 %0, %1" : "=v"(f) : "v"(x));
-    else asm("v_cvt_f32_ubyte3_e32 %0, %1" : "=v"(f) : "v"(x));
-    return f;
-}
-__device__ __forceinline__ uint4 dequant_u8x8(uint32_t lo, uint32_t hi, float d, float c) {
-    float f[8];
-    f[0] = __builtin_fmaf(byte_f32<0>(lo), d, c);
-    f[1] = __builtin_fmaf(byte_f32<1>(lo), d, c);
-    f[2] = __builtin_fmaf(byte_f32<2>(lo), d, c);
-    f[3] = __builtin_fmaf(byte_f32<3>(lo), d, c);
-    f[4] = __builtin_fmaf(byte_f32<0>(hi), d, c);
-    f[5] = __builtin_fmaf(byte_f32<1>(hi), d, c);
-    f[6] = __builtin_fmaf(byte_f32<2>(hi), d, c);
-    f[7] = __builtin_fmaf(byte_f32<3>(hi), d, c);
-    return make_uint4(pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]), pack_bf16(f[4], f[5]), pack_bf16(f[6], f[7]));
-}
-// One dword of a T4M chunk (4 bytes of one block: low nibbles = elements 4 kq + i, high = 16 + 4 kq + i) -> the
-// lane's 8 bf16 of that block.
-__device__ __forceinline__ uint4 dequant_q4m(uint32_t w, float d, float c) {
-    return dequant_u8x8(w & 0x0F0F0F0Fu, (w >> 4) & 0x0F0F0F0Fu, d, c);
-}
 
 }  // namespace
 
@@ -173,43 +127,25 @@ __device__ __forceinline__ uint4 dequant_q4m(uint32_t w, float d, float c) {
 // ALONE: see run_gemm_bf16_nv. (Eight waves of one token tile: two workgroups share a CU if they take at most 128 registers. Q4_K took 130:
 // bounded it spills 12 bytes, 9472 columns x 5000 rows 42.7 -> 31.9 us at 128 tokens with the slices that allows. The 8-bit formats
 // would spill 24 to 44 bytes, 33.6 -> 43.9 us on 14336 -> 4096: they keep a CU to a workgroup.)
-template <int FMT, bool OUT_BF16, int NV, int WAVES, int NT, bool ALONE>
-__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 : 2) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
+template <int FMT, bool OUT_BF16, int NV, int NT, bool ALONE>
+__global__ __launch_bounds__(64 * WAVES, NV == 1 && !ALONE ? 4 : 2) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
                                                         void* __restrict__ yv) {
     extern __shared__ uint4 bfrag[];  // [2][4 blocks][NT row tiles][64 lanes]
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t n = lane & 15;
-    constexpr int DT = (NT + WAVES - 1) / WAVES;  // row tiles a wave dequantizes (with NT = 7 the last wave has one fewer)
     const uint32_t all_steps = (w.n_in + 127) / 128, kblocks = 4 * all_steps;  // == t4m_steps(n_in)
     const uint32_t per_z = (all_steps + gridDim.z - 1) / gridDim.z;
     const uint32_t step0 = blockIdx.z * per_z;              // this slice's K-steps: step0 .. step0 + nsteps
     const uint32_t nsteps = min(all_steps, step0 + per_z) - step0;
     const uint32_t ntiles = row_tiles(w.n_out);
     const uint32_t nt0 = blockIdx.x * NT;               // first row tile of the workgroup
-    // the wave's token tiles: mt0, mt0 + WAVES, ... (NV of them: 2, or 1 when the whole launch has at most 64 tokens per
-    // workgroup row, so that a few tokens do not pay for 256)
+    // the wave's token tiles: mt0, mt0 + WAVES, ... (NV of them)
     const uint32_t mt0 = blockIdx.y * (WAVES * NV) + wave;
 
-    // the row tiles this wave dequantizes
-    const uint8_t* wbase[2];
-    const float* sbase[2] = {nullptr, nullptr};  // FP8: the block scales of the tile's rows
-#pragma unroll
-    for (int i = 0; i < DT; i++) {
-        const uint32_t tile = min(nt0 + DT * wave + i, ntiles - 1);
-        if (t4_geometry(FMT)) {
-            wbase[i] = w.p0 + ((size_t)tile * all_steps + step0) * (FMT == FMT_MXFP4 ? T4X_REC : T4M_REC);  // (T4N_REC == T4M_REC)
-        } else if (q8_format(FMT)) {  // the tile's records; load_raw indexes them from the matrix's first step
-            wbase[i] = w.p0 + (size_t)tile * t8_steps(w.n_in) * (FMT == FMT_Q8F ? T8F_REC : T8_REC);
-        } else if (k45_format(FMT)) {
-            wbase[i] = w.p0 + (size_t)tile * tk4_sbs(w.n_in) * (FMT == FMT_Q5_K ? TK5_REC : TK4_REC);
-        } else if (FMT == FMT_Q6_K) {
-            wbase[i] = w.p0 + (size_t)tile * t6k_steps(w.n_in) * T6K_REC;
-        } else {
-            const uint32_t row = min(tile * 16 + n, w.n_out - 1);
-            wbase[i] = w.p0 + fp8_offset(w, row, 128 * (size_t)step0 + 32 * (lane >> 4));
-            sbase[i] = reinterpret_cast<const float*>(w.p1) + (size_t)(tile * 16 / w.br) * ((w.n_in + w.bc - 1) / w.bc);  // indexed by the absolute column block
-        }
-    }
+    // the row tile this wave dequantizes (with NT = 7 the eighth wave has none)
+    const bool has_tile = NT == WAVES || wave < (uint32_t)NT;
+    const uint32_t tile = min(nt0 + wave, ntiles - 1);
+    const uint8_t* wbase = tile_records<FMT>(w, tile, lane);
     // A fragments of the wave's token tiles (tiles past the end repeat the last one; their rows are not stored)
     const uint4* abase[NV];
 #pragma unroll
@@ -221,167 +157,15 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    struct Raw {
-        uint4 c, c2;    // Q4M, Q4_K: one chunk; Q8: the chunks of the step's two records; Q6_K: low nibbles, high bit pairs; FP8: 32 row bytes
-        uint32_t m[4];  // the row's scale words (Q4M: scales, offsets; FP8: the block scale's bits)
+    // `s`: a step of this slice
+    auto load_raw = [&](RawTile& r, uint32_t s) {
+        if (has_tile) load_tile<FMT>(r, w, wbase, tile, step0 + s, lane);
     };
-    auto load_raw_tile = [&](Raw* r, int i, uint32_t s) {  // the records of the wave's row tile i at step s
-        if (NT % WAVES == 0 || DT * wave + i < NT) {  // (with NT = 7 the eighth wave has no tile)
-            if (FMT == FMT_NVFP4) {  // the row's eight sub-block scale bytes, and the matrix's scale of this step's columns
-                const uint8_t* rec = wbase[i] + (size_t)s * T4N_REC;
-                r[i].c = *reinterpret_cast<const uint4*>(rec + 16 * lane);
-                const uint2 sv = *reinterpret_cast<const uint2*>(rec + 1024 + 8 * n);
-                r[i].m[0] = sv.x;
-                r[i].m[1] = sv.y;
-                const uint32_t tile = min(nt0 + DT * wave + i, ntiles - 1);
-                r[i].m[2] = w.br ? __float_as_uint(reinterpret_cast<const float*>(w.p1)[(size_t)(min(tile * 16 + n, w.n_out - 1) / w.br) * ((w.n_in + w.bc - 1) / w.bc) +
-                                                                                    (128 * (step0 + s)) / w.bc])
-                                 : 0x3F800000u;
-            } else if (t4m_format(FMT)) {
-                const uint8_t* rec = wbase[i] + (size_t)s * (FMT == FMT_MXFP4 ? T4X_REC : T4M_REC);
-                r[i].c = *reinterpret_cast<const uint4*>(rec + 16 * lane);
-                r[i].m[0] = *reinterpret_cast<const uint32_t*>(rec + 1024 + 4 * n);
-                if (FMT != FMT_MXFP4) r[i].m[1] = *reinterpret_cast<const uint32_t*>(rec + 1088 + 4 * n);
-            } else if (q8_format(FMT)) {  // a step of 128 columns is two records of 64 (past the row's last record: that one again,
-                                          // which dequant_tile zeroes: nothing here may depend on a loaded value, or the request
-                                          // would be waited for where it is made)
-                constexpr uint32_t REC = FMT == FMT_Q8F ? T8F_REC : T8_REC;
-                const uint32_t nrec = t8_steps(w.n_in);
+    auto dequant = [&](const RawTile& r, uint32_t buf, uint32_t s) {  // the wave's row tile, 4 blocks
+        if (!has_tile) return;
+        uint4* dst = bfrag + ((size_t)(buf * 4) * NT + wave) * 64 + lane;  // block b: + b * NT * 64
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const uint8_t* rec = wbase[i] + (size_t)min(2 * (step0 + s) + h, nrec - 1) * REC;
-                    const uint4 v = *reinterpret_cast<const uint4*>(rec + 16 * lane);
-                    if (h) r[i].c2 = v;
-                    else r[i].c = v;
-                    if (FMT == FMT_Q8F) {
-                        const uint2 sc = *reinterpret_cast<const uint2*>(rec + 1024 + 8 * n);
-                        r[i].m[2 * h] = sc.x;
-                        r[i].m[2 * h + 1] = sc.y;
-                    } else {
-                        r[i].m[h] = *reinterpret_cast<const uint32_t*>(rec + 1024 + 4 * n);
-                    }
-                }
-            } else if (k45_format(FMT)) {  // half a super-block record: sub-blocks 4 (sa & 1) .. + 3
-                const uint32_t sa = step0 + s;
-                const uint8_t* rec = wbase[i] + (size_t)(sa >> 1) * (FMT == FMT_Q5_K ? TK5_REC : TK4_REC);
-                r[i].c = *reinterpret_cast<const uint4*>(rec + (sa & 1) * 1024 + 16 * lane);
-                if (FMT == FMT_Q5_K) r[i].c2.x = *reinterpret_cast<const uint32_t*>(rec + TK4_REC + (sa & 1) * 256 + 4 * lane);
-                r[i].m[0] = *reinterpret_cast<const uint32_t*>(rec + 2048 + 16 * n + 4 * (sa & 1));
-                r[i].m[1] = *reinterpret_cast<const uint32_t*>(rec + 2048 + 16 * n + 8 + 4 * (sa & 1));
-                r[i].m[2] = *reinterpret_cast<const uint32_t*>(rec + 2304 + 4 * n);
-            } else if (FMT == FMT_Q6_K) {
-                const uint8_t* rec = wbase[i] + (size_t)(step0 + s) * T6K_REC;
-                r[i].c = *reinterpret_cast<const uint4*>(rec + 16 * lane);
-                const uint2 hb = *reinterpret_cast<const uint2*>(rec + 1024 + 8 * lane);
-                r[i].c2.x = hb.x;
-                r[i].c2.y = hb.y;
-                const uint2 sc = *reinterpret_cast<const uint2*>(rec + 1536 + 8 * n);
-                r[i].m[0] = sc.x;
-                r[i].m[1] = sc.y;
-                r[i].m[2] = *reinterpret_cast<const uint16_t*>(rec + 1664 + 2 * n);
-            } else {
-                const uint8_t* p = wbase[i] + (w.group == 1 ? 2048 : 128) * (size_t)s;
-                r[i].c = *reinterpret_cast<const uint4*>(p);
-                r[i].c2 = *reinterpret_cast<const uint4*>(p + fp8_second_chunk(w));
-                r[i].m[0] = __float_as_uint(sbase[i][(128 * (step0 + s)) / w.bc]);
-            }
-        }
-    };
-    auto load_raw = [&](Raw* r, uint32_t s) {
-        load_raw_tile(r, 0, s);
-        if (DT == 2) load_raw_tile(r, 1, s);
-    };
-    // `s`: the step the records belong to (of this slice)
-    auto dequant_tile = [&](const Raw& r, int i, uint32_t buf, uint32_t s) {  // one of the wave's row tiles, 4 blocks
-        if (NT % WAVES != 0 && DT * wave + i >= NT) return;
-        uint4* dst = bfrag + ((size_t)(buf * 4) * NT + DT * wave + i) * 64 + lane;  // block b: + b * NT * 64
-        if (FMT == FMT_NVFP4) {  // as MXFP4 below with a scale per 16: the low nibbles' sub-block 2 b, the high nibbles' 2 b + 1
-            const uint32_t cw[4] = {r.c.x, r.c.y, r.c.z, r.c.w};
-            const float g = __uint_as_float(r.m[2]);
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const uint32_t sw = r.m[b >> 1] >> (16 * (b & 1));
-                const float d0 = ue4m3_half(sw) * g, d1 = ue4m3_half(sw >> 8) * g;
-                const uint32_t lo = mxfp4_values<12>(cw[b] & 0x0F0F0F0Fu), hi = mxfp4_values<12>((cw[b] >> 4) & 0x0F0F0F0Fu);
-                const float c0 = -12.0f * d0, c1 = -12.0f * d1;
-                dst[b * NT * 64] = make_uint4(pack_bf16(__builtin_fmaf(byte_f32<0>(lo), d0, c0), __builtin_fmaf(byte_f32<1>(lo), d0, c0)),
-                                              pack_bf16(__builtin_fmaf(byte_f32<2>(lo), d0, c0), __builtin_fmaf(byte_f32<3>(lo), d0, c0)),
-                                              pack_bf16(__builtin_fmaf(byte_f32<0>(hi), d1, c1), __builtin_fmaf(byte_f32<1>(hi), d1, c1)),
-                                              pack_bf16(__builtin_fmaf(byte_f32<2>(hi), d1, c1), __builtin_fmaf(byte_f32<3>(hi), d1, c1)));
-            }
-        } else if (FMT == FMT_MXFP4) {  // the code's doubled value + 12 as an unsigned byte, times the block's power of two: exact in bf16
-            const uint32_t cw[4] = {r.c.x, r.c.y, r.c.z, r.c.w};
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const float d = e8m0_half((r.m[0] >> (8 * b)) & 0xFF);
-                dst[b * NT * 64] = dequant_u8x8(mxfp4_values<12>(cw[b] & 0x0F0F0F0Fu), mxfp4_values<12>((cw[b] >> 4) & 0x0F0F0F0Fu), d, -12.0f * d);
-            }
-        } else if (FMT == FMT_Q40) {  // the block's own scale: word b / 2, half b % 2; (nib - 8) * d
-            const uint32_t cw[4] = {r.c.x, r.c.y, r.c.z, r.c.w};
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const float d = f16_bits_to_f32((uint16_t)((b & 1) ? r.m[b >> 1] >> 16 : r.m[b >> 1] & 0xFFFF));
-                dst[b * NT * 64] = dequant_q4m(cw[b], d, -8.0f * d);
-            }
-        } else if (FMT == FMT_Q4M) {
-            const uint32_t cw[4] = {r.c.x, r.c.y, r.c.z, r.c.w};
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int g = b >> 1;
-                const float d = f16_bits_to_f32((uint16_t)(g ? r.m[0] >> 16 : r.m[0] & 0xFFFF));
-                const float off = bf16_bits_to_f32((uint16_t)(g ? r.m[1] >> 16 : r.m[1] & 0xFFFF));
-                dst[b * NT * 64] = dequant_q4m(cw[b], d, off - 8.0f * d);
-            }
-        } else if (q8_format(FMT)) {  // block b = 2 h + e: codes 8 kq .. + 7 of block e of record h; q * d as (q + 128) * d - 128 d
-            const uint32_t cw[8] = {r.c.x, r.c.y, r.c.z, r.c.w, r.c2.x, r.c2.y, r.c2.z, r.c2.w};
-            const bool past = 2 * (step0 + s) + 1 >= t8_steps(w.n_in);  // the step's second record lies past the row
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int h = b >> 1, e = b & 1;
-                float d = FMT == FMT_Q8F ? __uint_as_float(r.m[b]) : f16_bits_to_f32((uint16_t)(e ? r.m[h] >> 16 : r.m[h] & 0xFFFF));
-                if (h && past) d = 0.0f;
-                dst[b * NT * 64] = dequant_u8x8(cw[2 * b] ^ 0x80808080u, cw[2 * b + 1] ^ 0x80808080u, d, -128.0f * d);
-            }
-        } else if (k45_format(FMT)) {  // block b = 2 jj + e: the low (e = 0) or high nibbles of the chunk's byte pair jj
-            const float d = f16_bits_to_f32((uint16_t)(r.m[2] & 0xFFFF)), dmin = f16_bits_to_f32((uint16_t)(r.m[2] >> 16));
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int jj = b >> 1, e = b & 1;
-                const uint32_t lo = jj ? r.c.z : r.c.x, hi = jj ? r.c.w : r.c.y;
-                const float sc = (float)((r.m[0] >> (8 * b)) & 0xFF), mn = (float)((r.m[1] >> (8 * b)) & 0xFF);
-                uint32_t w0 = (lo >> (4 * e)) & 0x0F0F0F0Fu, w1 = (hi >> (4 * e)) & 0x0F0F0F0Fu;
-                if (FMT == FMT_Q5_K) {  // the fifth bits of the block's two dwords: bits 8 k + 2 b and 8 k + 2 b + 1 of the plane
-                    w0 |= ((r.c2.x >> (2 * b)) & 0x01010101u) << 4;
-                    w1 |= ((r.c2.x >> (2 * b + 1)) & 0x01010101u) << 4;
-                }
-                dst[b * NT * 64] = dequant_u8x8(w0, w1, d * sc, -(dmin * mn));
-            }
-        } else if (FMT == FMT_Q6_K) {  // block b = 2 h + e: codes 8 e .. + 7 of the lane's 16 columns of half h
-            const float d = f16_bits_to_f32((uint16_t)(r.m[2] & 0xFFFF));
-            const uint32_t kq = lane >> 4;
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int h = b >> 1, e = b & 1;
-                const uint32_t src = e ? (h ? r.c.w : r.c.y) : (h ? r.c.z : r.c.x), hh = (h ? r.c2.y : r.c2.x) >> (4 * e);
-                const uint32_t w0 = (src & 0x0F0F0F0Fu) | ((hh & 0x03030303u) << 4);
-                const uint32_t w1 = ((src >> 4) & 0x0F0F0F0Fu) | (((hh >> 2) & 0x03030303u) << 4);
-                const float dsc = d * (float)(int)(int8_t)((r.m[h] >> (8 * kq)) & 0xFF);
-                dst[b * NT * 64] = dequant_u8x8(w0, w1, dsc, -32.0f * dsc);
-            }
-        } else {
-            const uint32_t cw[8] = {r.c.x, r.c.y, r.c.z, r.c.w, r.c2.x, r.c2.y, r.c2.z, r.c2.w};
-            const float sc = __uint_as_float(r.m[0]);
-#pragma unroll
-            for (int b = 0; b < 4; b++) {  // bytes 8 b .. 8 b + 7 of the lane's 32
-                const f32x2 v0 = __builtin_amdgcn_cvt_pk_f32_fp8((int)cw[2 * b], false);
-                const f32x2 v1 = __builtin_amdgcn_cvt_pk_f32_fp8((int)cw[2 * b], true);
-                const f32x2 v2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)cw[2 * b + 1], false);
-                const f32x2 v3 = __builtin_amdgcn_cvt_pk_f32_fp8((int)cw[2 * b + 1], true);
-                const uint32_t o[4] = {pack_bf16(v0.x * sc, v0.y * sc), pack_bf16(v1.x * sc, v1.y * sc),
-                                       pack_bf16(v2.x * sc, v2.y * sc), pack_bf16(v3.x * sc, v3.y * sc)};
-                dst[b * NT * 64] = make_uint4(o[0], o[1], o[2], o[3]);
-            }
-        }
+        for (int b = 0; b < 4; b++) dst[b * NT * 64] = tile_block<FMT>(r, w, b, step0 + s, lane);
     };
     auto read_b = [&](uint4* dst, uint32_t buf, uint32_t b) {
 #pragma unroll
@@ -403,20 +187,18 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 
     // memory a whole K-step (four blocks, ~2000 MFMA cycles) ahead; the packed records of the next step two blocks
     // before they are dequantized into the other LDS buffer. Each fragment has one home, refilled in place right after
     // its last use.
-    constexpr bool EARLY_RAW = OXHIP_GEMM_EARLY_RAW;
-    Raw raw[DT];
+    RawTile raw;
     load_raw(raw, 0);
     uint4 a_cur[AR][NV], b_cur[NT];
     const uint32_t last = nsteps - 1, last_blk = 4 * nsteps - 1;
 #pragma unroll
     for (int b = 0; b < AR; b++) read_a(a_cur[b], min((uint32_t)b, last_blk));
-    dequant_tile(raw[0], 0, 0, 0);
-    if (DT == 2) dequant_tile(raw[DT - 1], 1, 0, 0);
+    dequant(raw, 0, 0);
     load_raw(raw, min(1u, last));
     lds_barrier();
     read_b(b_cur, 0, 0);
     // One K-step; every step does the same work, so that the loop is one body whose accumulators stay in place: the
-    // records of the next step are dequantized into the other LDS buffer during blocks 0 and 1 (with 8 waves: block 0
+    // records of the next step are dequantized into the other LDS buffer during blocks 0 and 1 (block 0
     // by the waves 0-3, block 1 by the waves 4-7, which share their SIMDs with them), block 3 refills from
     // that buffer after the barrier, and the step after next is requested during block 2. Past the end the indices
     // repeat the last step: a little work that nobody reads, instead of separate loop tails.
@@ -435,20 +217,12 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 
                 else b_cur[j] = bfrag[(((buf ^ 1) * 4) * NT + j) * 64 + lane];
             }
             read_a(a_cur[b % AR], min(4 * s + b + AR, last_blk));
-            if (DT == 1) {
-                if (b == (int)(wave >> 2)) {
-                    dequant_tile(raw[0], 0, buf ^ 1, min(s + 1, last));
-                    load_raw_tile(raw, 0, min(s + 2, last));
-                }
-            } else if (EARLY_RAW) {  // a tile's records of the step after next are requested as soon as its registers are free
-                if (b < 2) {
-                    dequant_tile(raw[b < DT ? b : 0], b, buf ^ 1, min(s + 1, last));
-                    load_raw_tile(raw, b, min(s + 2, last));
-                }
-            } else {
-                if (b == 0) dequant_tile(raw[0], 0, buf ^ 1, min(s + 1, last));
-                if (b == 1) dequant_tile(raw[DT - 1], 1, buf ^ 1, min(s + 1, last));
-                if (b == 2) load_raw(raw, min(s + 2, last));
+            if (b == (int)(wave >> 2)) {
+                dequant(raw, buf ^ 1, min(s + 1, last));
+                // (Q4_K: the compiler would put the request among the conversions, 14336 rows x 2048 tokens 234 us, 226 this way; the
+                // other formats are no faster)
+                if constexpr (FMT == FMT_Q4_K) __builtin_amdgcn_sched_barrier(0);
+                load_raw(raw, min(s + 2, last));
             }
         }
     }
@@ -538,10 +312,8 @@ static void run_gemm_reduce(const float* partial, size_t n, uint32_t slices, voi
     else out_bf16 ? go(gemm_reduce_kernel<true, 4, false>) : go(gemm_reduce_kernel<false, 4, false>);
 }
 
-// Token tiles per wave and waves per workgroup: one tile and four waves when the launch has at most four tiles (64 tokens),
-// one tile and eight waves up to eight tiles (128 tokens), else two tiles and eight waves.
+// Token tiles per wave: one when the launch has at most eight tiles (128 tokens), else two.
 static int gemm_nv(size_t mtiles) { return mtiles <= 8 ? 1 : 2; }
-static int gemm_waves(size_t mtiles) { return mtiles <= 4 ? 4 : 8; }  // (5 to 8 token tiles: eight waves of one tile each)
 
 // Row tiles per workgroup (8, or 7 with two token tiles per wave) and K slices of a launch: the pair that costs least, in units
 // of one K-step of an eight-tile workgroup (0.9 us with one token tile per wave, 1.2 to 1.5 us with two):
@@ -551,9 +323,7 @@ static int gemm_waves(size_t mtiles) { return mtiles <= 4 ? 4 : 8; }  // (5 to 8
 //     in 8 slices, 21.2 in 10.
 //   1 for every million partial sums written and read back, 1.9 for those past six million, and 2 for the launch that adds them
 //     (14336 -> 4096, MLX 4-bit, 420 tokens, 4 slices -> 8: 6.9 million more, as many steps, 63.6 -> 69.7 us).
-// Any number of slices counts, not only powers of two: 9472 columns, MLX 4-bit x 9000 rows are 71 workgroups of 74 steps, at
-// 24 tokens 36 us in 3 slices, 38.7 in 4 (284 workgroups), 27.9 in 7 (497); 4352 columns, Q6_K x 5001 rows at 24 tokens
-// 20.7 us in 4, 18.4 in 6 (240 workgroups), 20.6 in 8. With two tiles: 14336 -> 4096, MLX 4-bit, 1100 tokens (160 workgroups) 167.6 us
+// Any number of slices counts, not only powers of two. With two tiles: 14336 -> 4096, MLX 4-bit, 1100 tokens (160 workgroups) 167.6 us
 // whole, 153.0 in 3 slices, 190.8 in 2; FP8 7168 x 18432 at 1100 tokens 397 us whole, 331 in 3. Four steps per slice at least
 // (7168 -> 1536, Q8_0, 200 tokens: 30.7 us at 14 steps, 24.4 at 7, 23.5 at 5).
 // Seven row tiles: 14336 rows x 512 tokens are one round of 256 workgroups of 112 rows instead of 224 of 128, 63 -> 60 us: a step of
@@ -564,11 +334,11 @@ struct GemmPlan {
 };
 static GemmPlan gemm_plan(const WeightView& w, size_t mtiles) {
     const bool one = gemm_nv(mtiles) == 1;
-    const uint32_t per_wg = gemm_waves(mtiles) * gemm_nv(mtiles), cols = (uint32_t)((mtiles + per_wg - 1) / per_wg);
+    const uint32_t per_wg = WAVES * gemm_nv(mtiles), cols = (uint32_t)((mtiles + per_wg - 1) / per_wg);
     const uint32_t steps = (w.n_in + 127) / 128;
-    const bool alone = !one || (gemm_waves(mtiles) == 8 && q8_format(w.fmt));
-    // (Eight waves of one tile: eight slices at most, 14336 -> 4096, MLX 4-bit at 70 tokens 29.1 us in 8 and 30.2 in 16.)
-    const uint32_t most = one && gemm_waves(mtiles) == 8 ? 8 : 16;
+    const bool alone = !one || q8_format(w.fmt);
+    // (One token tile per wave: eight slices at most, 14336 -> 4096, MLX 4-bit at 70 tokens 29.1 us in 8 and 30.2 in 16.)
+    const uint32_t most = one ? 8 : 16;
     const double millions = (double)mtiles * 16 * w.n_out * 1e-6;
     auto sums = [](double m) { return m < 6 ? m : 6 + 1.9 * (m - 6); };
     GemmPlan best{WG_NT, 1};
@@ -597,7 +367,7 @@ static GemmPlan gemm_plan(const WeightView& w, size_t mtiles) {
 uint32_t gemm_k_slices(const WeightView& w, size_t mtiles) { return gemm_plan(w, mtiles).slices; }
 
 namespace {
-template <int FMT, int NV, int NT, int WAVES = (NV == 1 ? 4 : 8)>
+template <int FMT, int NV, int NT>
 hipError_t run_gemm_bf16_nv(const WeightView& w, const void* apk, size_t t, size_t mtiles, void* y, bool out_bf16, float* partial,
                          hipStream_t s) {
     const uint32_t slices = gemm_k_slices(w, mtiles);
@@ -613,14 +383,14 @@ hipError_t run_gemm_bf16_nv(const WeightView& w, const void* apk, size_t t, size
     // Eight waves of one token tile that leave a second workgroup no room on their CU: the 8-bit formats always; Q4_K in launches of
     // at most a workgroup per CU, which need none, while the spill of the bounded kernel costs a start half a microsecond later
     // (2048 columns x 7168 rows at 80 tokens, 224 workgroups: 19.0 us bounded, 18.4 this way).
-    constexpr bool ALWAYS = NV == 1 && WAVES == 8 && q8_format(FMT), CHOICE = NV == 1 && WAVES == 8 && FMT == FMT_Q4_K;
+    constexpr bool ALWAYS = NV == 1 && q8_format(FMT), CHOICE = NV == 1 && FMT == FMT_Q4_K;
     span_start(s);
     if (CHOICE && (uint64_t)grid.x * grid.y * grid.z <= 256) {
-        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, WAVES, NT, CHOICE || ALWAYS>);
-        else go(gemm_bf16_kernel<FMT, false, NV, WAVES, NT, CHOICE || ALWAYS>);
+        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, NT, CHOICE || ALWAYS>);
+        else go(gemm_bf16_kernel<FMT, false, NV, NT, CHOICE || ALWAYS>);
     } else {
-        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, WAVES, NT, ALWAYS>);
-        else go(gemm_bf16_kernel<FMT, false, NV, WAVES, NT, ALWAYS>);
+        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, NT, ALWAYS>);
+        else go(gemm_bf16_kernel<FMT, false, NV, NT, ALWAYS>);
     }
     if (e != hipSuccess) return e;
     e = hipGetLastError();
@@ -632,8 +402,7 @@ hipError_t run_gemm_bf16_nv(const WeightView& w, const void* apk, size_t t, size
 template <int FMT>
 hipError_t run_gemm_bf16(const WeightView& w, const void* apk, size_t t, size_t mtiles, void* y, bool out_bf16, float* partial,
                          hipStream_t s) {
-    if (gemm_nv(mtiles) == 1 && gemm_waves(mtiles) == 4) return run_gemm_bf16_nv<FMT, 1, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
-    if (gemm_nv(mtiles) == 1) return run_gemm_bf16_nv<FMT, 1, WG_NT, 8>(w, apk, t, mtiles, y, out_bf16, partial, s);
+    if (gemm_nv(mtiles) == 1) return run_gemm_bf16_nv<FMT, 1, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
     if (gemm_plan(w, mtiles).nt == 7) return run_gemm_bf16_nv<FMT, 2, 7>(w, apk, t, mtiles, y, out_bf16, partial, s);
     return run_gemm_bf16_nv<FMT, 2, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
 }

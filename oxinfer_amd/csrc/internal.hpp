@@ -223,6 +223,10 @@ hipError_t launch_quantize_pack_i8(const void* x, bool src_bf16, size_t t, const
 hipError_t launch_gemm_i8(const WeightView& w, const void* frag, const void* xs, const void* fs, size_t t, float* y, int32_t* dump, hipStream_t s);
 hipError_t launch_gemm_bf16(const WeightView& w, const void* apk, size_t t, size_t mtiles, void* y, bool out_bf16, float* partial,
                             hipStream_t s);
+// gemm_short.hip: the same product for at most 64 tokens, from the same fragments
+bool gemm_short_ok(size_t t);
+uint32_t gemm_short_slices(const WeightView& w, size_t t);
+hipError_t launch_gemm_short(const WeightView& w, const void* apk, size_t t, void* y, bool out_bf16, float* partial, hipStream_t s);
 hipError_t launch_quantize_act_fp8(const void* x, bool src_bf16, size_t t, size_t n_in, size_t mtiles, size_t kblocks, void* out,
                                    float* sx, hipStream_t s);
 uint32_t gemm_fp8_k_slices(const WeightView& w, size_t mtiles);

@@ -212,6 +212,47 @@ def test_gemm_bf16_random_shapes_match_oracle(be, oxref):
             assert np.isfinite(y).all() and row_err(y, ref) < 2e-2, (name, n_out, n_in, t, xd.dtype, ob)
 
 
+def any_weight(be, oxref, name, n_out, n_in, seed):
+    """(uploaded weight, its dequantized rows) of any format that the bf16 GEMM takes."""
+    from oxinfer_amd import synth
+    if name == "MLX":
+        raw, (q, s16, off) = mlx_case(oxref, n_out, n_in, seed)
+        return be.upload_mlx_q4(*raw, 64, n_out, n_in), oxref.dequant_rows_q4(q, s16, off, 64, n_out, n_in)
+    if name == "Q8":
+        q, sc = synth.q8_matrix(n_out, n_in, seed)
+        return be.upload_q8(q, sc, n_out, n_in), oxref.q8_dequant_rows(q, sc, n_out, n_in)
+    if name == "FP8":
+        w = be.upload_fp8(*synth.fp8_e4m3(n_out, n_in, seed), n_out, n_in)
+        return w, be.dequantize(w).cpu().numpy()
+    if name == "NVFP4":
+        w = be.upload_nvfp4(synth.gguf_nvfp4(n_out, n_in, seed)[0], n_out, n_in)
+        return w, be.dequantize(w).cpu().numpy()
+    raw = gguf_raw(name, n_out, n_in, seed)
+    return be.upload_gguf(GGUF_KINDS[name], raw, n_out, n_in), oxref.dequantize_rows(GGUF_KINDS[name], raw, n_out, n_in)
+
+
+@pytest.mark.parametrize("n_out,n_in", [(40, 256), (2050, 512), (4100, 512), (8210, 256), (12300, 256), (40, 8192), (2050, 12288), (4100, 12288)])
+@pytest.mark.parametrize("name", ["MLX", "Q8", "FP8", "NVFP4", "Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K", "MXFP4"])
+def test_gemm_up_to_64_tokens(be, oxref, name, n_out, n_in):
+    """The kernel of at most 64 tokens in all its forms: one to four row tiles per workgroup (3, 129, 257, 514 and 769 tiles, the last
+    group ragged), fewer steps than waves, rows in two, three and four slices, and the edges of one to four token tiles. Against the
+    product of the operands rounded to bf16 in 64 bits: 1e-3 as above, the f32 sums themselves being off by 6e-6 at most."""
+    import torch
+    from oxinfer_amd import synth
+    w, wf = any_weight(be, oxref, name, n_out, n_in, 41)
+    assert w is not None, be.last_error()
+    wb = torch.from_numpy(synth.bf16_round(wf)).cuda().double()
+    x64 = torch.from_numpy(synth.activations(64, n_in, 42, bf16=True)).cuda()
+    for t in (1, 16, 17, 32, 33, 48, 49, 64):
+        if name == "FP8" and t <= 32:  # (a kernel of its own, which scales the blocks' sums: its weights are not rounded)
+            continue
+        x = x64[:t].contiguous()
+        ref = (x.double() @ wb.T).cpu().numpy()
+        assert row_err(be.gemm(w, x).cpu().numpy(), ref) < 1e-3, t
+        yb = be.gemm(w, x.to(torch.bfloat16), out_bf16=True).float().cpu().numpy()
+        assert row_err(yb, ref) < 1e-3 + 2**-8, t  # (the result rounded to bf16)
+
+
 @pytest.mark.parametrize("n_out,n_in", [(40, 640), (130, 96)])
 def test_gemm_bf16_q8_matrix_matches_oracle(be, oxref, n_out, n_in):
     """QMatrix (int8 codes, f32 scale per 32; src/quant.rs:128-133) through the same kernel."""
