@@ -51,6 +51,7 @@ class QActC(C.Structure):
 
 
 _lib = None
+_torch = None
 
 
 def library_path():
@@ -59,14 +60,14 @@ def library_path():
 
 def load_library():
     """Loads liboxinfer_hip.so (built in-tree by `python -m oxinfer_amd.build`). Raises if it is missing."""
-    global _lib
+    global _lib, _torch
     if _lib is not None:
         return _lib
     if not os.path.exists(_SO):
         raise RuntimeError(f"{_SO} is not built: run `python -m oxinfer_amd.build` (hipcc, gfx950). "
                            "There is no CPU fallback in this package.")
     try:
-        import torch  # noqa: F401  (its bundled HIP runtime must be the one this process uses)
+        import torch as _torch  # (its bundled HIP runtime must be the one this process uses)
     except ImportError:
         pass
     lib = C.CDLL(_SO)
@@ -382,8 +383,14 @@ class HipBackend:
     # ---- device-pointer entry points -------------------------------------------------------
     @staticmethod
     def _stream():
-        import torch
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        """The current torch stream of the current device, as the handle that the library takes. By torch's accessor of the handle
+        itself where it has one: building a torch Stream object for its handle took 3 us of the 6.5 us that a call of one launch
+        takes, this 0.2 us (a 4096 x 4096 product of one token, two calls: 14.5 -> 9.3 us)."""
+        c = _torch._C
+        try:
+            return c._cuda_getCurrentRawStream(c._cuda_getDevice())
+        except AttributeError:
+            return _torch.cuda.current_stream().cuda_stream
 
     def quantize_act(self, x, out=None):
         """x: torch f32 [t, n_in] on the device -> QAct (device)."""

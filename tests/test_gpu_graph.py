@@ -235,6 +235,25 @@ def test_norm_on_both_sides_of_the_workgroup_limit(be, n, rows):
         assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
 
 
+def test_calls_go_to_the_current_torch_stream(be):
+    """The handle that a call passes on is that of torch's current stream, inside and outside of a stream's context and in every thread."""
+    import threading
+    import torch
+
+    def current():
+        return be._stream(), torch.cuda.current_stream().cuda_stream
+    side = torch.cuda.Stream()
+    seen = [current()]
+    with torch.cuda.stream(side):
+        seen.append(current())
+        t = threading.Thread(target=lambda: seen.append(current()))  # (a thread starts on the default stream)
+        t.start()
+        t.join()
+    seen.append(current())
+    assert all(a == b for a, b in seen) and [a for a, _ in seen] == [0, side.cuda_stream, 0, 0]
+
+
+
 def test_norm_rounds_the_reciprocal_root_correctly(be):
     """r = m^(-1/2) is the f32 value nearest to the exact one also where that lies closest to the middle between two f32 values: the
     4096 such means of [1, 4) (every exponent's r is one of theirs, times a power of two). A row's squares add up to 32 m in f32, and
