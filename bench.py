@@ -449,7 +449,7 @@ def bench_moe(be, torch, synth, steps, warmup, pool_gb, t, experts, int8=False):
                 roofline={"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                           "frac": round(ach / HBM_PEAK_GBS, 4),
                           "traffic": profile_traffic(f"moe_t{t}.md") if t in (1, 256) and not int8 else None,
-                          "kernel": "moe_bf16_kernel<4> (grouped)" if prefill_form else "decode_mfma_kernel<6, *, false, true, true> (grouped)",
+                          "kernel": "moe_bf16_kernel (grouped)" if prefill_form else "decode_mfma_kernel<6, *, false, true, true> (grouped)",
                           "bytes_per_launch": nbytes, "avg_launch_us": round(ms * 1e3, 2)},
                 tflops=round(flops / (ms * 1e-3) / 1e12, 2))
 

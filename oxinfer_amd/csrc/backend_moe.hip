@@ -1,5 +1,6 @@
 // Backend::upload_moe / moe / matvec_rows (src/gpu.rs:165, :206-248 of the reference) over the grouped
 // decode kernel, plus their device-pointer forms.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
@@ -30,6 +31,9 @@ size_t up256(size_t v) { return (v + 255) / 256 * 256; }
 
 constexpr size_t COMB_GROUPS = 4096;  // row groups of the down projection that may meet through counters (h <= 65536)
 
+// The most chunks of up to 32 rows that a plan of the bf16 prefill form can cut.
+size_t bf16_chunks(size_t pairs, size_t n_exp) { return (pairs < n_exp ? pairs : n_exp) + pairs / 32 + 1; }
+
 // The scratch of one pass, carved from one allocation.
 struct Scratch {
     int* row_of;
@@ -41,7 +45,7 @@ struct Scratch {
     float* a;       // [pairs][inter]
     oxhip_qact aq;  // a quantized
     float* o;       // [pairs][h]
-    void* fx;       // bf16 fragments of the chunks' rows of x, and of a (the prefill form: chunks of up to 16 rows)
+    void* fx;       // the prefill form's bf16 rows of x, and its chunks' fragments of a
     void* fa;
     uint32_t* counters;  // arrival counters of the down launch's row groups (zero between launches)
     uint32_t max_chunks;
@@ -71,10 +75,9 @@ Scratch carve(uint8_t* base, size_t t, size_t pairs, size_t n_exp, size_t h, siz
     s.a = reinterpret_cast<float*>(take(pairs * inter * 4));
     s.aq = carve_qact(take(qact_bytes(pairs, inter)), pairs, inter);
     s.o = reinterpret_cast<float*>(take(pairs * h * 4));
-    const size_t chunks16 = (pairs < n_exp ? pairs : n_exp) + pairs / 16 + 1;
     const bool prefill = pairs / n_exp >= 6 && h % 128 == 0 && inter % 128 == 0;
-    s.fx = take(prefill ? moe_bf16_frag_bytes(chunks16, h) : 0);
-    s.fa = take(prefill ? moe_bf16_frag_bytes(chunks16, inter) : 0);
+    s.fx = take(prefill ? moe_bf16_row_bytes(t, h) : 0);
+    s.fa = take(prefill ? moe_bf16_frag_bytes(bf16_chunks(pairs, n_exp), inter) : 0);
     s.bytes = off;
     return s;
 }
@@ -131,10 +134,9 @@ int moe_pass(oxhip_ctx* c, oxhip_moe* m, const float* x, size_t t, const uint32_
     // Prefill passes over MLX 4-bit experts (six or more routed rows per expert on average) take the bf16 form: see
     // moe_bf16.hip. OXHIP_MOE_INT8 (oxhip_moe_set_mode) keeps the integer path (the 1e-3 accuracy class) at any size.
     const bool fused = m->up.empty();
-    const size_t grid_chunks16 = (pairs < m->n_exp ? pairs : m->n_exp) + pairs / 16 + 1;
     const bool bf16_form = avg >= 6 && fused && moe_bf16_ok(m->gate_up[0]->v) && moe_bf16_ok(m->down[0]->v) && m->mode != OXHIP_MOE_INT8 &&
-                           reinterpret_cast<uintptr_t>(x) % 16 == 0 && grid_chunks16 <= 65535;
-    if (bf16_form) max_rows = 16;
+                           reinterpret_cast<uintptr_t>(x) % 16 == 0 && (pairs < m->n_exp ? pairs : m->n_exp) + pairs / 16 + 1 <= 65535;
+    if (bf16_form) max_rows = 32;
     if (!bf16_form) {
         // The grouped integer kernel stages a chunk's activations in LDS, one set per group of 8 rows: long rows take
         // smaller chunks (checked for every projection before anything is launched).
@@ -156,27 +158,24 @@ int moe_pass(oxhip_ctx* c, oxhip_moe* m, const float* x, size_t t, const uint32_
     // One token over fused gate / up experts needs no plan: chunk j is route j (see GroupView::direct); its routing
     // and the quantization of x share a launch, and the pass is three launches.
     const bool direct = !bf16_form && t == 1 && fused && decode_grouped_glu_ok(m->gate_up[0]->v, inter) && row_tiles((uint32_t)h) <= COMB_GROUPS;
-    if (!routed && !(direct && m->n_exp <= 256)) {
+    const bool beside = m->n_exp <= 256;  // the routing kernel has room for other work beside it
+    if (bf16_form) {
+        if (!routed && beside) HIP_TRY(launch_route_rows(rin.logits, t, m->n_exp, k, ridx_out, rw_out, rin.stride, rin.expert_scale, x, m->gate_up[0]->v, sc.fx, s), "route + rows launch");
+        else HIP_TRY(launch_moe_rows(x, t, m->gate_up[0]->v, sc.fx, s), "moe rows launch");
+    }
+    if (!routed && !((direct || bf16_form) && beside)) {
         HIP_TRY(launch_route_top_k(rin.logits, t, m->n_exp, k, ridx_out, rw_out, s, rin.stride, rin.expert_scale), "route_top_k launch");
         routed = true;
     }
     if (bf16_form) {
         HIP_TRY(launch_moe_plan(route_idx, pairs, k, m->n_exp, max_rows, sc.row_of, sc.src, sc.chunks, sc.nchunks, s), "moe plan launch");
-        HIP_TRY(launch_moe_pack_bf16(x, h, sc.src, sc.chunks, sc.nchunks, grid_chunks, sc.fx, s, moe_bf16_std_geometry(m->gate_up[0]->v)), "moe pack launch");
+        // (about as many chunks as there will be: an expert has a last one, half full on average, and its rows past 16 in 32s before it)
+        const size_t chunks = std::min(m->n_exp, pairs) + (avg > 16 ? (pairs - 16 * m->n_exp) / 32 : 0);
+        g.rowmap = sc.src;
         g.bases = m->bases_gu;
-        if (moe_bf16_glu_ok(m->gate_up[0]->v, inter, grid_chunks)) {
-            // the gate / up launch pairs gate and up tiles per workgroup, applies the activation and writes the down projection's fragments
-            HIP_TRY(launch_moe_bf16(m->gate_up[0]->v, g, grid_chunks, sc.fx, nullptr, s, inter, m->act_kind, m->act_param, moe_bf16_std_geometry(m->down[0]->v),
-                                    sc.fa),
-                    "moe gate launch");
-        } else {
-            HIP_TRY(launch_moe_bf16(m->gate_up[0]->v, g, grid_chunks, sc.fx, sc.gu, s), "moe gate launch");
-            HIP_TRY(launch_moe_act_pack_bf16(sc.gu, sc.gu + inter, 2 * inter, inter, m->act_kind, m->act_param, sc.chunks, sc.nchunks, grid_chunks, sc.fa, s,
-                                             moe_bf16_std_geometry(m->down[0]->v)),
-                    "moe act launch");
-        }
+        HIP_TRY(launch_moe_bf16_gate(m->gate_up[0]->v, m->down[0]->v, g, grid_chunks, (uint32_t)chunks, sc.fx, t, m->act_kind, m->act_param, sc.fa, s), "moe gate launch");
         g.bases = m->bases_dn;
-        HIP_TRY(launch_moe_bf16(m->down[0]->v, g, grid_chunks, sc.fa, sc.o, s), "moe down launch");
+        HIP_TRY(launch_moe_bf16_down(m->down[0]->v, g, grid_chunks, (uint32_t)chunks, sc.fa, sc.o, s), "moe down launch");
     } else {
         if (direct) {
             if (!routed) HIP_TRY(launch_route_quantize(rin.logits, 1, m->n_exp, k, ridx_out, rw_out, rin.stride, rin.expert_scale, x, h, sc.xa, s), "route + quantize launch");

@@ -238,6 +238,9 @@ hipError_t launch_route_top_k(const float* logits, size_t t, size_t n, size_t k,
 // microseconds of latency); n <= 256.
 hipError_t launch_route_quantize(const float* logits, size_t t, size_t n, size_t k, uint32_t* idx, float* w, size_t stride,
                                  const float* expert_scale, const float* x, size_t h, const oxhip_qact& o, hipStream_t s);
+// route_top_k and launch_moe_rows (for experts like `w`) of the same t rows in one launch; n <= 256.
+hipError_t launch_route_rows(const float* logits, size_t t, size_t n, size_t k, uint32_t* idx, float* wts, size_t stride, const float* expert_scale, const float* x,
+                             const WeightView& w, void* rows, hipStream_t s);
 hipError_t launch_moe_plan(const uint32_t* route_idx, size_t pairs, size_t k, size_t n_exp, uint32_t chunk_rows, int* row_of, int* src,
                            int4* chunks, int* nchunks, hipStream_t s);
 hipError_t launch_moe_front(const uint32_t* route_idx, size_t pairs, size_t k, size_t n_exp, uint32_t chunk_rows, int* row_of, int* src,
@@ -256,17 +259,14 @@ hipError_t launch_router_logits(const float* x, const float* router, const float
 hipError_t launch_rmsnorm_quantize(const float* x, const float* w_f32, const uint16_t* w_bf16, float eps, size_t t, size_t n, float* out,
                                    const oxhip_qact* q, hipStream_t s, float pre = 1.0f, bool add = false, size_t x_stride = 0,
                                    size_t out_stride = 0);
-// The bf16 form of the grouped expert matmuls for prefill passes (moe_bf16.hip): MLX 4-bit weights, chunks of <= 16 rows.
+// The bf16 form of the grouped expert matmuls for prefill passes (moe_bf16.hip): fused gate / up experts, chunks of <= 32 rows.
 bool moe_bf16_ok(const WeightView& w);
-bool moe_bf16_std_geometry(const WeightView& w);  // its fragments hold a block's columns as 8 kq + j (Q8_0, Q4_K), not as T4M records do
+size_t moe_bf16_row_bytes(size_t t, size_t n_in);
 size_t moe_bf16_frag_bytes(size_t max_chunks, size_t n_in);
-hipError_t launch_moe_pack_bf16(const float* x, size_t n_in, const int* rowmap, const int4* chunks, const int* nchunks, uint32_t max_chunks,
-                                void* frag, hipStream_t s, bool std_geometry = false);
-hipError_t launch_moe_act_pack_bf16(const float* g, const float* u, size_t stride, size_t inter, uint32_t kind, float param, const int4* chunks,
-                                    const int* nchunks, uint32_t max_chunks, void* frag, hipStream_t s, bool std_geometry = false);
-bool moe_bf16_glu_ok(const WeightView& w, size_t inter, uint32_t max_chunks);  // the gate / up launch can apply the activation and write the down projection's fragments
-hipError_t launch_moe_bf16(const WeightView& w, const GroupView& g, uint32_t max_chunks, const void* frag, float* out, hipStream_t s,
-                           size_t glu_inter = 0, uint32_t act_kind = 0, float act_param = 0.0f, bool std_out = false, void* out_frag = nullptr);
+hipError_t launch_moe_rows(const float* x, size_t t, const WeightView& w, void* rows, hipStream_t s);
+hipError_t launch_moe_bf16_gate(const WeightView& w, const WeightView& down, const GroupView& g, uint32_t max_chunks, uint32_t chunks, const void* rows, size_t t,
+                                uint32_t act_kind, float act_param, void* frag, hipStream_t s);
+hipError_t launch_moe_bf16_down(const WeightView& w, const GroupView& g, uint32_t max_chunks, uint32_t chunks, const void* frag, float* out, hipStream_t s);
 
 hipError_t launch_fill_zero(uint32_t* p, size_t n, hipStream_t s);  // n dwords, by a kernel on `s`
 

@@ -4,6 +4,7 @@
 // re-quantization of its output, and the weighted combination in route order.
 #include "act_body.hpp"
 #include "internal.hpp"
+#include "moe_rows.hpp"
 
 namespace oxhip {
 
@@ -155,6 +156,30 @@ hipError_t launch_route_quantize(const float* logits, size_t t, size_t n, size_t
         route_quantize_kernel<2><<<grid, 512, 0, s>>>(logits, st, (uint32_t)n, (uint32_t)k, idx, w, expert_scale, (uint32_t)t, x, nblocks, qact_out(o));
     else
         route_quantize_kernel<4><<<grid, 512, 0, s>>>(logits, st, (uint32_t)n, (uint32_t)k, idx, w, expert_scale, (uint32_t)t, x, nblocks, qact_out(o));
+    return hipGetLastError();
+}
+
+// Workgroups 0 .. t - 1 route a token each; the others make the bf16 prefill form's rows of x (moe_row_unit).
+template <int PER, bool STD>
+__global__ __launch_bounds__(512) void route_rows_kernel(const float* __restrict__ logits, uint32_t stride, uint32_t n, uint32_t k, uint32_t* __restrict__ idx,
+                                                         float* __restrict__ wts, const float* __restrict__ expert_scale, uint32_t t, const float* __restrict__ x,
+                                                         size_t units, uint4* __restrict__ xb, float* __restrict__ sums) {
+    if (blockIdx.x < t) route_top_k_body<PER, 8>(logits, stride, n, k, idx, wts, expert_scale, blockIdx.x);
+    else moe_row_unit<STD>(x, (size_t)(blockIdx.x - t) * 512 + threadIdx.x, units, xb, sums);
+}
+
+hipError_t launch_route_rows(const float* logits, size_t t, size_t n, size_t k, uint32_t* idx, float* wts, size_t stride, const float* expert_scale, const float* x,
+                             const WeightView& w, void* rows, hipStream_t s) {
+    const size_t units = t * w.n_in / 8;
+    if (!units) return hipSuccess;
+    if (n > 256) return hipErrorInvalidValue;
+    uint4* xb = static_cast<uint4*>(rows);
+    float* sums = reinterpret_cast<float*>(xb + units);
+    auto go = [&](auto kern) {
+        kern<<<(unsigned)(t + (units + 511) / 512), 512, 0, s>>>(logits, (uint32_t)(stride ? stride : n), (uint32_t)n, (uint32_t)k, idx, wts, expert_scale, (uint32_t)t, x, units, xb, sums);
+    };
+    if (n <= 128) std_columns(w.fmt) ? go(route_rows_kernel<2, true>) : go(route_rows_kernel<2, false>);
+    else std_columns(w.fmt) ? go(route_rows_kernel<4, true>) : go(route_rows_kernel<4, false>);
     return hipGetLastError();
 }
 

@@ -238,6 +238,56 @@ def test_moe_prefill_rows_do_not_depend_on_the_batch(be, oxref, mlx_experts):
         assert np.array_equal(ys.view(np.uint32), y[keep].view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt", ["mlx", "Q4_K", "Q8_0", "Q4_0", "MXFP4", "mlx, Q8_0 down"])
+@pytest.mark.parametrize("h,inter", [(2304, 384), (256, 256), (4096, 256)])  # staged in three phases and one, an odd number of steps; one; four and one
+def test_moe_prefill_chunks(be, oxref, fmt, h, inter):
+    """The bf16 form's chunks at the edges of its token tiles and of a chunk (experts of 33, 32, 17, 16 and 1 rows): within 6e-3 of the
+    reference's grouped f32 path on activations that are bf16 values already (as in test_moe_gguf_experts), and bit for bit the same
+    where the tokens, and with them the rows' places, come in another order."""
+    from oxinfer_amd import synth
+    if fmt == "Q4_K":
+        inter = (inter + 255) // 256 * 256  # whole super-blocks
+    rows = [33, 32, 17, 16, 1]
+    ne, t = len(rows), sum(rows)
+    kinds = {"Q4_K": (Q4_K, synth.gguf_q4_k), "Q8_0": (Q8_0, synth.gguf_q8_0), "Q4_0": (Q4_0, synth.gguf_q4_0), "MXFP4": (MXFP4, synth.gguf_mxfp4)}
+
+    def experts(f, n, c, seed):
+        """(raw, dequantized f32 rows, descriptor) of each expert"""
+        out = []
+        for e in range(ne):
+            if f == "mlx":
+                raw = synth.mlx_q4(n, c, seed + e)
+                out.append((raw, oxref.dequant_rows_q4(*oxref.from_mlx_q4(*raw, n, c, 64), 64, n, c), be.desc_mlx_q4(*raw, 64, n, c)))
+            else:
+                kind, make = kinds[f]
+                raw = make(n, c, seed + e)
+                out.append((raw, oxref.dequantize_rows(kind, raw, n, c), be.desc_gguf(kind, raw, n, c)))
+        return out
+
+    first, second = ("mlx", "Q8_0") if "down" in fmt else (fmt, fmt)
+    gu, dn = experts(first, 2 * inter, h, 2500), experts(second, h, inter, 2600)
+    dev = be.upload_moe([e[2] for e in gu], [e[2] for e in dn], h, inter)
+    assert dev is not None, be.last_error()
+    idx = np.repeat(np.arange(ne, dtype=np.uint32), rows)[:, None]
+    w = np.ones((t, 1), np.float32)
+    x = synth.bf16_round(synth.activations(t, h, 2700))
+    ref = np.zeros((t, h))
+    for e in range(ne):
+        at = idx[:, 0] == e
+        p = x[at].astype(np.float64) @ gu[e][1].astype(np.float64).T
+        g, u = p[:, :inter], p[:, inter:]
+        ref[at] = (g / (1.0 + np.exp(-g)) * u) @ dn[e][1].astype(np.float64).T
+    results = []
+    for order in (np.arange(t), np.random.default_rng(5).permutation(t)):
+        y = np.zeros((t, h), np.float32)
+        assert be.moe(np.ascontiguousarray(x[order]), t, h, inter, np.ascontiguousarray(idx[order]), w, 1, dev, y), be.last_error()
+        back = np.zeros_like(y)
+        back[order] = y
+        results.append(back)
+    assert row_err(results[0], ref.astype(np.float32)) < 6e-3
+    assert np.array_equal(results[0].view(np.uint32), results[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("fmt", ["mlx", "Q4_K", "Q8_0", "Q4_0", "MXFP4"])
 def test_moe_few_rows_per_expert(be, oxref, fmt):
     """A launch's chunks of up to four rows run in another form than its longer ones, and below three routed rows per expert the
