@@ -298,7 +298,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     // The records' scales: a request costs the memory pipeline the same for 64 bytes as for 1 KiB, and one per step
     // and scale word (1 to 3) would cost more than the weights themselves. So one request serves four steps: lane group
     // kq asks for the words of step `first + kq` (row n of it), and at step first + q every lane takes them from lane
-    // 16 q + n. Q8_0: {d of the two blocks}; Q4_K: {four sub-block scales, four mins, (d, dmin)}: this step's four
+    // 16 q + n (scales_of). Q8_0: {d of the two blocks}; Q4_K: {four sub-block scales, four mins, (d, dmin)}: this step's four
     // sub-blocks are 4 (s & 1) .. + 3 of the super-block; MLX: {d of the two groups, offsets of the two groups}.
     // (The scale words are ordinary loads, not read-once ones like the codes: a record is not a whole number of cache lines,
     // so its scales share a line with the next record's first codes, and a line that came in as read-once is gone again
@@ -333,10 +333,36 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
             m[1] = gload<uint32_t>(rec + 1088 + 4 * n);
         }
     };
+    // Step q of the four takes its words from lane group q, lane 16 q + n. MLX 4-bit by swaps of 32 and 16 lanes, which leave a word of two
+    // steps in all lane groups each: a lane-to-lane read goes through the LDS pipe, and the step waits for it and for every LDS read ahead of
+    // it. (MoE, 128 experts of 2048 / 768, one token 18.4 -> 18.0 us, 24 tokens 64.8 -> 63.2; two layers at 16 tokens 127.9 -> 126.7. The
+    // other formats are bound by the swaps' issue: 4096 x 4096 at one token Q4_0 4.94 -> 5.12, Q8_0 5.38 -> 5.62, MXFP4 5.33 -> 5.47, Q4_K
+    // 5.46 -> 5.56 there and 6.39 -> 6.25 at eight, Q6_K and Q5_K 1 % either way.)
+    // scur: the words as they came; snear, sfar: of step q + 1 and of steps 2 and 3.
+    constexpr bool SWAPS = FMT == FMT_Q4M;
     const int take0 = (int)(4 * n);  // byte index of lane n for the lane-to-lane read; + 64 q: lane 16 q + n
-    auto scales_of = [&](const uint32_t* grp, int q, uint32_t* m) {
+    uint32_t scur[NM], snear[SWAPS ? NM : 1], sfar[SWAPS ? NM : 1];
+    auto scales_of = [&](int q, uint32_t* m) {
 #pragma unroll
-        for (int j = 0; j < NM; j++) m[j] = (uint32_t)__builtin_amdgcn_ds_bpermute(take0 + 64 * q, (int)grp[j]);
+        for (int j = 0; j < NM; j++) {
+            if constexpr (SWAPS) {
+                if (q & 1) {
+                    m[j] = snear[j];
+                    continue;
+                }
+                uint32_t both = sfar[j];
+                if (q == 0) {
+                    const auto v = __builtin_amdgcn_permlane32_swap(scur[j], scur[j], false, false);  // {lane groups 0, 1, 0, 1}, {2, 3, 2, 3}
+                    both = v[0];
+                    sfar[j] = v[1];
+                }
+                const auto v = __builtin_amdgcn_permlane16_swap(both, both, false, false);
+                m[j] = v[0];
+                snear[j] = v[1];
+            } else {
+                m[j] = (uint32_t)__builtin_amdgcn_ds_bpermute(take0 + 64 * q, (int)scur[j]);
+            }
+        }
     };
 
     float acc[NG][4];
@@ -726,7 +752,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     // regrouping them): its waits are counted against that order
     static_assert(PF % 4 == 0, "a request for scales serves four steps");
     Step<FMT> ring[PF];
-    uint32_t snext[PF / 4][NM], scur[NM];
+    uint32_t snext[PF / 4][NM];
 #pragma unroll
     for (int p = 0; p < PF; p++) {
         if (p % 4 == 0) {
@@ -858,7 +884,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
                 load_scales(snext[p / 4], sb + PF + p);
             }
             uint32_t sw[NM];
-            scales_of(scur, p % 4, sw);
+            scales_of(p % 4, sw);
             compute_step(ring[p], sw, sb + p);
             load_step(ring[p], min(sb + PF + p, slast));
             step_done();
@@ -872,7 +898,7 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
         }
         if (sb + p < s1) {
             uint32_t sw[NM];
-            scales_of(scur, p % 4, sw);
+            scales_of(p % 4, sw);
             compute_step(ring[p], sw, sb + p);
             step_done();
         }
