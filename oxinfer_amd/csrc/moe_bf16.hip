@@ -18,7 +18,7 @@
 // What bounds it: instruction issue (82 of 203 thousand cycles per SIMD were vector instructions and matrix instructions, half of a wave's time
 // waiting, before the steps named below) and the rounds of workgroups. 128 experts of 2048 / 768, 256 tokens, routing to combination, before
 // (chunks of 16 rows, an expert with more streamed and unpacked twice; words met through ds_bpermute; a launch that packed the gathered
-// rows) -> this: MLX 4-bit 123.5 -> 107.4 us, Q4_0 145 -> 110, MXFP4 175 -> 131, Q4_K 153 -> 131, Q8_0 206 -> 184 (the last four with the tracer).
+// rows) -> this: MLX 4-bit 123.5 -> 105 us, Q4_0 145 -> 104, MXFP4 175 -> 127, Q4_K 153 -> 125, Q8_0 206 -> 177 (the last four with the tracer).
 #include "act_body.hpp"
 #include "internal.hpp"
 #include "layout.hpp"
@@ -84,9 +84,10 @@ constexpr uint32_t PHASE = 16;            // steps x token tiles staged at a tim
 constexpr uint32_t UNIT_LDS = 4096 + 512;  // bytes of one: fragments and sums
 
 // One token tile (TT = 1: up to 16 rows) or two of a chunk; see moe_bf16_kernel.
-template <int RT, int FMT, int TT>
-__device__ __forceinline__ void moe_bf16_body(const WeightView& w, const uint8_t* expert, uint32_t first, uint32_t rows, uint32_t c, uint32_t gx, const MoeRows& in,
-                                              uint32_t kw, const MoeGlu& glu, float* __restrict__ out, float* lds) {
+template <int RT, int FMT, int TT, bool REP>
+__device__ __forceinline__ void moe_bf16_body(const WeightView& w, const uint8_t* expert, uint32_t first, uint32_t rows, uint32_t c, uint32_t gx0, const MoeRows& in,
+                                              uint32_t kw, uint32_t runs, const MoeGlu& glu, float* __restrict__ out, float* lds) {
+    const uint32_t nrep = REP ? runs : 1;
     constexpr bool STD = std_columns(FMT), Q8 = FMT == FMT_Q8_0, PER32 = FMT != FMT_Q4M;  // PER32: a scale per block of 32 instead of a scale and an offset per 64
     constexpr uint32_t P = PHASE / TT;  // steps of a phase
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -95,14 +96,17 @@ __device__ __forceinline__ void moe_bf16_body(const WeightView& w, const uint8_t
     const uint32_t kwsh = (uint32_t)__builtin_ctz(kw), ng = 8u >> kwsh, rg = wave >> kwsh, kwave = wave & (kw - 1);
     // (with the activation fused: the first half of the row groups takes gate tiles, the second the up tiles of the same rows)
     const uint32_t half = ng >> 1, gtiles = glu.inter / 16;
-    const uint32_t tile0 = !glu.inter ? (gx * ng + rg) * RT : (gx * half + (rg < half ? rg : rg - half)) * RT;
     const uint32_t tend = glu.inter ? gtiles : ntiles, tadd = glu.inter && rg >= half ? gtiles : 0u;
     const gbytes base = as_global(expert);
-    gbytes wp[RT];
+    gbytes wp[RT];  // (of the run of row tiles that requests go to)
     constexpr uint32_t REC = FMT == FMT_MXFP4 ? T4X_REC : T4M_REC;
     const size_t tile_bytes = Q8 ? (size_t)t8_steps(w.n_in) * T8_REC : FMT == FMT_Q4_K ? (size_t)tk4_sbs(w.n_in) * TK4_REC : (size_t)nsteps * REC;
+    auto point_at = [&](uint32_t gx) {
+        const uint32_t tile0 = !glu.inter ? (gx * ng + rg) * RT : (gx * half + (rg < half ? rg : rg - half)) * RT;
 #pragma unroll
-    for (int r = 0; r < RT; r++) wp[r] = base + (size_t)(min(tile0 + r, tend - 1) + tadd) * tile_bytes;
+        for (int r = 0; r < RT; r++) wp[r] = base + (size_t)(min(tile0 + r, tend - 1) + tadd) * tile_bytes;
+    };
+    point_at(gx0 * nrep);
     const uint32_t cnt = (nsteps - kwave + kw - 1) >> kwsh, ilast = cnt - 1;  // kw <= nsteps
 
     struct St {
@@ -194,7 +198,7 @@ __device__ __forceinline__ void moe_bf16_body(const WeightView& w, const uint8_t
         flive = fr < rows, slive = sr < rows;
         frow = (uint32_t)in.rowmap[first + (flive ? fr : 0)], srow = (uint32_t)in.rowmap[first + (slive ? sr : 0)];
     }
-    auto stage = [&](uint32_t ph) {
+    auto stage = [&](uint32_t ph, bool begin) {
         uint32_t tid = threadIdx.x;
         asm volatile("" : "+v"(tid));  // (or every piece's address would be made ahead of the phases and kept)
         const uint32_t s0 = ph * P, ns = min(P, nsteps - s0), total = ns * TT * 256, stotal = ns * TT * NS;
@@ -216,7 +220,7 @@ __device__ __forceinline__ void moe_bf16_body(const WeightView& w, const uint8_t
                                                 : in.sums + ((size_t)(2 * c + tile) * nsteps + step) * 64 + (PER32 ? 16 : 32) * b + (u & 15);
                     sm[k] = PER32 ? at[0] : at[0] + at[in.rowmap ? 1 : 16];
                 }
-                if (ph == 0) {
+                if (begin) {
                     load_scales(0);
 #pragma unroll
                     for (int p = 0; p < PF; p++) load(ring[p], (uint32_t)p);
@@ -240,10 +244,6 @@ __device__ __forceinline__ void moe_bf16_body(const WeightView& w, const uint8_t
     };
 
     f32x4 acc[RT][TT];
-#pragma unroll
-    for (int r = 0; r < RT; r++)
-#pragma unroll
-        for (int tt = 0; tt < TT; tt++) acc[r][tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     // The offsets' terms: one f32 matrix instruction (rows = tokens, K = 4) for the four blocks of a step (Q4_K) or the groups of two steps
     // (MLX 4-bit; `second`: there is a second one).
     auto offsets = [&](int r, float cc, uint32_t sl, bool second) {
@@ -343,24 +343,52 @@ __device__ __forceinline__ void moe_bf16_body(const WeightView& w, const uint8_t
             }
         }
     };
-    const uint32_t nph = (nsteps + P - 1) / P;
-    uint32_t i = 0;
-    for (uint32_t ph = 0; ph < nph; ph++) {
-        if (ph) __syncthreads();
-        stage(ph);
-        __syncthreads();
-        // (kw divides a phase's steps, and leaves each wave an even number of them)
-        const uint32_t iend = min((cnt + 1) & ~1u, (ph + 1) * (P >> kwsh));
-        for (; i < iend; i += PF) {
-            if (i < cnt) unfold(kwave + kw * i - ph * P, i + 1 < cnt);
+    const uint32_t nph = (nsteps + P - 1) / P, even = (cnt + 1) & ~1u;
+    for (uint32_t rep = 0; rep < nrep; rep++) {
+        const uint32_t gx = gx0 * nrep + rep;
 #pragma unroll
-            for (int p = 0; p < PF; p++) {
-                if (i + p < cnt) compute(ring[p], p, kwave + kw * (i + p) - ph * P);
-                load(ring[p], i + PF + p);
+        for (int r = 0; r < RT; r++)
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++) acc[r][tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        uint32_t i = 0;
+        for (uint32_t ph = 0; ph < nph; ph++) {
+            if (rep == 0 || nph > 1) {  // (rows staged whole serve all runs)
+                if (rep + ph) __syncthreads();
+                stage(ph, rep + ph == 0);
+                __syncthreads();
             }
-            load_scales(i + PF);
+            // (kw divides a phase's steps, and leaves each wave an even number of them)
+            const uint32_t iend = min(even, (ph + 1) * (P >> kwsh));
+            for (; i < iend; i += PF) {
+                if (i < cnt) unfold(kwave + kw * i - ph * P, i + 1 < cnt);
+                // (the run's last two steps make room for the next run's first)
+                const bool over = i + PF >= even && rep + 1 < nrep;
+                const uint32_t next = over ? 0 : i + PF;
+                if (over) point_at(gx + 1);
+#pragma unroll
+                for (int p = 0; p < PF; p++) {
+                    if (i + p < cnt) compute(ring[p], p, kwave + kw * (i + p) - ph * P);
+                    load(ring[p], next + p);
+                }
+                load_scales(next);
+            }
+        }
+        if (kw > 1 || glu.inter) break;  // (one run: the waves' sums meet in LDS)
+        // D[token 4 kq + e][row n]
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            const uint32_t row = ((gx * ng + rg) * RT + r) * 16 + n;
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const uint32_t tok = 16 * tt + 4 * kq + e;
+                    if (tok < rows && row < w.n_out) out[(size_t)(first + tok) * w.n_out + row] = acc[r][tt][e];
+                }
         }
     }
+    if (kw == 1 && !glu.inter) return;
+    const uint32_t gx = gx0;
     __syncthreads();  // the sums overwrite the fragments
     f32x4* red = reinterpret_cast<f32x4*>(lds);  // [wave][RT][TT][64]
 #pragma unroll
@@ -425,9 +453,10 @@ __device__ __forceinline__ void moe_bf16_body(const WeightView& w, const uint8_t
 // and meet in LDS in wave order. A workgroup's item (moe_bf16_item): a run of (8 / kw) RT row tiles of a chunk {expert, first row, rows <= 32}.
 // The chunk's rows (4 KiB per step and tile of 16) are staged into LDS, 64 KiB at a time: all eight waves multiply the same rows (each wave
 // asking memory for them costs more than the weights), and two workgroups share a CU. out [gathered row][n_out] f32.
-template <int RT, int FMT>
+// REP: an item is `nrep` such runs of row tiles, one after the other over the same staged rows (kw = 1, no activation).
+template <int RT, int FMT, bool REP>
 __global__ __launch_bounds__(512, 4) void moe_bf16_kernel(WeightView w, const uint8_t* const* __restrict__ bases, const int4* __restrict__ chunks,
-                                                          const int* __restrict__ nchunks, MoeRows in, uint32_t kw, uint32_t nx, MoeGlu glu,
+                                                          const int* __restrict__ nchunks, MoeRows in, uint32_t kw, uint32_t nrep, uint32_t nx, MoeGlu glu,
                                                           float* __restrict__ out) {
     extern __shared__ __align__(16) float lds[];
     uint32_t gx, c;
@@ -437,8 +466,8 @@ __global__ __launch_bounds__(512, 4) void moe_bf16_kernel(WeightView w, const ui
     ch.x = __builtin_amdgcn_readfirstlane(ch.x), ch.y = __builtin_amdgcn_readfirstlane(ch.y), ch.z = __builtin_amdgcn_readfirstlane(ch.z);
     const uint64_t eb = reinterpret_cast<uint64_t>(bases[ch.x]);
     const uint8_t* expert = reinterpret_cast<const uint8_t*>((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(eb >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)eb));
-    if (ch.z <= 16) moe_bf16_body<RT, FMT, 1>(w, expert, (uint32_t)ch.y, (uint32_t)ch.z, c, gx, in, kw, glu, out, lds);
-    else moe_bf16_body<RT, FMT, 2>(w, expert, (uint32_t)ch.y, (uint32_t)ch.z, c, gx, in, kw, glu, out, lds);
+    if (ch.z <= 16) moe_bf16_body<RT, FMT, 1, REP>(w, expert, (uint32_t)ch.y, (uint32_t)ch.z, c, gx, in, kw, nrep, glu, out, lds);
+    else moe_bf16_body<RT, FMT, 2, REP>(w, expert, (uint32_t)ch.y, (uint32_t)ch.z, c, gx, in, kw, nrep, glu, out, lds);
 }
 
 }  // namespace
@@ -473,29 +502,39 @@ hipError_t run_moe_bf16(const WeightView& w, const GroupView& g, uint32_t max_ch
     // K over two or four waves where one wave per row would leave fewer workgroups than places
     uint32_t rt = 2, kw = 1;
     while (kw < 4 && nsteps / (2 * kw) >= 4 && (uint64_t)nx_of(rt, kw) * max_chunks < 512) kw *= 2;
-    // Row tiles per wave: what takes fewer rounds of workgroups over the 512 places, a round as long as its waves' row tiles x steps and
-    // six more for its staging and its end. Two against three, 256 tokens, MLX 4-bit: 128 experts of 2048 / 768, gate / up 64.2 and 55.6 us
-    // (768 and 512 workgroups), down 36.1 and 39.2; 32 experts 38.9 and 48.5, 24.9 and 24.2; Q4_K, 64 experts of 2560 / 1024 95.6 and 119.7,
-    // 51.9 and 60.6. (Four row tiles spill in the form of two token tiles: 76. Q8_0 keeps to two, its steps being two records a tile.)
-    if (FMT != FMT_Q8_0 && kw == 1) {
-        auto rounds = [&](uint32_t r) {
-            const uint64_t items = (uint64_t)nx_of(r, 1) * chunks;
-            return ((items > 16 ? items - 16 : 1) + 511) / 512 * (r * nsteps + 6);
-        };
-        if (rounds(3) < rounds(2)) rt = 3;
+    // Row tiles per wave, and runs of them that a workgroup takes one after the other with one staging (the down projection's rows fit a
+    // phase): what takes fewer rounds of workgroups over the 512 places, a round as long as its waves' row tiles x steps and six more for its staging
+    // and its end. At 256 tokens, MLX 4-bit: gate / up launch, two tiles and three, 128 experts of 2048 / 768 64.2 and 55.6 us (768 and 512
+    // workgroups), 32 experts 38.9 and 48.5; down launch, one run of two tiles, of three, two, three and four of two, 128 experts 34.5, 36.3, 33.6, 38.0
+    // and 34.4, 32 experts (two tiles, 320 workgroups) 23.4, 22.4, 24.9, 23.5 and 27.2. (Four row tiles spill in the form of two token tiles: 76.)
+    uint32_t nrep = 1;
+    if (kw == 1) {
+        uint64_t least = ~0ull;
+        for (uint32_t r = 2; r <= (FMT == FMT_Q8_0 ? 2u : 3u); r++)  // (Q8_0, a step being two records per row tile, keeps to two and one; three and several runs would spill)
+            for (uint32_t n = 1; n <= (r == 2 && FMT != FMT_Q8_0 && !glu.inter && 2 * nsteps <= PHASE ? 4u : 1u); n++) {
+                const uint64_t items = (uint64_t)((nx_of(r, 1) + n - 1) / n) * chunks;
+                const uint64_t cost = ((items > 16 ? items - 16 : 1) + 511) / 512 * (n * r * nsteps + 6);
+                if (cost < least) {
+                    least = cost;
+                    rt = r;
+                    nrep = n;
+                }
+            }
     }
-    const uint32_t nx = nx_of(rt, kw);
+    const uint32_t nx = (nx_of(rt, kw) + nrep - 1) / nrep;
     const size_t lds = PHASE * UNIT_LDS;
     const dim3 grid((nx * max_chunks + 7) / 8 * 8);  // every XCD's share of the items (moe_bf16_item), whatever the chunk count turns out to be
     auto go = [&](auto kern) -> hipError_t {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
-        kern<<<grid, 512, lds, s>>>(w, g.bases, g.chunks, g.nchunks, in, kw, nx, glu, out);
+        kern<<<grid, 512, lds, s>>>(w, g.bases, g.chunks, g.nchunks, in, kw, nrep, nx, glu, out);
         return hipGetLastError();
     };
-    if (rt == 2) return go(moe_bf16_kernel<2, FMT>);
-    if constexpr (FMT != FMT_Q8_0) return go(moe_bf16_kernel<3, FMT>);
-    return hipErrorInvalidValue;
+    if constexpr (FMT != FMT_Q8_0) {
+        if (nrep > 1) return go(moe_bf16_kernel<2, FMT, true>);
+        if (rt == 3) return go(moe_bf16_kernel<3, FMT, false>);
+    }
+    return go(moe_bf16_kernel<2, FMT, false>);
 }
 hipError_t launch_moe_bf16(const WeightView& w, const GroupView& g, uint32_t max_chunks, const MoeRows& in, const MoeGlu& glu, uint32_t chunks, float* out, hipStream_t s) {
     if (!moe_bf16_ok(w) || (glu.inter && (w.n_out != 2 * glu.inter || glu.inter % 128))) return hipErrorInvalidValue;

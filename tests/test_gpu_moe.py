@@ -239,8 +239,9 @@ def test_moe_prefill_rows_do_not_depend_on_the_batch(be, oxref, mlx_experts):
 
 
 @pytest.mark.parametrize("fmt", ["mlx", "Q4_K", "Q8_0", "Q4_0", "MXFP4", "mlx, Q8_0 down"])
-@pytest.mark.parametrize("h,inter", [(2304, 384), (256, 256), (4096, 256)])  # staged in three phases and one, an odd number of steps; one; four and one
-def test_moe_prefill_chunks(be, oxref, fmt, h, inter):
+# staged in three phases and one, an odd number of steps; one; four and one; enough workgroups for several runs of row tiles per workgroup
+@pytest.mark.parametrize("h,inter,copies", [(2304, 384, 1), (256, 256, 1), (4096, 256, 1), (2048, 384, 14)])
+def test_moe_prefill_chunks(be, oxref, fmt, h, inter, copies):
     """The bf16 form's chunks at the edges of its token tiles and of a chunk (experts of 33, 32, 17, 16 and 1 rows): within 6e-3 of the
     reference's grouped f32 path on activations that are bf16 values already (as in test_moe_gguf_experts), and bit for bit the same
     where the tokens, and with them the rows' places, come in another order."""
@@ -266,14 +267,15 @@ def test_moe_prefill_chunks(be, oxref, fmt, h, inter):
 
     first, second = ("mlx", "Q8_0") if "down" in fmt else (fmt, fmt)
     gu, dn = experts(first, 2 * inter, h, 2500), experts(second, h, inter, 2600)
-    dev = be.upload_moe([e[2] for e in gu], [e[2] for e in dn], h, inter)
+    dev = be.upload_moe([e[2] for e in gu] * copies, [e[2] for e in dn] * copies, h, inter)
     assert dev is not None, be.last_error()
-    idx = np.repeat(np.arange(ne, dtype=np.uint32), rows)[:, None]
+    t *= copies
+    idx = np.repeat(np.arange(ne * copies, dtype=np.uint32), rows * copies)[:, None]
     w = np.ones((t, 1), np.float32)
     x = synth.bf16_round(synth.activations(t, h, 2700))
     ref = np.zeros((t, h))
     for e in range(ne):
-        at = idx[:, 0] == e
+        at = idx[:, 0] % ne == e
         p = x[at].astype(np.float64) @ gu[e][1].astype(np.float64).T
         g, u = p[:, :inter], p[:, inter:]
         ref[at] = (g / (1.0 + np.exp(-g)) * u) @ dn[e][1].astype(np.float64).T
