@@ -18,7 +18,7 @@
 // What bounds it: instruction issue (82 of 203 thousand cycles per SIMD were vector instructions and matrix instructions, half of a wave's time
 // waiting, before the steps named below) and the rounds of workgroups. 128 experts of 2048 / 768, 256 tokens, routing to combination, before
 // (chunks of 16 rows, an expert with more streamed and unpacked twice; words met through ds_bpermute; a launch that packed the gathered
-// rows) -> this: MLX 4-bit 123.5 -> 105 us, Q4_0 145 -> 104, MXFP4 175 -> 127, Q4_K 153 -> 125, Q8_0 206 -> 177 (the last four with the tracer).
+// rows) -> this: MLX 4-bit 123.5 -> 103 us, Q4_0 145 -> 104, MXFP4 175 -> 127, Q4_K 153 -> 125, Q8_0 206 -> 177 (the last four with the tracer).
 #include "act_body.hpp"
 #include "internal.hpp"
 #include "layout.hpp"
