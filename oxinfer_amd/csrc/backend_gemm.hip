@@ -39,13 +39,13 @@ int gemm_bf16_run(DevBuf& ws, const oxhip_weight* w, const void* x, bool x_bf16,
     }
     const size_t mtiles = (t + 15) / 16, kblocks = 4 * (size_t)((w->v.n_in + 127) / 128);
     const size_t pack_bytes = align_up(mtiles * kblocks * 64 * 16, 256);
-    const bool few = gemm_short_ok(t);  // up to 64 tokens
-    const uint32_t slices = few ? gemm_short_slices(w->v, t) : gemm_k_slices(w->v, mtiles);
+    const ShortPlan few = t <= 64 ? short_plan(w->v.fmt, w->v.n_out, w->v.n_in, t) : ShortPlan{0, 1};
+    const uint32_t slices = few.rt ? few.slices : gemm_k_slices(w->v, mtiles);
     const size_t bytes = pack_bytes + (slices > 1 ? (size_t)slices * t * w->v.n_out * 4 : 0);
     if (!grow_ws(ws, bytes, s)) return 0;
     HIP_TRY(launch_pack_a(x, x_bf16, gemm_bf16_pack_mode(w->v), t, w->v.n_in, mtiles, kblocks, ws.p, s), "gemm pack launch");
     float* partial = reinterpret_cast<float*>(static_cast<uint8_t*>(ws.p) + pack_bytes);
-    HIP_TRY(few ? launch_gemm_short(w->v, ws.p, t, y, y_bf16, partial, s) : launch_gemm_bf16(w->v, ws.p, t, mtiles, y, y_bf16, partial, s), "gemm launch");
+    HIP_TRY(few.rt ? launch_gemm_short(w->v, ws.p, t, few, y, y_bf16, partial, s) : launch_gemm_bf16(w->v, ws.p, t, mtiles, y, y_bf16, partial, s), "gemm launch");
     return 1;
 }
 

@@ -13,9 +13,9 @@
 // dequantize at the same time: the waves 0-3 do so in a step's first block, the waves 4-7 in its second. Sharing the
 // token dimension keeps the activation requests at one per fragment and workgroup (sharing the rows instead would
 // request every fragment twice and run into the vector memory path's 64 bytes per cycle and CU). A
-// launch of 65 to 128 tokens runs one tile per wave (34 -> 27 us on the Llama-8B MLP shapes against two); up to 64 tokens are
-// gemm_short.hip's.
-//   B (weights): each K-step of 128 the waves dequantize the step's 8 row tiles (one each) from the packed
+// launch of 65 to 128 tokens runs one tile per wave (34 -> 27 us on the Llama-8B MLP shapes against two), one of at most 64 four waves
+// of one tile (64 tokens x 128 rows per workgroup) where gemm_short.hip's kernel would take longer (short_plan).
+//   B (weights): each K-step of 128 the waves dequantize the step's 8 row tiles (one each; two each with 4 waves) from the packed
 //     records into bf16 MFMA fragments in LDS (double-buffered, one barrier per step); every wave then reads all
 //     8 x 4 fragments with ds_read_b128. A weight is dequantized once per workgroup: (code - 8) * d + offset in
 //     f32 as one fma(code, d, offset - 8 d), rounded to bf16. The GGUF formats likewise, from their own records:
@@ -111,8 +111,7 @@ hipError_t launch_pack_a(const void* x, bool src_bf16, int mode, size_t t, size_
 
 namespace {
 
-constexpr int WG_NT = 8;   // row tiles per workgroup (128 rows), or 7 where that fills more CUs (gemm_plan)
-constexpr int WAVES = 8;
+constexpr int WG_NT = GEMM_WG_NT;
 constexpr int AR = 4;      // blocks of A fragments held ahead (a whole K-step: two starve the FP8 shapes, whose activations do not stay in L2)
 
 }  // namespace
@@ -127,12 +126,13 @@ constexpr int AR = 4;      // blocks of A fragments held ahead (a whole K-step: 
 // ALONE: see run_gemm_bf16_nv. (Eight waves of one token tile: two workgroups share a CU if they take at most 128 registers. Q4_K took 130:
 // bounded it spills 12 bytes, 9472 columns x 5000 rows 42.7 -> 31.9 us at 128 tokens with the slices that allows. The 8-bit formats
 // would spill 24 to 44 bytes, 33.6 -> 43.9 us on 14336 -> 4096: they keep a CU to a workgroup.)
-template <int FMT, bool OUT_BF16, int NV, int NT, bool ALONE>
-__global__ __launch_bounds__(64 * WAVES, NV == 1 && !ALONE ? 4 : 2) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
+template <int FMT, bool OUT_BF16, int NV, int WAVES, int NT, bool ALONE>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 : 2) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
                                                         void* __restrict__ yv) {
     extern __shared__ uint4 bfrag[];  // [2][4 blocks][NT row tiles][64 lanes]
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t n = lane & 15;
+    constexpr int DT = (NT + WAVES - 1) / WAVES;  // row tiles a wave dequantizes
     const uint32_t all_steps = (w.n_in + 127) / 128, kblocks = 4 * all_steps;  // == t4m_steps(n_in)
     const uint32_t per_z = (all_steps + gridDim.z - 1) / gridDim.z;
     const uint32_t step0 = blockIdx.z * per_z;              // this slice's K-steps: step0 .. step0 + nsteps
@@ -142,10 +142,15 @@ __global__ __launch_bounds__(64 * WAVES, NV == 1 && !ALONE ? 4 : 2) void gemm_bf
     // the wave's token tiles: mt0, mt0 + WAVES, ... (NV of them)
     const uint32_t mt0 = blockIdx.y * (WAVES * NV) + wave;
 
-    // the row tile this wave dequantizes (with NT = 7 the eighth wave has none)
-    const bool has_tile = NT == WAVES || wave < (uint32_t)NT;
-    const uint32_t tile = min(nt0 + wave, ntiles - 1);
-    const uint8_t* wbase = tile_records<FMT>(w, tile, lane);
+    // the row tiles this wave dequantizes (with NT = 7 the eighth wave has none)
+    const bool has_tile = NT == DT * WAVES || wave < (uint32_t)NT;
+    uint32_t tile[DT];
+    const uint8_t* wbase[DT];
+#pragma unroll
+    for (int i = 0; i < DT; i++) {
+        tile[i] = min(nt0 + DT * wave + i, ntiles - 1);
+        wbase[i] = tile_records<FMT>(w, tile[i], lane);
+    }
     // A fragments of the wave's token tiles (tiles past the end repeat the last one; their rows are not stored)
     const uint4* abase[NV];
 #pragma unroll
@@ -158,12 +163,12 @@ __global__ __launch_bounds__(64 * WAVES, NV == 1 && !ALONE ? 4 : 2) void gemm_bf
         for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     // `s`: a step of this slice
-    auto load_raw = [&](RawTile& r, uint32_t s) {
-        if (has_tile) load_tile<FMT>(r, w, wbase, tile, step0 + s, lane);
+    auto load_raw = [&](RawTile& r, int i, uint32_t s) {
+        if (has_tile) load_tile<FMT>(r, w, wbase[i], tile[i], step0 + s, lane);
     };
-    auto dequant = [&](const RawTile& r, uint32_t buf, uint32_t s) {  // the wave's row tile, 4 blocks
+    auto dequant = [&](const RawTile& r, int i, uint32_t buf, uint32_t s) {  // the wave's row tile i, 4 blocks
         if (!has_tile) return;
-        uint4* dst = bfrag + ((size_t)(buf * 4) * NT + wave) * 64 + lane;  // block b: + b * NT * 64
+        uint4* dst = bfrag + ((size_t)(buf * 4) * NT + DT * wave + i) * 64 + lane;  // block b: + b * NT * 64
 #pragma unroll
         for (int b = 0; b < 4; b++) dst[b * NT * 64] = tile_block<FMT>(r, w, b, step0 + s, lane);
     };
@@ -187,21 +192,24 @@ __global__ __launch_bounds__(64 * WAVES, NV == 1 && !ALONE ? 4 : 2) void gemm_bf
     // memory a whole K-step (four blocks, ~2000 MFMA cycles) ahead; the packed records of the next step two blocks
     // before they are dequantized into the other LDS buffer. Each fragment has one home, refilled in place right after
     // its last use.
-    RawTile raw;
-    load_raw(raw, 0);
+    RawTile raw[DT];
+#pragma unroll
+    for (int i = 0; i < DT; i++) load_raw(raw[i], i, 0);
     uint4 a_cur[AR][NV], b_cur[NT];
     const uint32_t last = nsteps - 1, last_blk = 4 * nsteps - 1;
 #pragma unroll
     for (int b = 0; b < AR; b++) read_a(a_cur[b], min((uint32_t)b, last_blk));
-    dequant(raw, 0, 0);
-    load_raw(raw, min(1u, last));
+#pragma unroll
+    for (int i = 0; i < DT; i++) dequant(raw[i], i, 0, 0);
+#pragma unroll
+    for (int i = 0; i < DT; i++) load_raw(raw[i], i, min(1u, last));
     lds_barrier();
     read_b(b_cur, 0, 0);
     // One K-step; every step does the same work, so that the loop is one body whose accumulators stay in place: the
-    // records of the next step are dequantized into the other LDS buffer during blocks 0 and 1 (block 0
+    // records of the next step are dequantized into the other LDS buffer during blocks 0 and 1 (with eight waves block 0
     // by the waves 0-3, block 1 by the waves 4-7, which share their SIMDs with them), block 3 refills from
-    // that buffer after the barrier, and the step after next is requested during block 2. Past the end the indices
-    // repeat the last step: a little work that nobody reads, instead of separate loop tails.
+    // that buffer after the barrier, and a tile of the step after next is requested as soon as its registers are free. Past the end
+    // the indices repeat the last step: a little work that nobody reads, instead of separate loop tails.
     for (uint32_t s = 0; s < nsteps; s++) {
         const uint32_t buf = s & 1;
 #pragma unroll
@@ -217,12 +225,14 @@ __global__ __launch_bounds__(64 * WAVES, NV == 1 && !ALONE ? 4 : 2) void gemm_bf
                 else b_cur[j] = bfrag[(((buf ^ 1) * 4) * NT + j) * 64 + lane];
             }
             read_a(a_cur[b % AR], min(4 * s + b + AR, last_blk));
-            if (b == (int)(wave >> 2)) {
-                dequant(raw, buf ^ 1, min(s + 1, last));
-                // (Q4_K: the compiler would put the request among the conversions, 14336 rows x 2048 tokens 234 us, 226 this way; the
-                // other formats are no faster)
-                if constexpr (FMT == FMT_Q4_K) __builtin_amdgcn_sched_barrier(0);
-                load_raw(raw, min(s + 2, last));
+            if (DT == 2 ? b < 2 : b == (int)(wave >> 2)) {
+                const int i = DT == 2 ? b & 1 : 0;
+                dequant(raw[i], i, buf ^ 1, min(s + 1, last));
+                // (Left to itself the compiler puts the request among the conversions. Q4_K 14336 rows x 2048 tokens 234 us, 226 this way; four
+                // waves, medians of 24 calls of up to 64 tokens: Q5_K 0.89 of the time, MXFP4 0.90, Q4_0 0.95, MLX 4-bit, Q8 and Q6_K 0.96
+                // to 0.98, Q4_K, FP8 and NVFP4 the same; FP8 at 200 tokens 60.0 -> 58.4 us on 9472 x 8960. The others are no faster.)
+                if constexpr (FMT == FMT_Q4_K || WAVES == 4 || (FMT == FMT_FP8 && NV == 2)) __builtin_amdgcn_sched_barrier(0);
+                load_raw(raw[i], i, min(s + 2, last));
             }
         }
     }
@@ -312,62 +322,12 @@ static void run_gemm_reduce(const float* partial, size_t n, uint32_t slices, voi
     else out_bf16 ? go(gemm_reduce_kernel<true, 4, false>) : go(gemm_reduce_kernel<false, 4, false>);
 }
 
-// Token tiles per wave: one when the launch has at most eight tiles (128 tokens), else two.
-static int gemm_nv(size_t mtiles) { return mtiles <= 8 ? 1 : 2; }
-
-// Row tiles per workgroup (8, or 7 with two token tiles per wave) and K slices of a launch: the pair that costs least, in units
-// of one K-step of an eight-tile workgroup (0.9 us with one token tile per wave, 1.2 to 1.5 us with two):
-//   rounds of workgroups over the 256 CUs x K-steps per slice. Two workgroups with one token tile per wave share a CU and
-//     take 1.55 steps' time for a step of each; a workgroup with two tiles per wave, or with eight waves of an 8-bit format, has
-//     its CU to itself. A slice of four steps costs 4.65 (the pipeline fills as often): 5120 -> 2816, MLX 4-bit, 100 tokens 20.2 us
-//     in 8 slices, 21.2 in 10.
-//   1 for every million partial sums written and read back, 1.9 for those past six million, and 2 for the launch that adds them
-//     (14336 -> 4096, MLX 4-bit, 420 tokens, 4 slices -> 8: 6.9 million more, as many steps, 63.6 -> 69.7 us).
-// Any number of slices counts, not only powers of two. With two tiles: 14336 -> 4096, MLX 4-bit, 1100 tokens (160 workgroups) 167.6 us
-// whole, 153.0 in 3 slices, 190.8 in 2; FP8 7168 x 18432 at 1100 tokens 397 us whole, 331 in 3. Four steps per slice at least
-// (7168 -> 1536, Q8_0, 200 tokens: 30.7 us at 14 steps, 24.4 at 7, 23.5 at 5).
-// Seven row tiles: 14336 rows x 512 tokens are one round of 256 workgroups of 112 rows instead of 224 of 128, 63 -> 60 us: a step of
-// theirs costs 0.94 of one of eight, not 7/8 (counted as 7/8, 8192 rows x 512 tokens of 4096 columns went from 256 workgroups in two
-// slices to 148 of seven tiles whole, Q4_K 46.5 -> 53.2 us; 7895 x 5888 at 224 tokens 37.1 -> 39.6).
-struct GemmPlan {
-    uint32_t nt, slices;
-};
-static GemmPlan gemm_plan(const WeightView& w, size_t mtiles) {
-    const bool one = gemm_nv(mtiles) == 1;
-    const uint32_t per_wg = WAVES * gemm_nv(mtiles), cols = (uint32_t)((mtiles + per_wg - 1) / per_wg);
-    const uint32_t steps = (w.n_in + 127) / 128;
-    const bool alone = !one || q8_format(w.fmt);
-    // (One token tile per wave: eight slices at most, 14336 -> 4096, MLX 4-bit at 70 tokens 29.1 us in 8 and 30.2 in 16.)
-    const uint32_t most = one ? 8 : 16;
-    const double millions = (double)mtiles * 16 * w.n_out * 1e-6;
-    auto sums = [](double m) { return m < 6 ? m : 6 + 1.9 * (m - 6); };
-    GemmPlan best{WG_NT, 1};
-    double least = 0;
-    for (uint32_t nt : {(uint32_t)WG_NT, 7u}) {
-        if (one && nt == 7) break;
-        const uint64_t wgs = (uint64_t)((row_tiles(w.n_out) + nt - 1) / nt) * cols;
-        for (uint32_t z = 1; z <= most; z++) {
-            const uint32_t per = (steps + z - 1) / z;
-            if (z > 1 && steps / z < 4) break;
-            // every slice must own a step: the kernel gives slice i the steps from i * per (33 steps in 8 slices of 5 would
-            // start the last one past the end)
-            if ((z - 1) * per >= steps) continue;
-            const uint64_t rounds = (wgs * z + 255) / 256;
-            const double held = alone ? (double)rounds : (double)(rounds / 2) * 1.55 + (double)(rounds % 2);
-            const double cost = held * (per < 5 && z > 1 ? per + 0.65 : per) * (nt == 7 ? 0.94 : 1.0) + (z > 1 ? sums(z * millions) + 2 : 0);
-            if ((nt == WG_NT && z == 1) || cost < least) {
-                least = cost;
-                best = GemmPlan{nt, z};
-            }
-        }
-    }
-    return best;
-}
+static GemmPlan gemm_plan(const WeightView& w, size_t mtiles) { return gemm_plan(w.fmt, w.n_out, w.n_in, mtiles); }
 
 uint32_t gemm_k_slices(const WeightView& w, size_t mtiles) { return gemm_plan(w, mtiles).slices; }
 
 namespace {
-template <int FMT, int NV, int NT>
+template <int FMT, int NV, int WAVES, int NT>
 hipError_t run_gemm_bf16_nv(const WeightView& w, const void* apk, size_t t, size_t mtiles, void* y, bool out_bf16, float* partial,
                          hipStream_t s) {
     const uint32_t slices = gemm_k_slices(w, mtiles);
@@ -383,14 +343,14 @@ hipError_t run_gemm_bf16_nv(const WeightView& w, const void* apk, size_t t, size
     // Eight waves of one token tile that leave a second workgroup no room on their CU: the 8-bit formats always; Q4_K in launches of
     // at most a workgroup per CU, which need none, while the spill of the bounded kernel costs a start half a microsecond later
     // (2048 columns x 7168 rows at 80 tokens, 224 workgroups: 19.0 us bounded, 18.4 this way).
-    constexpr bool ALWAYS = NV == 1 && q8_format(FMT), CHOICE = NV == 1 && FMT == FMT_Q4_K;
+    constexpr bool ALWAYS = NV == 1 && WAVES == 8 && q8_format(FMT), CHOICE = NV == 1 && WAVES == 8 && FMT == FMT_Q4_K;
     span_start(s);
     if (CHOICE && (uint64_t)grid.x * grid.y * grid.z <= 256) {
-        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, NT, CHOICE || ALWAYS>);
-        else go(gemm_bf16_kernel<FMT, false, NV, NT, CHOICE || ALWAYS>);
+        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, WAVES, NT, CHOICE || ALWAYS>);
+        else go(gemm_bf16_kernel<FMT, false, NV, WAVES, NT, CHOICE || ALWAYS>);
     } else {
-        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, NT, ALWAYS>);
-        else go(gemm_bf16_kernel<FMT, false, NV, NT, ALWAYS>);
+        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, WAVES, NT, ALWAYS>);
+        else go(gemm_bf16_kernel<FMT, false, NV, WAVES, NT, ALWAYS>);
     }
     if (e != hipSuccess) return e;
     e = hipGetLastError();
@@ -402,9 +362,10 @@ hipError_t run_gemm_bf16_nv(const WeightView& w, const void* apk, size_t t, size
 template <int FMT>
 hipError_t run_gemm_bf16(const WeightView& w, const void* apk, size_t t, size_t mtiles, void* y, bool out_bf16, float* partial,
                          hipStream_t s) {
-    if (gemm_nv(mtiles) == 1) return run_gemm_bf16_nv<FMT, 1, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
-    if (gemm_plan(w, mtiles).nt == 7) return run_gemm_bf16_nv<FMT, 2, 7>(w, apk, t, mtiles, y, out_bf16, partial, s);
-    return run_gemm_bf16_nv<FMT, 2, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
+    if (gemm_waves(mtiles) == 4) return run_gemm_bf16_nv<FMT, 1, 4, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
+    if (gemm_nv(mtiles) == 1) return run_gemm_bf16_nv<FMT, 1, 8, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
+    if (gemm_plan(w, mtiles).nt == 7) return run_gemm_bf16_nv<FMT, 2, 8, 7>(w, apk, t, mtiles, y, out_bf16, partial, s);
+    return run_gemm_bf16_nv<FMT, 2, 8, WG_NT>(w, apk, t, mtiles, y, out_bf16, partial, s);
 }
 }  // namespace
 

@@ -6,17 +6,17 @@
 // takes the K-steps v, v + 8, ... (of its slice), so that a workgroup reads one contiguous window of its tiles' records, turns each
 // record into operands in registers and multiplies it with the fragments of all its NTT token tiles: 4 NTT RT matrix instructions a step,
 // no barrier, no weight through LDS. The eight sums meet in LDS once, in wave order. (Sharing the operands of 128 rows through LDS, as
-// gemm.hip does for more tokens, put two barriers' waits and a trip through LDS into each of the six to sixteen steps that a workgroup
-// has here, and needed K slices, and a launch to add them, for almost every matrix.)
-// The fragments are requested by every wave that needs them, RT records to a fragment, so RT is as large as keeps the CUs busy: see
-// short_plan. A step's registers are refilled where they are used up, the fragments a step ahead, the records two (three: no gain, the
-// kernels of four row tiles spill; read-once requests for the records: 10 to 30 % slower, the other side of a line of scales is lost).
+// gemm.hip does for more tokens, puts two barriers' waits and a trip through LDS into each of the six to sixteen steps that a workgroup
+// has here, and needs K slices, and a launch to add them, for almost every matrix.)
+// The fragments are requested by every wave that needs them, RT records to a fragment: row tiles, K slices and the sizes where gemm.hip's
+// way is the faster one all the same are short_plan's (gemm_plan.hpp). A step's registers are refilled where they are used up, the fragments
+// a step ahead, the records two (three: no gain, the kernels of four row tiles spill; read-once requests for the records: 10 to 30 %
+// slower, the other side of a line of scales is lost).
 //
-// Whole calls on the device, packing included, before (gemm.hip's kernel with four waves of one token tile) -> this, at 24 / 43 / 64 tokens:
-// MLX 4-bit 4096 x 4096 14.2 / 16.6 / 17.6 -> 9.2 / 11.3 / 12.4 us, 14336 x 4096 24.4 / 25.2 / 25.9 -> 17.0 / 19.0 / 20.3, 4096 x 14336
-// 24.0 / 24.6 / 25.1 -> 19.4 / 21.9 / 23.6; Q4_K 15.6 / 17.4 / 19.2 -> 10.3 / 11.7 / 13.2, 27.5 / 27.6 / 29.0 -> 18.9 / 20.5 / 21.9,
-// 26.7 / 27.2 / 28.1 -> 21.9 / 23.7 / 25.4; Q6_K 5001 x 4352 at 43 tokens 19.6 -> 14.0; NVFP4 4096 x 4096 23.6 / 25.1 / 26.8 -> 12.5 / 13.2 / 13.9.
-#include <algorithm>
+// Whole calls on the device, packing included, weights in HBM (in brackets: in the Infinity Cache), gemm.hip's four waves -> this, at 24 / 43 /
+// 64 tokens: MLX 4-bit 4096 x 4096 15.3 / 16.6 / 18.2 -> 11.4 / 13.8 / 15.5 us (13.4 / 15.1 / 16.7 -> 8.8 / 10.3 / 12.0), 14336 x 4096 25.8 / 27.2 / 28.6
+// -> 21.3 / 23.5 / 25.5 (22.5 / 23.9 / 25.3 -> 15.5 / 17.4 / 19.3); Q4_K 16.9 / 18.2 / 20.2 -> 12.0 / 14.1 / 15.8, 29.6 / 31.0 / 32.0 -> 22.9 / 25.0 / 27.1;
+// Q6_K 5001 x 4352 at 43 tokens 21.8 -> 18.3 (18.9 -> 13.2); NVFP4 4096 x 4096 24.2 / 25.5 / 26.9 -> 13.7 / 14.7 / 16.0.
 #include <type_traits>
 
 #include "gemm_tile.hpp"
@@ -112,49 +112,13 @@ __global__ __launch_bounds__(64 * KW, 2) void gemm_short_kernel(WeightView w, co
     }
 }
 
-// Row tiles per workgroup and K slices, by measuring 30 shapes from 1024 x 2048 to 14336 x 14336 in up to five formats (device time of
-// whole calls, Q4_K at 24 and 64 tokens where nothing else is said): few enough row tiles that the 256 CUs have a workgroup each, and
-// no fewer, since the workgroups of a launch request the whole activations once each.
-//   4096 x 4096, MLX 4-bit: one row tile 9.8 and 13.1 us, two (128 workgroups) 11.4 and 14.0, four 14.7 and 19.0.
-//   5001 x 4352, MLX 4-bit: two (157 workgroups) 12.0 and 14.9, one (313: some CUs have two) 13.9 and 19.9, four 15.5 and 19.0.
-//   12000 x 4096: three (250 workgroups) 16.4 and 19.1, two (375) 19.1 and 25.4, four (188) 17.9 and 21.5; 8320 rows 15.4 and 18.9, 17.7
-//   and 24.7, 17.4 and 21.3. 14336 x 4096, MLX 4-bit: four (224 workgroups) 17.2 and 20.2, two (448) 17.0 and 23.4, one 21.7 and 30.6.
-// K slices cost a launch that adds them. They pay where rows are long and the row tiles do not fill the CUs (1024 x 14336: whole 19.4 and
-// 28.4, in four slices 12.9 and 17.4; x 8192 13.6 and 18.4, 10.2 and 13.0; x 4096 9.7 and 12.6, 9.1 and 10.8, which the host's third
-// launch takes back), or where they let a workgroup have more row tiles, which halves the fragments' requests:
-//   4096 x 14336, MLX 4-bit: one tile, whole 19.3 and 29.2 us (24.3 at 48 tokens), two tiles in two slices 19.1 and 24.9 (22.4).
-//   4096 x 11008 at 48 / 64 tokens 19.4 / 24.5, 19.4 / 22.6; 3000 x 8192 at 40 / 64 16.7 / 19.4, 16.8 / 18.5.
-//   5120 x 12288: two tiles, whole 27.1 and 31.0, four in three slices (240 workgroups) 21.2 and 25.9; FP8 at 64 28.0 and 25.6.
-//   7168 x 18432 at 64: FP8 54.1 and (four, two slices) 47.4, Q8_0 56.9 and 52.0, Q6_K 49.3 and 47.6, MLX 4-bit 38.3 and 37.7.
-//   7168 x 14336 is better whole (Q5_K 32.5 and 36.6; 30.9 and 37.6), as are 8192 x 8192 and 14336 rows of 8192 and 14336 columns.
-// (Q8 at four token tiles keeps to three row tiles: four would spill.)
-struct ShortPlan {
-    uint32_t rt, slices;
-};
-ShortPlan short_plan(const WeightView& w, size_t t) {
-    const uint32_t tiles = row_tiles(w.n_out), steps = (w.n_in + 127) / 128;
-    if (tiles <= 128) return {1, steps >= 64 ? std::min(4u, 256 / tiles) : 1};
-    if (tiles <= 256) return steps * t >= 4000 ? ShortPlan{2, 2} : ShortPlan{1, 1};
-    const uint32_t most = w.fmt == FMT_Q8F && t > 48 ? 3 : 4;
-    if (tiles <= 512) return steps >= (tiles <= 340 ? 96 : 128) ? ShortPlan{most, tiles <= 340 ? 3u : 2u} : ShortPlan{2, 1};
-    return {tiles <= 768 ? 3u : most, 1};
-}
-
-}  // namespace
-
-bool gemm_short_ok(size_t t) { return t <= 64; }
-uint32_t gemm_short_slices(const WeightView& w, size_t t) { return short_plan(w, t).slices; }
-
-namespace {
-
 template <int FMT>
-hipError_t run_short(const WeightView& w, const void* apk, size_t t, void* y, bool out_bf16, float* partial, hipStream_t s) {
-    const ShortPlan p = short_plan(w, t);
+hipError_t run_short(const WeightView& w, const void* apk, size_t t, const ShortPlan& p, void* y, bool out_bf16, float* partial, hipStream_t s) {
     const uint32_t mtiles = (uint32_t)((t + 15) / 16);
     hipError_t e = hipSuccess;
     auto go = [&](auto ntt, auto rt) {
         constexpr int NTT = decltype(ntt)::value, RT = decltype(rt)::value;
-        if constexpr (!(FMT == FMT_Q8F && NTT * RT == 16)) {
+        if constexpr (short_form(FMT, NTT, RT)) {
             auto kern = gemm_short_kernel<FMT, NTT, RT>;
             constexpr size_t lds = (size_t)KW * RT * NTT * 1024;
             e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -181,19 +145,19 @@ hipError_t run_short(const WeightView& w, const void* apk, size_t t, void* y, bo
 
 }  // namespace
 
-// `apk`: the fragments that launch_pack_a makes in gemm_bf16_pack_mode; `partial`: gemm_short_slices() * t * n_out floats, if more than one.
-hipError_t launch_gemm_short(const WeightView& w, const void* apk, size_t t, void* y, bool out_bf16, float* partial, hipStream_t s) {
+// `apk`: the fragments that launch_pack_a makes in gemm_bf16_pack_mode; `partial`: p.slices * t * n_out floats, if more than one.
+hipError_t launch_gemm_short(const WeightView& w, const void* apk, size_t t, const ShortPlan& p, void* y, bool out_bf16, float* partial, hipStream_t s) {
     switch (w.fmt) {
-        case FMT_Q4M: return run_short<FMT_Q4M>(w, apk, t, y, out_bf16, partial, s);
-        case FMT_Q40: return run_short<FMT_Q40>(w, apk, t, y, out_bf16, partial, s);
-        case FMT_MXFP4: return run_short<FMT_MXFP4>(w, apk, t, y, out_bf16, partial, s);
-        case FMT_NVFP4: return run_short<FMT_NVFP4>(w, apk, t, y, out_bf16, partial, s);
-        case FMT_Q8_0: return run_short<FMT_Q8_0>(w, apk, t, y, out_bf16, partial, s);
-        case FMT_Q8F: return run_short<FMT_Q8F>(w, apk, t, y, out_bf16, partial, s);
-        case FMT_Q4_K: return run_short<FMT_Q4_K>(w, apk, t, y, out_bf16, partial, s);
-        case FMT_Q5_K: return run_short<FMT_Q5_K>(w, apk, t, y, out_bf16, partial, s);
-        case FMT_Q6_K: return run_short<FMT_Q6_K>(w, apk, t, y, out_bf16, partial, s);
-        case FMT_FP8: return run_short<FMT_FP8>(w, apk, t, y, out_bf16, partial, s);
+        case FMT_Q4M: return run_short<FMT_Q4M>(w, apk, t, p, y, out_bf16, partial, s);
+        case FMT_Q40: return run_short<FMT_Q40>(w, apk, t, p, y, out_bf16, partial, s);
+        case FMT_MXFP4: return run_short<FMT_MXFP4>(w, apk, t, p, y, out_bf16, partial, s);
+        case FMT_NVFP4: return run_short<FMT_NVFP4>(w, apk, t, p, y, out_bf16, partial, s);
+        case FMT_Q8_0: return run_short<FMT_Q8_0>(w, apk, t, p, y, out_bf16, partial, s);
+        case FMT_Q8F: return run_short<FMT_Q8F>(w, apk, t, p, y, out_bf16, partial, s);
+        case FMT_Q4_K: return run_short<FMT_Q4_K>(w, apk, t, p, y, out_bf16, partial, s);
+        case FMT_Q5_K: return run_short<FMT_Q5_K>(w, apk, t, p, y, out_bf16, partial, s);
+        case FMT_Q6_K: return run_short<FMT_Q6_K>(w, apk, t, p, y, out_bf16, partial, s);
+        case FMT_FP8: return run_short<FMT_FP8>(w, apk, t, p, y, out_bf16, partial, s);
         default: return hipErrorInvalidValue;
     }
 }

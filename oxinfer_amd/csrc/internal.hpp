@@ -8,6 +8,7 @@
 #include <string>
 
 #include "../../include/oxhip.h"
+#include "gemm_plan.hpp"
 
 namespace oxhip {
 
@@ -32,7 +33,6 @@ namespace oxhip {
 //   NVFP4 p0      T4N records (layout.hpp); p1 f32 scales on top of the decoded values [ceil(n_out/br)][ceil(n_in/bc)],
 //                 or none (br == 0). Float-stored like FP8: f32 activations at decode sizes.
 // ------------------------------------------------------------------------------------------------
-enum Fmt : int { FMT_Q4 = 0, FMT_Q8_0 = 1, FMT_Q4_K = 2, FMT_Q6_K = 3, FMT_FP8 = 4, FMT_BF16 = 5, FMT_Q4M = 6, FMT_Q8F = 7, FMT_Q40 = 8, FMT_Q5_K = 9, FMT_MXFP4 = 10, FMT_NVFP4 = 11 };
 // the formats of the matrix-core decode kernels (decode_mfma.hip); the two Q8 kinds carry no sums or offsets
 inline bool mfma_decode_format(int f) { return f == FMT_Q8_0 || f == FMT_Q8F || f == FMT_Q4_K || f == FMT_Q6_K || f == FMT_Q4M || f == FMT_Q40 || f == FMT_Q5_K || f == FMT_MXFP4; }
 // the two 4-bit formats in T4M records (MLX: a scale and an offset per 64; GGUF Q4_0: a scale per 32)
@@ -223,10 +223,8 @@ hipError_t launch_quantize_pack_i8(const void* x, bool src_bf16, size_t t, const
 hipError_t launch_gemm_i8(const WeightView& w, const void* frag, const void* xs, const void* fs, size_t t, float* y, int32_t* dump, hipStream_t s);
 hipError_t launch_gemm_bf16(const WeightView& w, const void* apk, size_t t, size_t mtiles, void* y, bool out_bf16, float* partial,
                             hipStream_t s);
-// gemm_short.hip: the same product for at most 64 tokens, from the same fragments
-bool gemm_short_ok(size_t t);
-uint32_t gemm_short_slices(const WeightView& w, size_t t);
-hipError_t launch_gemm_short(const WeightView& w, const void* apk, size_t t, void* y, bool out_bf16, float* partial, hipStream_t s);
+// gemm_short.hip: the same product for at most 64 tokens, from the same fragments, as short_plan cuts it (rt > 0)
+hipError_t launch_gemm_short(const WeightView& w, const void* apk, size_t t, const ShortPlan& p, void* y, bool out_bf16, float* partial, hipStream_t s);
 hipError_t launch_quantize_act_fp8(const void* x, bool src_bf16, size_t t, size_t n_in, size_t mtiles, size_t kblocks, void* out,
                                    float* sx, hipStream_t s);
 uint32_t gemm_fp8_k_slices(const WeightView& w, size_t mtiles);

@@ -231,11 +231,17 @@ def any_weight(be, oxref, name, n_out, n_in, seed):
     return be.upload_gguf(GGUF_KINDS[name], raw, n_out, n_in), oxref.dequantize_rows(GGUF_KINDS[name], raw, n_out, n_in)
 
 
-@pytest.mark.parametrize("n_out,n_in", [(40, 256), (2050, 512), (4100, 512), (8210, 256), (12300, 256), (40, 8192), (2050, 12288), (4100, 12288)])
+# (tests/test_gemm_plan.py holds these sizes to the forms that the test below names)
+SHORT_SIZES = [(40, 256), (2050, 512), (4100, 512), (8210, 256), (12300, 256), (40, 8192), (2050, 12288), (4100, 12288), (37001, 256), (2251, 14336)]
+SHORT_TOKENS = (1, 16, 17, 32, 33, 48, 49, 64)
+
+
+@pytest.mark.parametrize("n_out,n_in", SHORT_SIZES)
 @pytest.mark.parametrize("name", ["MLX", "Q8", "FP8", "NVFP4", "Q4_0", "Q8_0", "Q4_K", "Q5_K", "Q6_K", "MXFP4"])
 def test_gemm_up_to_64_tokens(be, oxref, name, n_out, n_in):
-    """The kernel of at most 64 tokens in all its forms: one to four row tiles per workgroup (3, 129, 257, 514 and 769 tiles, the last
-    group ragged), fewer steps than waves, rows in two, three and four slices, and the edges of one to four token tiles. Against the
+    """The kernels of at most 64 tokens in all their forms: gemm_short.hip's one to four row tiles per workgroup (3, 129, 257, 514 and 769
+    tiles, the last group ragged), fewer steps than waves, rows in three and four slices, gemm.hip's four waves whole and in slices (2313 tiles,
+    the last group ragged, and 141), and the edges of one to four token tiles. Against the
     product of the operands rounded to bf16 in 64 bits: 1e-3 as above, the f32 sums themselves being off by 6e-6 at most."""
     import torch
     from oxinfer_amd import synth
@@ -243,7 +249,7 @@ def test_gemm_up_to_64_tokens(be, oxref, name, n_out, n_in):
     assert w is not None, be.last_error()
     wb = torch.from_numpy(synth.bf16_round(wf)).cuda().double()
     x64 = torch.from_numpy(synth.activations(64, n_in, 42, bf16=True)).cuda()
-    for t in (1, 16, 17, 32, 33, 48, 49, 64):
+    for t in SHORT_TOKENS:
         if name == "FP8" and t <= 32:  # (a kernel of its own, which scales the blocks' sums: its weights are not rounded)
             continue
         x = x64[:t].contiguous()
