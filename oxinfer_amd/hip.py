@@ -385,12 +385,15 @@ class HipBackend:
     def _stream():
         """The current torch stream of the current device, as the handle that the library takes. By torch's accessor of the handle
         itself where it has one: building a torch Stream object for its handle took 3 us of the 6.5 us that a call of one launch
-        takes, this 0.2 us (a 4096 x 4096 product of one token, two calls: 14.5 -> 9.3 us)."""
-        c = _torch._C
+        takes, this 0.2 us (a 4096 x 4096 product of one token, two calls: 14.5 -> 9.3 us). (`_cuda_getDevice` initialises the device
+        as torch's own calls do, or raises as they do.)"""
+        torch = _torch
+        if torch is None:
+            import torch
         try:
-            return c._cuda_getCurrentRawStream(c._cuda_getDevice())
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
         except AttributeError:
-            return _torch.cuda.current_stream().cuda_stream
+            return torch.cuda.current_stream().cuda_stream
 
     def quantize_act(self, x, out=None):
         """x: torch f32 [t, n_in] on the device -> QAct (device)."""
