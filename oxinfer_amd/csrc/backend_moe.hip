@@ -1,11 +1,11 @@
 // Backend::upload_moe / moe / matvec_rows (src/gpu.rs:165, :206-248 of the reference) over the grouped
 // decode kernel, plus their device-pointer forms.
-#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
 
 #include "backend.hpp"
+#include "moe_plan.hpp"
 
 using namespace oxhip;
 
@@ -30,9 +30,6 @@ bool mfma_format(const oxhip_weight* w) { return w->v.fmt == FMT_Q8_0 || w->v.fm
 size_t up256(size_t v) { return (v + 255) / 256 * 256; }
 
 constexpr size_t COMB_GROUPS = 4096;  // row groups of the down projection that may meet through counters (h <= 65536)
-
-// The most chunks of up to 32 rows that a plan of the bf16 prefill form can cut.
-size_t bf16_chunks(size_t pairs, size_t n_exp) { return (pairs < n_exp ? pairs : n_exp) + pairs / 32 + 1; }
 
 // The scratch of one pass, carved from one allocation.
 struct Scratch {
@@ -77,7 +74,7 @@ Scratch carve(uint8_t* base, size_t t, size_t pairs, size_t n_exp, size_t h, siz
     s.o = reinterpret_cast<float*>(take(pairs * h * 4));
     const bool prefill = pairs / n_exp >= 6 && h % 128 == 0 && inter % 128 == 0;
     s.fx = take(prefill ? moe_bf16_row_bytes(t, h) : 0);
-    s.fa = take(prefill ? moe_bf16_frag_bytes(bf16_chunks(pairs, n_exp), inter) : 0);
+    s.fa = take(prefill ? moe_bf16_frag_bytes(moe_most_chunks(pairs, n_exp), inter) : 0);
     s.bytes = off;
     return s;
 }
@@ -169,13 +166,12 @@ int moe_pass(oxhip_ctx* c, oxhip_moe* m, const float* x, size_t t, const uint32_
     }
     if (bf16_form) {
         HIP_TRY(launch_moe_plan(route_idx, pairs, k, m->n_exp, max_rows, sc.row_of, sc.src, sc.chunks, sc.nchunks, s), "moe plan launch");
-        // (about as many chunks as there will be: an expert has a last one, half full on average, and its rows past 16 in 32s before it)
-        const size_t chunks = std::min(m->n_exp, pairs) + (avg > 16 ? (pairs - 16 * m->n_exp) / 32 : 0);
+        const uint32_t chunks = moe_expected_chunks(pairs, m->n_exp);
         g.rowmap = sc.src;
         g.bases = m->bases_gu;
-        HIP_TRY(launch_moe_bf16_gate(m->gate_up[0]->v, m->down[0]->v, g, grid_chunks, (uint32_t)chunks, sc.fx, t, m->act_kind, m->act_param, sc.fa, s), "moe gate launch");
+        HIP_TRY(launch_moe_bf16_gate(m->gate_up[0]->v, m->down[0]->v, g, grid_chunks, chunks, sc.fx, t, m->act_kind, m->act_param, sc.fa, s), "moe gate launch");
         g.bases = m->bases_dn;
-        HIP_TRY(launch_moe_bf16_down(m->down[0]->v, g, grid_chunks, (uint32_t)chunks, sc.fa, sc.o, s), "moe down launch");
+        HIP_TRY(launch_moe_bf16_down(m->down[0]->v, g, grid_chunks, chunks, sc.fa, sc.o, s), "moe down launch");
     } else {
         if (direct) {
             if (!routed) HIP_TRY(launch_route_quantize(rin.logits, 1, m->n_exp, k, ridx_out, rw_out, rin.stride, rin.expert_scale, x, h, sc.xa, s), "route + quantize launch");

@@ -22,9 +22,8 @@
 #include "act_body.hpp"
 #include "internal.hpp"
 #include "layout.hpp"
+#include "moe_plan.hpp"
 #include "moe_rows.hpp"
-
-#include <algorithm>
 
 namespace oxhip {
 
@@ -80,7 +79,7 @@ __device__ __forceinline__ T gload_at(gbytes base, uint32_t voff) {
     return gload<T>((gbytes)u + voff);
 }
 
-constexpr uint32_t PHASE = 16;            // steps x token tiles staged at a time
+constexpr uint32_t PHASE = MOE_PHASE;
 constexpr uint32_t UNIT_LDS = 4096 + 512;  // bytes of one: fragments and sums
 
 // One token tile (TT = 1: up to 16 rows) or two of a chunk; see moe_bf16_kernel.
@@ -494,45 +493,18 @@ hipError_t launch_moe_rows(const float* x, size_t t, const WeightView& w, void* 
 namespace {
 template <int FMT>
 hipError_t run_moe_bf16(const WeightView& w, const GroupView& g, uint32_t max_chunks, const MoeRows& in, const MoeGlu& glu, uint32_t chunks, float* out, hipStream_t s) {
-    const uint32_t nsteps = w.n_in / 128, tiles = glu.inter ? glu.inter / 16 : row_tiles(w.n_out);
-    auto nx_of = [&](uint32_t r, uint32_t k) {
-        const uint32_t per = (8 / k) * r / (glu.inter ? 2 : 1);
-        return (tiles + per - 1) / per;
-    };
-    // K over two or four waves where one wave per row would leave fewer workgroups than places
-    uint32_t rt = 2, kw = 1;
-    while (kw < 4 && nsteps / (2 * kw) >= 4 && (uint64_t)nx_of(rt, kw) * max_chunks < 512) kw *= 2;
-    // Row tiles per wave, and runs of them that a workgroup takes one after the other with one staging (the down projection's rows fit a
-    // phase): what takes fewer rounds of workgroups over the 512 places, a round as long as its waves' row tiles x steps and six more for its staging
-    // and its end. At 256 tokens, MLX 4-bit: gate / up launch, two tiles and three, 128 experts of 2048 / 768 64.2 and 55.6 us (768 and 512
-    // workgroups), 32 experts 38.9 and 48.5; down launch, one run of two tiles, of three, two, three and four of two, 128 experts 34.5, 36.3, 33.6, 38.0
-    // and 34.4, 32 experts (two tiles, 320 workgroups) 23.4, 22.4, 24.9, 23.5 and 27.2. (Four row tiles spill in the form of two token tiles: 76.)
-    uint32_t nrep = 1;
-    if (kw == 1) {
-        uint64_t least = ~0ull;
-        for (uint32_t r = 2; r <= (FMT == FMT_Q8_0 ? 2u : 3u); r++)  // (Q8_0, a step being two records per row tile, keeps to two and one; three and several runs would spill)
-            for (uint32_t n = 1; n <= (r == 2 && FMT != FMT_Q8_0 && !glu.inter && 2 * nsteps <= PHASE ? 4u : 1u); n++) {
-                const uint64_t items = (uint64_t)((nx_of(r, 1) + n - 1) / n) * chunks;
-                const uint64_t cost = ((items > 16 ? items - 16 : 1) + 511) / 512 * (n * r * nsteps + 6);
-                if (cost < least) {
-                    least = cost;
-                    rt = r;
-                    nrep = n;
-                }
-            }
-    }
-    const uint32_t nx = (nx_of(rt, kw) + nrep - 1) / nrep;
+    const MoePlan p = moe_plan(FMT, w.n_out, w.n_in, glu.inter, max_chunks, chunks);
     const size_t lds = PHASE * UNIT_LDS;
-    const dim3 grid((nx * max_chunks + 7) / 8 * 8);  // every XCD's share of the items (moe_bf16_item), whatever the chunk count turns out to be
+    const dim3 grid((p.nx * max_chunks + 7) / 8 * 8);  // every XCD's share of the items (moe_bf16_item), whatever the chunk count turns out to be
     auto go = [&](auto kern) -> hipError_t {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
-        kern<<<grid, 512, lds, s>>>(w, g.bases, g.chunks, g.nchunks, in, kw, nrep, nx, glu, out);
+        kern<<<grid, 512, lds, s>>>(w, g.bases, g.chunks, g.nchunks, in, p.kw, p.nrep, p.nx, glu, out);
         return hipGetLastError();
     };
     if constexpr (FMT != FMT_Q8_0) {
-        if (nrep > 1) return go(moe_bf16_kernel<2, FMT, true>);
-        if (rt == 3) return go(moe_bf16_kernel<3, FMT, false>);
+        if (p.nrep > 1) return go(moe_bf16_kernel<2, FMT, true>);
+        if (p.rt == 3) return go(moe_bf16_kernel<3, FMT, false>);
     }
     return go(moe_bf16_kernel<2, FMT, false>);
 }

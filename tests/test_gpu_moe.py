@@ -222,7 +222,8 @@ def test_moe_gguf_experts(be, oxref, kind):
 
 def test_moe_prefill_rows_do_not_depend_on_the_batch(be, oxref, mlx_experts):
     """In the bf16 form too every (token, row) sum is formed on its own in a fixed order: a token's output is
-    bit-identical whichever other tokens share the pass (and its expert's chunks)."""
+    bit-identical whichever other tokens share the pass (and its expert's chunks). (Where the launches split K over the same number of
+    waves, here none: that number goes by the pass's size, and the order of a sum's terms with it.)"""
     from oxinfer_amd import synth
     ne, h, inter, raw_gu, raw_dn, _, _ = mlx_experts
     k, t = 3, 40
@@ -238,9 +239,15 @@ def test_moe_prefill_rows_do_not_depend_on_the_batch(be, oxref, mlx_experts):
         assert np.array_equal(ys.view(np.uint32), y[keep].view(np.uint32))
 
 
+# staged in three phases and one, an odd number of steps; one; four and one; three row tiles per wave in the down launch; two, three (the last
+# ending past the matrix) and four runs of row tiles per workgroup there, three row tiles per wave in the gate / up launch, the last group
+# ragged (24 copies) or not (32). tests/test_moe_plan.py holds them to that.
+CHUNK_SIZES = [(2304, 384, 1), (256, 256, 1), (4096, 256, 1), (2048, 384, 14), (2048, 384, 16), (2048, 512, 24), (2048, 384, 32)]
+CHUNK_ROWS = [33, 32, 17, 16, 1]  # of the experts
+
+
 @pytest.mark.parametrize("fmt", ["mlx", "Q4_K", "Q8_0", "Q4_0", "MXFP4", "mlx, Q8_0 down"])
-# staged in three phases and one, an odd number of steps; one; four and one; enough workgroups for several runs of row tiles per workgroup
-@pytest.mark.parametrize("h,inter,copies", [(2304, 384, 1), (256, 256, 1), (4096, 256, 1), (2048, 384, 14)])
+@pytest.mark.parametrize("h,inter,copies", CHUNK_SIZES)
 def test_moe_prefill_chunks(be, oxref, fmt, h, inter, copies):
     """The bf16 form's chunks at the edges of its token tiles and of a chunk (experts of 33, 32, 17, 16 and 1 rows): within 6e-3 of the
     reference's grouped f32 path on activations that are bf16 values already (as in test_moe_gguf_experts), and bit for bit the same
@@ -248,7 +255,7 @@ def test_moe_prefill_chunks(be, oxref, fmt, h, inter, copies):
     from oxinfer_amd import synth
     if fmt == "Q4_K":
         inter = (inter + 255) // 256 * 256  # whole super-blocks
-    rows = [33, 32, 17, 16, 1]
+    rows = CHUNK_ROWS
     ne, t = len(rows), sum(rows)
     kinds = {"Q4_K": (Q4_K, synth.gguf_q4_k), "Q8_0": (Q8_0, synth.gguf_q8_0), "Q4_0": (Q4_0, synth.gguf_q4_0), "MXFP4": (MXFP4, synth.gguf_mxfp4)}
 
