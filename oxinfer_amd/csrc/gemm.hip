@@ -123,11 +123,10 @@ constexpr int AR = 4;      // blocks of A fragments held ahead (a whole K-step: 
 // FMT: FMT_Q4M (tile-packed MLX 4-bit), FMT_Q8_0 / FMT_Q8F / FMT_Q4_K / FMT_Q6_K (their tile records) or FMT_FP8 (e4m3 bytes with 128 x 128 block scales: the bytes are
 // exact in bf16, the block scale multiplies in f32 before the rounding, and a lane takes 32 consecutive row bytes
 // per step, which pack_a's mode 2 mirrors on the activation side).
-// ALONE: see run_gemm_bf16_nv. (Eight waves of one token tile: two workgroups share a CU if they take at most 128 registers. Q4_K took 130:
-// bounded it spills 12 bytes, 9472 columns x 5000 rows 42.7 -> 31.9 us at 128 tokens with the slices that allows. The 8-bit formats
-// would spill 24 to 44 bytes, 33.6 -> 43.9 us on 14336 -> 4096: they keep a CU to a workgroup.)
-template <int FMT, bool OUT_BF16, int NV, int WAVES, int NT, bool ALONE>
-__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 : 2) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
+// (Eight waves of one token tile: two workgroups share a CU if they take at most 128 registers. The 8-bit formats would spill 24 to 40
+// bytes, 33.6 -> 43.9 us on 14336 -> 4096: they keep a CU to a workgroup.)
+template <int FMT, bool OUT_BF16, int NV, int WAVES, int NT>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !q8_format(FMT) ? 4 : 2) void gemm_bf16_kernel(WeightView w, const uint4* __restrict__ apk, uint32_t t, uint32_t mtiles,
                                                         void* __restrict__ yv) {
     extern __shared__ uint4 bfrag[];  // [2][4 blocks][NT row tiles][64 lanes]
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -230,7 +229,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 1 : NV == 1 && !ALONE ? 4 
                 dequant(raw[i], i, buf ^ 1, min(s + 1, last));
                 // (Left to itself the compiler puts the request among the conversions. Q4_K 14336 rows x 2048 tokens 234 us, 226 this way; four
                 // waves, medians of 24 calls of up to 64 tokens: Q5_K 0.89 of the time, MXFP4 0.90, Q4_0 0.95, MLX 4-bit, Q8 and Q6_K 0.96
-                // to 0.98, Q4_K, FP8 and NVFP4 the same; FP8 at 200 tokens 60.0 -> 58.4 us on 9472 x 8960. The others are no faster.)
+                // to 0.98, Q4_K, FP8 and NVFP4 the same; FP8 past 128 tokens 0.98 to 0.99. The others are no faster.)
                 if constexpr (FMT == FMT_Q4_K || WAVES == 4 || (FMT == FMT_FP8 && NV == 2)) __builtin_amdgcn_sched_barrier(0);
                 load_raw(raw[i], i, min(s + 2, last));
             }
@@ -340,18 +339,9 @@ hipError_t run_gemm_bf16_nv(const WeightView& w, const void* apk, size_t t, size
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e == hipSuccess) kern<<<grid, 64 * WAVES, lds, s>>>(w, static_cast<const uint4*>(apk), (uint32_t)t, (uint32_t)mtiles, dst);
     };
-    // Eight waves of one token tile that leave a second workgroup no room on their CU: the 8-bit formats always; Q4_K in launches of
-    // at most a workgroup per CU, which need none, while the spill of the bounded kernel costs a start half a microsecond later
-    // (2048 columns x 7168 rows at 80 tokens, 224 workgroups: 19.0 us bounded, 18.4 this way).
-    constexpr bool ALWAYS = NV == 1 && WAVES == 8 && q8_format(FMT), CHOICE = NV == 1 && WAVES == 8 && FMT == FMT_Q4_K;
     span_start(s);
-    if (CHOICE && (uint64_t)grid.x * grid.y * grid.z <= 256) {
-        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, WAVES, NT, CHOICE || ALWAYS>);
-        else go(gemm_bf16_kernel<FMT, false, NV, WAVES, NT, CHOICE || ALWAYS>);
-    } else {
-        if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, WAVES, NT, ALWAYS>);
-        else go(gemm_bf16_kernel<FMT, false, NV, WAVES, NT, ALWAYS>);
-    }
+    if (direct_bf16) go(gemm_bf16_kernel<FMT, true, NV, WAVES, NT>);
+    else go(gemm_bf16_kernel<FMT, false, NV, WAVES, NT>);
     if (e != hipSuccess) return e;
     e = hipGetLastError();
     span_stop(s);
