@@ -335,8 +335,8 @@ __device__ __forceinline__ void decode_body(WeightView w, QActView xa, uint32_t 
     };
     // Step q of the four takes its words from lane group q, lane 16 q + n. MLX 4-bit by swaps of 32 and 16 lanes, which leave a word of two
     // steps in all lane groups each: a lane-to-lane read goes through the LDS pipe, and the step waits for it and for every LDS read ahead of
-    // it. (MoE, 128 experts of 2048 / 768, one token 18.4 -> 18.0 us, 24 tokens 64.8 -> 63.2; two layers at 16 tokens 127.9 -> 126.7. The
-    // other formats are bound by the swaps' issue: 4096 x 4096 at one token Q4_0 4.94 -> 5.12, Q8_0 5.38 -> 5.62, MXFP4 5.33 -> 5.47, Q4_K
+    // it. (Worth little: eight matrices at seven token counts 0.992 of the time in the median, 1.016 at most; MoE, 128 experts of 2048 / 768, at
+    // one and 24 tokens 1 %, within a run's spread. The other formats are bound by the swaps' issue: 4096 x 4096 at one token Q4_0 4.94 -> 5.12, Q8_0 5.38 -> 5.62, MXFP4 5.33 -> 5.47, Q4_K
     // 5.46 -> 5.56 there and 6.39 -> 6.25 at eight, Q6_K and Q5_K 1 % either way.)
     // scur: the words as they came; snear, sfar: of step q + 1 and of steps 2 and 3.
     constexpr bool SWAPS = FMT == FMT_Q4M;

@@ -6,9 +6,10 @@
 // bound it. Here the routed tokens of a chunk (up to 32 rows of one expert, one or two tiles of 16) go in as bf16 and a weight is the bf16
 // value 128 + nibble, two of them made by one mask (nibbles 16 bits apart, | 0x4300). The matrix cores form
 //     D = sum (128 + nib) x - 136 sum x = sum (nib - 8) x
-// exactly in f32 (the second term is what the accumulator starts from), per group of 64 columns in MLX 4-bit, per block of 32 in the others,
-// and y += d D costs one multiply-add per (row, token, group). The offsets of MLX 4-bit and Q4_K, off sum x, are one more matrix
-// instruction in f32 (K = four groups or blocks). MXFP4 goes in as 128 + 12 + the doubled E2M1 value. Q8_0's code q as the byte m = q + 128 =
+// in f32 (the second term is what the accumulator starts from), per group of 64 columns in MLX 4-bit, per block of 32 in the others,
+// and y += d D costs one multiply-add per (row, token, group). Codes and single products are exact; the sums are rounded, and what cancels in
+// them leaves an error of the order of 2^-24 x 136 sum |x| (Q8_0: 2^-24 x 2304 sum |x|). The offsets of MLX 4-bit and Q4_K, off sum x, are
+// one more matrix instruction in f32 (K = four groups or blocks). MXFP4 goes in as 128 + 12 + the doubled E2M1 value. Q8_0's code q as the byte m = q + 128 =
 // 16 H + L, both nibbles as 128 + nibble in two matrix instructions: sum q x = 16 D_H + (D_L - 2304 sum x).
 // This is the reference's own prefill form: from 8 rows on its
 // experts run a grouped f32 GEMM over exact activations with Act::scalar between the two (src/moe.rs:735-827,
@@ -452,7 +453,9 @@ __device__ __forceinline__ void moe_bf16_body(const WeightView& w, const uint8_t
 // and meet in LDS in wave order. A workgroup's item (moe_bf16_item): a run of (8 / kw) RT row tiles of a chunk {expert, first row, rows <= 32}.
 // The chunk's rows (4 KiB per step and tile of 16) are staged into LDS, 64 KiB at a time: all eight waves multiply the same rows (each wave
 // asking memory for them costs more than the weights), and two workgroups share a CU. out [gathered row][n_out] f32.
-// REP: an item is `nrep` such runs of row tiles, one after the other over the same staged rows (kw = 1, no activation).
+// REP: an item is `nrep` such runs of row tiles, one after the other over the same staged rows (kw = 1, no activation). (These forms keep 37
+// to 76 scalar registers in vector lanes, the others 0 to 23: the bodies of one and two token tiles, the activation and the waves' join are
+// one kernel. No form spills vector registers.)
 template <int RT, int FMT, bool REP>
 __global__ __launch_bounds__(512, 4) void moe_bf16_kernel(WeightView w, const uint8_t* const* __restrict__ bases, const int4* __restrict__ chunks,
                                                           const int* __restrict__ nchunks, MoeRows in, uint32_t kw, uint32_t nrep, uint32_t nx, MoeGlu glu,
@@ -471,6 +474,8 @@ __global__ __launch_bounds__(512, 4) void moe_bf16_kernel(WeightView w, const ui
 
 }  // namespace
 
+// (Rows of up to 4096 columns: the form once staged a chunk's rows whole. It stages them in phases now, but longer rows have not been measured
+// here against the integer kernels, which they keep.)
 bool moe_bf16_ok(const WeightView& w) {
     if (w.n_in % 128 || w.n_in < 128 || w.n_in > 4096) return false;
     return t4m_format(w.fmt) || w.fmt == FMT_Q8_0 || (w.fmt == FMT_Q4_K && w.n_in % 256 == 0);
